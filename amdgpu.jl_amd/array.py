@@ -202,6 +202,27 @@ _waiting: set = set()          # (device, stream) keys whose workspace has been 
 _sort_tmps: dict = {}          # (device, stream) -> temporaries of sorts whose record has not been read
 
 
+# Pinned host words that a kernel writes its scalar result to (the count behind x[mask]): the host reads them after the
+# stream synchronisation it needs anyway, with no device-to-host copy in between.  A slot belongs to one call from take to
+# give, whatever thread or stream it runs on; the free list holds at most as many as calls have been in flight at once.
+_free_slots: list = []
+SLOT_BYTES = 128
+
+
+def take_slot():
+    """(address, NumPy bytes, tensor) of a free pinned slot; hand it back with ``give_slot``."""
+    try:
+        return _free_slots.pop()
+    except IndexError:
+        t = torch.empty(SLOT_BYTES, dtype=torch.uint8, pin_memory=True)
+        return t.data_ptr(), t.numpy(), t
+
+
+def give_slot(slot) -> None:
+    if len(_free_slots) < 64:
+        _free_slots.append(slot)
+
+
 def note_waiting_call() -> None:
     """The call being issued on the current stream polls other workgroups through the stream's workspace."""
     _waiting.add((torch.cuda.current_device(), stream_ptr()))

@@ -7,10 +7,11 @@ the native scan and ``rk_findall_scatter``."""
 from __future__ import annotations
 
 import numpy as np
+import torch
 
 from . import _lib as L
 from .accumulate import accumulate
-from .array import ROCArray, note_waiting_call, stream_ptr, workspace
+from .array import ROCArray, check_waits, device, give_slot, note_waiting_call, stream_ptr, take_slot, workspace
 from .mapreduce import count
 
 
@@ -58,15 +59,36 @@ def findall_two_pass(bools: ROCArray) -> ROCArray:
     return ys
 
 
+def _select(x: ROCArray, mask: ROCArray) -> ROCArray:
+    """``x[mask]`` with a mask of x's shape: count, allocate, then one streaming pass that moves the selected elements
+    (no index array in between)."""
+    n = len(x)
+    if n == 0:
+        return ROCArray(dims=(0,), dtype=x.dtype)
+    st = stream_ptr()
+    nbytes = int(L.lib.rk_mask_tmp_bytes(n))
+    tmp = torch.empty(nbytes, dtype=torch.uint8, device=device())
+    ws, ws_bytes = workspace()
+    slot = take_slot()
+    L.check(L.lib.rk_mask_count(mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes, st), "rk_mask_count")
+    check_waits()                           # the host waits here anyway: the place to learn of a give-up
+    torch.cuda.current_stream().synchronize()
+    total = int(slot[1][:8].view(np.int64)[0])
+    give_slot(slot)
+    y = ROCArray(dims=(total,), dtype=x.dtype)
+    if total > 0:
+        L.check(L.lib.rk_mask_select(mask.ptr, n, x.ptr, y.ptr, x.dtype.itemsize, total, tmp.data_ptr(), nbytes, st), "rk_mask_select")
+    return y
+
+
 def getindex_mask(x: ROCArray, mask: ROCArray) -> ROCArray:
     """``x[mask]`` for a mask of x's shape, or ``x[:, ..., :, mask]`` for a Bool vector along the last dim
-    (test/hip_rocarray/indexing.jl:5-18): ``Base.to_index`` turns the mask into ``findall(mask)``
-    (indexing.jl:1), then the selected slices are gathered."""
+    (test/hip_rocarray/indexing.jl:5-18).  The first moves the selected elements in one pass over the mask; for the second
+    ``Base.to_index`` turns the mask into ``findall(mask)`` (indexing.jl:1) and the selected slices are gathered."""
     if mask.dtype != np.bool_:
         raise L.UnsupportedError(L.RK_ERR_UNSUPPORTED, "logical indexing needs a Bool mask")
     if mask.dims == x.dims:
-        inner, nsrc, lead = 1, len(x), ()
-        idx = findall(mask.reshape(len(mask)))
+        return _select(x, mask)
     elif mask.ndim == 1 and x.ndim >= 1 and mask.dims[0] == x.dims[-1]:
         lead = x.dims[:-1]
         inner, nsrc = int(np.prod(lead, dtype=np.int64)), x.dims[-1]

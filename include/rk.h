@@ -379,6 +379,23 @@ RK_API int32_t rk_findall(const uint8_t* bools, int ndim, const int64_t* shape, 
 RK_API int32_t rk_gather_slices(const void* x, const int64_t* idx, void* y, size_t elsize,
                          int64_t inner, int64_t nidx, int64_t nsrc, void* stream);
 
+/* ---- logical indexing ------------------------------------------------------------------------
+ * y = x[mask] for a Bool mask of x's shape (test/hip_rocarray/indexing.jl:5-18) without the index
+ * array of findall in between.  The caller allocates y between the two calls:
+ *   rk_mask_count   writes the number of true entries to `count_out` (Int64; device memory, or
+ *                   pinned host memory to be read after the stream has been synchronised) and
+ *                   leaves in `tmp` where every stretch of the mask starts in the result.
+ *                   Needs a workspace.
+ *   rk_mask_select  y[k] = the element of x at the k-th true entry, k < nsel = that count; mask and
+ *                   `tmp` as rk_mask_count left them.
+ * `tmp`: caller-owned, 256-byte aligned, rk_mask_tmp_bytes(n) bytes, any contents before the
+ * count.  Elements are opaque (`elsize` = 1, 2, 4, 8 or 16); only bit 0 of a Bool byte counts. */
+RK_API size_t  rk_mask_tmp_bytes(int64_t n);
+RK_API int32_t rk_mask_count(const uint8_t* mask, int64_t n, int64_t* count_out, void* tmp, size_t tmp_bytes,
+                      void* ws, size_t ws_bytes, void* stream);
+RK_API int32_t rk_mask_select(const uint8_t* mask, int64_t n, const void* x, void* y, size_t elsize, int64_t nsel,
+                       const void* tmp, size_t tmp_bytes, void* stream);
+
 /* ---- reverse / reverse! -------------------------------------------------------------------
  * Replaces both `_reverse!` kernels of src/kernels/reverse.jl: out of place (`:59-88`, y != x)
  * and in place (`:92-122`, y == x; partially overlapping x and y are not allowed).

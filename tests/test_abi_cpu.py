@@ -224,6 +224,17 @@ def test_volumerhs_and_scatter_validation(L):
     assert ga(one, one, two, 3, 3, 5, 7, None) == L.RK_ERR_UNSUPPORTED
     assert ga(one, one, two, 4, -1, 5, 7, None) == L.RK_ERR_INVALID_ARGUMENT
     assert ga(None, None, None, 4, 3, 0, 7, None) == L.RK_SUCCESS
+    mb, mc, ms = L.lib.rk_mask_tmp_bytes, L.lib.rk_mask_count, L.lib.rk_mask_select
+    assert mb(0) == 256 and mb(1 << 26) % 256 == 0 and mb(1 << 26) < (1 << 20)
+    assert mc(None, 5, one, big, 1 << 20, big, 16 << 20, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert mc(one, 5, None, big, 1 << 20, big, 16 << 20, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert mc(one, 5, one, None, 1 << 20, big, 16 << 20, None) == L.RK_ERR_WORKSPACE
+    assert mc(one, 5, one, big, 8, big, 16 << 20, None) == L.RK_ERR_WORKSPACE
+    assert mc(one, 5, one, big, 1 << 20, None, 0, None) == L.RK_ERR_WORKSPACE
+    assert ms(one, 5, None, one, 4, 3, big, 1 << 20, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert ms(one, 5, one, one, 3, 3, big, 1 << 20, None) == L.RK_ERR_UNSUPPORTED
+    assert ms(one, 5, one, one, 4, 3, None, 0, None) == L.RK_ERR_WORKSPACE
+    assert ms(None, 5, None, None, 4, 0, None, 0, None) == L.RK_SUCCESS
     f = L.lib.rk_findall
     assert f(None, 1, L.shape_array((5,)), one, None, two, 16 << 20, None) == L.RK_ERR_INVALID_ARGUMENT
     assert f(one, 1, L.shape_array((5,)), None, None, two, 16 << 20, None) == L.RK_ERR_INVALID_ARGUMENT

@@ -92,6 +92,32 @@ def test_selection_by_mask(rk, orc, dtype):
     assert rk.getindex_mask(rk.ROCArray(x), rk.ROCArray(np.zeros((33, 65), dtype=bool))).dims == (0,)
 
 
+@pytest.mark.parametrize("n", [1, 15, 63, 4095, 4096, 4097, 65535, 65536, 65537, 16 * 65536 + 5, (1 << 24) + 3, (1 << 26) + 4097])
+def test_mask_select_edges(rk, n):
+    # tile (4096), group (16 or 64 tiles) and completion-ticket edges of the count; every density class of the list in LDS
+    rng = np.random.default_rng(n)
+    x = rng.integers(0, 1 << 31, n).astype(np.uint32).view(np.float32)
+    dx = rk.ROCArray(x)
+    for dens in (0.0, 0.01, 0.5, 1.0) if n < 1 << 24 else (0.4,):
+        m = rng.random(n) < dens
+        if dens == 0.5:
+            m[n // 2:] = True                                       # a full stretch behind a mixed one
+        got = rk.Array(rk.getindex_mask(dx, rk.ROCArray(m)))
+        assert np.array_equal(got.view(np.uint32), x[m].view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [np.int8, np.int16, np.int32, np.int64])
+def test_mask_select_unaligned(rk, dtype):
+    # mask and x that start at odd addresses (views), element sizes 1 to 8
+    rng = np.random.default_rng(3)
+    n = 200_003
+    x, m = rng.integers(-100, 100, n).astype(dtype), rng.random(n) < 0.3
+    dx, dm = rk.ROCArray(x), rk.ROCArray(m)
+    for a, b in ((2, n), (8, n - 1), (17, n - 70_000)):
+        got = rk.Array(rk.getindex_mask(dx.view_range(a, b), dm.view_range(a, b)))
+        assert np.array_equal(got, x[a - 1:b][m[a - 1:b]])
+
+
 def test_the_paths_the_tunables_select():
     """RK_SELECT_ORDERED=0 (persistent workgroups fed by a tile counter) and RK_SCAN_DYNAMIC_IDS=1 (the same for the
     long scans) are read once per process, so they are exercised in a child process: findall and a long cumsum against
