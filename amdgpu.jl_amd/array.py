@@ -193,13 +193,11 @@ def workspace(min_bytes: int = 0):
 
 
 # ---- give-ups of bounded waits -------------------------------------------------------------------------
-# The single-pass scans, the one-pass findall and the small sorts wait on other workgroups with a budget; a kernel that
-# runs out of it records that in the workspace (the sort: in its temporary) and finishes with meaningless results.
-# The mirror reads those records where it synchronises anyway -- Array(x), item() -- for every workspace and sort
-# temporary that such a kernel has used on the current stream since the last look, and raises.
+# The single-pass scans and the one-pass findall wait on other workgroups with a budget; a kernel that runs out of it
+# records that in the workspace and finishes with meaningless results.  The mirror reads the record where it synchronises
+# anyway -- Array(x), item() -- when such a kernel has used the stream's workspace since the last look, and raises.
 _staging: dict = {}            # (device, stream) -> pinned bytes for scalar fetches (item())
 _waiting: set = set()          # (device, stream) keys whose workspace has been handed to a kernel with bounded waits
-_sort_tmps: dict = {}          # (device, stream) -> temporaries of sorts whose record has not been read
 
 
 # Pinned host words that a kernel writes its scalar result to (the count behind x[mask]): the host reads them after the
@@ -228,14 +226,6 @@ def note_waiting_call() -> None:
     _waiting.add((torch.cuda.current_device(), stream_ptr()))
 
 
-def note_sort(tmp: "torch.Tensor") -> None:
-    """Keeps a sort's temporary until its record has been read (instead of freeing it at once)."""
-    pending = _sort_tmps.setdefault((torch.cuda.current_device(), stream_ptr()), [])
-    pending.append(tmp)
-    if len(pending) > 16:                   # a long run of sorts without a fetch: read the records rather than hoard memory
-        check_waits()
-
-
 def check_waits() -> None:
     """Reads the give-up records of the current stream (synchronises it when there are any to read); raises
     ``WaitError`` after preparing the workspace again."""
@@ -253,11 +243,5 @@ def check_waits() -> None:
                 failed = "a scan or findall on this stream"
             elif st != L.RK_SUCCESS:
                 L.check(st, "rk_workspace_status")
-    for tmp in _sort_tmps.pop(key, ()):
-        st = L.lib.rk_sort_status(tmp.data_ptr(), tmp.numel(), stream_ptr())
-        if st == L.RK_ERR_WAIT:
-            failed = "a sort on this stream"
-        elif st != L.RK_SUCCESS:
-            L.check(st, "rk_sort_status")
     if failed is not None:
         raise L.WaitError(L.RK_ERR_WAIT, failed)

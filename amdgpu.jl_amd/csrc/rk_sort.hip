@@ -1,28 +1,27 @@
 // sort! / sortperm! of vectors (src/kernels/sorting.jl:1-3, which forwards to AcceleratedKernels' merge sort):
 // least-significant-digit radix sort, 8 bits per pass.
 //
-//   sort_init_kernel     clears the control block (and the tile descriptors of small sorts); no memset: graph-safe
-//   sort_pass_kernel     a tile of 4096 keys ranks its keys by digit (wave-level match by ballots, counts in LDS), learns
-//                        how many keys of each digit the earlier tiles hold, reorders the tile in LDS and writes runs of
-//                        equal digits.  The kernel is bound by its vector instructions (about 75 a key, 32 of them the
-//                        match), not by memory.
-//   sort_finish_kernel   moves the result into the caller's array when an odd number of passes ran
-//
-// Up to 256 tiles (RK_SORT_LOOKBACK_TILES; 2^20 keys) the counts of the earlier tiles come from a chained look-back (tiles in
-// ticket order publish their 256 counts, one lane per digit walks back), and a pass reads and writes every key once:
-//   sort_min_kernel      integers: one read of the keys for the smallest mapped key, which every key is taken relative to
-//   sort_hist_kernel     one read of the keys: the 256-bin histogram of every digit at once
-//   sort_plan_kernel     exclusive scan of every histogram = first output slot of each digit value; passes whose
-//                        digit is the same for all keys are skipped (small-range integers need 1-2 passes);
-//                        records which buffer each remaining pass reads
-// Beyond that the walk becomes the bottleneck -- a descriptor is 2 KiB per step against 16 KiB of keys per tile, and the
-// tiles in flight resolve their prefixes nearly one after the other (2^22 Float32: 388 us against 146 us) -- so large
-// sorts count before every pass instead:
-//   sort_minmax_kernel   integers only: smallest and largest key in one read; passes above the range are skipped
+//   sort_init_kernel     clears the control block; no memset: graph-safe
+//   sort_range_kernel    one read of the keys: smallest and largest key (integers) and the bits that differ between keys;
+//                        the workgroup that finishes last decides which passes run (a digit that is the same in every key
+//                        needs none) and which buffer each of them reads
+// and for every pass
 //   sort_upsweep_kernel  the 256 digit counts of every tile (one more read of the keys, at streaming speed)
-//   sort_tilescan_kernel exclusive scan of the counts down the tiles in one launch (chunks of tiles; the workgroup
-//                        that finishes last scans the chunk totals and the digit totals)
-// and their pass kernel gives each XCD a contiguous eighth of the tiles.
+//   sort_pass_kernel     a tile of 4096 keys ranks its keys by digit (wave-level match by ballots, counts in LDS), reorders
+//                        the tile in LDS and writes runs of equal digits.  The kernel is bound by its vector instructions
+//                        (about 75 a key, 32 of them the match), not by memory.
+//
+// How a tile learns where its digits go:
+//   up to 256 tiles (2^20 keys)  every workgroup of the pass sums the columns of the table of counts itself (256 rows of
+//                        512 bytes out of L2, one or two rounds of loads): nothing waits for anything.  These sorts are bound
+//                        by latency -- a tile or less per compute unit -- so a tile is 16 waves with 4 keys a lane, not
+//                        4 waves with 16.  A chained look-back in their place resolved the tiles nearly one after the
+//                        other: 22 us a pass for 10^6 Int64 keys with their permutation.
+//   beyond               sort_tilescan_kernel: exclusive scan of the counts down the tiles in one launch (chunks of tiles; the
+//                        workgroup that finishes last scans the chunk totals and the digit totals); the pass kernel gives
+//                        each XCD a contiguous eighth of the tiles.
+// Large sorts of floats run every pass (their digits are hardly ever constant) and do without the range read.
+//   sort_finish_kernel   moves the result of sort! into the caller's array when an odd number of passes ran
 //
 // Keys are mapped to unsigned integers that sort like Base.isless (-0.0 < 0.0, NaN last; sortperm makes every NaN the
 // canonical one so that they are equal keys, sort! keeps their bit patterns), complemented for rev=true; the mapping is
@@ -33,25 +32,25 @@
 #include <type_traits>
 
 #include "rk_common.hpp"
-#include "rk_scan_impl.hpp"
 
 namespace rk {
 
 constexpr int SORT_BLOCK = 256;
-constexpr int SORT_NW = SORT_BLOCK / WAVE;
 constexpr int SORT_MAX_PASSES = 8;
 
 struct SortCtl {                                  // head of the caller's temporary buffer
-    uint32_t hist[SORT_MAX_PASSES][256];          // counts, then (sort_plan_kernel) exclusive prefix sums
-    uint32_t ticket[SORT_MAX_PASSES];
+    uint32_t hist[SORT_MAX_PASSES][256];          // large sorts: first output slot of every digit value (sort_tilescan_kernel)
+    // everything from here on is cleared by sort_init_kernel
     uint32_t skip[SORT_MAX_PASSES];
     uint32_t src_is_b[SORT_MAX_PASSES];           // the pass reads buffer B (1) or A (0)
-    uint32_t first_pass, last_pass, nexec;
-    uint32_t wait_failed;                         // a look-back gave up its bounded wait (WaitCtl); read by rk_sort_status
-    unsigned long long inv_min;                   // ~(smallest mapped key), kept as a maximum so that zero is its identity
-    unsigned long long key_max;                   // largest mapped key (large integer sorts: range = key_max - smallest)
     uint32_t scan_ticket[SORT_MAX_PASSES];        // sort_tilescan_kernel: workgroups that have stored their chunk totals
+    uint32_t first_pass, last_pass, nexec;
+    uint32_t range_ticket;                        // sort_range_kernel: workgroups that have added their part
+    unsigned long long inv_min;                   // ~(smallest mapped key), kept as a maximum so that zero is its identity
+    unsigned long long key_max;                   // largest mapped key (integers: range = key_max - smallest)
+    unsigned long long varying;                   // bits that are not the same in all mapped keys
 };
+constexpr int SORT_CTL_CLEAR = (int)((sizeof(SortCtl) - offsetof(SortCtl, skip)) / sizeof(uint32_t));
 
 // ---- key <-> ordered unsigned integer -----------------------------------------------------------------
 template <typename T> struct SortKey;
@@ -144,22 +143,10 @@ template <typename T> __device__ __forceinline__ T dec_bits(typename SortKey<T>:
 
 template <typename U> __device__ __forceinline__ uint32_t digit_of(U u, int pass) { return (uint32_t)(u >> (8 * pass)) & 0xffu; }
 
-// Mask of the lanes of `valid` whose digit equals this lane's.  Per bit of the digit: e = all ones where the bit is
-// set, m = ballot of the bit; (m ^ e) has a one exactly for the lanes that differ from this lane in that bit.
-__device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t valid) {
-    uint32_t diff_lo = 0, diff_hi = 0;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-        const uint32_t e = (uint32_t)__builtin_amdgcn_sbfe((int)d, b, 1);
-        const uint64_t m = __ballot(e != 0u);
-        diff_lo |= (uint32_t)m ^ e;
-        diff_hi |= (uint32_t)(m >> 32) ^ e;
-    }
-    return ~(((uint64_t)diff_hi << 32) | diff_lo) & valid;
-}
-// The same for the ranking of the pass kernel, which is bound by its vector instructions: four per bit (sign-extended
-// bit, compare into a lane mask, and one three-input bit operation same &= ~(m ^ e) for each half of the wave)
-// instead of the six the compiler makes of the plain form.  Call with all 64 lanes active.
+// Mask of the lanes whose digit equals this lane's, as two halves.  Per bit of the digit: e = all ones where the bit is
+// set, m = ballot of the bit; (m ^ e) has a one exactly for the lanes that differ from this lane in that bit.  Four vector
+// instructions a bit (sign-extended bit, compare into a lane mask, and one three-input bit operation same &= ~(m ^ e) for
+// each half of the wave) instead of the six the compiler makes of the plain form.  Call with all 64 lanes active.
 __device__ __forceinline__ void match_digit_halves(uint32_t d, uint32_t& same_lo, uint32_t& same_hi) {
     same_lo = ~0u;
     same_hi = ~0u;
@@ -173,42 +160,50 @@ __device__ __forceinline__ void match_digit_halves(uint32_t d, uint32_t& same_lo
     }
 }
 
-// Histogram updates in LDS.  Evenly spread digits go in with one LDS atomic per lane.  When many lanes hold the same
-// digit (exponent bytes, the high bytes of small integers) those atomics would queue up on one LDS word, so the
-// lanes are matched first and one lane per digit value adds the whole group.  digits_skewed() is the wave-uniform
-// test: do at least 8 lanes share the first lane's digit?
+// Wave-uniform test of a digit for the counting kernel: do at least 8 lanes share the first lane's digit?
 __device__ __forceinline__ bool digits_skewed(uint32_t d, bool valid) {
     const uint64_t active = __ballot(valid);
     if (active == 0ull) return false;
     const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, __ffsll((unsigned long long)active) - 1);
     return __popcll(__ballot(valid && d == d0)) >= 8;
 }
-__device__ __forceinline__ void count_digit(uint32_t* row, uint32_t d, bool valid, bool skewed) {
-    if (skewed) {
-        const uint64_t active = __ballot(valid);
-        if (active == 0ull) return;
-        const int first = __ffsll((unsigned long long)active) - 1;
-        const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, first);
-        if (__ballot(valid && d == d0) == active) {                       // one value in the whole wave
-            if (lane_id() == first) atomicAdd(&row[d0], (uint32_t)__popcll(active));
-            return;
-        }
-        const uint64_t peers = match_digit(d, active);
-        if (valid && lane_id() == __ffsll((unsigned long long)peers) - 1) atomicAdd(&row[d], (uint32_t)__popcll(peers));
-    } else if (valid) atomicAdd(&row[d], 1u);
+// ---- plan: which passes run and what they read --------------------------------------------------------------------
+// relative: keys are taken relative to the smallest one (integers), so digits above their range are zero in every key, and
+// so are low digits in which the keys do not differ.  Otherwise (floats) a digit in which no two keys differ is skipped:
+// their exponent bytes are constant or not whatever is subtracted.
+__device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool relative, unsigned long long range, unsigned long long varying,
+                                               int first_reads_b) {
+    uint32_t src_b = first_reads_b ? 1u : 0u, nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
+    for (int p = 0; p < passes; ++p) {
+        const unsigned long long upto = p == 7 ? ~0ull : (1ull << (8 * (p + 1))) - 1ull;
+        const bool skip = relative ? (range >> (8 * p)) == 0ull || (varying & upto) == 0ull : ((varying >> (8 * p)) & 0xffull) == 0ull;
+        ctl->skip[p] = skip ? 1u : 0u;
+        if (skip) continue;
+        ctl->src_is_b[p] = src_b;
+        src_b ^= 1u;
+        if (first == 0xffffffffu) first = (uint32_t)p;
+        last = (uint32_t)p;
+        ++nexec;
+    }
+    ctl->first_pass = first;
+    ctl->last_pass = last;
+    ctl->nexec = nexec;
 }
 
-// ---- init: clear control block and descriptors ------------------------------------------------------------
-// min_is_zero: the keys are not taken relative to their smallest (floats: the read that finds it saves no pass), so the
-// control block starts with ~0 in inv_min, i.e. a smallest mapped key of 0.
-__global__ __launch_bounds__(256) void sort_init_kernel(uint64_t* words, int64_t nwords, int min_is_zero) {
-    constexpr int64_t INV_MIN_WORD = (int64_t)(offsetof(SortCtl, inv_min) / sizeof(uint64_t));
-    static_assert(offsetof(SortCtl, inv_min) % sizeof(uint64_t) == 0, "inv_min is one of the cleared words");
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords; i += (int64_t)gridDim.x * 256)
-        words[i] = (min_is_zero && i == INV_MIN_WORD) ? ~0ull : 0ull;
+// ---- init: clear the control block ----------------------------------------------------------------------------------
+// all_passes: large sorts of floats, which run every pass on keys that are not taken relative to the smallest one; their
+// plan is made here.
+__global__ __launch_bounds__(256) void sort_init_kernel(SortCtl* ctl, int all_passes, int first_reads_b) {
+    for (int i = threadIdx.x; i < SORT_CTL_CLEAR; i += 256) ctl->skip[i] = 0u;
+    if (all_passes == 0) return;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        ctl->inv_min = ~0ull;
+        sort_make_plan(ctl, all_passes, false, 0ull, ~0ull, first_reads_b);
+    }
 }
 
-// The two whole-array reads below take 16-byte vectors from the aligned body [head, head + nvec * VEC) of the keys
+// The whole-array read below takes 16-byte vectors from the aligned body [head, head + nvec * VEC) of the keys
 // and single elements from the few keys in front of and behind it.
 template <typename T, typename F>
 __device__ __forceinline__ void for_each_key(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, F&& f) {
@@ -249,166 +244,76 @@ __device__ __forceinline__ void for_each_key(const T* __restrict__ keys, int64_t
     }
 }
 
-// ---- smallest mapped key ---------------------------------------------------------------------------------------
+// ---- smallest and largest key, varying bits -----------------------------------------------------------------------------
+// One read at streaming speed.  Integers are taken relative to the smallest key: small-range integers then need one or two
+// passes.  The workgroup whose ticket is the last makes the plan.
+constexpr int RANGE_BLOCK = 1024;       // few, large workgroups: each ends with device-wide atomics on shared words
 template <typename T>
-__global__ __launch_bounds__(256) void sort_min_kernel(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, int rev,
-                                                       SortCtl* ctl) {
+__global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, int rev,
+                                                                 int first_reads_b, SortCtl* ctl) {
     typedef typename SortKey<T>::U U;
+    typedef unsigned long long W;
     constexpr int VEC = 16 / sizeof(T);
-    __shared__ unsigned long long part[SORT_NW];
-    unsigned long long inv = 0;                  // max of ~u
-    for_each_key<T>(keys, n, head, nvec, [&](const U (&k)[VEC], int cnt) {
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-            if (j < cnt) {
-                const unsigned long long x = (unsigned long long)(U)~enc_bits<T>(k[j], rev, (U)0);
-                inv = x > inv ? x : inv;
-            }
-        }
-    });
-    // one device-wide atomic per workgroup: atomics on one address complete one after the other
-    inv = wave_reduce(inv, OpMax());
-    if (lane_id() == 0) part[threadIdx.x / WAVE] = inv;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int w = 1; w < SORT_NW; ++w) inv = part[w] > inv ? part[w] : inv;
-        if (inv != 0ull) atomicMax(&ctl->inv_min, inv);
-    }
-}
-
-// ---- smallest and largest mapped key (large integer sorts) ------------------------------------------------------------
-// Keys are taken relative to the smallest one, so their range tells which digits are zero in every key: the passes of
-// those digits are skipped.  One read at streaming speed; the large sorts do without the histogram read below.
-constexpr int MINMAX_BLOCK = 1024;      // few, large workgroups: each ends with two device-wide atomics on shared words
-template <typename T>
-__global__ __launch_bounds__(MINMAX_BLOCK) void sort_minmax_kernel(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, int rev,
-                                                                   SortCtl* ctl) {
-    typedef typename SortKey<T>::U U;
-    constexpr int VEC = 16 / sizeof(T);
-    __shared__ U part[2][MINMAX_BLOCK / WAVE];
-    U mn = (U)~(U)0, mx = 0;
+    constexpr bool RELATIVE = std::is_integral<T>::value;
+    __shared__ W part[3][RANGE_BLOCK / WAVE];
+    const U u0 = enc_bits<T>(__builtin_bit_cast(U, keys[0]), rev, (U)0);
+    U mn = u0, mx = u0, var = 0;
     for_each_key<T>(keys, n, head, nvec, [&](const U (&k)[VEC], int cnt) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
             if (j < cnt) {
                 const U u = enc_bits<T>(k[j], rev, (U)0);
-                mn = u < mn ? u : mn;
-                mx = u > mx ? u : mx;
+                if (RELATIVE) { mn = u < mn ? u : mn; mx = u > mx ? u : mx; }
+                var |= (U)(u ^ u0);
             }
         }
     });
-    mn = wave_reduce(mn, OpMin());
-    mx = wave_reduce(mx, OpMax());
-    if (lane_id() == 0) { part[0][threadIdx.x / WAVE] = mn; part[1][threadIdx.x / WAVE] = mx; }
+    W inv = wave_reduce((W)(U)~mn, OpMax()), top = wave_reduce((W)mx, OpMax()), dif = wave_reduce((W)var, OpOr());
+    if (lane_id() == 0) { part[0][threadIdx.x / WAVE] = inv; part[1][threadIdx.x / WAVE] = top; part[2][threadIdx.x / WAVE] = dif; }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < MINMAX_BLOCK / WAVE; ++w) { mn = part[0][w] < mn ? part[0][w] : mn; mx = part[1][w] > mx ? part[1][w] : mx; }
-        const unsigned long long inv = (unsigned long long)(U)~mn;
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < RANGE_BLOCK / WAVE; ++w) {
+        inv = part[0][w] > inv ? part[0][w] : inv;
+        top = part[1][w] > top ? part[1][w] : top;
+        dif |= part[2][w];
+    }
+    if (RELATIVE) {
         if (inv != 0ull) atomicMax(&ctl->inv_min, inv);
-        if (mx != 0) atomicMax(&ctl->key_max, (unsigned long long)mx);
+        if (top != 0ull) atomicMax(&ctl->key_max, top);
     }
+    if (dif != 0ull) atomicOr(&ctl->varying, dif);
+    publish_barrier();
+    if (atomicAdd(&ctl->range_ticket, 1u) != gridDim.x - 1u) return;
+    if (!RELATIVE) ctl->inv_min = ~0ull;                     // the smallest key is taken as 0
+    const W smallest = (W)(U)~(U)load_agent(&ctl->inv_min);
+    sort_make_plan(ctl, (int)sizeof(T), RELATIVE, RELATIVE ? load_agent(&ctl->key_max) - smallest : 0ull, load_agent(&ctl->varying), first_reads_b);
 }
 
-// ---- all digit histograms in one read -------------------------------------------------------------------------
-template <typename T, int PASSES>
-__global__ __launch_bounds__(256) void sort_hist_kernel(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, int rev,
-                                                        SortCtl* ctl) {
-    typedef typename SortKey<T>::U U;
-    __shared__ uint32_t h[PASSES][256];
-    const U umin = (U)~ctl->inv_min;
-    for (int i = threadIdx.x; i < PASSES * 256; i += 256) (&h[0][0])[i] = 0;
-    __syncthreads();
-    constexpr int VEC = 16 / sizeof(T);
-    for_each_key<T>(keys, n, head, nvec, [&](const U (&k)[VEC], int cnt) {
-        U u[VEC];
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) u[j] = enc_bits<T>(k[j], rev, umin);
-#pragma unroll
-        for (int p = 0; p < PASSES; ++p) {
-            const bool skewed = digits_skewed(digit_of(u[0], p), true);       // judged on the first key of the vector
-#pragma unroll
-            for (int j = 0; j < VEC; ++j) count_digit(h[p], digit_of(u[j], p), j < cnt, skewed);
-        }
-    });
-    __syncthreads();
-    for (int i = threadIdx.x; i < PASSES * 256; i += 256) {
-        const uint32_t c = (&h[0][0])[i];
-        if (c) atomicAdd(&ctl->hist[0][0] + i, c);
-    }
-}
-
-// ---- plan: scan the histograms, decide which passes run and what they read ---------------------------------------
-// one workgroup of 256 threads; lane d owns digit value d.  mode 0: from the histograms of sort_hist_kernel.
-// mode 1 (large sorts of integers): from the range of the keys, histograms come later, pass by pass.
-// mode 2 (large sorts of floats): every pass runs, keys are not taken relative to the smallest.
-__global__ __launch_bounds__(256) void sort_plan_kernel(SortCtl* ctl, int passes, uint32_t n, int first_reads_b, int mode) {
-    __shared__ uint32_t wsum[SORT_NW];
-    __shared__ int any_full;
-    const int d = threadIdx.x, wave = d / WAVE, lane = d % WAVE;
-    if (mode == 0) {
-        for (int p = 0; p < passes; ++p) {
-            const uint32_t c = ctl->hist[p][d];
-            if (d == 0) any_full = 0;
-            __syncthreads();
-            if (c == n) any_full = 1;
-            const uint32_t inc = wave_scan_inclusive(c, OpAdd(), 0u);
-            if (lane == WAVE - 1) wsum[wave] = inc;
-            __syncthreads();
-            uint32_t base = 0;
-            for (int w = 0; w < wave; ++w) base += wsum[w];
-            ctl->hist[p][d] = base + inc - c;
-            if (d == 0) ctl->skip[p] = any_full ? 1u : 0u;
-            __syncthreads();
-        }
-    } else if (d == 0) {
-        if (mode == 2) ctl->inv_min = ~0ull;                          // smallest key taken as 0
-        const unsigned long long umin = ~ctl->inv_min;                 // high bits beyond the key width: ones in both, cancel below
-        const unsigned long long range = mode == 2 ? ~0ull : ctl->key_max - (umin & (passes == 8 ? ~0ull : ((1ull << (8 * passes)) - 1ull)));
-        for (int p = 0; p < passes; ++p) ctl->skip[p] = (range >> (8 * p)) == 0ull ? 1u : 0u;
-    }
-    if (d == 0) {
-        uint32_t src_b = first_reads_b ? 1u : 0u, nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
-        for (int p = 0; p < passes; ++p) {
-            if (ctl->skip[p]) continue;
-            ctl->src_is_b[p] = src_b;
-            src_b ^= 1u;
-            if (first == 0xffffffffu) first = (uint32_t)p;
-            last = (uint32_t)p;
-            ++nexec;
-        }
-        ctl->first_pass = first;
-        ctl->last_pass = last;
-        ctl->nexec = nexec;
-    }
-}
-
-// ---- digit counts of every tile (large sorts) ---------------------------------------------------------------------
+// ---- digit counts of every tile -----------------------------------------------------------------------------------
 // Same tiles as sort_pass_kernel, one per workgroup; the order of the keys inside the tile does not matter here, so
-// aligned full tiles are read as 16-byte vectors.  One LDS atomic per key into one of UPS_SUB histograms per wave,
+// aligned full tiles are read as 16-byte vectors.  One LDS atomic per key into one of SUB histograms per wave,
 // chosen by the lane: skewed digits (exponent bytes, the high bytes of small integers) then queue up 16 deep on a
 // counter instead of 64 deep, and no lane has to find out who else holds its digit.
-constexpr int UPS_SUB = 4;
-
-template <typename T, int ITEMS>
-__global__ __launch_bounds__(SORT_BLOCK, 8) void sort_upsweep_kernel(const T* __restrict__ orig, const typename SortKey<T>::U* buf_a,
-                                                                  const typename SortKey<T>::U* buf_b, uint32_t n, int pass, int rev,
-                                                                  const SortCtl* ctl, uint32_t* __restrict__ tile_count) {
+template <typename T, int BLOCK, int ITEMS, int SUB, typename C>
+__global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restrict__ orig, const typename SortKey<T>::U* buf_a,
+                                                                const typename SortKey<T>::U* buf_b, uint32_t n, int pass, int rev,
+                                                                const SortCtl* ctl, C* __restrict__ tile_count) {
     typedef typename SortKey<T>::U U;
-    constexpr int TILE = SORT_BLOCK * ITEMS;
+    constexpr int TILE = BLOCK * ITEMS, NW = BLOCK / WAVE;
+    static_assert(sizeof(C) == 4 || TILE < 65536, "a count fits the table's type");
     constexpr int VEC = 16 / (int)sizeof(T), NV = ITEMS / VEC;
     typedef typename VecOf<U, VEC>::type VU;
-    __shared__ uint32_t cnt[SORT_NW * UPS_SUB][256];
+    __shared__ uint32_t cnt[NW * SUB][256];
     if (ctl->skip[pass]) return;
     const bool first = (uint32_t)pass == ctl->first_pass;
     const U* in = first ? (const U*)orig : (ctl->src_is_b[pass] != 0u ? buf_b : buf_a);
     const U umin = (U)~ctl->inv_min;
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-    for (int i = tid; i < SORT_NW * UPS_SUB * 256; i += SORT_BLOCK) (&cnt[0][0])[i] = 0;
+    for (int i = tid; i < NW * SUB * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
     const uint32_t tile = blockIdx.x;
     const uint32_t e0 = tile * (uint32_t)TILE;
     const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
-    uint32_t* row = cnt[wave * UPS_SUB + (lane & (UPS_SUB - 1))];
+    uint32_t* row = cnt[wave * SUB + (lane & (SUB - 1))];
     // When many lanes hold the same digit (judged on every fourth key) the two most frequent values -- as seen from the
     // first lane still in play -- are taken out with a ballot each and added by that lane alone; uniform floats have
     // 50% and 37% of their keys in two values of the exponent digit.
@@ -432,11 +337,13 @@ __global__ __launch_bounds__(SORT_BLOCK, 8) void sort_upsweep_kernel(const T* __
     };
     // (the two read paths share no variables: merged into one key array they made the compiler shuffle it through
     // private memory)
-    if (e0 + (uint32_t)TILE <= n && (((uintptr_t)(in + e0)) & 15) == 0) {
+    bool vectors = false;
+    if constexpr (NV > 0) vectors = e0 + (uint32_t)TILE <= n && (((uintptr_t)(in + e0)) & 15) == 0;
+    if (vectors) {
         const VU* vin = (const VU*)(in + e0);
-        VU v[NV];
+        VU v[NV > 0 ? NV : 1];
 #pragma unroll
-        for (int r = 0; r < NV; ++r) v[r] = vin[r * SORT_BLOCK + tid];
+        for (int r = 0; r < NV; ++r) v[r] = vin[r * BLOCK + tid];
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < NV; ++r) {
@@ -463,10 +370,11 @@ __global__ __launch_bounds__(SORT_BLOCK, 8) void sort_upsweep_kernel(const T* __
         }
     }
     __syncthreads();
+    if (BLOCK > 256 && tid >= 256) return;
     uint32_t c = 0;
 #pragma unroll
-    for (int w = 0; w < SORT_NW * UPS_SUB; ++w) c += cnt[w][tid];
-    tile_count[(uint64_t)tile * 256 + tid] = c;
+    for (int w = 0; w < NW * SUB; ++w) c += cnt[w][tid];
+    tile_count[(uint64_t)tile * 256 + tid] = (C)c;
 }
 
 // ---- where every tile's keys go (large sorts) --------------------------------------------------------------------------
@@ -550,7 +458,7 @@ __device__ __forceinline__ uint32_t ts_scan_groups(const uint32_t* x, uint32_t* 
 __global__ __launch_bounds__(TS_BLOCK) void sort_tilescan_kernel(SortCtl* ctl, int pass, uint32_t* count, uint32_t ntiles, uint32_t chunk_rows,
                                                                  uint32_t* chunk_total, uint32_t* chunk_prefix) {
     __shared__ uint32_t gsum[2][TS_GROUPS][256];
-    __shared__ uint32_t wsum[SORT_NW];
+    __shared__ uint32_t wsum[256 / WAVE];
     __shared__ uint32_t lds_ticket;
     if (ctl->skip[pass]) return;
     const uint32_t d = threadIdx.x & 255u, g = threadIdx.x >> 8, chunk = blockIdx.x, nchunks = gridDim.x;
@@ -581,32 +489,38 @@ __global__ __launch_bounds__(TS_BLOCK) void sort_tilescan_kernel(SortCtl* ctl, i
 }
 
 // ---- one pass ----------------------------------------------------------------------------------------------------
-// Tile = 256 threads x ITEMS keys.  Wave w owns the w-th quarter of the tile; its item i of lane l is key
-// i * 64 + l of that quarter (coalesced loads; the order (i, l) is memory order, which the ranking keeps).
-// desc[tile][digit]: low half = count, high half = (pass + 1) << 2 | status (1 = count of this tile only,
-// 2 = count of this and all earlier tiles); written and read with relaxed device-scope atomics, so the count
-// always travels with its tag.
+// Tile = BLOCK threads x ITEMS keys.  Wave w owns the w-th part of the tile; its item i of lane l is key
+// i * 64 + l of that part (coalesced loads; the order (i, l) is memory order, which the ranking keeps).
+// DIRECT: `counts` are the raw counts of every tile (uint16, a row of 256 a tile) and the workgroup sums the columns it
+// needs itself; otherwise they are the exclusive counts of sort_tilescan_kernel.
 // waves per SIMD the register allocation aims at: the kernel is bound by its vector instructions, and three or four
 // waves hide the latencies (measured: 4 against 6 workgroups a CU differ by 4%)
-template <typename T, bool PERM, bool COUNTED> constexpr int sort_pass_waves() { return (COUNTED && !PERM && sizeof(T) <= 4) ? 4 : 3; }
+template <typename T, bool PERM, bool DIRECT> constexpr int sort_pass_waves() { return (DIRECT || (!PERM && sizeof(T) <= 4)) ? 4 : 3; }
 
-template <typename T, int ITEMS, bool PERM, bool COUNTED>
-__global__ __launch_bounds__(SORT_BLOCK, (sort_pass_waves<T, PERM, COUNTED>())) void sort_pass_kernel(const T* __restrict__ orig, typename SortKey<T>::U* buf_a,
+template <typename T, int BLOCK, int ITEMS, bool PERM, bool DIRECT>
+__global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void sort_pass_kernel(const T* __restrict__ orig, typename SortKey<T>::U* buf_a,
                                                                typename SortKey<T>::U* buf_b, uint32_t* val_a, uint32_t* val_b,
-                                                               int64_t* __restrict__ perm_out, uint32_t n, int pass, int rev, SortCtl* ctl,
-                                                               uint64_t* desc, const uint32_t* __restrict__ tile_before,
+                                                               int64_t* __restrict__ perm_out, uint32_t n, int pass, int rev, const SortCtl* ctl,
+                                                               const void* __restrict__ counts,
                                                                const uint32_t* __restrict__ chunk_prefix, uint32_t chunk_rows,
-                                                               uint32_t ntiles, long long wait_rounds, uint32_t xcd_chunk) {
+                                                               uint32_t ntiles, uint32_t xcd_chunk) {
     typedef typename SortKey<T>::U U;
-    constexpr int TILE = SORT_BLOCK * ITEMS;
+    constexpr int TILE = BLOCK * ITEMS, NW = BLOCK / WAVE;
+    constexpr int GROUPS = DIRECT ? BLOCK / 128 : 1;       // groups of rows of the table, 128 lanes (two counts each) a group
     __shared__ U lds_keys[TILE];
     __shared__ uint32_t lds_vals[PERM ? TILE : 1];
-    __shared__ uint32_t cnt[SORT_NW][256];        // per wave and digit: count, then slot in the sorted tile of the wave's first key of the digit
+    __shared__ uint32_t cnt[NW][256];             // per wave and digit: count, then slot in the sorted tile of the wave's first key of the digit
     __shared__ uint32_t goff[256];                // global slot of the digit's first key of this tile, minus its slot in the sorted tile
-    __shared__ uint32_t wsum[SORT_NW];
-    __shared__ uint32_t lds_tile;
+    __shared__ uint32_t wsum[2][256 / WAVE];
+    __shared__ uint2 part_before[GROUPS][DIRECT ? 128 : 1], part_all[GROUPS][DIRECT ? 128 : 1];
 
-    if (ctl->skip[pass]) return;
+    const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+    if (ctl->skip[pass]) {
+        // all keys equal: no pass ran, and the last one writes the identity permutation
+        if (PERM && pass == (int)sizeof(T) - 1 && ctl->nexec == 0u)
+            for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < (int64_t)n; i += (int64_t)gridDim.x * BLOCK) perm_out[i] = i + 1;
+        return;
+    }
     const bool first = (uint32_t)pass == ctl->first_pass, last = (uint32_t)pass == ctl->last_pass;
     const U umin = (U)~ctl->inv_min;
     const bool src_b = ctl->src_is_b[pass] != 0u;
@@ -614,259 +528,232 @@ __global__ __launch_bounds__(SORT_BLOCK, (sort_pass_waves<T, PERM, COUNTED>())) 
     U* dst = src_b ? buf_a : buf_b;
     const uint32_t* vsrc = src_b ? val_b : val_a;
     uint32_t* vdst = src_b ? val_a : val_b;
-    const uint32_t tag_a = ((uint32_t)(pass + 1) << 2) | 1u, tag_p = ((uint32_t)(pass + 1) << 2) | 2u;
-    for (uint32_t round = 0;; ++round) {
-        // everything derived from the thread's index is computed again for every tile: hoisted out of this loop it
-        // would sit in some 35 registers (16 of them tid + i * 256) across the whole kernel
-        int tid = threadIdx.x;
-        asm volatile("" : "+v"(tid));
-        const int wave = tid / WAVE, lane = tid % WAVE;
-        if (!COUNTED && tid == 0) {
-            // once a look-back of this call has given up its wait the result is lost: no further tile starts
-            const uint32_t failed = __hip_atomic_load(&ctl->wait_failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t ticket = atomicAdd(&ctl->ticket[pass], 1u);
-            lds_tile = failed != 0u ? ntiles : ticket;
-        }
-        for (int i = tid; i < SORT_NW * 256; i += SORT_BLOCK) (&cnt[0][0])[i] = 0;
-        __syncthreads();
-        uint32_t tile = COUNTED ? blockIdx.x + round * gridDim.x : lds_tile;
-        if (COUNTED && xcd_chunk != 0u) {
-            const uint32_t i = (blockIdx.x >> 3) + round * (gridDim.x >> 3);
-            tile = i < xcd_chunk ? (blockIdx.x & 7u) * xcd_chunk + i : ntiles;
-        }
-        if (tile >= ntiles) return;
-        const uint32_t e0 = tile * (uint32_t)TILE;
-        const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
+    for (int i = tid; i < NW * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
+    __syncthreads();
+    uint32_t tile = blockIdx.x;
+    if (!DIRECT && xcd_chunk != 0u) {
+        const uint32_t i = blockIdx.x >> 3;
+        tile = i < xcd_chunk ? (blockIdx.x & 7u) * xcd_chunk + i : ntiles;
+    }
+    if (tile >= ntiles) return;
+    const uint32_t e0 = tile * (uint32_t)TILE;
+    const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
 
-        // Every tile but the last is full: its code carries no bounds checks (they cost an exec-mask save and a
-        // branch per key and round).
-        auto sort_tile = [&](auto full_tile) {
-            constexpr bool FULL = decltype(full_tile)::value;
-            // load (and map on the first pass)
-            U key[ITEMS];
-            uint32_t val[PERM ? ITEMS : 1];
-            uint32_t rank[ITEMS];
-    #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) {
-                const uint32_t e = woff + i * WAVE;
-                key[i] = (U)~(U)0;
-                if (FULL || e < n) key[i] = in[e];
+    // Every tile but the last is full: its code carries no bounds checks (they cost an exec-mask save and a
+    // branch per key and round).
+    auto sort_tile = [&](auto full_tile) {
+        constexpr bool FULL = decltype(full_tile)::value;
+        // load (and map on the first pass)
+        U key[ITEMS];
+        uint32_t val[PERM ? ITEMS : 1];
+        uint32_t rank[ITEMS];
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t e = woff + i * WAVE;
+            key[i] = (U)~(U)0;
+            if (FULL || e < n) key[i] = in[e];
+        }
+        if constexpr (PERM) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) val[i] = woff + i * WAVE;              // first pass: the key's own index
+            if (!first) {
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i)
+                    if (FULL || woff + i * WAVE < n) val[i] = vsrc[woff + i * WAVE];
             }
-            if constexpr (PERM) {
-    #pragma unroll
-                for (int i = 0; i < ITEMS; ++i) val[i] = woff + i * WAVE;              // first pass: the key's own index
-                if (!first) {
-    #pragma unroll
-                    for (int i = 0; i < ITEMS; ++i)
-                        if (FULL || woff + i * WAVE < n) val[i] = vsrc[woff + i * WAVE];
+        }
+        if constexpr (DIRECT) {
+            // columns of the table of counts: all rows, and the rows of the tiles in front.  At most 256 rows, 16 in flight.
+            const uint32_t c = (uint32_t)tid & 127u, g = (uint32_t)tid >> 7;
+            const uint32_t* col = (const uint32_t*)counts + c;
+            uint2 bef = {0u, 0u}, sum = {0u, 0u};
+            constexpr uint32_t UNR = 16;
+            for (uint32_t r0 = g; r0 < ntiles; r0 += GROUPS * UNR) {
+                uint32_t w[UNR];
+#pragma unroll
+                for (uint32_t u = 0; u < UNR; ++u) {
+                    const uint32_t r = r0 + u * GROUPS;
+                    w[u] = col[(uint64_t)(r < ntiles ? r : ntiles - 1u) * 128];
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < UNR; ++u) {
+                    const uint32_t r = r0 + u * GROUPS;
+                    const uint32_t lo = r < ntiles ? w[u] & 0xffffu : 0u, hi = r < ntiles ? w[u] >> 16 : 0u;
+                    sum.x += lo;
+                    sum.y += hi;
+                    bef.x += r < tile ? lo : 0u;
+                    bef.y += r < tile ? hi : 0u;
                 }
             }
-            if (first) {
-    #pragma unroll
-                for (int i = 0; i < ITEMS; ++i) key[i] = enc_bits<T>(key[i], rev, umin);    // padding keys are never counted
+            part_before[g][c] = bef;
+            part_all[g][c] = sum;
+        }
+        if (first) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) key[i] = enc_bits<T>(key[i], rev, umin);    // padding keys are never counted
+        }
+        // rank inside the wave: lanes with the same digit find each other with 8 ballots; every lane reads the
+        // wave's counter of its digit -- the rank of the group's first key -- and then the lowest lane of the group
+        // adds the size of the group to it.  LDS executes the instructions of one wave in order, so the read of
+        // the next round sees this add, and the 16 rounds queue up back to back; a result is used two rounds later.
+        uint32_t* wcnt = cnt[wave];
+        constexpr int DEPTH = 2;                       // counter reads in flight before their result is used
+        uint32_t pend_before[DEPTH], pend_below[DEPTH];
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const bool valid = FULL || woff + i * WAVE < n;
+            const uint32_t d = digit_of(key[i], pass);
+            uint32_t same_lo, same_hi;
+            match_digit_halves(d, same_lo, same_hi);
+            if (!FULL) {
+                const uint64_t vm = __ballot(valid);
+                same_lo &= (uint32_t)vm;
+                same_hi &= (uint32_t)(vm >> 32);
             }
-            // rank inside the wave: lanes with the same digit find each other with 8 ballots; every lane reads the
-            // wave's counter of its digit -- the rank of the group's first key -- and then the lowest lane of the group
-            // adds the size of the group to it.  LDS executes the instructions of one wave in order, so the read of
-            // the next round sees this add, and the 16 rounds queue up back to back; a result is used two rounds later.
-            uint32_t* wcnt = cnt[wave];
-            constexpr int DEPTH = 2;                       // counter reads in flight before their result is used
-            uint32_t pend_before[DEPTH], pend_below[DEPTH];
-    #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) {
-                const bool valid = FULL || woff + i * WAVE < n;
-                const uint32_t d = digit_of(key[i], pass);
-                uint32_t same_lo, same_hi;
-                match_digit_halves(d, same_lo, same_hi);
-                if (!FULL) {
-                    const uint64_t vm = __ballot(valid);
-                    same_lo &= (uint32_t)vm;
-                    same_hi &= (uint32_t)(vm >> 32);
-                }
-                const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
-                const uint32_t before = __hip_atomic_load(&wcnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                __builtin_amdgcn_wave_barrier();
-                if (valid && below == 0u) {
-                    const uint32_t total = (uint32_t)__builtin_popcount(same_lo) + (uint32_t)__builtin_popcount(same_hi);
-                    __hip_atomic_fetch_add(&wcnt[d], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                }
-                if (i >= DEPTH) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
-                pend_before[i % DEPTH] = before;
-                pend_below[i % DEPTH] = below;
-                __builtin_amdgcn_sched_barrier(0);
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
+            const uint32_t before = __hip_atomic_load(&wcnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+            __builtin_amdgcn_wave_barrier();
+            if (valid && below == 0u) {
+                const uint32_t total = (uint32_t)__builtin_popcount(same_lo) + (uint32_t)__builtin_popcount(same_hi);
+                __hip_atomic_fetch_add(&wcnt[d], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
             }
-    #pragma unroll
-            for (int i = ITEMS; i < ITEMS + DEPTH; ++i) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
-            __syncthreads();
-            // digit d = tid: count of the tile and of each wave
-            uint32_t wave_count[SORT_NW];
-            uint32_t count = 0;
-    #pragma unroll
-            for (int w = 0; w < SORT_NW; ++w) {
+            if (i >= DEPTH) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
+            pend_before[i % DEPTH] = before;
+            pend_below[i % DEPTH] = below;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = ITEMS; i < ITEMS + DEPTH; ++i) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
+        __syncthreads();
+        // digit d = tid (the first 256 threads): count of the tile and of each wave, first slot inside the sorted tile
+        // (exclusive scan over the digits) and in the whole output
+        uint32_t wave_count[NW];
+        uint32_t count = 0, excl = 0, all = 0, inc = 0, inc_all = 0;
+        const bool has_digit = BLOCK == 256 || tid < 256;
+        if (has_digit) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
                 wave_count[w] = cnt[w][tid];
                 count += wave_count[w];
             }
-            // publish the count, then look back over the earlier tiles for this digit
-            uint64_t* my = desc + (uint64_t)tile * 256 + tid;
-            uint32_t excl = 0;
-            if constexpr (COUNTED) {
-                excl = tile_before[(uint64_t)tile * 256 + tid] + chunk_prefix[(uint64_t)(tile / chunk_rows) * 256 + tid];
-            } else if (tile == 0) {
-                __hip_atomic_store(my, ((uint64_t)tag_p << 32) | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                __hip_atomic_store(my, ((uint64_t)tag_a << 32) | count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                // walk back over the earlier tiles, LB descriptors per round trip: sum counts until one that already
-                // includes its own predecessors; a descriptor that is not written yet is polled again
-                constexpr int LB = 8;
-                int64_t t = (int64_t)tile - 1;
-                bool done = false;
-                const WaitCtl wc{&ctl->wait_failed, wait_rounds, 0, 1u};     // the control block belongs to this call alone
-                long long rounds = 0;
-                while (!done) {
-                    uint64_t w[LB];
-    #pragma unroll
-                    for (int j = 0; j < LB; ++j) {
-                        w[j] = ((uint64_t)tag_p << 32);                       // in front of tile 0: nothing, and final
-                        if (t - j >= 0) w[j] = __hip_atomic_load(desc + (uint64_t)(t - j) * 256 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    }
-                    int j = 0;
-    #pragma unroll
-                    for (; j < LB; ++j) {
-                        const uint32_t tg = (uint32_t)(w[j] >> 32);
-                        if (tg != tag_a && tg != tag_p) break;
-                        excl += (uint32_t)w[j];
-                        if (tg == tag_p) { done = true; break; }
-                    }
-                    t -= j;
-                    if (!done && j == 0) {
-                        // every lane counts its own rounds (a lane per digit); one giving up makes all others follow
-                        if (wait_give_up(wc, rounds)) break;
-                        __builtin_amdgcn_s_sleep(2);
-                    }
+            if constexpr (DIRECT) {
+#pragma unroll
+                for (int g = 0; g < GROUPS; ++g) {
+                    const uint2 b = part_before[g][tid >> 1], a = part_all[g][tid >> 1];
+                    excl += (tid & 1) ? b.y : b.x;
+                    all += (tid & 1) ? a.y : a.x;
                 }
-                __hip_atomic_store(my, ((uint64_t)tag_p << 32) | (uint64_t)(excl + count), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                inc_all = wave_scan_inclusive(all, OpAdd(), 0u);
+                if (lane == WAVE - 1) wsum[1][wave] = inc_all;
+            } else {
+                excl = ((const uint32_t*)counts)[(uint64_t)tile * 256 + tid] + chunk_prefix[(uint64_t)(tile / chunk_rows) * 256 + tid];
             }
-            // first slot of every digit inside the sorted tile: exclusive scan of the counts over the 256 digits
-            const uint32_t inc = wave_scan_inclusive(count, OpAdd(), 0u);
-            if (lane == WAVE - 1) wsum[wave] = inc;
-            __syncthreads();
-            uint32_t start = inc - count;
-            for (int w = 0; w < wave; ++w) start += wsum[w];
-            goff[tid] = ctl->hist[pass][tid] + excl - start;
-    #pragma unroll
-            for (int w = 0; w < SORT_NW; ++w) {
+            inc = wave_scan_inclusive(count, OpAdd(), 0u);
+            if (lane == WAVE - 1) wsum[0][wave] = inc;
+        }
+        __syncthreads();
+        if (has_digit) {
+            uint32_t start = inc - count, base = DIRECT ? inc_all - all : ctl->hist[pass][tid];
+            for (int w = 0; w < wave; ++w) {
+                start += wsum[0][w];
+                if (DIRECT) base += wsum[1][w];
+            }
+            goff[tid] = base + excl - start;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
                 cnt[w][tid] = start;
                 start += wave_count[w];
             }
-            __syncthreads();
-            // reorder the tile in LDS.  Reads first, writes after, so that the 16 table reads are in flight together.
-    #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) {
-                uint32_t d = digit_of(key[i], pass);
-                asm volatile("" : "+v"(d));            // computed again here: 16 LDS addresses kept from the ranking cost a wave of occupancy
-                rank[i] += wcnt[d];
+        }
+        __syncthreads();
+        // reorder the tile in LDS.  Reads first, writes after, so that the 16 table reads are in flight together.
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            uint32_t d = digit_of(key[i], pass);
+            asm volatile("" : "+v"(d));            // computed again here: 16 LDS addresses kept from the ranking cost a wave of occupancy
+            rank[i] += wcnt[d];
+        }
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (FULL || woff + i * WAVE < n) {
+                lds_keys[rank[i]] = key[i];
+                if constexpr (PERM) lds_vals[rank[i]] = val[i];
             }
-    #pragma unroll
+        }
+        __syncthreads();
+        // write runs of equal digits: thread q takes the q-th key of the sorted tile.  Again all reads of a kind
+        // together; `last` is decided once, not per key.
+        const uint32_t valid_n = n - e0 < (uint32_t)TILE ? n - e0 : (uint32_t)TILE;
+        U out_key[ITEMS];
+        uint32_t slot[ITEMS];
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t q = (uint32_t)tid + i * BLOCK;
+            out_key[i] = (U)0;
+            if (FULL || q < valid_n) out_key[i] = lds_keys[q];
+        }
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) slot[i] = goff[digit_of(out_key[i], pass)] + (uint32_t)tid + i * BLOCK;
+        auto writable = [&](int i) { return FULL || (uint32_t)tid + i * BLOCK < valid_n; };
+        if constexpr (PERM) {
+            uint32_t out_val[ITEMS];
+#pragma unroll
             for (int i = 0; i < ITEMS; ++i) {
-                if (FULL || woff + i * WAVE < n) {
-                    lds_keys[rank[i]] = key[i];
-                    if constexpr (PERM) lds_vals[rank[i]] = val[i];
-                }
+                out_val[i] = 0;
+                if (FULL || (uint32_t)tid + i * BLOCK < valid_n) out_val[i] = lds_vals[(uint32_t)tid + i * BLOCK];
             }
-            __syncthreads();
-            // write runs of equal digits: thread q takes the q-th key of the sorted tile.  Again all reads of a kind
-            // together; `last` is decided once, not per key.
-            const uint32_t valid_n = n - e0 < (uint32_t)TILE ? n - e0 : (uint32_t)TILE;
-            U out_key[ITEMS];
-            uint32_t slot[ITEMS];
-    #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) {
-                const uint32_t q = (uint32_t)tid + i * SORT_BLOCK;
-                out_key[i] = (U)0;
-                if (FULL || q < valid_n) out_key[i] = lds_keys[q];
-            }
-    #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) slot[i] = goff[digit_of(out_key[i], pass)] + (uint32_t)tid + i * SORT_BLOCK;
-            // slot < n always holds in a sound sort.  After a look-back has given up its wait (WaitCtl) the offsets are
-            // too small and this pass leaves holes; the next pass then reads keys the histograms never counted, and
-            // its slots can lie anywhere: keep every store inside the arrays.  (The large sorts count every tile of
-            // every pass themselves and wait for nobody.)
-            auto writable = [&](int i) { return (FULL || (uint32_t)tid + i * SORT_BLOCK < valid_n) && (COUNTED || slot[i] < n); };
-            if constexpr (PERM) {
-                uint32_t out_val[ITEMS];
-    #pragma unroll
-                for (int i = 0; i < ITEMS; ++i) {
-                    out_val[i] = 0;
-                    if (FULL || (uint32_t)tid + i * SORT_BLOCK < valid_n) out_val[i] = lds_vals[(uint32_t)tid + i * SORT_BLOCK];
-                }
-                if (last) {
-    #pragma unroll
-                    for (int i = 0; i < ITEMS; ++i) if (writable(i)) perm_out[slot[i]] = (int64_t)out_val[i] + 1;
-                } else {
-    #pragma unroll
-                    for (int i = 0; i < ITEMS; ++i) if (writable(i)) { dst[slot[i]] = out_key[i]; vdst[slot[i]] = out_val[i]; }
-                }
-            } else if (last) {
-    #pragma unroll
-                for (int i = 0; i < ITEMS; ++i) if (writable(i)) ((T*)dst)[slot[i]] = dec_bits<T>(out_key[i], rev, umin);
+            if (last) {
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) if (writable(i)) perm_out[slot[i]] = (int64_t)out_val[i] + 1;
             } else {
-    #pragma unroll
-                for (int i = 0; i < ITEMS; ++i) if (writable(i)) dst[slot[i]] = out_key[i];
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) if (writable(i)) { dst[slot[i]] = out_key[i]; vdst[slot[i]] = out_val[i]; }
             }
-        };
-        if (e0 + (uint32_t)TILE <= n) sort_tile(std::true_type{}); else sort_tile(std::false_type{});
-        __syncthreads();      // LDS is reused by the next tile
-    }
+        } else if (last) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) if (writable(i)) ((T*)dst)[slot[i]] = dec_bits<T>(out_key[i], rev, umin);
+        } else {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) if (writable(i)) dst[slot[i]] = out_key[i];
+        }
+    };
+    if (e0 + (uint32_t)TILE <= n) sort_tile(std::true_type{}); else sort_tile(std::false_type{});
 }
 
 // ---- finish ------------------------------------------------------------------------------------------------------
-// sort: after an odd number of passes the result sits in buffer B.  sortperm: no pass ran = identity permutation.
+// sort!: after an odd number of passes the result sits in buffer B.
 template <typename W>
-__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, W* a, const W* b, int64_t nwords, int64_t* perm_out, int64_t n) {
-    const uint32_t nexec = ctl->nexec;
-    if (perm_out != nullptr) {
-        if (nexec != 0u) return;
-        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) perm_out[i] = i + 1;
-        return;
-    }
-    if ((nexec & 1u) == 0u) return;
+__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, W* a, const W* b, int64_t nwords) {
+    if ((ctl->nexec & 1u) == 0u) return;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords; i += (int64_t)gridDim.x * 256) a[i] = b[i];
 }
 
 // ---- host --------------------------------------------------------------------------------------------------------
+constexpr int64_t SORT_TILE = 4096;               // keys per tile: 256 lanes x 16 (large sorts) or 1024 x 4
+constexpr int SORT_ITEMS = (int)SORT_TILE / SORT_BLOCK;
+constexpr int DIRECT_BLOCK = 1024, DIRECT_ITEMS = (int)SORT_TILE / DIRECT_BLOCK;
+constexpr uint32_t DIRECT_TILES = 256;            // up to here a pass sums the columns of the table of counts itself
+
 struct SortLayout {
-    size_t desc_off, clear_end, chunk_total_off, chunk_prefix_off, keys_b_off, keys_a_off, val_a_off, val_b_off, total;
+    size_t count_off, chunk_total_off, chunk_prefix_off, keys_b_off, keys_a_off, val_a_off, val_b_off, total;
     uint32_t ntiles, chunk_rows, nchunks;
-    bool counted;          // large sort: desc_off holds the per-tile digit counts (uint32) instead of descriptors
+    bool direct;
 };
 
-// keys per lane and tile: 16 for every key size (8 was tried for 8-byte keys: 5.2 instead of 4.4 ms for 2^26 Float64)
-constexpr int sort_items_for(size_t) { return 16; }
-template <typename T> constexpr int sort_items() { return sort_items_for(sizeof(T)); }
-
-// More tiles than this: count first, no look-back (RK_SORT_LOOKBACK_TILES).
-static uint32_t sort_lookback_tiles() {
-    static const uint32_t v = [] { const char* e = std::getenv("RK_SORT_LOOKBACK_TILES"); const long x = e ? std::atol(e) : 0; return x > 0 ? (uint32_t)x : 256u; }();
-    return v;
-}
-
-static SortLayout sort_layout(size_t key_size, int items, int64_t n, bool perm) {
+static SortLayout sort_layout(size_t key_size, int64_t n, bool perm) {
     SortLayout l{};
-    const int64_t tile = (int64_t)SORT_BLOCK * items;
-    l.ntiles = (uint32_t)((n + tile - 1) / tile);
+    l.ntiles = (uint32_t)((n + SORT_TILE - 1) / SORT_TILE);
     size_t off = (sizeof(SortCtl) + 255) & ~(size_t)255;
-    l.counted = l.ntiles > sort_lookback_tiles();
-    l.desc_off = off;
-    if (l.counted) {
-        l.clear_end = off;                                   // only the control block needs clearing
+    l.direct = l.ntiles <= DIRECT_TILES;
+    l.count_off = off;
+    if (l.direct) {
+        off += (size_t)l.ntiles * 256 * sizeof(uint16_t);
+    } else {
         off += (size_t)l.ntiles * 256 * sizeof(uint32_t);
         l.chunk_rows = (l.ntiles + TS_MAX_CHUNKS - 1) / TS_MAX_CHUNKS;
         l.nchunks = (l.ntiles + l.chunk_rows - 1) / l.chunk_rows;
         l.chunk_total_off = off;  off += (size_t)TS_MAX_CHUNKS * 256 * sizeof(uint32_t);
         l.chunk_prefix_off = off; off += (size_t)TS_MAX_CHUNKS * 256 * sizeof(uint32_t);
-    } else {
-        off += (size_t)l.ntiles * 256 * sizeof(uint64_t);
-        l.clear_end = off;
     }
     const size_t kbytes = ((size_t)n * key_size + 255) & ~(size_t)255, vbytes = ((size_t)n * 4 + 255) & ~(size_t)255;
     l.keys_b_off = off; off += kbytes;
@@ -879,95 +766,72 @@ static SortLayout sort_layout(size_t key_size, int items, int64_t n, bool perm) 
     return l;
 }
 
-template <typename T>
+template <typename T, bool PERM>
 static int32_t sort_typed(void* keys, int64_t* perm_out, int64_t n, int rev, void* tmp, size_t tmp_bytes, hipStream_t stream) {
     typedef typename SortKey<T>::U U;
-    constexpr int ITEMS = sort_items<T>();
     constexpr int PASSES = (int)sizeof(T);
-    const bool perm = perm_out != nullptr;
-    const SortLayout l = sort_layout(sizeof(T), ITEMS, n, perm);
+    const SortLayout l = sort_layout(sizeof(T), n, PERM);
     if (tmp == nullptr || !is_aligned(tmp, 256) || tmp_bytes < l.total) return RK_ERR_WORKSPACE;
     char* base = (char*)tmp;
     SortCtl* ctl = (SortCtl*)base;
-    uint64_t* desc = (uint64_t*)(base + l.desc_off);
     U* buf_b = (U*)(base + l.keys_b_off);
-    U* buf_a = perm ? (U*)(base + l.keys_a_off) : (U*)keys;
-    uint32_t* val_a = perm ? (uint32_t*)(base + l.val_a_off) : nullptr;
-    uint32_t* val_b = perm ? (uint32_t*)(base + l.val_b_off) : nullptr;
+    U* buf_a = PERM ? (U*)(base + l.keys_a_off) : (U*)keys;
+    uint32_t* val_a = PERM ? (uint32_t*)(base + l.val_a_off) : nullptr;
+    uint32_t* val_b = PERM ? (uint32_t*)(base + l.val_b_off) : nullptr;
     const int cus = device_info().cus;
 
-    const int64_t init_words = (int64_t)(l.clear_end / sizeof(uint64_t));
-    int64_t g = (init_words + 255) / 256;
-    if (g > cus * 16) g = cus * 16;
-    // floats: no read for the smallest key.  Relative keys let small-range integers skip passes (1000 .. 1255: one pass
-    // instead of two); the exponent bytes of floats are constant or not whatever is subtracted, and the histograms of the
-    // small sorts find constant digits by themselves.
     constexpr bool FLOAT_KEYS = !std::is_integral<T>::value;
-    sort_init_kernel<<<(unsigned)g, 256, 0, stream>>>((uint64_t*)base, init_words, FLOAT_KEYS ? 1 : 0);
+    const bool all_passes = FLOAT_KEYS && !l.direct;
+    const int first_reads_b = PERM ? 1 : 0;          // sortperm: the first pass reads the caller's keys and writes buffer A
+    sort_init_kernel<<<1, 256, 0, stream>>>(ctl, all_passes ? PASSES : 0, first_reads_b);
     RK_LAUNCH_CHECK();
-    g = (n + 256 * 16 - 1) / (256 * 16);
-    if (g > cus * 8) g = cus * 8;
-    constexpr int KVEC = 16 / (int)sizeof(T);
-    int64_t head = (int64_t)(((16 - ((uintptr_t)keys & 15)) & 15) / sizeof(T));
-    if (head > n) head = n;
-    const int64_t nvec = (n - head) / KVEC;
-    // few workgroups: each ends with device-wide atomics on shared words (1 for the minimum, 256 per digit position)
-    const unsigned gmin = (unsigned)(g < cus * 2 ? g : cus * 2), ghist = (unsigned)(g < cus * 4 ? g : cus * 4);
-    // sortperm: the first pass reads the caller's keys and should write buffer A, i.e. "reads B"
-    if (!l.counted) {
-        if (!FLOAT_KEYS) {
-            sort_min_kernel<T><<<gmin, 256, 0, stream>>>((const T*)keys, n, head, nvec, rev, ctl);
-            RK_LAUNCH_CHECK();
-        }
-        sort_hist_kernel<T, PASSES><<<ghist, 256, 0, stream>>>((const T*)keys, n, head, nvec, rev, ctl);
+    if (!all_passes) {
+        constexpr int KVEC = 16 / (int)sizeof(T);
+        int64_t head = (int64_t)(((16 - ((uintptr_t)keys & 15)) & 15) / sizeof(T));
+        if (head > n) head = n;
+        const int64_t nvec = (n - head) / KVEC;
+        // 4 vectors a lane and few workgroups: each ends with device-wide atomics on shared words
+        int64_t g = (nvec + RANGE_BLOCK * 4 - 1) / (RANGE_BLOCK * 4);
+        if (g > cus * 2) g = cus * 2;
+        if (g < 1) g = 1;
+        sort_range_kernel<T><<<(unsigned)g, RANGE_BLOCK, 0, stream>>>((const T*)keys, n, head, nvec, rev, first_reads_b, ctl);
         RK_LAUNCH_CHECK();
-        sort_plan_kernel<<<1, 256, 0, stream>>>(ctl, PASSES, (uint32_t)n, perm ? 1 : 0, 0);
-    } else if (std::is_integral<T>::value) {
-        sort_minmax_kernel<T><<<gmin, MINMAX_BLOCK, 0, stream>>>((const T*)keys, n, head, nvec, rev, ctl);
-        RK_LAUNCH_CHECK();
-        sort_plan_kernel<<<1, 256, 0, stream>>>(ctl, PASSES, (uint32_t)n, perm ? 1 : 0, 1);
-    } else {
-        // floats: the digits of a large array are hardly ever constant, so no read is spent on finding out
-        sort_plan_kernel<<<1, 256, 0, stream>>>(ctl, PASSES, (uint32_t)n, perm ? 1 : 0, 2);
     }
-    RK_LAUNCH_CHECK();
-    // tunables, read once: workgroups of the pass kernel per CU (RK_SORT_WGS_PER_CU), XCD-contiguous tiles (RK_SORT_XCD=0: off).
-    // Large sorts launch one workgroup per tile unless told otherwise: the hardware's dispatcher balances the load
-    // better than a fixed share of tiles per resident workgroup (2^26 Float32: 866 against 986 us with 4 a CU).
-    static const int wgs_per_cu = [] { const char* e = std::getenv("RK_SORT_WGS_PER_CU"); const int x = e ? std::atoi(e) : 0; return x > 0 ? x : 0; }();
+    // tunable, read once: XCD-contiguous tiles (RK_SORT_XCD=0: off).  Large sorts launch one workgroup per tile: the
+    // hardware's dispatcher balances the load better than a fixed share of tiles per resident workgroup (2^26 Float32:
+    // 866 against 986 us with 4 a CU), and each XCD takes a contiguous eighth of the tiles, so the runs that neighbouring
+    // tiles write next to each other meet in one L2 (workgroups go to the XCDs round-robin by their index).
     static const int xcd_map = [] { const char* e = std::getenv("RK_SORT_XCD"); return e ? std::atoi(e) : 1; }();
-    unsigned pgrid;
-    if (l.counted && wgs_per_cu == 0) pgrid = (l.ntiles + 7u) & ~7u;
-    else { const unsigned cap = (unsigned)(cus * (wgs_per_cu > 0 ? wgs_per_cu : 6)); pgrid = l.ntiles < cap ? l.ntiles : cap; }
-    // large sorts: each XCD takes a contiguous eighth of the tiles, so the runs that neighbouring tiles write next to
-    // each other meet in one L2 (workgroups go to the XCDs round-robin by their index)
-    const uint32_t xcd_chunk = (xcd_map != 0 && l.counted && pgrid % 8u == 0u) ? (l.ntiles + 7u) / 8u : 0u;
-    uint32_t* tile_count = (uint32_t*)desc;
-    uint32_t* chunk_total = l.counted ? (uint32_t*)(base + l.chunk_total_off) : nullptr;
-    uint32_t* chunk_prefix = l.counted ? (uint32_t*)(base + l.chunk_prefix_off) : nullptr;
-    const long long wb = wait_budget();
+    const unsigned pgrid = (l.ntiles + 7u) & ~7u;
+    const uint32_t xcd_chunk = xcd_map != 0 ? (l.ntiles + 7u) / 8u : 0u;
     for (int p = 0; p < PASSES; ++p) {
-        if (l.counted) {
-            sort_upsweep_kernel<T, ITEMS><<<l.ntiles, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, tile_count);
+        if (l.direct) {
+            uint16_t* counts = (uint16_t*)(base + l.count_off);
+            sort_upsweep_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, 1, uint16_t><<<l.ntiles, DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
             RK_LAUNCH_CHECK();
-            sort_tilescan_kernel<<<l.nchunks, TS_BLOCK, 0, stream>>>(ctl, p, tile_count, l.ntiles, l.chunk_rows, chunk_total, chunk_prefix);
-            RK_LAUNCH_CHECK();
-            if (perm) sort_pass_kernel<T, ITEMS, true, true><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, desc, tile_count, chunk_prefix, l.chunk_rows, l.ntiles, wb, xcd_chunk);
-            else sort_pass_kernel<T, ITEMS, false, true><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, nullptr, nullptr, nullptr, (uint32_t)n, p, rev, ctl, desc, tile_count, chunk_prefix, l.chunk_rows, l.ntiles, wb, xcd_chunk);
+            sort_pass_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, PERM, true><<<l.ntiles, DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, nullptr, 1u, l.ntiles, 0u);
         } else {
-            if (perm) sort_pass_kernel<T, ITEMS, true, false><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, desc, nullptr, nullptr, 1u, l.ntiles, wb, 0u);
-            else sort_pass_kernel<T, ITEMS, false, false><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, nullptr, nullptr, nullptr, (uint32_t)n, p, rev, ctl, desc, nullptr, nullptr, 1u, l.ntiles, wb, 0u);
+            uint32_t* counts = (uint32_t*)(base + l.count_off);
+            uint32_t* chunk_total = (uint32_t*)(base + l.chunk_total_off);
+            uint32_t* chunk_prefix = (uint32_t*)(base + l.chunk_prefix_off);
+            sort_upsweep_kernel<T, SORT_BLOCK, SORT_ITEMS, 4, uint32_t><<<l.ntiles, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
+            RK_LAUNCH_CHECK();
+            sort_tilescan_kernel<<<l.nchunks, TS_BLOCK, 0, stream>>>(ctl, p, counts, l.ntiles, l.chunk_rows, chunk_total, chunk_prefix);
+            RK_LAUNCH_CHECK();
+            sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, chunk_prefix, l.chunk_rows, l.ntiles, xcd_chunk);
         }
         RK_LAUNCH_CHECK();
     }
-    const int64_t nwords = ((int64_t)n * (int64_t)sizeof(T) + 3) / 4;
-    g = ((perm ? n : nwords) + 255) / 256;
-    if (g > cus * 16) g = cus * 16;
-    // whole 32-bit words: buffers are 256-byte padded, the caller's array is at least element-aligned; 16-bit keys
-    // with an odd count copy one element more than n only inside buffer padding on the source side -- so copy by element there
-    if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (uint16_t*)keys, (const uint16_t*)buf_b, perm ? 0 : n, perm_out, n);
-    else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (uint32_t*)keys, (const uint32_t*)buf_b, perm ? 0 : nwords, perm_out, n);
-    RK_LAUNCH_CHECK();
+    if (!PERM && !(all_passes && PASSES % 2 == 0)) {
+        // whole 32-bit words: buffers are 256-byte padded, the caller's array is at least element-aligned; 16-bit keys
+        // with an odd count copy one element more than n only inside buffer padding on the source side -- so copy by element there
+        const int64_t nwords = sizeof(T) == 2 ? n : ((int64_t)n * (int64_t)sizeof(T) + 3) / 4;
+        int64_t g = (nwords + 255) / 256;
+        if (g > cus * 16) g = cus * 16;
+        if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (uint16_t*)keys, (const uint16_t*)buf_b, nwords);
+        else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (uint32_t*)keys, (const uint32_t*)buf_b, nwords);
+        RK_LAUNCH_CHECK();
+    }
     return RK_SUCCESS;
 }
 
@@ -987,9 +851,10 @@ using namespace rk;
 extern "C" size_t rk_sort_tmp_bytes(rk_dtype dt, int64_t n, int32_t with_perm) {
     size_t ks = 0;
     if (!sort_dtype_size((int)dt, &ks) || n <= 0) return 256;
-    return sort_layout(ks, sort_items_for(ks), n, with_perm != 0).total;
+    return sort_layout(ks, n, with_perm != 0).total;
 }
 
+template <bool PERM>
 static int32_t sort_dispatch(rk_dtype dt, void* keys, int64_t* perm_out, int64_t n, int32_t rev, void* tmp, size_t tmp_bytes, void* stream) {
     size_t ks = 0;
     if (!sort_dtype_size((int)dt, &ks)) return ((int)dt >= RK_F32 && (int)dt <= RK_I16) ? RK_ERR_UNSUPPORTED : RK_ERR_INVALID_ARGUMENT;
@@ -998,32 +863,31 @@ static int32_t sort_dispatch(rk_dtype dt, void* keys, int64_t* perm_out, int64_t
     if (keys == nullptr || !is_aligned(keys, ks)) return RK_ERR_INVALID_ARGUMENT;
     if (n >= ((int64_t)1 << 31)) return RK_ERR_TOO_LARGE;
     hipStream_t st = (hipStream_t)stream;
-    const int r = (rev ? SORT_REV : 0) | (perm_out == nullptr ? SORT_KEEP_NAN : 0);
+    const int r = (rev ? SORT_REV : 0) | (PERM ? 0 : SORT_KEEP_NAN);
     switch ((int)dt) {
-        case RK_F32: return sort_typed<float>(keys, perm_out, n, r, tmp, tmp_bytes, st);
-        case RK_F64: return sort_typed<double>(keys, perm_out, n, r, tmp, tmp_bytes, st);
-        case RK_I32: return sort_typed<int32_t>(keys, perm_out, n, r, tmp, tmp_bytes, st);
-        case RK_I64: return sort_typed<int64_t>(keys, perm_out, n, r, tmp, tmp_bytes, st);
-        case RK_F16: return sort_typed<half_bits>(keys, perm_out, n, r, tmp, tmp_bytes, st);
-        default:     return sort_typed<int16_t>(keys, perm_out, n, r, tmp, tmp_bytes, st);
+        case RK_F32: return sort_typed<float, PERM>(keys, perm_out, n, r, tmp, tmp_bytes, st);
+        case RK_F64: return sort_typed<double, PERM>(keys, perm_out, n, r, tmp, tmp_bytes, st);
+        case RK_I32: return sort_typed<int32_t, PERM>(keys, perm_out, n, r, tmp, tmp_bytes, st);
+        case RK_I64: return sort_typed<int64_t, PERM>(keys, perm_out, n, r, tmp, tmp_bytes, st);
+        case RK_F16: return sort_typed<half_bits, PERM>(keys, perm_out, n, r, tmp, tmp_bytes, st);
+        default:     return sort_typed<int16_t, PERM>(keys, perm_out, n, r, tmp, tmp_bytes, st);
     }
 }
 
+// No kernel of the sort waits for another workgroup, so there is no give-up to report.
 extern "C" int32_t rk_sort_status(const void* tmp, size_t tmp_bytes, void* stream) {
     if (tmp == nullptr) return RK_ERR_INVALID_ARGUMENT;
     if (!is_aligned(tmp, 256) || tmp_bytes < sizeof(SortCtl)) return RK_ERR_WORKSPACE;
-    uint32_t failed = 0;
-    RK_HIP(hipMemcpyAsync(&failed, (const char*)tmp + offsetof(SortCtl, wait_failed), sizeof(failed), hipMemcpyDeviceToHost, (hipStream_t)stream));
     RK_HIP(hipStreamSynchronize((hipStream_t)stream));
-    return failed != 0u ? RK_ERR_WAIT : RK_SUCCESS;
+    return RK_SUCCESS;
 }
 
 extern "C" int32_t rk_sort(rk_dtype dt, void* keys, int64_t n, int32_t rev, void* tmp, size_t tmp_bytes, void* stream) {
-    return sort_dispatch(dt, keys, nullptr, n, rev, tmp, tmp_bytes, stream);
+    return sort_dispatch<false>(dt, keys, nullptr, n, rev, tmp, tmp_bytes, stream);
 }
 
 extern "C" int32_t rk_sortperm(rk_dtype dt, const void* keys, int64_t* perm_out, int64_t n, int32_t rev, void* tmp, size_t tmp_bytes,
                                void* stream) {
     if (n > 0 && perm_out == nullptr) return RK_ERR_INVALID_ARGUMENT;
-    return sort_dispatch(dt, (void*)keys, perm_out, n, rev, tmp, tmp_bytes, stream);
+    return sort_dispatch<true>(dt, (void*)keys, perm_out, n, rev, tmp, tmp_bytes, stream);
 }

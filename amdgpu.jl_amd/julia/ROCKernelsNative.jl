@@ -84,28 +84,19 @@ function workspace(minbytes::Integer = 0)
 end
 
 # ---- give-ups of bounded waits ---------------------------------------------------------------------------------
-# The scans across rows, the scan of 8-byte / unaligned lines and sorts of up to 2^20 keys wait on other workgroups with
-# a budget; a kernel that runs out of it records that in the workspace (the sort: in its temporary) and finishes with
-# meaningless results.  The records are read where the host waits for the device anyway -- Array(x), a scalar fetch --
-# for every workspace and sort temporary such a kernel has used on the task's stream since the last look; a give-up
-# prepares the workspace again and throws.  (The single-pass scan of long lines and findall never give up.)
+# The scans across rows and the scan of 8-byte / unaligned lines wait on other workgroups with a budget; a kernel that
+# runs out of it records that in the workspace and finishes with meaningless results.  The record is read where the host
+# waits for the device anyway -- Array(x), a scalar fetch -- when such a kernel has used the workspace of the task's stream
+# since the last look; a give-up prepares the workspace again and throws.  (The single-pass scan of long lines and findall never give up.)
 const waiting = Set{Tuple{Int,Ptr{Cvoid}}}()                                  # streams whose workspace a waiting kernel has used
-const sort_tmps = Dict{Tuple{Int,Ptr{Cvoid}},Vector{ROCArray{UInt8,1}}}()     # temporaries of small sorts, record unread
 note_waiting_call() = lock(() -> push!(waiting, (AMDGPU.device_id(AMDGPU.device()), stream_ptr())), workspaces_lock)
-function note_sort(tmp::ROCArray{UInt8,1}, n::Integer)
-    n > (1 << 20) && return AMDGPU.unsafe_free!(tmp)       # large sorts count before every pass and wait for nobody
-    key = (AMDGPU.device_id(AMDGPU.device()), stream_ptr())
-    pending = lock(() -> push!(get!(sort_tmps, key, ROCArray{UInt8,1}[]), tmp), workspaces_lock)
-    length(pending) > 16 && check_waits()                  # a long run of sorts without a fetch: read rather than hoard
-    return nothing
-end
 function check_waits()
     key = (AMDGPU.device_id(AMDGPU.device()), stream_ptr())
     failed = false
-    ws, tmps = lock(workspaces_lock) do
+    ws = lock(workspaces_lock) do
         w = key in waiting ? get(workspaces, key, nothing) : nothing
         delete!(waiting, key)
-        (w, pop!(sort_tmps, key, ROCArray{UInt8,1}[]))
+        w
     end
     if ws !== nothing
         st = ccall((:rk_workspace_status, librk[]), Int32, (Ptr{Cvoid}, Csize_t, Ptr{Cvoid}), pointer(ws), length(ws), stream_ptr())
@@ -115,11 +106,6 @@ function check_waits()
         else
             check(st)
         end
-    end
-    for tmp in tmps
-        st = ccall((:rk_sort_status, librk[]), Int32, (Ptr{Cvoid}, Csize_t, Ptr{Cvoid}), pointer(tmp), sizeof(tmp), stream_ptr())
-        AMDGPU.unsafe_free!(tmp)
-        st == RK_ERR_WAIT ? (failed = true) : check(st)
     end
     failed && throw(RKError(RK_ERR_WAIT))
     return nothing
@@ -689,7 +675,7 @@ function enable_sort!()
             st = ccall((:rk_sort, librk[]), Int32, (Cint, Ptr{Cvoid}, Int64, Int32, Ptr{Cvoid}, Csize_t, Ptr{Cvoid}),
                        rk_dtype(T), pointer(x), n, rev, pointer(tmp), sizeof(tmp), stream_ptr())
         end
-        note_sort(tmp, n)                                           # freed at once, or kept until its record has been read
+        AMDGPU.unsafe_free!(tmp)                                    # stream-ordered
         declined(st) && return (AMDGPU.AK.sort!(x; rev); x)          # rk_sort validates before it writes
         check(st)
         return x
@@ -711,7 +697,7 @@ function enable_sort!()
             st = ccall((:rk_sortperm, librk[]), Int32, (Cint, Ptr{Cvoid}, Ptr{Int64}, Int64, Int32, Ptr{Cvoid}, Csize_t, Ptr{Cvoid}),
                        rk_dtype(T), pointer(x), pointer(ix), n, rev, pointer(tmp), sizeof(tmp), stream_ptr())
         end
-        note_sort(tmp, n)
+        AMDGPU.unsafe_free!(tmp)
         declined(st) && return (AMDGPU.AK.sortperm!(ix, x; rev); ix)
         check(st)
         return ix

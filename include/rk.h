@@ -114,8 +114,8 @@ RK_API size_t  rk_workspace_bytes(rk_opkind kind, rk_dtype dt, int ndim, const i
  * Call once per allocation, before its first use. */
 RK_API int32_t rk_workspace_init(void* ws, size_t ws_bytes, void* stream);
 
-/* Bounded waits.  The single-pass scan, the one-pass findall and the sort hand values from
- * workgroup to workgroup through the workspace (the sort: through its temporary); the
+/* Bounded waits.  The single-pass scan and the one-pass findall hand values from
+ * workgroup to workgroup through the workspace; the
  * receiving side polls.  With a prepared workspace used by one call at a time such a wait
  * ends within microseconds.  A workspace that was never prepared, or that two calls use at
  * the same time, could make it wait for ever -- a hung GPU -- so every wait counts its
@@ -132,8 +132,8 @@ RK_API int32_t rk_workspace_init(void* ws, size_t ws_bytes, void* stream);
  *   rk_workspace_status  SYNCHRONISES `stream`, then returns RK_ERR_WAIT if any call on the
  *                        workspace gave up a wait since it was last prepared, else
  *                        RK_SUCCESS.  After RK_ERR_WAIT call rk_workspace_init again.
- *   rk_sort_status       the same for the temporary of rk_sort / rk_sortperm (no
- *                        preparation needed afterwards: every sort clears its temporary).
+ *   rk_sort_status       the same for the temporary of rk_sort / rk_sortperm.  No kernel of
+ *                        the sort waits for another workgroup: RK_SUCCESS.
  *   rk_accumulate_static_status   the same for the library's own array behind
  *                        rk_accumulate_static on the current device; after RK_ERR_WAIT the
  *                        array has been prepared again before the call returns. */

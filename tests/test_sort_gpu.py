@@ -106,6 +106,30 @@ def test_full_size_sort(rk, orc):
     assert np.array_equal(p, orc.sortperm(k, True))
 
 
+@pytest.mark.parametrize("tiles", [1, 2, 7, 8, 9, 127, 128, 129, 255, 256, 257])
+@pytest.mark.parametrize("dtype", [np.int16, np.float32, np.int64])
+def test_table_of_counts_edges(rk, orc, dtype, tiles):
+    # up to 256 tiles of 4096 keys every workgroup sums the columns of the table of counts itself (8 groups of rows, 16 rows
+    # a round): one key more and less than whole tiles around the edges of the groups and of the dispatch
+    rng = np.random.default_rng(tiles)
+    for n in (tiles * 4096 - 1, tiles * 4096, tiles * 4096 + 1):
+        x = _rand(rng, dtype, n)
+        assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(x))), orc.sort(x))
+        assert np.array_equal(rk.Array(rk.sortperm(rk.ROCArray(x), rev=True)), orc.sortperm(x, True))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+def test_constant_digits(rk, orc, dtype):
+    # digits in which no two keys differ are skipped: low ones (whole numbers as floats, multiples of 65536), high ones, a
+    # middle one that only relative keys carry into, none at all
+    rng = np.random.default_rng(17)
+    for n in (50_000, 300_000):
+        _check(rk, orc, rng.integers(-500, 500, n).astype(dtype))
+        _check(rk, orc, (rng.integers(-500, 500, n) * 65536).astype(dtype))
+        _check(rk, orc, (rng.integers(0, 2, n) * (1 << 24) + 255).astype(dtype))
+        _check(rk, orc, np.full(n, 3, dtype=dtype))
+
+
 # More than 256 tiles of 4096 keys: the sort counts the digits of every tile before each pass (no look-back).
 LARGE = 1024 * 4096 + 4096 * 3 + 37
 
