@@ -920,6 +920,154 @@ __global__ __launch_bounds__(BLOCK) void bc_flat_kernel(const BcFlatArgs a) {
     store_nt((V*)a.dest + i, o);
 }
 
+// A matrix against row and column vectors (C .= A .+ r .* c), one element type, every array of it 16-byte aligned where it
+// is dense: the lean form of rows and indexed mode.  The general kernels fetch each operand's pointer, strides and type
+// through branches of their own and split the linear index by three divisions; here the arguments are one compact block,
+// a wave takes 64 vectors of the destination's linear order as in bc_flat_kernel, and the column of a lane comes from one
+// multiplication.  Bound by memory: C .= A .+ r .* c back to back, indexed mode -> here, 8191 x 4099 Float32 56.1 -> 46.5 us
+// (5.8 TB/s), 4097 x 4099 Float64 55.1 -> 46.1, 1001 x 33521 54.2 -> 46.8, 65537 x 511 53.9 -> 45.7; C .= A .- r 46.3 -> 43.2,
+// 48.7 -> 44.3, 46.3 -> 42.7, 46.1 -> 43.6.  Workgroups of 256 threads: 45.3 and 43.7 us at 8191 x 4099, 46.4 and 44.7 for
+// 8192 x 4096 (64: 45.2 and 42.8).
+struct BcMatArgs {
+    uint32_t    total, rows;
+    uint32_t    recip;                      // floor(2^32 / rows)
+    void*       dest;
+    const void* ptr[4];
+    uint64_t    scalar[4];                  // bits of the value in the compute type
+    int64_t     col_step[4];                // BC_MAT_ROW: elements from one column's value to the next
+    int32_t     kind[4];
+    int32_t     n_operands, n_tokens;
+    int32_t     tokens[RK_MAX_PROGRAM];
+    int32_t     post;                       // always 0: homogeneous programs round nowhere
+};
+enum { BC_MAT_SCALAR, BC_MAT_DENSE, BC_MAT_ROW, BC_MAT_COLUMN };   // ROW: one value a column of the matrix; COLUMN: one a row
+
+template <typename Eval, typename CT, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void bc_matrix_kernel(const BcMatArgs a) {
+    constexpr int FV = 16 / sizeof(CT);
+    typedef typename VecOf<CT, FV>::type V;
+    const uint32_t e0 = (blockIdx.x * BLOCK + threadIdx.x) * (uint32_t)FV;      // total < 2^31
+    if (e0 >= a.total) return;
+    // the estimate is at most one too small for any 32-bit dividend
+    uint32_t col = __umulhi(e0, a.recip), row = e0 - col * a.rows;
+    if (row >= a.rows) { ++col; row -= a.rows; }
+    if (a.total - e0 < (uint32_t)FV) {           // the last lane of a ragged total: element by element
+        for (uint32_t e = e0; e < a.total; ++e) {
+            CT in[RK_MAX_OPERANDS][1], out[1];
+#pragma unroll
+            for (int k = 0; k < Eval::NOPS; ++k) {
+                if (k >= a.n_operands) continue;
+                const CT* p = (const CT*)a.ptr[k];
+                if (a.kind[k] == BC_MAT_SCALAR) __builtin_memcpy(&in[k][0], &a.scalar[k], sizeof(CT));
+                else in[k][0] = p[a.kind[k] == BC_MAT_DENSE ? (int64_t)e : a.kind[k] == BC_MAT_ROW ? col * a.col_step[k] : (int64_t)row];
+            }
+            Eval::template run<CT, 1>(a, in, out, (CT*)nullptr);
+            ((CT*)a.dest)[e] = out[0];
+            if (++row == a.rows) { row = 0; ++col; }
+        }
+        return;
+    }
+    // lanes whose vector ends in the next column (columns hold at least one vector, so it meets one column end at most)
+    const uint32_t left = a.rows - row;          // elements of this column from the first one on
+    const bool crosses = left < (uint32_t)FV;
+    const bool any_crosses = __ballot(crosses) != 0ull;
+    CT in[RK_MAX_OPERANDS][FV];
+#pragma unroll
+    for (int k = 0; k < Eval::NOPS; ++k) {
+        if (k >= a.n_operands) continue;
+        const CT* p = (const CT*)a.ptr[k];
+        if (a.kind[k] == BC_MAT_DENSE) {
+            const V x = load_nt((const V*)(p + e0));
+#pragma unroll
+            for (int j = 0; j < FV; ++j) in[k][j] = x[j];
+        } else if (a.kind[k] == BC_MAT_ROW) {
+            const CT x = p[col * a.col_step[k]];
+#pragma unroll
+            for (int j = 0; j < FV; ++j) in[k][j] = x;
+            if (any_crosses) {
+                const CT y = p[(crosses ? col + 1u : col) * a.col_step[k]];
+#pragma unroll
+                for (int j = 1; j < FV; ++j) in[k][j] = (uint32_t)j < left ? x : y;
+            }
+        } else if (a.kind[k] == BC_MAT_COLUMN) {
+            if (!any_crosses) {
+                const V x = load_elems<CT, FV>(p + row);
+#pragma unroll
+                for (int j = 0; j < FV; ++j) in[k][j] = x[j];
+            } else {
+                // the column's last FV elements (or those from `row` on), then the head of the next column
+                const uint32_t start = crosses ? a.rows - (uint32_t)FV : row, d = row - start;
+                const V x = load_elems<CT, FV>(p + start), y = load_elems<CT, FV>(p);
+#pragma unroll
+                for (int j = 0; j < FV; ++j) {
+                    CT v = x[j];
+#pragma unroll
+                    for (int s = 1; s < FV; ++s)
+                        if (d == (uint32_t)s) v = j + s < FV ? x[j + s < FV ? j + s : 0] : y[j + s >= FV ? j + s - FV : 0];
+                    in[k][j] = v;
+                }
+            }
+        } else {
+            CT x;
+            __builtin_memcpy(&x, &a.scalar[k], sizeof(CT));
+#pragma unroll
+            for (int j = 0; j < FV; ++j) in[k][j] = x;
+        }
+    }
+    CT out[FV];
+    Eval::template run<CT, FV>(a, in, out, (CT*)nullptr);
+    V o;
+#pragma unroll
+    for (int j = 0; j < FV; ++j) o[j] = out[j];
+    store_nt((V*)((CT*)a.dest + e0), o);
+}
+
+// Fills `f` when bc_matrix_kernel takes the call: two merged dims, dense destination, and every operand a scalar, dense,
+// one value a column or one value a row.
+// Columns that are no whole number of vectors: at least 32 vectors long, so that a wave meets three column ends at most.
+// Shorter ones stay with indexed mode, whose two loads per vector are unconditional (C .= A .- r, indexed mode against
+// this kernel: 5 x 6710886 Float32 49.6 against 54.0 us, 17 x 1973790 47.5 / 52.0, 33 x 1016801 Float64 96.6 / 108.6; the
+// other way round at 100 x 335544 Float32: 51.7 / 43.0, C .= A .+ r .* c 53.7 / 46.5).
+// Columns of whole vectors never split a vector, however short: 4-byte types leave rows mode (16 x 2097152 Float32 48.3 ->
+// 43.7 us, 8192 x 4096 45.1 -> 42.8, C .= A .+ r .* c 48.0 -> 46.3 and 45.1 -> 45.2); 8-byte types stay (4096^2 Float64:
+// C .= A .+ r .* c 44.5 against 45.2 us here, C .= A .- r 45.0 against 44.3).
+template <typename CT>
+static bool bc_matrix_args(const BcArgs& a, BcMatArgs& f) {
+    constexpr int FV = 16 / sizeof(CT);
+    if (a.ndim != 2 || a.n_operands > 4 || a.post != 0) return false;
+    if (a.total >= (1ll << 31)) return false;
+    if (a.indexed != 0 ? a.shape[0] < 32 * FV : sizeof(CT) != 4) return false;
+    if (a.dest_stride0 != 1 || a.dest_stride[0] != a.shape[0] || !is_aligned(a.dest, 16)) return false;
+    std::memset(&f, 0, sizeof(f));
+    for (int k = 0; k < a.n_operands; ++k) {
+        const BcOperand& o = a.op[k];
+        f.ptr[k] = o.ptr;
+        if (o.ptr == nullptr) {
+            const CT x = (o.dtype == RK_F32 || o.dtype == RK_F64 || o.dtype == RK_F16) ? (CT)o.sf : (CT)o.si;
+            std::memcpy(&f.scalar[k], &x, sizeof(CT));
+            f.kind[k] = BC_MAT_SCALAR;
+        } else if (o.stride0 == 1 && o.stride[0] == a.shape[0]) {
+            if (!is_aligned(o.ptr, 16)) return false;
+            f.kind[k] = BC_MAT_DENSE;
+        } else if (o.stride0 == 0) {
+            f.kind[k] = BC_MAT_ROW;
+            f.col_step[k] = o.stride[0];
+        } else if (o.stride0 == 1 && o.stride[0] == 0) {
+            f.kind[k] = BC_MAT_COLUMN;
+        } else {
+            return false;
+        }
+    }
+    f.total = (uint32_t)a.total;
+    f.rows = (uint32_t)a.shape[0];
+    f.recip = (uint32_t)((1ull << 32) / (uint64_t)a.shape[0]);
+    f.dest = a.dest;
+    f.n_operands = a.n_operands;
+    f.n_tokens = a.n_tokens;
+    for (int i = 0; i < a.n_tokens; ++i) f.tokens[i] = a.tokens[i];
+    return true;
+}
+
 static int tune_bc_narrow16() {
     const char* e = std::getenv("RK_BC_NARROW16");
     return e ? std::atoi(e) : 1;
@@ -1083,6 +1231,16 @@ static int32_t bc_launch(const BcArgs& a, bool vec, bool rows, hipStream_t strea
             const int64_t blocks = (f.nvec + FB - 1) / FB;
             if (blocks > 0x7fffffff) return RK_ERR_TOO_LARGE;
             bc_flat_kernel<Eval, CT, FB><<<(unsigned)blocks, FB, lds, stream>>>(f);
+            RK_LAUNCH_CHECK();
+            return RK_SUCCESS;
+        }
+    }
+    if constexpr (!Eval::USES_LDS && Eval::NOPS <= 4 && !EvalFlatOnly<Eval>::value) {
+        BcMatArgs f;
+        if (rows && vec && homog && bc_matrix_args<CT>(a, f)) {
+            constexpr uint32_t FV = 16 / (uint32_t)sizeof(CT);
+            const uint32_t nvec = (f.total + FV - 1) / FV;
+            bc_matrix_kernel<Eval, CT, BC_FLAT_BLOCK><<<(nvec + BC_FLAT_BLOCK - 1) / BC_FLAT_BLOCK, BC_FLAT_BLOCK, 0, stream>>>(f);
             RK_LAUNCH_CHECK();
             return RK_SUCCESS;
         }

@@ -470,3 +470,26 @@ def test_short_odd_first_dim(rk, shape, others):
     rk.materialize_(dest, L(dA) + np.float32(0))
     rk.materialize_(dest, L(dest) * L(dv) + L(du))
     np.testing.assert_array_equal(rk.Array(dest), A * v + u)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+@pytest.mark.parametrize("m,n", [(127, 5), (128, 3), (129, 4), (130, 3), (131, 5), (257, 33), (255, 1025), (63, 9), (65, 7),
+                                 (4, 1000), (8, 3), (1003, 2), (5001, 7)])
+def test_matrix_against_row_and_column(rk, dtype, m, n):
+    """Column lengths on both sides of the whole-vector and 32-vector lines, vectors that end in the next column at every
+    offset, ragged totals; every operand kind in every slot.  + - * on integer-valued data: exact in every type."""
+    rng = _rng(m * 7919 + n)
+    u = lambda *s: rng.integers(-50, 51, s).astype(dtype)
+    A, B, r, c, s = u(m, n), u(m, n), u(1, n), u(m, 1), dtype(3)
+    dA, dB, dr, dc = (rk.ROCArray(v) for v in (A, B, r, c))
+    L = rk.lazy
+    for got, want in ((rk.materialize(L(dA) + L(dr) * L(dc)), A + r * c),
+                      (rk.materialize(L(dr) + L(dA) * L(dc)), r + A * c),
+                      (rk.materialize(L(dA) - L(dr)), A - r),
+                      (rk.materialize(L(dc) - L(dA)), c - A),
+                      (rk.materialize(L(dr) * L(dc)), r * c),
+                      (rk.materialize((L(dA) - L(dr)) * s), (A - r) * s),
+                      (rk.materialize(L(dA) * L(dc) + L(dB)), A * c + B)):
+        assert np.array_equal(rk.Array(got), want)
+    out = rk.materialize_(dA, L(dA) + L(dr) * L(dc))           # in place
+    assert out is dA and np.array_equal(rk.Array(dA), A + r * c)
