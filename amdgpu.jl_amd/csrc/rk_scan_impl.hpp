@@ -1725,12 +1725,42 @@ __device__ __forceinline__ void rows_lookback(const T (&tot)[VEC], T (&base)[VEC
     }
 }
 
+// How scan_rows_ordered_kernel cuts a row into column strips: `lanes` vectors each, and with per_xcd != 0 the strips of an
+// XCD (chains are dealt to the XCDs round-robin) are neighbours.
+struct RowStrips {
+    int64_t strips;
+    int     lanes;
+    int64_t per_xcd;
+};
+// Rows of whole 128-byte lines: strips of a whole wave, in order (4096 x 16000 Float32 96.4 us; with neighbours on one XCD
+// 97.7).  Other rows: two strips share the line at their common edge, which two XCDs fetch and write in part each; with
+// neighbours on one XCD its L2 joins them (8191 x 8001 111.7 -> 106.4 us, 6001 x 10922 116.7 -> 112.5).  That needs a
+// multiple of 8 strips, which also makes the launch order safe (rows_chains_stay_on_their_xcd) and so does without the
+// tile counter: narrower strips are worth it as long as 42 of the 64 lanes work (4097 x 16000, 24 strips of 43 lanes
+// instead of 17: 119.7 -> 114.6; 3001 x 21800, 47 lanes: 124.8 -> 119.1; 20001 x 3200, 63 lanes: 116.7 -> 109.3; 2561 x
+// 25600, 41 lanes: 125.2 and 124.9; 1279 x 51200, 40 lanes: 127.9 -> 133.6).
+constexpr int ROWS_MIN_LANES = 42;
+inline RowStrips row_strips(int64_t inner, size_t esz, int vec, bool may_narrow) {
+    const int64_t cols = (int64_t)WAVE * vec;
+    RowStrips rs{(inner + cols - 1) / cols, WAVE, 0};
+    if (inner * (int64_t)esz % 128 == 0) return rs;
+    const int64_t even = (rs.strips + 7) / 8 * 8;
+    const int lanes = (int)((inner + even * vec - 1) / (even * vec));
+    if (rs.strips % 8 != 0) {
+        if (!may_narrow || lanes < ROWS_MIN_LANES) return rs;
+        rs.strips = even;
+        rs.lanes = lanes;
+    }
+    rs.per_xcd = rs.strips / 8;
+    return rs;
+}
+
 // NW waves hold rows; one more wave holds none and does the publishing and the look-back.  The registers a kernel
 // needs are the maximum over its branches, so the row data (32 registers) and the look-back's working set no longer
 // add up: 64 registers suffice and two workgroups share a compute unit (with wave 0 doing both, 25 registers spilled).
 template <typename In, typename T, typename Out, typename Op, int NW, int R>
 __global__ __launch_bounds__((NW + 1) * WAVE, 8) void scan_rows_ordered_kernel(const In* __restrict__ in, Out* __restrict__ out, ScanGeom g, T init,
-                                                                               int inclusive, Op op, int64_t strips, int64_t nchains,
+                                                                               int inclusive, Op op, RowStrips rs, int64_t nchains,
                                                                                int64_t nslices, T* payload, unsigned long long* counter,
                                                                                uint32_t* tickets, int ticket_group, uint64_t* desc,
                                                                                int64_t desc_capacity, WaitCtl wc, int dynamic_ids) {
@@ -1762,16 +1792,18 @@ __global__ __launch_bounds__((NW + 1) * WAVE, 8) void scan_rows_ordered_kernel(c
         for (int j = 0; j < VEC; ++j) lds_base[lane * VEC + j] = base[j];
         __syncthreads();
     } else {
-        const int64_t o = chain / strips, strip = chain - o * strips;
+        const int64_t o = chain / rs.strips, nth = chain - o * rs.strips;
+        const int64_t strip = rs.per_xcd != 0 ? (nth & 7) * rs.per_xcd + (nth >> 3) : nth;
+        const int64_t strip_col = strip * (rs.lanes * VEC);
         // rows that are no whole number of vectors: the last vector starts VEC elements before the row's end (see
         // scan_strided_kernel); payloads are per lane slot, the same columns in every tile of the strip
         constexpr bool ANY_ALIGN = sizeof(In) >= 4 && OutElemVectors<Out, T>::value;
-        const int64_t nominal = strip * COLS + (int64_t)lane * VEC;
-        const bool live = nominal < g.inner;
+        const int64_t nominal = strip_col + (int64_t)lane * VEC;
+        const bool live = lane < rs.lanes && nominal < g.inner;
         const int64_t col0 = (ANY_ALIGN && live && nominal + VEC > g.inner) ? g.inner - VEC : nominal;
         // wave-uniform row addresses + a 32-bit offset per lane (the rows of a wave are the same for all its lanes)
         const int64_t row0 = slice * (NW * R) + (int64_t)__builtin_amdgcn_readfirstlane(wave) * R;
-        const int64_t shift = strip * COLS >= VEC ? strip * COLS - VEC : 0;     // the first lane of a strip may reach back VEC columns
+        const int64_t shift = strip_col >= VEC ? strip_col - VEC : 0;           // the first lane of a strip may reach back VEC columns
         const int64_t wave_e0 = o * g.inner * g.mid + row0 * g.inner + shift;
         const unsigned loff = (unsigned)(col0 - shift);
         const int64_t left = g.mid - row0;
@@ -2012,12 +2044,17 @@ inline int32_t scan_across_rows(const In* in, Out* out, const ScanGeom& g, T ini
         // the payloads of all tiles and groups must fit the partials area.  8-byte values too: 2048 x 16384 Float64 103 us against 139
         // for the three passes, 4096 x 4096 Int64 54 against 70.
         constexpr int NW = 15, R = sizeof(In) >= 4 ? 10 : 8;     // 15 waves of rows + 1 for the look-back (Bool -> Int64 with ten rows: 20 registers spilled)
-        const int64_t nchains = strips * g.outer, nslices = (g.mid + NW * R - 1) / (NW * R), ntiles = nchains * nslices;
+        const int64_t nslices = (g.mid + NW * R - 1) / (NW * R);
+        auto needs = [&](int64_t chains) { return chains * (nslices + 2 * ((nslices + ROWS_GROUP - 1) / ROWS_GROUP)) * cols * (int64_t)sizeof(T); };
+        // (1- and 2-byte elements, whose vectors have to be aligned, keep strips of a whole wave in order)
+        RowStrips rs = sizeof(In) >= 4 ? row_strips(g.inner, sizeof(In), VEC, true) : RowStrips{strips, WAVE, 0};
+        if (sizeof(In) >= 4 && (rs.strips * g.outer >= cus * 4 || needs(rs.strips * g.outer) > (int64_t)scratch_bytes)) rs = row_strips(g.inner, sizeof(In), VEC, false);
+        const int64_t nchains = rs.strips * g.outer, ntiles = nchains * nslices;
         const int64_t ngroups = (nslices + ROWS_GROUP - 1) / ROWS_GROUP * nchains;
         if (vec && ws != nullptr && tune_scan_rows_ordered() != 0 && nchains < cus * 4 && nslices >= 4 &&
             (size_t)((ntiles + 2 * ngroups) * cols) * sizeof(T) <= scratch_bytes && (size_t)(ntiles + ngroups) * sizeof(uint64_t) <= ws->desc_bytes) {
             scan_rows_ordered_kernel<In, T, Out, Op, NW, R><<<(unsigned)ntiles, (NW + 1) * WAVE, 0, stream>>>(
-                in, out, g, init, inclusive, op, strips, nchains, nslices, (T*)scratch, (unsigned long long*)&ws->hdr->scan_counter,
+                in, out, g, init, inclusive, op, rs, nchains, nslices, (T*)scratch, (unsigned long long*)&ws->hdr->scan_counter,
                 ws->tickets, ordered_ticket_group(ntiles), ws->desc, (int64_t)(ws->desc_bytes / sizeof(uint64_t)), wait_ctl(ws->hdr),
                 ordered_dynamic_ids(ntiles, (NW + 1) * WAVE, rows_chains_stay_on_their_xcd(nchains)));
             RK_LAUNCH_CHECK();

@@ -463,6 +463,26 @@ def test_scans_across_rows_that_are_no_whole_vectors(rk, orc, shape):
             assert np.array_equal(rk.Array(dx), want.astype(dtype))
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64, np.float32])
+@pytest.mark.parametrize("vectors", [328, 336, 337, 512, 513, 1009, 2050])
+@pytest.mark.parametrize("extra,outer", [(0, 1), (1, 1), (1, 3)])
+def test_strips_of_rows_that_are_no_whole_lines(rk, orc, dtype, vectors, extra, outer):
+    """cumsum(A; dims=2) by tiles of rows: rows of whole 128-byte lines keep strips of 64 vectors in order; other rows are
+    cut into a multiple of 8 strips (narrower ones where at least 42 lanes of 64 work: up to 328 vectors
+    are 41 lanes in 8 strips, 329 .. 336 are 42), neighbours on one XCD.  Whole vectors and one element more.  Integer-valued: exact."""
+    dt = np.dtype(dtype)
+    inner, mid = vectors * (16 // dt.itemsize) + extra, 601 + 149 * outer
+    x = np.random.default_rng(vectors + outer).integers(-9, 10, (inner, mid, outer)).astype(dtype)
+    d = rk.ROCArray(x)
+    want = np.cumsum(x, axis=1, dtype=np.int64).astype(dtype)
+    assert np.array_equal(rk.Array(rk.cumsum(d, dims=2)), want)
+    got = rk.Array(rk.accumulate("add", d, dims=2, init=dt.type(4), inclusive=False))
+    assert np.array_equal(got, want - x + dt.type(4))
+    if extra == 0:
+        rk.accumulate_("add", d, d, dims=2)                             # in place
+        assert np.array_equal(rk.Array(d), want)
+
+
 @pytest.mark.parametrize("shape", [(100, 50_000), (65, 30_011), (128, 9_000), (95, 20_000, 2), (32, 100_001), (33, 40_000, 3), (16, 33_000, 5),
                                    (64, 2_000, 3), (31, 70_000), (128, 4_001), (48, 1921), (17, 200_000)])
 def test_short_rows_several_to_a_load(rk, orc, shape):
