@@ -125,6 +125,7 @@ PROTOTYPES = {
                                    C.c_void_p]),
     "rk_sort_tmp_bytes": (C.c_size_t, [C.c_int, C.c_int64, C.c_int32]),
     "rk_sort": (C.c_int32, [C.c_int, C.c_void_p, C.c_int64, C.c_int32, C.c_void_p, C.c_size_t, C.c_void_p]),
+    "rk_sort_to": (C.c_int32, [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_void_p, C.c_size_t, C.c_void_p]),
     "rk_sortperm": (C.c_int32, [C.c_int, C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_void_p, C.c_size_t, C.c_void_p]),
     "rk_permutedims": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, _I64P, C.POINTER(C.c_int32), C.c_void_p]),
     "rk_reverse": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, _I64P, C.c_uint32, C.c_void_p]),

@@ -680,6 +680,21 @@ function enable_sort!()
         check(st)
         return x
     end
+    @eval function Base.sort(x::ROCVector{T}; rev::Bool=false, lt=isless, by=identity, kwargs...) where {T<:SORTABLE}
+        flip = native_order(lt)
+        n = length(x)
+        (flip !== nothing && isempty(kwargs) && by === identity && n > 1) || return sort!(copy(x); rev, lt, by, kwargs...)
+        y = similar(x)
+        tmp = ROCVector{UInt8}(undef, ccall((:rk_sort_tmp_bytes, librk[]), Csize_t, (Cint, Int64, Int32), rk_dtype(T), n, 0))
+        GC.@preserve x y tmp begin
+            st = ccall((:rk_sort_to, librk[]), Int32, (Cint, Ptr{Cvoid}, Ptr{Cvoid}, Int64, Int32, Ptr{Cvoid}, Csize_t, Ptr{Cvoid}),
+                       rk_dtype(T), pointer(x), pointer(y), n, xor(rev, flip), pointer(tmp), sizeof(tmp), stream_ptr())
+        end
+        AMDGPU.unsafe_free!(tmp)
+        declined(st) && return sort!(copyto!(y, x); rev, lt)
+        check(st)
+        return y
+    end
     @eval function Base.sortperm!(ix::ROCVector{Int}, x::ROCVector{T}; rev::Bool=false, lt=isless, by=identity, kwargs...) where {T<:SORTABLE}
         flip = native_order(lt)
         (flip !== nothing && isempty(kwargs)) || return (AMDGPU.AK.sortperm!(ix, x; rev, lt, by, kwargs...); ix)

@@ -69,9 +69,17 @@ def sort_(x: ROCArray, *, rev: bool = False, lt=None, by=None) -> ROCArray:
 def sort(x: ROCArray, *, rev: bool = False, lt=None, by=None) -> ROCArray:
     """``sort(x; rev, lt, by)``: sorted copy."""
     rev = bool(rev) != _check(x, lt, by)
+    n = len(x)
+    if n <= 1:
+        return x.copy()
     if by is not None:
-        return _gather(x, sortperm(_keys(x, by), rev=rev)) if len(x) > 1 else x.copy()
-    return sort_(x.copy(), rev=rev)
+        return _gather(x, sortperm(_keys(x, by), rev=rev))
+    code = x.code                                # (an element type without a sort is refused before anything is allocated)
+    y = ROCArray(dims=x.dims, dtype=x.dtype)
+    tmp = _tmp(code, n, False)
+    L.check(L.lib.rk_sort_to(code, x.ptr, y.ptr, n, 1 if rev else 0, tmp.data_ptr(), tmp.numel(), stream_ptr()), "rk_sort_to")
+    tmp.record_stream(torch.cuda.current_stream())
+    return y
 
 
 def sortperm_(ix: ROCArray, x: ROCArray, *, rev: bool = False, lt=None, by=None) -> ROCArray:

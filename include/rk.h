@@ -425,6 +425,8 @@ RK_API int32_t rk_permutedims(const void* src, void* dst, size_t elsize, int ndi
  * themselves is by bit pattern).  Stable: sortperm keeps equal keys -- all NaNs count as equal --
  * in index order, also with rev != 0, like Base.
  *   rk_sort      sorts `keys` in place.
+ *   rk_sort_to   leaves `keys` untouched and writes the sorted keys to `out` (`sort(x)`): the same array or one that
+ *                shares no element with it (RK_ERR_INVALID_ARGUMENT otherwise).
  *   rk_sortperm  leaves `keys` untouched and writes the 1-based permutation (Int64) to
  *                `perm_out`; unlike `sortperm!(ix, x)` it does not read an initial `ix`
  *                (the reference always passes 1:n, src/kernels/sorting.jl:3).
@@ -433,6 +435,8 @@ RK_API int32_t rk_permutedims(const void* src, void* dst, size_t elsize, int ndi
 RK_API size_t  rk_sort_tmp_bytes(rk_dtype dt, int64_t n, int32_t with_perm);
 RK_API int32_t rk_sort(rk_dtype dt, void* keys, int64_t n, int32_t rev, void* tmp, size_t tmp_bytes,
                 void* stream);
+RK_API int32_t rk_sort_to(rk_dtype dt, const void* keys, void* out, int64_t n, int32_t rev, void* tmp,
+                          size_t tmp_bytes, void* stream);
 RK_API int32_t rk_sortperm(rk_dtype dt, const void* keys, int64_t* perm_out, int64_t n, int32_t rev,
                     void* tmp, size_t tmp_bytes, void* stream);
 

@@ -215,6 +215,11 @@ def test_volumerhs_and_scatter_validation(L):
     assert so(L.RK_F32, one, 10, 0, big, 16, None) == L.RK_ERR_WORKSPACE
     assert so(L.RK_F32, one, 1 << 31, 0, big, 1 << 40, None) == L.RK_ERR_TOO_LARGE
     assert so(L.RK_F32, None, 0, 0, None, 0, None) == L.RK_SUCCESS
+    to = L.lib.rk_sort_to
+    assert to(L.RK_F32, one, None, 10, 0, big, 1 << 30, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert to(L.RK_F32, one, C.c_void_p(0x1004), 10, 0, big, 1 << 30, None) == L.RK_ERR_INVALID_ARGUMENT     # overlaps the keys
+    assert to(L.RK_U8, one, big, 10, 0, big, 1 << 30, None) == L.RK_ERR_UNSUPPORTED
+    assert to(L.RK_F32, None, None, 0, 0, None, 0, None) == L.RK_SUCCESS
     assert sp(L.RK_I64, one, None, 10, 0, big, 1 << 30, None) == L.RK_ERR_INVALID_ARGUMENT
     n = 1 << 20
     assert tb(L.RK_F32, n, 0) >= 4 * n and tb(L.RK_F32, n, 1) >= 16 * n and tb(L.RK_F32, n, 0) < 5 * n

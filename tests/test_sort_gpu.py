@@ -170,6 +170,25 @@ def test_large_unaligned_view(rk, orc):
     assert np.array_equal(got[:3], x[:3]) and np.array_equal(got[LARGE + 6:], x[LARGE + 6:])
 
 
+@pytest.mark.parametrize("dtype", TYPES)
+@pytest.mark.parametrize("n", [2, 4097, (1 << 20) + 1, (1 << 20) + 8191 * 3])
+def test_sorted_copy_by_number_of_passes(rk, orc, dtype, n):
+    """sort(x) reads x in its first pass and writes another array: keys that differ in no digit (no pass runs: a copy), in
+    one, in an odd and an even number, and in all of them; x starts at an odd element and stays as it was."""
+    rng = np.random.default_rng(n)
+    dt = np.dtype(dtype)
+    whole = _rand(rng, dtype, n + 1)
+    cases = [np.full(n + 1, whole[0], dtype=dtype), whole]
+    if dt.kind == "i":
+        cases += [rng.integers(0, 1 << min(bits, 8 * dt.itemsize - 1), n + 1).astype(dtype) for bits in (8, 16, 24)]
+    for x in cases:
+        for rev in (False, True):
+            xd = rk.ROCArray(x)
+            got = rk.Array(rk.sort(xd.view_range(2, n + 1), rev=rev))
+            assert np.array_equal(got, orc.sort(x[1:], rev))
+            assert np.array_equal(rk.Array(xd), x)
+
+
 @pytest.mark.parametrize("dtype", [np.int16, np.float32, np.float64])
 def test_unaligned_views(rk, orc, dtype):
     # keys that start 1 .. 9 elements into a buffer: the vector body of the whole-array reads starts later
