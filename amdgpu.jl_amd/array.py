@@ -7,6 +7,8 @@ memory and the stream, nothing else: no torch kernel runs on the path.
 """
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import torch
 
@@ -30,14 +32,14 @@ def dtype_code(dt) -> int:
 
 
 def device() -> torch.device:
-    if not torch.cuda.is_available():
+    if not (torch.cuda.is_initialized() or torch.cuda.is_available()):
         raise RuntimeError("no GPU visible: ROCArray needs a HIP device (there is no CPU path)")
     return torch.device("cuda", torch.cuda.current_device())
 
 
 def stream_ptr() -> int:
     """The current (task-local, in the reference: src/tls.jl:71-86) stream as a hipStream_t."""
-    return int(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 class ROCArray:
@@ -56,7 +58,7 @@ class ROCArray:
             self.dims = tuple(int(d) for d in dims)
             self.dtype = np.dtype(dtype)
             self.offset = 0
-            nbytes = int(np.prod(self.dims, dtype=np.int64)) * self.dtype.itemsize
+            nbytes = math.prod(self.dims) * self.dtype.itemsize
             self.buf = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device())
             return
         host = np.asarray(data)
@@ -80,13 +82,13 @@ class ROCArray:
         return self.dims[d - 1] if d <= len(self.dims) else 1
 
     def __len__(self) -> int:
-        return int(np.prod(self.dims, dtype=np.int64))
+        return math.prod(self.dims)
 
     length = __len__
 
     @property
     def ptr(self) -> int:
-        return int(self.buf.data_ptr()) + self.offset
+        return self.buf.data_ptr() + self.offset
 
     @property
     def code(self) -> int:
@@ -124,7 +126,7 @@ class ROCArray:
     def reshape(self, *dims):
         if len(dims) == 1 and isinstance(dims[0], (tuple, list)):
             dims = tuple(dims[0])
-        if int(np.prod(dims, dtype=np.int64)) != len(self):
+        if math.prod(dims) != len(self):
             raise L.DimensionMismatch(L.RK_ERR_DIMENSION, "reshape")
         return ROCArray(buf=self.buf, dims=dims, dtype=self.dtype, offset=self.offset)
 
@@ -200,7 +202,7 @@ _staging: dict = {}            # (device, stream) -> pinned bytes for scalar fet
 _waiting: set = set()          # (device, stream) keys whose workspace has been handed to a kernel with bounded waits
 
 
-# Pinned host words that a kernel writes its scalar result to (the count behind x[mask]): the host reads them after the
+# Pinned host words that a kernel writes its scalar results to (the count behind x[mask], sum(x), findmax(x)): the host reads them after the
 # stream synchronisation it needs anyway, with no device-to-host copy in between.  A slot belongs to one call from take to
 # give, whatever thread or stream it runs on; the free list holds at most as many as calls have been in flight at once.
 _free_slots: list = []
@@ -219,6 +221,12 @@ def take_slot():
 def give_slot(slot) -> None:
     if len(_free_slots) < 64:
         _free_slots.append(slot)
+
+
+def await_slot() -> None:
+    """The host waits for the current stream, and with it for the words that its kernels write to a slot."""
+    check_waits()                           # the place to learn of a give-up
+    torch.cuda.current_stream().synchronize()
 
 
 def note_waiting_call() -> None:

@@ -11,7 +11,7 @@ import torch
 
 from . import _lib as L
 from .accumulate import accumulate
-from .array import ROCArray, check_waits, device, give_slot, note_waiting_call, stream_ptr, take_slot, workspace
+from .array import ROCArray, await_slot, device, give_slot, note_waiting_call, stream_ptr, take_slot, workspace
 from .mapreduce import count
 
 
@@ -71,8 +71,7 @@ def _select(x: ROCArray, mask: ROCArray) -> ROCArray:
     ws, ws_bytes = workspace()
     slot = take_slot()
     L.check(L.lib.rk_mask_count(mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes, st), "rk_mask_count")
-    check_waits()                           # the host waits here anyway: the place to learn of a give-up
-    torch.cuda.current_stream().synchronize()
+    await_slot()
     total = int(slot[1][:8].view(np.int64)[0])
     give_slot(slot)
     y = ROCArray(dims=(total,), dtype=x.dtype)

@@ -14,7 +14,8 @@ import ctypes as C
 import numpy as np
 
 from . import _lib as L
-from .array import ROCArray, dtype_code, stream_ptr, workspace
+from .array import ROCArray, await_slot, dtype_code, give_slot, stream_ptr, take_slot, workspace
+from .views import ROCView
 
 # f of mapreduce(f, op, A): enumerated, like the C ABI
 identity, abs2, abs_ = "identity", "abs2", "abs"
@@ -125,16 +126,24 @@ def mapreducedim_(f, op: str, R: ROCArray, A: ROCArray, init=None) -> ROCArray:
     return R
 
 
+def _dense_args(f, prog, op, A, R_code, R_ptr, init, R_dtype, mask):
+    """(foreign function, its name, arguments up to the stream) of a reduction of a dense array."""
+    ws, ws_bytes = workspace()
+    tail = (_OP[op], A.code, R_code, A.ptr, A.ndim, L.shape_array(A.dims), mask, R_ptr, _scalar_buffer(init, R_dtype), ws, ws_bytes)
+    if callable(f):
+        return L.lib.rk_mapreduce_program, "rk_mapreduce_program", (prog,) + tail
+    return L.lib.rk_mapreduce, "rk_mapreduce", (_MAP[f],) + tail
+
+
 def _launch_mapreducedim(f, op, R, A, init, mask):
     """Zero-argument callable that enqueues the reduction on the current stream."""
-    ws, ws_bytes = workspace()
-    ibuf = _scalar_buffer(init, R.dtype)
-    from .views import ROCView
     if isinstance(R, ROCView) or isinstance(A, ROCView):
         # wrapper arrays (transpose, PermutedDimsArray): rk_mapreduce_strided renumbers the dims; closures for f and
         # views with gaps are not native here
         if callable(f):
             raise L.UnsupportedError(L.RK_ERR_UNSUPPORTED, "a closure for f over a wrapper array: copy(view) first")
+        ws, ws_bytes = workspace()
+        ibuf = _scalar_buffer(init, R.dtype)
         rdims = tuple(R.dims) + (1,) * (A.ndim - R.ndim)
         rstr = (tuple(R.strides) if isinstance(R, ROCView) else _dense_strides(R.dims)) + (0,) * (A.ndim - R.ndim)
         astr = tuple(A.strides) if isinstance(A, ROCView) else _dense_strides(A.dims)
@@ -148,13 +157,8 @@ def _launch_mapreducedim(f, op, R, A, init, mask):
         def launch_strided():
             L.check(fn(*args, stream_ptr()), name)
         return launch_strided
-    if callable(f):
-        prog, _ = _map_program(f, A.dtype)
-        args = (prog, _OP[op], A.code, R.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, R.ptr, ibuf, ws, ws_bytes)
-        fn, name = L.lib.rk_mapreduce_program, "rk_mapreduce_program"
-    else:
-        args = (_MAP[f], _OP[op], A.code, R.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, R.ptr, ibuf, ws, ws_bytes)
-        fn, name = L.lib.rk_mapreduce, "rk_mapreduce"
+    prog = _map_program(f, A.dtype)[0] if callable(f) else None
+    fn, name, args = _dense_args(f, prog, op, A, R.code, R.ptr, init, R.dtype, mask)
 
     def launch():
         L.check(fn(*args, stream_ptr()), name)
@@ -182,9 +186,10 @@ def mapreduce(f, op: str, A: ROCArray, dims=None, init=None):
     traced into a program that the reduction kernels evaluate on the loaded values (one pass over A); the result
     eltype is ``promote_op(op, T, T)`` with T the eltype of ``f(x)``, as GPUArrays infers it."""
     mask = _dims_mask(dims, A.ndim)
+    prog = None
     if callable(f):
         try:
-            _, mapped = _map_program(f, A.dtype)
+            prog, mapped = _map_program(f, A.dtype)
         except L.UnsupportedError:
             # a closure the reduction kernels do not interpret (too long, pow or trigonometry, another array, a result
             # in another float type): map first -- one fused broadcast kernel -- then reduce the mapped array
@@ -203,11 +208,28 @@ def mapreduce(f, op: str, A: ROCArray, dims=None, init=None):
             return out_dt.type(neutral)
         R = ROCArray(np.full(_reduced_dims(A.dims, mask), neutral, dtype=out_dt))
         return R
-    rshape = (1,) * A.ndim if dims is None else _reduced_dims(A.dims, mask)
-    R = ROCArray(dims=rshape, dtype=out_dt)
-    mapreducedim_(f, op, R, A, init=init)
+    if isinstance(A, ROCView):
+        R = ROCArray(dims=(1,) * A.ndim if dims is None else _reduced_dims(A.dims, mask), dtype=out_dt)
+        mapreducedim_(f, op, R, A, init=init)
+        return R.item() if dims is None else R
+    # a dense array: R is reduced along exactly `dims` by construction, and f has been traced (once)
+    if prog is None and f not in _MAP:
+        raise L.UnsupportedError(L.RK_ERR_UNSUPPORTED, f"map {f!r}")
+    for d, n in enumerate(A.dims):
+        if n == 1:
+            mask &= ~(1 << d)                       # as mapreducedim! sees it: R has A's extent there
     if dims is None:
-        return R.item()
+        # the kernel writes the value to pinned host memory: no result array, no copy
+        slot = take_slot()
+        fn, name, args = _dense_args(f, prog, op, A, dtype_code(out_dt), slot[0], init, out_dt, mask)
+        L.check(fn(*args, stream_ptr()), name)
+        await_slot()
+        value = slot[1][:out_dt.itemsize].view(out_dt)[0].copy()
+        give_slot(slot)
+        return value
+    R = ROCArray(dims=_reduced_dims(A.dims, mask), dtype=out_dt)
+    fn, name, args = _dense_args(f, prog, op, A, R.code, R.ptr, init, out_dt, mask)
+    L.check(fn(*args, stream_ptr()), name)
     return R
 
 
@@ -336,12 +358,22 @@ def _findminmax(A, want_max: bool, dims):
     if len(A) == 0:
         raise ValueError("reducing over an empty collection is not allowed")
     mask = _dims_mask(dims, A.ndim)
+    if dims is None and not isinstance(A, ROCView):
+        # value and CartesianIndex go straight to pinned host memory: no result arrays, no copies
+        ws, ws_bytes = workspace()
+        slot = take_slot()
+        L.check(L.lib.rk_findminmax(1 if want_max else 0, A.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, slot[0],
+                                    slot[0] + 16, ws, ws_bytes, stream_ptr()), "rk_findminmax")
+        await_slot()
+        value = slot[1][:A.dtype.itemsize].view(A.dtype)[0].copy()
+        c = tuple(int(v) for v in slot[1][16:16 + 8 * A.ndim].view(np.int64))
+        give_slot(slot)
+        return value, (c[0] if A.ndim == 1 else c)
     rshape = (1,) * A.ndim if dims is None else _reduced_dims(A.dims, mask)
     vals = ROCArray(dims=rshape, dtype=A.dtype)
     # Array{CartesianIndex{N}}: N Int64 per element; kept as an Int64 array with a leading dim N
     idx = ROCArray(dims=(A.ndim,) + rshape, dtype=np.int64)
     ws, ws_bytes = workspace()
-    from .views import ROCView
     if isinstance(A, ROCView):
         # wrapper arrays (transpose, PermutedDimsArray): the index comes back in the wrapper's coordinates; orders of
         # dims for which the first of equal winners or the output layout would differ raise UnsupportedError

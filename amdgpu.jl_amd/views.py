@@ -6,6 +6,8 @@ triple; it can be an operand or the destination of a broadcast (``rk_broadcast_s
 Reductions, scans and the other dense kernels take dense arrays only: their ``ptr`` is what those ops read, and a view has none."""
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 from . import _lib as L
@@ -27,7 +29,7 @@ class ROCView:
         return len(self.dims)
 
     def __len__(self) -> int:
-        return int(np.prod(self.dims, dtype=np.int64))
+        return math.prod(self.dims)
 
     @property
     def code(self) -> int:
