@@ -4,7 +4,8 @@
 //   sort_init_kernel     clears the control block; no memset: graph-safe
 //   sort_range_kernel    one read of the keys: smallest and largest key (integers) and the bits that differ between keys;
 //                        the workgroup that finishes last decides which passes run (a digit that is the same in every key
-//                        needs none) and which buffer each of them reads
+//                        needs none) and which buffer each of them reads.  (Integers are taken relative to the smallest key;
+//                        small sorts can drop further passes when they have seen the relative keys: sort_refine_plan)
 // and for every pass
 //   sort_upsweep_kernel  the 256 digit counts of every tile (one more read of the keys, at streaming speed)
 //   sort_pass_kernel     a tile of 4096 keys ranks its keys by digit (wave-level match by ballots, counts in LDS), reorders
@@ -39,7 +40,10 @@ constexpr int SORT_BLOCK = 256;
 constexpr int SORT_MAX_PASSES = 8;
 
 struct SortCtl {                                  // head of the caller's temporary buffer
-    uint32_t hist[SORT_MAX_PASSES][256];          // large sorts: first output slot of every digit value (sort_tilescan_kernel)
+    union {
+        uint32_t hist[SORT_MAX_PASSES][256];      // large sorts: first output slot of every digit value (sort_tilescan_kernel)
+        unsigned long long tile_bits[256];        // small sorts of integers: bits set in any relative key of a tile (first pass)
+    };
     // everything from here on is cleared by sort_init_kernel
     uint32_t skip[SORT_MAX_PASSES];
     uint32_t src_is_b[SORT_MAX_PASSES];           // the pass reads buffer B (1) or A (0)
@@ -49,6 +53,7 @@ struct SortCtl {                                  // head of the caller's tempor
     unsigned long long inv_min;                   // ~(smallest mapped key), kept as a maximum so that zero is its identity
     unsigned long long key_max;                   // largest mapped key (integers: range = key_max - smallest)
     unsigned long long varying;                   // bits that are not the same in all mapped keys
+    uint32_t refine, unused;                      // integers: a digit below the highest may be zero in every relative key
 };
 constexpr int SORT_CTL_CLEAR = (int)((sizeof(SortCtl) - offsetof(SortCtl, skip)) / sizeof(uint32_t));
 
@@ -128,8 +133,8 @@ template <> struct SortKey<double> {
 // `rev` here is a set of flags: bit 0 = descending order, bit 1 = keep NaN bit patterns (SORT_KEEP_NAN).
 constexpr int SORT_REV = 1, SORT_KEEP_NAN = 2;
 // the same mapping on the raw bit pattern: one load path serves the first pass (caller's keys) and the later ones
-// and relative to the smallest mapped key of the array: small-range integers (and floats of one binade) then have
-// constant high digits, whose passes are skipped
+// and, for integers, relative to the smallest mapped key of the array: small-range integers then have constant high digits,
+// whose passes are skipped
 template <typename T> __device__ __forceinline__ typename SortKey<T>::U enc_bits(typename SortKey<T>::U raw, int rev, typename SortKey<T>::U umin) {
     typedef typename SortKey<T>::U U;
     const U u = SortKey<T>::enc(__builtin_bit_cast(T, raw), (rev & SORT_KEEP_NAN) != 0);
@@ -184,10 +189,12 @@ __device__ __forceinline__ bool digits_skewed(uint32_t d, bool valid) {
 }
 // ---- plan: which passes run and what they read --------------------------------------------------------------------
 // relative: keys are taken relative to the smallest one (integers), so digits above their range are zero in every key, and
-// so are low digits in which the keys do not differ.  Otherwise (floats) a digit in which no two keys differ is skipped:
-// their exponent bytes are constant or not whatever is subtracted.
+// so are low digits in which the keys do not differ.  (Digits between them that are zero in every relative key show only once
+// the smallest key is known, and `sampled`, the bits of some relative keys, rules most of them out: sort_refine_plan.)
+// Otherwise (floats) a digit in which no two keys differ is skipped: their exponent bytes are constant or not whatever is
+// subtracted.
 __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool relative, unsigned long long range, unsigned long long varying,
-                                               int first_reads_b) {
+                                               unsigned long long sampled, int first_reads_b) {
     uint32_t src_b = first_reads_b ? 1u : 0u, nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
     for (int p = 0; p < passes; ++p) {
         const unsigned long long upto = p == 7 ? ~0ull : (1ull << (8 * (p + 1))) - 1ull;
@@ -197,12 +204,44 @@ __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool re
         ctl->src_is_b[p] = src_b;
         src_b ^= 1u;
         if (first == 0xffffffffu) first = (uint32_t)p;
+        else if (relative && (range >> (8 * p)) > 0xffull && ((sampled >> (8 * p)) & 0xffull) == 0ull) ctl->refine = 1u;
         last = (uint32_t)p;
         ++nexec;
     }
     ctl->first_pass = first;
     ctl->last_pass = last;
     ctl->nexec = nexec;
+}
+
+// Small sorts of integers, in their first pass: `bits` are those set in any relative key, and of the passes that are left only
+// those run whose digit has one: keys with an id in the upper half and a small number in the lower one are constant in the
+// digits between.  The last pass stays what it is -- the largest relative key has a bit in the highest digit of the range.
+// sort and sortperm of Int64[1000003], by the range alone -> so: (id << 32) + small number 105 -> 90 and 107 -> 74 us, only the
+// lowest and the highest byte varying 118 -> 66 and 123 -> 67.  Keys that differ in every digit are told by 64 of them
+// (sort_range_kernel) and do without: 137.0 and 137.7, 138.1 and 138.5.
+__device__ __forceinline__ void sort_refine_plan(SortCtl* ctl, int first, bool first_reads_b, int passes, unsigned long long bits) {
+    uint32_t src_b = first_reads_b ? 0u : 1u, nexec = 1;
+    for (int p = first + 1; p < passes; ++p) {
+        const bool skip = ((bits >> (8 * p)) & 0xffull) == 0ull;
+        ctl->skip[p] = skip ? 1u : 0u;
+        if (skip) continue;
+        ctl->src_is_b[p] = src_b;
+        src_b ^= 1u;
+        ++nexec;
+    }
+    ctl->nexec = nexec;
+}
+
+// What the plan says about one pass.  All words are asked for together: read where they are used, each waits for the branch
+// that the one before decides, round trips to memory in front of the keys (sortperm(Int64[1000003]) 138.6 against 136.6 us).
+struct SortStep {
+    uint32_t skip, src_b, first_pass, last_pass, refine;
+    unsigned long long inv_min;
+};
+__device__ __forceinline__ SortStep sort_step(const SortCtl* ctl, int pass) {
+    SortStep s{ctl->skip[pass], ctl->src_is_b[pass], ctl->first_pass, ctl->last_pass, ctl->refine, ctl->inv_min};
+    asm volatile("" : "+s"(s.skip), "+s"(s.src_b), "+s"(s.first_pass), "+s"(s.last_pass), "+s"(s.refine), "+s"(s.inv_min));
+    return s;
 }
 
 // ---- init: clear the control block ----------------------------------------------------------------------------------
@@ -214,7 +253,7 @@ __global__ __launch_bounds__(256) void sort_init_kernel(SortCtl* ctl, int all_pa
     __syncthreads();
     if (threadIdx.x == 0) {
         ctl->inv_min = ~0ull;
-        sort_make_plan(ctl, all_passes, false, 0ull, ~0ull, first_reads_b);
+        sort_make_plan(ctl, all_passes, false, 0ull, ~0ull, 0ull, first_reads_b);
     }
 }
 
@@ -272,6 +311,8 @@ __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __rest
     constexpr bool RELATIVE = std::is_integral<T>::value;
     __shared__ W part[3][RANGE_BLOCK / WAVE];
     const U u0 = enc_bits<T>(__builtin_bit_cast(U, keys[0]), rev, (U)0);
+    U sample = (U)0;                                         // 64 keys, evenly spread
+    if (RELATIVE && threadIdx.x < WAVE) sample = enc_bits<T>(__builtin_bit_cast(U, keys[(n - 1) * threadIdx.x / (WAVE - 1)]), rev, (U)0);
     U mn = u0, mx = u0, var = 0;
     for_each_key<T>(keys, n, head, nvec, [&](const U (&k)[VEC], int cnt) {
 #pragma unroll
@@ -286,22 +327,29 @@ __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __rest
     W inv = wave_reduce((W)(U)~mn, OpMax()), top = wave_reduce((W)mx, OpMax()), dif = wave_reduce((W)var, OpOr());
     if (lane_id() == 0) { part[0][threadIdx.x / WAVE] = inv; part[1][threadIdx.x / WAVE] = top; part[2][threadIdx.x / WAVE] = dif; }
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int w = 1; w < RANGE_BLOCK / WAVE; ++w) {
-        inv = part[0][w] > inv ? part[0][w] : inv;
-        top = part[1][w] > top ? part[1][w] : top;
-        dif |= part[2][w];
+    if (threadIdx.x >= WAVE) return;
+    int finishes_last = 0;
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < RANGE_BLOCK / WAVE; ++w) {
+            inv = part[0][w] > inv ? part[0][w] : inv;
+            top = part[1][w] > top ? part[1][w] : top;
+            dif |= part[2][w];
+        }
+        if (RELATIVE) {
+            if (inv != 0ull) atomicMax(&ctl->inv_min, inv);
+            if (top != 0ull) atomicMax(&ctl->key_max, top);
+        }
+        if (dif != 0ull) atomicOr(&ctl->varying, dif);
+        publish_barrier();
+        finishes_last = atomicAdd(&ctl->range_ticket, 1u) == gridDim.x - 1u;
+        if (!RELATIVE && finishes_last) ctl->inv_min = ~0ull;       // the smallest key is taken as 0
     }
-    if (RELATIVE) {
-        if (inv != 0ull) atomicMax(&ctl->inv_min, inv);
-        if (top != 0ull) atomicMax(&ctl->key_max, top);
-    }
-    if (dif != 0ull) atomicOr(&ctl->varying, dif);
-    publish_barrier();
-    if (atomicAdd(&ctl->range_ticket, 1u) != gridDim.x - 1u) return;
-    if (!RELATIVE) ctl->inv_min = ~0ull;                     // the smallest key is taken as 0
-    const W smallest = (W)(U)~(U)load_agent(&ctl->inv_min);
-    sort_make_plan(ctl, (int)sizeof(T), RELATIVE, RELATIVE ? load_agent(&ctl->key_max) - smallest : 0ull, load_agent(&ctl->varying), first_reads_b);
+    if (__builtin_amdgcn_readfirstlane(finishes_last) == 0) return;
+    const U smallest = (U)~(U)load_agent(&ctl->inv_min);
+    const W sampled = RELATIVE ? wave_reduce((W)(U)(sample - smallest), OpOr()) : 0ull;
+    if (threadIdx.x == 0)
+        sort_make_plan(ctl, (int)sizeof(T), RELATIVE, RELATIVE ? load_agent(&ctl->key_max) - (W)smallest : 0ull, load_agent(&ctl->varying), sampled,
+                       first_reads_b);
 }
 
 // ---- digit counts of every tile -----------------------------------------------------------------------------------
@@ -312,17 +360,20 @@ __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __rest
 template <typename T, int BLOCK, int ITEMS, int SUB, typename C>
 __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restrict__ orig, const typename SortKey<T>::U* buf_a,
                                                                 const typename SortKey<T>::U* buf_b, uint32_t n, int pass, int rev,
-                                                                const SortCtl* ctl, C* __restrict__ tile_count) {
+                                                                SortCtl* ctl, C* __restrict__ tile_count) {
     typedef typename SortKey<T>::U U;
     constexpr int TILE = BLOCK * ITEMS, NW = BLOCK / WAVE;
+    constexpr bool REFINE = std::is_integral<T>::value && sizeof(C) == 2;       // small sorts of integers: sort_refine_plan
     static_assert(sizeof(C) == 4 || TILE < 65536, "a count fits the table's type");
     constexpr int VEC = 16 / (int)sizeof(T), NV = ITEMS / VEC;
     typedef typename VecOf<U, VEC>::type VU;
     __shared__ uint32_t cnt[NW * SUB][256];
-    if (ctl->skip[pass]) return;
-    const bool first = (uint32_t)pass == ctl->first_pass;
-    const U* in = first ? (const U*)orig : (ctl->src_is_b[pass] != 0u ? buf_b : buf_a);
-    const U umin = (U)~ctl->inv_min;
+    __shared__ U wave_bits[REFINE ? NW : 1];
+    const SortStep step = sort_step(ctl, pass);
+    if (step.skip != 0u) return;
+    const bool first = (uint32_t)pass == step.first_pass, refine = REFINE && first && step.refine != 0u;
+    const U* in = first ? (const U*)orig : (step.src_b != 0u ? buf_b : buf_a);
+    const U umin = (U)~step.inv_min;
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
     for (int i = tid; i < NW * SUB * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
     const uint32_t tile = blockIdx.x;
@@ -333,6 +384,7 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
     // first lane still in play -- are taken out with a ballot each and added by that lane alone; uniform floats have
     // 50% and 37% of their keys in two values of the exponent digit.
     bool skewed = false;
+    U bits = (U)0;
     auto count = [&](uint32_t d, bool valid, int i) {
         if ((i & 3) == 0) skewed = digits_skewed(d, valid);
         if (skewed) {
@@ -366,6 +418,7 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
             for (int j = 0; j < VEC; ++j) {
                 U k = (U)v[r][j];
                 if (first) k = enc_bits<T>(k, rev, umin);
+                if (REFINE) bits |= k;
                 count(digit_of(k, pass), true, r * VEC + j);
             }
         }
@@ -381,10 +434,25 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             const U k = first ? enc_bits<T>(key[i], rev, umin) : key[i];
+            if (REFINE && woff + i * WAVE < n) bits |= k;
             count(digit_of(k, pass), woff + i * WAVE < n, i);
         }
     }
+    if constexpr (REFINE) {
+        if (refine) {
+            bits = (U)wave_reduce((unsigned long long)bits, OpOr());
+            if (lane == 0) wave_bits[wave] = bits;
+        }
+    }
     __syncthreads();
+    if constexpr (REFINE) {
+        if (refine && tid == 0) {
+            U all = (U)0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) all |= wave_bits[w];
+            ctl->tile_bits[tile] = (unsigned long long)all;
+        }
+    }
     if (BLOCK > 256 && tid >= 256) return;
     uint32_t c = 0;
 #pragma unroll
@@ -512,33 +580,55 @@ __global__ __launch_bounds__(TS_BLOCK) void sort_tilescan_kernel(SortCtl* ctl, i
 // waves hide the latencies (measured: 4 against 6 workgroups a CU differ by 4%)
 template <typename T, bool PERM, bool DIRECT> constexpr int sort_pass_waves() { return (DIRECT || (!PERM && sizeof(T) <= 4)) ? 4 : 3; }
 
+// One workgroup more than tiles, which in the first pass decides which of the others run, beside the tiles and not in front of
+// them (sort_refine_plan; it writes nothing that the first pass reads).
+template <typename T, bool DIRECT> constexpr bool sort_refines() { return DIRECT && std::is_integral<T>::value; }
+
 template <typename T, int BLOCK, int ITEMS, bool PERM, bool DIRECT>
 __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void sort_pass_kernel(const T* __restrict__ orig, typename SortKey<T>::U* buf_a,
                                                                typename SortKey<T>::U* buf_b, uint32_t* val_a, uint32_t* val_b,
-                                                               int64_t* __restrict__ perm_out, uint32_t n, int pass, int rev, const SortCtl* ctl,
+                                                               int64_t* __restrict__ perm_out, uint32_t n, int pass, int rev, SortCtl* ctl,
                                                                const void* __restrict__ counts,
                                                                const uint32_t* __restrict__ chunk_prefix, uint32_t chunk_rows,
                                                                uint32_t ntiles, uint32_t xcd_chunk) {
     typedef typename SortKey<T>::U U;
     constexpr int TILE = BLOCK * ITEMS, NW = BLOCK / WAVE;
     constexpr int GROUPS = DIRECT ? BLOCK / 128 : 1;       // groups of rows of the table, 128 lanes (two counts each) a group
+    constexpr bool REFINE = sort_refines<T, DIRECT>();
     __shared__ U lds_keys[TILE];
     __shared__ uint32_t lds_vals[PERM ? TILE : 1];
     __shared__ uint32_t cnt[NW][256];             // per wave and digit: count, then slot in the sorted tile of the wave's first key of the digit
     __shared__ uint32_t goff[256];                // global slot of the digit's first key of this tile, minus its slot in the sorted tile
     __shared__ uint32_t wsum[2][256 / WAVE];
+    __shared__ unsigned long long wave_bits[REFINE ? 256 / WAVE : 1];
     __shared__ uint2 part_before[GROUPS][DIRECT ? 128 : 1], part_all[GROUPS][DIRECT ? 128 : 1];
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-    if (ctl->skip[pass]) {
+    const SortStep step = sort_step(ctl, pass);
+    if (step.skip != 0u) {
         // all keys equal: no pass ran, and the last one writes the identity permutation
         if (PERM && pass == (int)sizeof(T) - 1 && ctl->nexec == 0u)
             for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < (int64_t)n; i += (int64_t)gridDim.x * BLOCK) perm_out[i] = i + 1;
         return;
     }
-    const bool first = (uint32_t)pass == ctl->first_pass, last = (uint32_t)pass == ctl->last_pass;
-    const U umin = (U)~ctl->inv_min;
-    const bool src_b = ctl->src_is_b[pass] != 0u;
+    const bool first = (uint32_t)pass == step.first_pass, last = (uint32_t)pass == step.last_pass;
+    const U umin = (U)~step.inv_min;
+    const bool src_b = step.src_b != 0u;
+    if constexpr (REFINE) {
+        if (blockIdx.x == ntiles) {               // one workgroup more than tiles: the plan, beside the first pass
+            if (!first || step.refine == 0u) return;
+            const unsigned long long b = wave_reduce((uint32_t)tid < ntiles ? ctl->tile_bits[tid] : 0ull, OpOr());
+            if (tid < 256 && lane == 0) wave_bits[wave] = b;
+            __syncthreads();
+            if (tid == 0) {
+                unsigned long long bits = 0;
+#pragma unroll
+                for (int w = 0; w < 256 / WAVE; ++w) bits |= wave_bits[w];
+                sort_refine_plan(ctl, pass, src_b, (int)sizeof(T), bits);
+            }
+            return;
+        }
+    }
     const U* in = first ? (const U*)orig : (src_b ? buf_b : buf_a);
     U* dst = src_b ? buf_a : buf_b;
     const uint32_t* vsrc = src_b ? val_b : val_a;
@@ -828,7 +918,7 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
             uint16_t* counts = (uint16_t*)(base + l.count_off);
             sort_upsweep_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, 1, uint16_t><<<l.ntiles, DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
             RK_LAUNCH_CHECK();
-            sort_pass_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, PERM, true><<<l.ntiles, DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, nullptr, 1u, l.ntiles, 0u);
+            sort_pass_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, PERM, true><<<l.ntiles + (sort_refines<T, true>() ? 1u : 0u), DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, nullptr, 1u, l.ntiles, 0u);
         } else {
             uint32_t* counts = (uint32_t*)(base + l.count_off);
             uint32_t* chunk_total = (uint32_t*)(base + l.chunk_total_off);

@@ -130,6 +130,44 @@ def test_constant_digits(rk, orc, dtype):
         _check(rk, orc, np.full(n, 3, dtype=dtype))
 
 
+def _passes_run(rk, x, perm):
+    """The number of passes that a small sort ran, from the control block at the head of its temporary: 256 digit counts
+    and three flags for each of 8 passes, the first and the last pass, then their number."""
+    import torch
+    from amdgpu_jl_amd import _lib as L
+    from amdgpu_jl_amd.array import stream_ptr
+    d = rk.ROCArray(x)
+    out = rk.ROCArray(dims=(x.size,), dtype=np.int64 if perm else x.dtype)
+    tmp = torch.empty(int(L.lib.rk_sort_tmp_bytes(d.code, x.size, int(perm))), dtype=torch.uint8, device="cuda")
+    f = L.lib.rk_sortperm if perm else L.lib.rk_sort_to
+    L.check(f(d.code, d.ptr, out.ptr, x.size, 0, tmp.data_ptr(), tmp.numel(), stream_ptr()), "sort")
+    at = 8 * 256 * 4 + 3 * 8 * 4 + 2 * 4
+    return int(tmp[at:at + 4].cpu().numpy().view(np.uint32)[0]), rk.Array(out)
+
+
+@pytest.mark.parametrize("perm", [False, True])
+@pytest.mark.parametrize("dtype", [np.int16, np.int32, np.int64])
+@pytest.mark.parametrize("n", [2, 4096, 4097, 300_000, 1 << 20])
+def test_digits_that_no_two_relative_keys_differ_in_run_no_pass(rk, orc, dtype, n, perm):
+    """Small integer sorts: a pass for every digit in which keys minus the smallest one differ, wherever it stands (an id in
+    the high digits and a small number, perhaps negative, in the low one; a step; a range that carries), and no other."""
+    rng = np.random.default_rng(n)
+    bits = 8 * np.dtype(dtype).itemsize
+    ids, small = rng.integers(0, 100, n).astype(np.int64), rng.integers(-100, 101, n).astype(np.int64)
+    wide = np.int64(1) << (bits - 8)
+    cases = [(ids - 50) * wide + (small + 100), (ids - 50) * wide + small, (ids - 50) * wide, small, small + 5000, small * 256 // 2,
+             np.full(n, -7, dtype=np.int64), rng.integers(-(1 << (bits - 1)), 1 << (bits - 1), n, dtype=np.int64)]
+    if bits >= 32:
+        cases.append((ids << (bits // 2)) + small * (small > 0))
+    for k in cases:
+        x = k.astype(dtype)
+        rel = np.bitwise_or.reduce(x.astype(np.int64).view(np.uint64) - np.uint64(int(x.min()) & (2 ** 64 - 1)))
+        want = sum(1 for p in range(bits // 8) if (int(rel) >> (8 * p)) & 255)
+        ran, got = _passes_run(rk, x, perm)
+        assert np.array_equal(got, orc.sortperm(x) if perm else orc.sort(x))
+        assert ran == want, (ran, want, hex(int(rel)))
+
+
 # More than 256 tiles of 4096 keys: the sort counts the digits of every tile before each pass (no look-back).
 LARGE = 1024 * 4096 + 4096 * 3 + 37
 
