@@ -202,15 +202,18 @@ _staging: dict = {}            # (device, stream) -> pinned bytes for scalar fet
 _waiting: set = set()          # (device, stream) keys whose workspace has been handed to a kernel with bounded waits
 
 
-# Pinned host words that a kernel writes its scalar results to (the count behind x[mask], sum(x), findmax(x)): the host reads them after the
-# stream synchronisation it needs anyway, with no device-to-host copy in between.  A slot belongs to one call from take to
-# give, whatever thread or stream it runs on; the free list holds at most as many as calls have been in flight at once.
+# Pinned host words that a kernel writes its scalar results to (the count behind x[mask], sum(x), findmax(x)): the host reads
+# them after the stream synchronisation it needs anyway, with no device-to-host copy in between.  A slot belongs to one call
+# from take_slot to give_slot, whatever thread or stream it runs on; the free list holds at most as many as calls have been
+# in flight at once.  PyTorch's pinned allocator does not know that a kernel writes to a slot by its address, so a slot whose
+# stream has not been waited for is kept for good.
 _free_slots: list = []
+_parked_slots: list = []
 SLOT_BYTES = 128
 
 
 def take_slot():
-    """(address, NumPy bytes, tensor) of a free pinned slot; hand it back with ``give_slot``."""
+    """(address, NumPy bytes, tensor) of a free pinned slot; ``fill_slot``, read, and hand it back with ``give_slot``."""
     try:
         return _free_slots.pop()
     except IndexError:
@@ -223,10 +226,29 @@ def give_slot(slot) -> None:
         _free_slots.append(slot)
 
 
-def await_slot() -> None:
-    """The host waits for the current stream, and with it for the words that its kernels write to a slot."""
-    check_waits()                           # the place to learn of a give-up
-    torch.cuda.current_stream().synchronize()
+def _rescue_slot(slot) -> None:
+    """After an exception between the launch and the end of the wait: back to the free list once the stream is done with
+    it, parked where that cannot be known (a stream that is being captured, a failed synchronisation)."""
+    _parked_slots.append(slot)
+    try:
+        if torch.cuda.is_current_stream_capturing():
+            return
+        torch.cuda.current_stream().synchronize()
+    except Exception:                       # the caller raises the first one
+        return
+    _parked_slots.remove(slot)
+    give_slot(slot)
+
+
+def fill_slot(slot, fn, name, args) -> None:
+    """Calls ``fn(*args, stream)``, which enqueues kernels that write scalars to the slot, and waits for the stream."""
+    try:
+        L.check(fn(*args, stream_ptr()), name)
+        check_waits()                       # the place to learn of a give-up
+        torch.cuda.current_stream().synchronize()
+    except BaseException:
+        _rescue_slot(slot)
+        raise
 
 
 def note_waiting_call() -> None:

@@ -11,7 +11,7 @@ import torch
 
 from . import _lib as L
 from .accumulate import accumulate
-from .array import ROCArray, await_slot, device, give_slot, note_waiting_call, stream_ptr, take_slot, workspace
+from .array import ROCArray, device, fill_slot, give_slot, note_waiting_call, stream_ptr, take_slot, workspace
 from .mapreduce import count
 
 
@@ -65,18 +65,17 @@ def _select(x: ROCArray, mask: ROCArray) -> ROCArray:
     n = len(x)
     if n == 0:
         return ROCArray(dims=(0,), dtype=x.dtype)
-    st = stream_ptr()
     nbytes = int(L.lib.rk_mask_tmp_bytes(n))
     tmp = torch.empty(nbytes, dtype=torch.uint8, device=device())
     ws, ws_bytes = workspace()
     slot = take_slot()
-    L.check(L.lib.rk_mask_count(mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes, st), "rk_mask_count")
-    await_slot()
+    fill_slot(slot, L.lib.rk_mask_count, "rk_mask_count", (mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes))
     total = int(slot[1][:8].view(np.int64)[0])
     give_slot(slot)
     y = ROCArray(dims=(total,), dtype=x.dtype)
     if total > 0:
-        L.check(L.lib.rk_mask_select(mask.ptr, n, x.ptr, y.ptr, x.dtype.itemsize, total, tmp.data_ptr(), nbytes, st), "rk_mask_select")
+        L.check(L.lib.rk_mask_select(mask.ptr, n, x.ptr, y.ptr, x.dtype.itemsize, total, tmp.data_ptr(), nbytes, stream_ptr()),
+                "rk_mask_select")
     return y
 
 

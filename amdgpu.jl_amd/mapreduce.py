@@ -14,7 +14,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib as L
-from .array import ROCArray, await_slot, dtype_code, give_slot, stream_ptr, take_slot, workspace
+from .array import ROCArray, dtype_code, fill_slot, give_slot, stream_ptr, take_slot, workspace
 from .views import ROCView
 
 # f of mapreduce(f, op, A): enumerated, like the C ABI
@@ -222,8 +222,7 @@ def mapreduce(f, op: str, A: ROCArray, dims=None, init=None):
         # the kernel writes the value to pinned host memory: no result array, no copy
         slot = take_slot()
         fn, name, args = _dense_args(f, prog, op, A, dtype_code(out_dt), slot[0], init, out_dt, mask)
-        L.check(fn(*args, stream_ptr()), name)
-        await_slot()
+        fill_slot(slot, fn, name, args)
         value = slot[1][:out_dt.itemsize].view(out_dt)[0].copy()
         give_slot(slot)
         return value
@@ -362,9 +361,8 @@ def _findminmax(A, want_max: bool, dims):
         # value and CartesianIndex go straight to pinned host memory: no result arrays, no copies
         ws, ws_bytes = workspace()
         slot = take_slot()
-        L.check(L.lib.rk_findminmax(1 if want_max else 0, A.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, slot[0],
-                                    slot[0] + 16, ws, ws_bytes, stream_ptr()), "rk_findminmax")
-        await_slot()
+        fill_slot(slot, L.lib.rk_findminmax, "rk_findminmax",
+                  (1 if want_max else 0, A.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, slot[0], slot[0] + 16, ws, ws_bytes))
         value = slot[1][:A.dtype.itemsize].view(A.dtype)[0].copy()
         c = tuple(int(v) for v in slot[1][16:16 + 8 * A.ndim].view(np.int64))
         give_slot(slot)

@@ -1,0 +1,73 @@
+"""Host-side bookkeeping of the Python mirror that needs no GPU: pinned slots of scalar results."""
+import numpy as np
+import pytest
+
+
+class _Stream:
+    def __init__(self, fail=False):
+        self.waits, self.fail = 0, fail
+
+    def synchronize(self):
+        self.waits += 1
+        if self.fail:
+            raise RuntimeError("stream error")
+
+
+@pytest.fixture()
+def slots(rk, monkeypatch):
+    """The module with one slot of ordinary memory and a stream that can be told to fail or to be capturing."""
+    from amdgpu_jl_amd import array
+    words = np.zeros(array.SLOT_BYTES, dtype=np.uint8)
+    slot = (words.ctypes.data, words, None)
+    state = dict(stream=_Stream(), capturing=False)
+    monkeypatch.setattr(array, "_free_slots", [slot])
+    monkeypatch.setattr(array, "_parked_slots", [])
+    monkeypatch.setattr(array, "check_waits", lambda: None)
+    monkeypatch.setattr(array, "stream_ptr", lambda: 0)
+    monkeypatch.setattr(array.torch.cuda, "current_stream", lambda *a: state["stream"])
+    monkeypatch.setattr(array.torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    return array, slot, state
+
+
+def test_a_slot_is_read_after_the_wait(slots):
+    array, slot, state = slots
+    got = array.take_slot()
+    assert got is slot and array._free_slots == []
+
+    def call(*args):
+        assert args == (slot[0], 3, 0) and state["stream"].waits == 0
+        slot[1][0] = 7
+        return 0
+    array.fill_slot(got, call, "call", (slot[0], 3))
+    assert got[1][0] == 7 and state["stream"].waits == 1
+    array.give_slot(got)
+    assert array._free_slots == [slot] and array._parked_slots == []
+
+
+@pytest.mark.parametrize("where", ["launch", "status", "wait"])
+@pytest.mark.parametrize("error", [ValueError, KeyboardInterrupt])
+def test_an_interrupted_fetch_waits_before_the_slot_is_used_again(slots, monkeypatch, where, error):
+    array, slot, state = slots
+
+    def stop(*args):
+        assert state["stream"].waits == 0
+        raise error()
+    if where == "wait":
+        monkeypatch.setattr(array, "check_waits", stop)
+    if where == "status":
+        error = array.L.RKError
+    call = {"launch": stop, "status": lambda *a: array.L.RK_ERR_WORKSPACE, "wait": lambda *a: 0}[where]
+    with pytest.raises(error):
+        array.fill_slot(array.take_slot(), call, "call", ())
+    assert state["stream"].waits == 1
+    assert array._free_slots == [slot] and array._parked_slots == []
+
+
+@pytest.mark.parametrize("why", ["capturing", "failed wait"])
+def test_a_slot_that_may_still_be_written_is_parked(slots, why):
+    array, slot, state = slots
+    state.update(capturing=why == "capturing", stream=_Stream(fail=True))
+    with pytest.raises(RuntimeError, match="stream error"):
+        array.fill_slot(array.take_slot(), lambda *a: 0, "call", ())
+    assert array._free_slots == [] and array._parked_slots == [slot]
+    assert state["stream"].waits == (1 if why == "capturing" else 2)

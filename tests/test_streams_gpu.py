@@ -68,3 +68,37 @@ def test_two_streams_beyond_residency(rk, orc):
             assert np.array_equal(rk.Array(cs), want_x)
             assert np.array_equal(rk.Array(c2), want_b)
             assert np.array_equal(rk.Array(fa), want_m)
+
+
+def test_scalars_fetched_by_two_threads_on_two_streams(rk):
+    """sum, findmax and x[mask] hand their scalars to the host through pinned slots that calls take from one free list: two
+    threads, each on a stream of its own, fetch different values at once and each gets its own.  Whole numbers: exact."""
+    import threading
+    failures, start = [], threading.Barrier(2)
+
+    def work(who):
+        try:
+            rng = np.random.default_rng(60 + who)
+            with torch.cuda.stream(torch.cuda.Stream()):
+                jobs = []
+                for n in (1000, 1 << 16, (1 << 20) + 3):
+                    x = rng.permutation(n).astype(np.int64) * (who + 1) - n
+                    m = rng.random(n) < 0.1 + 0.5 * who
+                    jobs.append((x, m, rk.ROCArray(x), rk.ROCArray(m), x.sum(), x.max(), int(x.argmax()) + 1, x[m]))
+                start.wait(timeout=60)
+                for it in range(100):
+                    x, m, dx, dm, total, top, at, some = jobs[it % len(jobs)]
+                    assert rk.sum(dx) == total
+                    assert rk.findmax(dx) == (top, at)
+                    got = rk.getindex_mask(dx, dm)
+                    assert len(got) == len(some)
+                    if it >= 97:
+                        assert np.array_equal(rk.Array(got), some)
+        except BaseException as e:                                  # an assertion in a thread would go unseen
+            failures.append(f"thread {who}: {e!r}")
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=100)
+    assert not failures and not any(t.is_alive() for t in threads), failures
