@@ -126,6 +126,7 @@ class ROCArray:
     def reshape(self, *dims):
         if len(dims) == 1 and isinstance(dims[0], (tuple, list)):
             dims = tuple(dims[0])
+        dims = tuple(int(d) for d in dims)
         if math.prod(dims) != len(self):
             raise L.DimensionMismatch(L.RK_ERR_DIMENSION, "reshape")
         return ROCArray(buf=self.buf, dims=dims, dtype=self.dtype, offset=self.offset)

@@ -1,4 +1,4 @@
-"""Host-side bookkeeping of the Python mirror that needs no GPU: pinned slots of scalar results."""
+"""Host-side parts of the Python mirror that need no GPU: pinned slots of scalar results, shapes."""
 import numpy as np
 import pytest
 
@@ -71,3 +71,16 @@ def test_a_slot_that_may_still_be_written_is_parked(slots, why):
         array.fill_slot(array.take_slot(), lambda *a: 0, "call", ())
     assert array._free_slots == [] and array._parked_slots == [slot]
     assert state["stream"].waits == (1 if why == "capturing" else 2)
+
+
+def test_reshape_counts_the_elements_of_the_dims_it_makes(rk):
+    """The check is on the whole numbers that become the result's dims, whatever type they come in."""
+    import torch
+    from amdgpu_jl_amd import _lib as L
+    x = rk.ROCArray(buf=torch.zeros(20, dtype=torch.uint8), dims=(5,), dtype=np.float32)
+    assert x.reshape(5, 1).dims == x.reshape((np.int32(5), 1.0)).dims == (5, 1)
+    for dims in ((2.5, 2), (4,), (5, 2)):
+        with pytest.raises(L.DimensionMismatch):
+            x.reshape(*dims)
+    y = rk.ROCArray(buf=torch.zeros(16, dtype=torch.uint8), dims=(4,), dtype=np.float32)
+    assert y.reshape(2.5, 2).dims == (2, 2)
