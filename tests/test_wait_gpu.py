@@ -1,10 +1,10 @@
 """Bounded waits: a look-back that cannot complete helps itself (single-pass scan of long lines, one-pass findall:
-exact results whatever happens) or gives up and records it (the other kernels); every kernel exits.
+exact results whatever happens) or gives up and records it (the other scans); every kernel exits.  Sorts wait for nobody.
 
 The condition is forced from the host: rk_set_wait_budget(1) lets a wait spend ONE unsuccessful poll, which in a scan of
 thousands of tiles some tile always exceeds (a predecessor's aggregate is not there yet at the first look).  The
-kernels run to their end with meaningless results, rk_workspace_status / rk_sort_status report RK_ERR_WAIT, and after
-preparing the workspace again the same call is correct.  No kernel faults, traps or hangs here."""
+kernels run to their end with meaningless results, rk_workspace_status reports RK_ERR_WAIT, and after preparing the
+workspace again the same call is correct.  No kernel faults, traps or hangs here."""
 import numpy as np
 import pytest
 
@@ -84,26 +84,26 @@ def test_findall_gives_up_and_recovers(rk, orc, tiny_budget):
     assert np.array_equal(rk.Array(ys), np.flatnonzero(b) + 1)
 
 
-def test_sort_gives_up_and_recovers(rk, orc, tiny_budget):
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("dtype", [np.float32, np.int64])
+def test_sorts_do_not_wait(rk, orc, tiny_budget, n, dtype):
+    """No kernel of the sort polls another workgroup, below and above the 2^20 keys where the passes change: whatever the
+    budget, the result is right and the status clean."""
     import torch
     L = tiny_budget
     from amdgpu_jl_amd.array import stream_ptr
     rng = np.random.default_rng(7)
-    # 2^20 keys: 256 tiles chained by look-back.  After a give-up no further tile starts and every store is kept inside
-    # the arrays (a pass that follows one with holes reads keys the histograms never counted).
-    k = rng.standard_normal(1 << 20).astype(np.float32)
+    k = rng.standard_normal(n).astype(dtype) if dtype == np.float32 else rng.integers(-2**62, 2**62, n)
     dk = rk.ROCArray(k)
-    tmp = torch.empty(int(L.lib.rk_sort_tmp_bytes(L.RK_F32, k.size, 0)), dtype=torch.uint8, device="cuda")
-    assert L.lib.rk_sort(L.RK_F32, dk.ptr, k.size, 0, tmp.data_ptr(), tmp.numel(), stream_ptr()) == 0
-    st = L.lib.rk_sort_status(tmp.data_ptr(), tmp.numel(), stream_ptr())
-    assert st in (0, L.RK_ERR_WAIT)
-    if st == 0:
-        assert np.array_equal(rk.Array(dk), np.sort(k))
-    L.lib.rk_set_wait_budget(0)
-    dk = rk.ROCArray(k)
-    assert L.lib.rk_sort(L.RK_F32, dk.ptr, k.size, 0, tmp.data_ptr(), tmp.numel(), stream_ptr()) == 0
+    tmp = torch.empty(int(L.lib.rk_sort_tmp_bytes(dk.code, n, 1)), dtype=torch.uint8, device="cuda")
+    ix = rk.ROCArray(dims=(n,), dtype=np.int64)
+    assert L.lib.rk_sortperm(dk.code, dk.ptr, ix.ptr, n, 0, tmp.data_ptr(), tmp.numel(), stream_ptr()) == 0
+    assert L.lib.rk_sort_status(tmp.data_ptr(), tmp.numel(), stream_ptr()) == 0
+    assert np.array_equal(rk.Array(ix), orc.sortperm(k))
+    assert L.lib.rk_sort(dk.code, dk.ptr, n, 0, tmp.data_ptr(), tmp.numel(), stream_ptr()) == 0
     assert L.lib.rk_sort_status(tmp.data_ptr(), tmp.numel(), stream_ptr()) == 0
     assert np.array_equal(rk.Array(dk), np.sort(k))
+    assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(k), rev=True)), np.sort(k)[::-1])
 
 
 def _alone_count(ws):
@@ -301,23 +301,17 @@ def test_mirror_raises_on_give_up(rk, orc, tiny_budget):
         assert np.array_equal(got, want)
     L.lib.rk_set_wait_budget(0)
     assert np.array_equal(rk.Array(rk.cumsum(x, dims=2)), want)  # the mirror prepared the workspace again
-    # findall and a small sort go the same way
+    # findall goes the same way
     L.lib.rk_set_wait_budget(1)
     b = rng.random(1 << 24) < 0.3
     db = rk.ROCArray(b)
-    k = rng.standard_normal(1 << 20).astype(np.float32)
     for _ in range(2):
         try:
             assert np.array_equal(rk.Array(rk.findall(db)), np.flatnonzero(b) + 1)
         except L.WaitError:
             pass
-        try:
-            assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(k))), np.sort(k))
-        except L.WaitError:
-            pass
     L.lib.rk_set_wait_budget(0)
     assert np.array_equal(rk.Array(rk.findall(db)), np.flatnonzero(b) + 1)
-    assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(k))), np.sort(k))
 
 
 def test_static_scratch_reports_and_recovers(rk, orc, tiny_budget):
