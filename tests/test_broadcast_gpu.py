@@ -493,3 +493,25 @@ def test_matrix_against_row_and_column(rk, dtype, m, n):
         assert np.array_equal(rk.Array(got), want)
     out = rk.materialize_(dA, L(dA) + L(dr) * L(dc))           # in place
     assert out is dA and np.array_equal(rk.Array(dA), A + r * c)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+@pytest.mark.parametrize("m,n", [(257, 33), (130, 7), (1003, 5), (128, 64)])
+def test_matrix_against_strided_and_odd_row_vectors(rk, dtype, m, n):
+    """Row vectors that are a row of a matrix (one value every `step` elements), every other column of one, backwards, or
+    start at an odd element of a buffer; column vectors at an odd element.  Integer-valued: exact."""
+    rng = _rng(m * 31 + n)
+    u = lambda *s: rng.integers(-50, 51, s).astype(dtype)
+    A, P, Q, v, w = u(m, n), u(9, n), u(5, 2 * n), u(n + 3), u(m + 3)
+    dA, dP, dQ, dv, dw = (rk.ROCArray(k) for k in (A, P, Q, v, w))
+    L = rk.lazy
+    rows = [(rk.view(dP, (4, 4), None), P[3:4, :]), (rk.view(dQ, (2, 2), (1, 2, 2 * n - 1)), Q[1:2, ::2]),
+            (rk.view(dP, (9, 9), (n, -1, 1)), P[8:9, ::-1]), (dv.view_range(2, n + 1).reshape(1, n), v[1:n + 1].reshape(1, n)),
+            (rk.transpose(dv.view_range(4, n + 3)), v[3:].reshape(1, n))]
+    cols = [(rk.ROCArray(w[:m].reshape(m, 1)), w[:m].reshape(m, 1)), (dw.view_range(2, m + 1).reshape(m, 1), w[1:m + 1].reshape(m, 1)),
+            (dw.view_range(4, m + 3), w[3:].reshape(m, 1))]
+    for dr, r in rows:
+        assert np.array_equal(rk.Array(rk.materialize(L(dA) - L(dr))), A - r)
+        for dc, c in cols:
+            assert np.array_equal(rk.Array(rk.materialize(L(dA) + L(dr) * L(dc))), A + r * c)
+            assert np.array_equal(rk.Array(rk.materialize(L(dr) * L(dc))), r * c)

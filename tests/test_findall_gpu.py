@@ -98,7 +98,7 @@ def test_mask_select_edges(rk, n):
     rng = np.random.default_rng(n)
     x = rng.integers(0, 1 << 31, n).astype(np.uint32).view(np.float32)
     dx = rk.ROCArray(x)
-    for dens in (0.0, 0.01, 0.5, 1.0) if n < 1 << 24 else (0.4,):
+    for dens in (0.0, 0.01, 0.5, 1.0) if n < 1 << 26 else (0.4,):
         m = rng.random(n) < dens
         if dens == 0.5:
             m[n // 2:] = True                                       # a full stretch behind a mixed one
@@ -116,6 +116,60 @@ def test_mask_select_unaligned(rk, dtype):
     for a, b in ((2, n), (8, n - 1), (17, n - 70_000)):
         got = rk.Array(rk.getindex_mask(dx.view_range(a, b), dm.view_range(a, b)))
         assert np.array_equal(got, x[a - 1:b][m[a - 1:b]])
+
+
+def _mask_calls(rk, mask, x, y, elsize, n, nsel=None, between=None):
+    """rk_mask_count and rk_mask_select on raw addresses; `between` runs after the count.  Returns the count."""
+    import torch
+    from amdgpu_jl_amd import _lib as L
+    from amdgpu_jl_amd.array import stream_ptr, workspace
+    tmp = torch.empty(int(L.lib.rk_mask_tmp_bytes(n)), dtype=torch.uint8, device="cuda")
+    total = torch.full((1,), -1, dtype=torch.int64, device="cuda")
+    ws, ws_bytes = workspace()
+    L.check(L.lib.rk_mask_count(mask, n, total.data_ptr(), tmp.data_ptr(), tmp.numel(), ws, ws_bytes, stream_ptr()), "count")
+    cnt = int(total.item())
+    if between is not None:
+        between()
+    L.check(L.lib.rk_mask_select(mask, n, x, y, elsize, cnt if nsel is None else nsel, tmp.data_ptr(), tmp.numel(), stream_ptr()), "select")
+    torch.cuda.synchronize()
+    return cnt
+
+
+@pytest.mark.parametrize("xoff,yoff", [(0, 0), (8, 0), (0, 8), (8, 24)])
+def test_mask_select_16_byte_elements(rk, xoff, yoff):
+    """Elements of 16 bytes need 8-byte alignment only (ComplexF64, pairs of Int64)."""
+    import torch
+    rng = np.random.default_rng(xoff + 3 * yoff)
+    n = 70_003
+    x, m = rng.integers(-2**62, 2**62, (n, 2)), rng.random(n) < 0.4
+    dx = torch.zeros(16 * n + 64, dtype=torch.uint8, device="cuda")
+    dx[xoff:xoff + 16 * n] = torch.from_numpy(x.view(np.uint8).reshape(-1).copy()).cuda()
+    dm, want = torch.from_numpy(m.view(np.uint8).copy()).cuda(), x[m]
+    dy = torch.full((16 * len(want) + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+    assert dx.data_ptr() % 16 == 0 and dy.data_ptr() % 16 == 0
+    assert _mask_calls(rk, dm.data_ptr(), dx.data_ptr() + xoff, dy.data_ptr() + yoff, 16, n) == len(want)
+    got = dy.cpu().numpy()
+    assert np.array_equal(got[yoff:yoff + 16 * len(want)].view(np.int64).reshape(-1, 2), want)
+    assert (got[:yoff] == 0xA5).all() and (got[yoff + 16 * len(want):] == 0xA5).all()
+
+
+@pytest.mark.parametrize("n", [100, 70_003, (1 << 24) + 5])
+def test_mask_bytes_and_the_bound_of_the_result(rk, n):
+    """Only bit 0 of a Bool byte counts, and no element is written past nsel: neither with a smaller one than the count nor
+    for a mask that gains entries between the two calls."""
+    import torch
+    rng = np.random.default_rng(n)
+    x = rng.integers(0, 1 << 31, n, dtype=np.int32)
+    m = rng.choice(np.array([0, 1, 2, 3, 254, 255], dtype=np.uint8), n)
+    dx, dm, want = torch.from_numpy(x).cuda(), torch.from_numpy(m).cuda(), x[(m & 1) == 1]
+    for nsel in (len(want), len(want) // 2):
+        dy = torch.full((len(want) + 16,), -7, dtype=torch.int32, device="cuda")
+        assert _mask_calls(rk, dm.data_ptr(), dx.data_ptr(), dy.data_ptr(), 4, n, nsel) == len(want)
+        got = dy.cpu().numpy()
+        assert np.array_equal(got[:nsel], want[:nsel]) and (got[nsel:] == -7).all()
+    dy = torch.full((len(want) + 16,), -7, dtype=torch.int32, device="cuda")
+    _mask_calls(rk, dm.data_ptr(), dx.data_ptr(), dy.data_ptr(), 4, n, between=lambda: dm.fill_(1))
+    assert (dy.cpu().numpy()[len(want):] == -7).all()
 
 
 def test_the_paths_the_tunables_select():

@@ -464,12 +464,13 @@ def test_scans_across_rows_that_are_no_whole_vectors(rk, orc, shape):
 
 
 @pytest.mark.parametrize("dtype", [np.int32, np.int64, np.float32])
-@pytest.mark.parametrize("vectors", [328, 336, 337, 512, 513, 1009, 2050])
+@pytest.mark.parametrize("vectors", [328, 336, 337, 512, 513, 1009, 2050, 4105])
 @pytest.mark.parametrize("extra,outer", [(0, 1), (1, 1), (1, 3)])
 def test_strips_of_rows_that_are_no_whole_lines(rk, orc, dtype, vectors, extra, outer):
     """cumsum(A; dims=2) by tiles of rows: rows of whole 128-byte lines keep strips of 64 vectors in order; other rows are
     cut into a multiple of 8 strips (narrower ones where at least 42 lanes of 64 work: up to 328 vectors
-    are 41 lanes in 8 strips, 329 .. 336 are 42), neighbours on one XCD.  Whole vectors and one element more.  Integer-valued: exact."""
+    are 41 lanes in 8 strips, 329 .. 336 are 42), neighbours on one XCD.  4105 vectors are 72 strips of 58 lanes, the last one
+    without a column.  Whole vectors and one element more.  Integer-valued: exact."""
     dt = np.dtype(dtype)
     inner, mid = vectors * (16 // dt.itemsize) + extra, 601 + 149 * outer
     x = np.random.default_rng(vectors + outer).integers(-9, 10, (inner, mid, outer)).astype(dtype)
