@@ -26,7 +26,7 @@ KNOWN = [
     ("bc_flat_kernel<EvalCopy", 16777216, "calibration: copy z .= x Float32[2^26]", 4 * M26 / KIB, 4 * M26 / KIB),
     ("bc_flat_kernel<EvalAxpbyExp", 16777216, "z .= a.*x .+ y.*exp.(w) Float32[2^26]", 12 * M26 / KIB, 4 * M26 / KIB),
     ("bc_flat_kernel<EvalAxpbyExp", 33554432, "cfg4a z .= a.*x .+ y.*exp.(w) 512^3", 12 * M27 / KIB, 4 * M27 / KIB),
-    ("bc_kernel<EvalAddMul", None, "cfg4b C .= A .+ r .* c 16384^2", 4 * (1 << 28) / KIB, 4 * (1 << 28) / KIB),
+    ("bc_matrix_kernel<EvalAddMul", None, "cfg4b C .= A .+ r .* c 16384^2", 4 * (1 << 28) / KIB, 4 * (1 << 28) / KIB),
     ("scan_ordered_kernel<int", 2097152, "cumsum Int32[2^26]", 4 * M26 / KIB, 4 * M26 / KIB),
     ("scan_ordered_kernel<int", 4194304, "cfg3a cumsum Int32[2^27]", 4 * M27 / KIB, 4 * M27 / KIB),
     ("scan_ordered_kernel<short", None, "cumsum Int16[2^26] (native narrow scan, 4 B/elt)", 2 * M26 / KIB, 2 * M26 / KIB),
