@@ -920,14 +920,16 @@ __global__ __launch_bounds__(BLOCK) void bc_flat_kernel(const BcFlatArgs a) {
     store_nt((V*)a.dest + i, o);
 }
 
-// A matrix against row and column vectors (C .= A .+ r .* c), one element type, every array of it 16-byte aligned where it
-// is dense: the lean form of rows and indexed mode.  The general kernels fetch each operand's pointer, strides and type
-// through branches of their own and split the linear index by three divisions; here the arguments are one compact block,
-// a wave takes 64 vectors of the destination's linear order as in bc_flat_kernel, and the column of a lane comes from one
-// multiplication.  Bound by memory: C .= A .+ r .* c back to back, indexed mode -> here, 8191 x 4099 Float32 56.1 -> 46.5 us
-// (5.8 TB/s), 4097 x 4099 Float64 55.1 -> 46.1, 1001 x 33521 54.2 -> 46.8, 65537 x 511 53.9 -> 45.7; C .= A .- r 46.3 -> 43.2,
-// 48.7 -> 44.3, 46.3 -> 42.7, 46.1 -> 43.6.  Workgroups of 256 threads: 45.3 and 43.7 us at 8191 x 4099, 46.4 and 44.7 for
-// 8192 x 4096 (64: 45.2 and 42.8).
+// A matrix against row and column vectors (C .= A .+ r .* c), one element type that is the compute type too (Float32, Float64
+// or Int64; Int32 and narrower types stay with the general kernels), every array of it 16-byte aligned where it is dense: the
+// lean form of rows and indexed mode.  The general kernels fetch each operand's pointer, strides and type through branches
+// of their own and split the linear index by three divisions; here the arguments are one compact block, a wave takes 64
+// vectors of the destination's linear order as in bc_flat_kernel, and the column of a lane comes from one multiplication.
+// Bound by memory (128.5 MiB read and 128.1 written of 128.1 each at 8191 x 4099).  C .= A .+ r .* c back to back on the same
+// arrays, indexed mode -> here: 8191 x 4099 Float32 56.1 -> 46.5 us (5.8 TB/s), 4097 x 4099 Float64 55.1 -> 46.1, 1001 x 33521
+// 54.2 -> 46.8, 65537 x 511 53.9 -> 45.7; C .= A .- r 46.3 -> 43.2, 48.7 -> 44.3, 46.3 -> 42.7, 46.1 -> 43.6.  With arrays that
+// change from call to call 8191 x 4099 takes 56.9 -> 48.9 (5.5 TB/s).  Workgroups of 256 threads: 45.3 and 43.7 us at 8191 x
+// 4099, 46.4 and 44.7 for 8192 x 4096 (64: 45.2 and 42.8).
 struct BcMatArgs {
     uint32_t    total, rows;
     uint32_t    recip;                      // floor(2^32 / rows)

@@ -313,20 +313,20 @@ __device__ __forceinline__ void publish_barrier() {
 }
 
 // ---- bounded waits ------------------------------------------------------------------------------------------
-// Every loop that polls memory written by another workgroup (look-back of the scans, of the select and of the
-// sort) counts its unsuccessful rounds.  When one wait has used `budget` rounds -- which only happens when the
+// Every loop that polls memory written by another workgroup (look-back of the scans and of the select) counts its
+// unsuccessful rounds.  When one wait has used `budget` rounds -- which only happens when the
 // state it polls is not what the protocol expects: a workspace that was never prepared, or one shared by calls
 // that run at the same time -- it writes the call's `stamp` into the word `failed`, stops waiting and carries on
 // with a meaningless value, so that every workgroup still runs to its end and the kernel exits normally.  All
 // waiters of the SAME call look at `failed` every few rounds and give up with the first one; a stamp left by an
 // earlier call (the word stays set until the host has read it and prepared the workspace again) is not theirs and
 // does not stop them.  The results of the call that gave up are wrong; the host learns of it through
-// rk_workspace_status / rk_sort_status.
+// rk_workspace_status.
 struct WaitCtl {
     uint32_t* failed;
     long long budget;       // unsuccessful poll rounds one wait may spend (a round is a device-coherent load: ~1 us)
     int       backoff;      // s_sleep units between rounds
-    uint32_t  stamp;        // nonzero mark of the running call: the scan epoch (set by the kernel), 1 in the sort's own control block
+    uint32_t  stamp;        // nonzero mark of the running call: the scan epoch (set by the kernel)
 };
 // Called once per unsuccessful round by (at least) one full wave; true = stop waiting.
 __device__ __forceinline__ bool wait_give_up(const WaitCtl& w, long long& rounds) {

@@ -1734,11 +1734,13 @@ struct RowStrips {
 };
 // Rows of whole 128-byte lines: strips of a whole wave, in order (4096 x 16000 Float32 96.4 us; with neighbours on one XCD
 // 97.7).  Other rows: two strips share the line at their common edge, which two XCDs fetch and write in part each; with
-// neighbours on one XCD its L2 joins them (8191 x 8001 111.7 -> 106.4 us, 6001 x 10922 116.7 -> 112.5).  That needs a
-// multiple of 8 strips, which also makes the launch order safe (rows_chains_stay_on_their_xcd) and so does without the
-// tile counter: narrower strips are worth it as long as 42 of the 64 lanes work (4097 x 16000, 24 strips of 43 lanes
-// instead of 17: 119.7 -> 114.6; 3001 x 21800, 47 lanes: 124.8 -> 119.1; 20001 x 3200, 63 lanes: 116.7 -> 109.3; 2561 x
-// 25600, 41 lanes: 125.2 and 124.9; 1279 x 51200, 40 lanes: 127.9 -> 133.6).
+// neighbours on one XCD its L2 serves part of those reads twice (8191 x 8001, 32 strips either way: 283 -> 268 MiB read of an
+// array of 250, 261 and 263 written -- the stores are non-temporal and stay in parts; 111.7 -> 106.4 us, 6001 x 10922 116.7 ->
+// 112.5).  That needs a multiple of 8 strips, which also makes the launch order safe (rows_chains_stay_on_their_xcd) and so does
+// without the tile counter: narrower strips are worth it as long as 42 of the 64 lanes work (4097 x 16000, 24 strips of 43
+// lanes instead of 17: 119.7 -> 114.6 although it reads 280 -> 277 and writes 263 -> 270 MiB; 3001 x 21800, 47 lanes: 124.8 ->
+// 119.1; 20001 x 3200, 63 lanes: 116.7 -> 109.3; 2561 x 25600, 41 lanes: 125.2 and 124.9; 1279 x 51200, 40 lanes: 127.9 -> 133.6).
+// Times back to back on one array; with arrays that change from call to call 4097 x 16000 takes 120.3 -> 117.5.
 constexpr int ROWS_MIN_LANES = 42;
 inline RowStrips row_strips(int64_t inner, size_t esz, int vec, bool may_narrow) {
     const int64_t cols = (int64_t)WAVE * vec;

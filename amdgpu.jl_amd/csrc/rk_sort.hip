@@ -10,7 +10,7 @@
 //   sort_upsweep_kernel  the 256 digit counts of every tile (one more read of the keys, at streaming speed)
 //   sort_pass_kernel     a tile of 4096 keys ranks its keys by digit (wave-level match by ballots, counts in LDS), reorders
 //                        the tile in LDS and writes runs of equal digits.  The kernel is bound by its vector instructions
-//                        (about 75 a key, 32 of them the match), not by memory.
+//                        (58 a key, 32 of them the match), not by memory.
 //
 // How a tile learns where its digits go:
 //   up to 256 tiles (2^20 keys)  every workgroup of the pass sums the columns of the table of counts itself (256 rows of
@@ -300,7 +300,8 @@ __device__ __forceinline__ void for_each_key(const T* __restrict__ keys, int64_t
 
 // ---- smallest and largest key, varying bits -----------------------------------------------------------------------------
 // One read at streaming speed.  Integers are taken relative to the smallest key: small-range integers then need one or two
-// passes.  The workgroup whose ticket is the last makes the plan.
+// passes.  The workgroup whose ticket is the last makes the plan; for integers it also looks at 64 keys relative to the
+// smallest, which tell nearly always that no further pass can be dropped.
 constexpr int RANGE_BLOCK = 1024;       // few, large workgroups: each ends with device-wide atomics on shared words
 template <typename T>
 __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, int rev,
@@ -840,7 +841,11 @@ __global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, co
 constexpr int64_t SORT_TILE = 4096;
 constexpr int SORT_ITEMS = (int)SORT_TILE / SORT_BLOCK;
 constexpr int DIRECT_BLOCK = 1024, DIRECT_ITEMS = (int)SORT_TILE / DIRECT_BLOCK;
-constexpr uint32_t DIRECT_TILES = 256;            // up to here a pass sums the columns of the table of counts itself
+// Up to here a pass sums the columns of the table of counts itself.  Every tile reads the counts of all tiles, so that traffic
+// grows with their square: sort!(Float32), summed here / by the tile scan, 0.75 x 2^20 keys 61.4 / 102 us, 2^20 64.6 / 112, 1.5 x
+// 2^20 98 / 117, 2^21 112 / 131, 2^22 267 / 136; Int64 2^20 139 / 249, 2^21 231 / 263, 2^22 560 / 321.  256 tiles are a workgroup
+// a compute unit and one word each in tile_bits; the times alone would allow 512.
+constexpr uint32_t DIRECT_TILES = 256;
 
 struct SortLayout {
     size_t count_off, chunk_total_off, chunk_prefix_off, keys_b_off, keys_a_off, val_a_off, val_b_off, total;

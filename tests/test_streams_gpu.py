@@ -1,7 +1,7 @@
 """Several streams at once, each with its own workspace: the boundary's contract is one workspace per stream, any
 number of streams concurrently (Julia tasks each own a stream, src/tls.jl:71-86).  Calls are enqueued round-robin on
-three streams without synchronising in between, so their kernels -- including the chained scans and the sort, whose
-workgroups wait on one another through the workspace -- overlap on the device; every result is checked afterwards."""
+three streams without synchronising in between, so their kernels -- including the chained scans, whose workgroups wait on
+one another through the workspace -- overlap on the device; every result is checked afterwards."""
 import numpy as np
 import pytest
 import torch
