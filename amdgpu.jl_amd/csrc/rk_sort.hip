@@ -1,11 +1,15 @@
 // sort! / sortperm! of vectors (src/kernels/sorting.jl:1-3, which forwards to AcceleratedKernels' merge sort):
 // least-significant-digit radix sort, 8 bits per pass.
 //
+// Three ways by the number of keys:
+//   up to 4096           one workgroup does all of it in LDS (sort_tiny_kernel, rk_sort_buckets.hpp).
+//   up to 2^20           keys of 4 and 8 bytes go through splitters into buckets that are sorted in LDS (rk_sort_buckets.hpp):
+//                        such sorts are bound by the latency of their kernels, and these are four or five whatever the width.
+//   more, and keys of 2 bytes, the radix passes of this file:
 //   sort_init_kernel     clears the control block; no memset: graph-safe
 //   sort_range_kernel    one read of the keys: smallest and largest key (integers) and the bits that differ between keys;
 //                        the workgroup that finishes last decides which passes run (a digit that is the same in every key
-//                        needs none) and which buffer each of them reads.  (Integers are taken relative to the smallest key;
-//                        small sorts can drop further passes when they have seen the relative keys: sort_refine_plan)
+//                        needs none) and which buffer each of them reads.  (Integers are taken relative to the smallest key.)
 // and for every pass
 //   sort_upsweep_kernel  the 256 digit counts of every tile (one more read of the keys, at streaming speed)
 //   sort_pass_kernel     a tile of 4096 keys ranks its keys by digit (wave-level match by ballots, counts in LDS), reorders
@@ -14,10 +18,8 @@
 //
 // How a tile learns where its digits go:
 //   up to 256 tiles (2^20 keys)  every workgroup of the pass sums the columns of the table of counts itself (256 rows of
-//                        512 bytes out of L2, one or two rounds of loads): nothing waits for anything.  These sorts are bound
-//                        by latency -- a tile or less per compute unit -- so a tile is 16 waves with 4 keys a lane, not
-//                        4 waves with 16.  A chained look-back in their place resolved the tiles nearly one after the
-//                        other: 22 us a pass for 10^6 Int64 keys with their permutation.
+//                        512 bytes out of L2, one or two rounds of loads): nothing waits for anything.  A tile or less per
+//                        compute unit: it is 16 waves with 4 keys a lane, not 4 waves with 16.
 //   beyond               sort_tilescan_kernel: exclusive scan of the counts down the tiles in one launch (chunks of tiles; the
 //                        workgroup that finishes last scans the chunk totals and the digit totals); the pass kernel gives
 //                        each XCD a contiguous eighth of the tiles.
@@ -40,10 +42,7 @@ constexpr int SORT_BLOCK = 256;
 constexpr int SORT_MAX_PASSES = 8;
 
 struct SortCtl {                                  // head of the caller's temporary buffer
-    union {
-        uint32_t hist[SORT_MAX_PASSES][256];      // large sorts: first output slot of every digit value (sort_tilescan_kernel)
-        unsigned long long tile_bits[256];        // small sorts of integers: bits set in any relative key of a tile (first pass)
-    };
+    uint32_t hist[SORT_MAX_PASSES][256];          // large sorts: first output slot of every digit value (sort_tilescan_kernel)
     // everything from here on is cleared by sort_init_kernel
     uint32_t skip[SORT_MAX_PASSES];
     uint32_t src_is_b[SORT_MAX_PASSES];           // the pass reads buffer B (1) or A (0)
@@ -53,7 +52,6 @@ struct SortCtl {                                  // head of the caller's tempor
     unsigned long long inv_min;                   // ~(smallest mapped key), kept as a maximum so that zero is its identity
     unsigned long long key_max;                   // largest mapped key (integers: range = key_max - smallest)
     unsigned long long varying;                   // bits that are not the same in all mapped keys
-    uint32_t refine, unused;                      // integers: a digit below the highest may be zero in every relative key
 };
 constexpr int SORT_CTL_CLEAR = (int)((sizeof(SortCtl) - offsetof(SortCtl, skip)) / sizeof(uint32_t));
 
@@ -189,12 +187,11 @@ __device__ __forceinline__ bool digits_skewed(uint32_t d, bool valid) {
 }
 // ---- plan: which passes run and what they read --------------------------------------------------------------------
 // relative: keys are taken relative to the smallest one (integers), so digits above their range are zero in every key, and
-// so are low digits in which the keys do not differ.  (Digits between them that are zero in every relative key show only once
-// the smallest key is known, and `sampled`, the bits of some relative keys, rules most of them out: sort_refine_plan.)
+// so are low digits in which the keys do not differ.
 // Otherwise (floats) a digit in which no two keys differ is skipped: their exponent bytes are constant or not whatever is
 // subtracted.
 __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool relative, unsigned long long range, unsigned long long varying,
-                                               unsigned long long sampled, int first_reads_b) {
+                                               int first_reads_b) {
     uint32_t src_b = first_reads_b ? 1u : 0u, nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
     for (int p = 0; p < passes; ++p) {
         const unsigned long long upto = p == 7 ? ~0ull : (1ull << (8 * (p + 1))) - 1ull;
@@ -204,7 +201,6 @@ __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool re
         ctl->src_is_b[p] = src_b;
         src_b ^= 1u;
         if (first == 0xffffffffu) first = (uint32_t)p;
-        else if (relative && (range >> (8 * p)) > 0xffull && ((sampled >> (8 * p)) & 0xffull) == 0ull) ctl->refine = 1u;
         last = (uint32_t)p;
         ++nexec;
     }
@@ -213,34 +209,15 @@ __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool re
     ctl->nexec = nexec;
 }
 
-// Small sorts of integers, in their first pass: `bits` are those set in any relative key, and of the passes that are left only
-// those run whose digit has one: keys with an id in the upper half and a small number in the lower one are constant in the
-// digits between.  The last pass stays what it is -- the largest relative key has a bit in the highest digit of the range.
-// sort and sortperm of Int64[1000003], by the range alone -> so: (id << 32) + small number 105 -> 90 and 107 -> 74 us, only the
-// lowest and the highest byte varying 118 -> 66 and 123 -> 67.  Keys that differ in every digit are told by 64 of them
-// (sort_range_kernel) and do without: 137.0 and 137.7, 138.1 and 138.5.
-__device__ __forceinline__ void sort_refine_plan(SortCtl* ctl, int first, bool first_reads_b, int passes, unsigned long long bits) {
-    uint32_t src_b = first_reads_b ? 0u : 1u, nexec = 1;
-    for (int p = first + 1; p < passes; ++p) {
-        const bool skip = ((bits >> (8 * p)) & 0xffull) == 0ull;
-        ctl->skip[p] = skip ? 1u : 0u;
-        if (skip) continue;
-        ctl->src_is_b[p] = src_b;
-        src_b ^= 1u;
-        ++nexec;
-    }
-    ctl->nexec = nexec;
-}
-
 // What the plan says about one pass.  All words are asked for together: read where they are used, each waits for the branch
 // that the one before decides, round trips to memory in front of the keys (sortperm(Int64[1000003]) 138.6 against 136.6 us).
 struct SortStep {
-    uint32_t skip, src_b, first_pass, last_pass, refine;
+    uint32_t skip, src_b, first_pass, last_pass;
     unsigned long long inv_min;
 };
 __device__ __forceinline__ SortStep sort_step(const SortCtl* ctl, int pass) {
-    SortStep s{ctl->skip[pass], ctl->src_is_b[pass], ctl->first_pass, ctl->last_pass, ctl->refine, ctl->inv_min};
-    asm volatile("" : "+s"(s.skip), "+s"(s.src_b), "+s"(s.first_pass), "+s"(s.last_pass), "+s"(s.refine), "+s"(s.inv_min));
+    SortStep s{ctl->skip[pass], ctl->src_is_b[pass], ctl->first_pass, ctl->last_pass, ctl->inv_min};
+    asm volatile("" : "+s"(s.skip), "+s"(s.src_b), "+s"(s.first_pass), "+s"(s.last_pass), "+s"(s.inv_min));
     return s;
 }
 
@@ -253,7 +230,7 @@ __global__ __launch_bounds__(256) void sort_init_kernel(SortCtl* ctl, int all_pa
     __syncthreads();
     if (threadIdx.x == 0) {
         ctl->inv_min = ~0ull;
-        sort_make_plan(ctl, all_passes, false, 0ull, ~0ull, 0ull, first_reads_b);
+        sort_make_plan(ctl, all_passes, false, 0ull, ~0ull, first_reads_b);
     }
 }
 
@@ -300,8 +277,7 @@ __device__ __forceinline__ void for_each_key(const T* __restrict__ keys, int64_t
 
 // ---- smallest and largest key, varying bits -----------------------------------------------------------------------------
 // One read at streaming speed.  Integers are taken relative to the smallest key: small-range integers then need one or two
-// passes.  The workgroup whose ticket is the last makes the plan; for integers it also looks at 64 keys relative to the
-// smallest, which tell nearly always that no further pass can be dropped.
+// passes.  The workgroup whose ticket is the last makes the plan.
 constexpr int RANGE_BLOCK = 1024;       // few, large workgroups: each ends with device-wide atomics on shared words
 template <typename T>
 __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, int rev,
@@ -312,8 +288,6 @@ __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __rest
     constexpr bool RELATIVE = std::is_integral<T>::value;
     __shared__ W part[3][RANGE_BLOCK / WAVE];
     const U u0 = enc_bits<T>(__builtin_bit_cast(U, keys[0]), rev, (U)0);
-    U sample = (U)0;                                         // 64 keys, evenly spread
-    if (RELATIVE && threadIdx.x < WAVE) sample = enc_bits<T>(__builtin_bit_cast(U, keys[(n - 1) * threadIdx.x / (WAVE - 1)]), rev, (U)0);
     U mn = u0, mx = u0, var = 0;
     for_each_key<T>(keys, n, head, nvec, [&](const U (&k)[VEC], int cnt) {
 #pragma unroll
@@ -347,10 +321,8 @@ __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __rest
     }
     if (__builtin_amdgcn_readfirstlane(finishes_last) == 0) return;
     const U smallest = (U)~(U)load_agent(&ctl->inv_min);
-    const W sampled = RELATIVE ? wave_reduce((W)(U)(sample - smallest), OpOr()) : 0ull;
     if (threadIdx.x == 0)
-        sort_make_plan(ctl, (int)sizeof(T), RELATIVE, RELATIVE ? load_agent(&ctl->key_max) - (W)smallest : 0ull, load_agent(&ctl->varying), sampled,
-                       first_reads_b);
+        sort_make_plan(ctl, (int)sizeof(T), RELATIVE, RELATIVE ? load_agent(&ctl->key_max) - (W)smallest : 0ull, load_agent(&ctl->varying), first_reads_b);
 }
 
 // ---- digit counts of every tile -----------------------------------------------------------------------------------
@@ -364,15 +336,13 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
                                                                 SortCtl* ctl, C* __restrict__ tile_count) {
     typedef typename SortKey<T>::U U;
     constexpr int TILE = BLOCK * ITEMS, NW = BLOCK / WAVE;
-    constexpr bool REFINE = std::is_integral<T>::value && sizeof(C) == 2;       // small sorts of integers: sort_refine_plan
     static_assert(sizeof(C) == 4 || TILE < 65536, "a count fits the table's type");
     constexpr int VEC = 16 / (int)sizeof(T), NV = ITEMS / VEC;
     typedef typename VecOf<U, VEC>::type VU;
     __shared__ uint32_t cnt[NW * SUB][256];
-    __shared__ U wave_bits[REFINE ? NW : 1];
     const SortStep step = sort_step(ctl, pass);
     if (step.skip != 0u) return;
-    const bool first = (uint32_t)pass == step.first_pass, refine = REFINE && first && step.refine != 0u;
+    const bool first = (uint32_t)pass == step.first_pass;
     const U* in = first ? (const U*)orig : (step.src_b != 0u ? buf_b : buf_a);
     const U umin = (U)~step.inv_min;
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
@@ -385,7 +355,6 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
     // first lane still in play -- are taken out with a ballot each and added by that lane alone; uniform floats have
     // 50% and 37% of their keys in two values of the exponent digit.
     bool skewed = false;
-    U bits = (U)0;
     auto count = [&](uint32_t d, bool valid, int i) {
         if ((i & 3) == 0) skewed = digits_skewed(d, valid);
         if (skewed) {
@@ -419,7 +388,6 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
             for (int j = 0; j < VEC; ++j) {
                 U k = (U)v[r][j];
                 if (first) k = enc_bits<T>(k, rev, umin);
-                if (REFINE) bits |= k;
                 count(digit_of(k, pass), true, r * VEC + j);
             }
         }
@@ -435,25 +403,10 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             const U k = first ? enc_bits<T>(key[i], rev, umin) : key[i];
-            if (REFINE && woff + i * WAVE < n) bits |= k;
             count(digit_of(k, pass), woff + i * WAVE < n, i);
         }
     }
-    if constexpr (REFINE) {
-        if (refine) {
-            bits = (U)wave_reduce((unsigned long long)bits, OpOr());
-            if (lane == 0) wave_bits[wave] = bits;
-        }
-    }
     __syncthreads();
-    if constexpr (REFINE) {
-        if (refine && tid == 0) {
-            U all = (U)0;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) all |= wave_bits[w];
-            ctl->tile_bits[tile] = (unsigned long long)all;
-        }
-    }
     if (BLOCK > 256 && tid >= 256) return;
     uint32_t c = 0;
 #pragma unroll
@@ -575,15 +528,11 @@ __global__ __launch_bounds__(TS_BLOCK) void sort_tilescan_kernel(SortCtl* ctl, i
 // ---- one pass ----------------------------------------------------------------------------------------------------
 // Tile = BLOCK threads x ITEMS keys.  Wave w owns the w-th part of the tile; its item i of lane l is key
 // i * 64 + l of that part (coalesced loads; the order (i, l) is memory order, which the ranking keeps).
-// DIRECT: `counts` are the raw counts of every tile (uint16, a row of 256 a tile) and the workgroup sums the columns it
+// DIRECT (keys of 2 bytes): `counts` are the raw counts of every tile (uint16, a row of 256 a tile) and the workgroup sums the columns it
 // needs itself; otherwise they are the exclusive counts of sort_tilescan_kernel.
 // waves per SIMD the register allocation aims at: the kernel is bound by its vector instructions, and three or four
 // waves hide the latencies (measured: 4 against 6 workgroups a CU differ by 4%)
 template <typename T, bool PERM, bool DIRECT> constexpr int sort_pass_waves() { return (DIRECT || (!PERM && sizeof(T) <= 4)) ? 4 : 3; }
-
-// One workgroup more than tiles, which in the first pass decides which of the others run, beside the tiles and not in front of
-// them (sort_refine_plan; it writes nothing that the first pass reads).
-template <typename T, bool DIRECT> constexpr bool sort_refines() { return DIRECT && std::is_integral<T>::value; }
 
 template <typename T, int BLOCK, int ITEMS, bool PERM, bool DIRECT>
 __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void sort_pass_kernel(const T* __restrict__ orig, typename SortKey<T>::U* buf_a,
@@ -595,13 +544,11 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
     typedef typename SortKey<T>::U U;
     constexpr int TILE = BLOCK * ITEMS, NW = BLOCK / WAVE;
     constexpr int GROUPS = DIRECT ? BLOCK / 128 : 1;       // groups of rows of the table, 128 lanes (two counts each) a group
-    constexpr bool REFINE = sort_refines<T, DIRECT>();
     __shared__ U lds_keys[TILE];
     __shared__ uint32_t lds_vals[PERM ? TILE : 1];
     __shared__ uint32_t cnt[NW][256];             // per wave and digit: count, then slot in the sorted tile of the wave's first key of the digit
     __shared__ uint32_t goff[256];                // global slot of the digit's first key of this tile, minus its slot in the sorted tile
     __shared__ uint32_t wsum[2][256 / WAVE];
-    __shared__ unsigned long long wave_bits[REFINE ? 256 / WAVE : 1];
     __shared__ uint2 part_before[GROUPS][DIRECT ? 128 : 1], part_all[GROUPS][DIRECT ? 128 : 1];
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
@@ -615,21 +562,6 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
     const bool first = (uint32_t)pass == step.first_pass, last = (uint32_t)pass == step.last_pass;
     const U umin = (U)~step.inv_min;
     const bool src_b = step.src_b != 0u;
-    if constexpr (REFINE) {
-        if (blockIdx.x == ntiles) {               // one workgroup more than tiles: the plan, beside the first pass
-            if (!first || step.refine == 0u) return;
-            const unsigned long long b = wave_reduce((uint32_t)tid < ntiles ? ctl->tile_bits[tid] : 0ull, OpOr());
-            if (tid < 256 && lane == 0) wave_bits[wave] = b;
-            __syncthreads();
-            if (tid == 0) {
-                unsigned long long bits = 0;
-#pragma unroll
-                for (int w = 0; w < 256 / WAVE; ++w) bits |= wave_bits[w];
-                sort_refine_plan(ctl, pass, src_b, (int)sizeof(T), bits);
-            }
-            return;
-        }
-    }
     const U* in = first ? (const U*)orig : (src_b ? buf_b : buf_a);
     U* dst = src_b ? buf_a : buf_b;
     const uint32_t* vsrc = src_b ? val_b : val_a;
@@ -835,6 +767,12 @@ __global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, co
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords; i += (int64_t)gridDim.x * 256) a[i] = from[i];
 }
 
+}  // namespace rk
+
+#include "rk_sort_buckets.hpp"
+
+namespace rk {
+
 // ---- host --------------------------------------------------------------------------------------------------------
 // keys per tile: 256 lanes x 16 (large sorts) or 1024 x 4.  (512 lanes x 16 for large sorts halve the table of counts, tile
 // scan 17.8 -> 15.7 us a pass of Float32[2^26], but the pass itself takes 141 instead of 121 us.)
@@ -843,24 +781,26 @@ constexpr int SORT_ITEMS = (int)SORT_TILE / SORT_BLOCK;
 constexpr int DIRECT_BLOCK = 1024, DIRECT_ITEMS = (int)SORT_TILE / DIRECT_BLOCK;
 // Up to here a pass sums the columns of the table of counts itself.  Every tile reads the counts of all tiles, so that traffic
 // grows with their square: sort!(Float32), summed here / by the tile scan, 0.75 x 2^20 keys 61.4 / 102 us, 2^20 64.6 / 112, 1.5 x
-// 2^20 98 / 117, 2^21 112 / 131, 2^22 267 / 136; Int64 2^20 139 / 249, 2^21 231 / 263, 2^22 560 / 321.  256 tiles are a workgroup
-// a compute unit and one word each in tile_bits; the times alone would allow 512.
+// 2^20 98 / 117, 2^21 112 / 131, 2^22 267 / 136.  256 tiles are a workgroup a compute unit.
 constexpr uint32_t DIRECT_TILES = 256;
 
 struct SortLayout {
     size_t count_off, chunk_total_off, chunk_prefix_off, keys_b_off, keys_a_off, val_a_off, val_b_off, total;
-    uint32_t ntiles, chunk_rows, nchunks;
-    bool direct;
+    size_t compact_off, spl_key_off, spl_pos_off, table_off, tile_min_off;
+    uint32_t ntiles, chunk_rows, nchunks, k;
+    bool tiny, direct, buckets;
 };
 
 static SortLayout sort_layout(size_t key_size, int64_t n, bool perm) {
     SortLayout l{};
     l.ntiles = (uint32_t)((n + SORT_TILE - 1) / SORT_TILE);
     size_t off = (sizeof(SortCtl) + 255) & ~(size_t)255;
+    l.tiny = n <= ST_MAX;
     l.direct = l.ntiles <= DIRECT_TILES;
+    l.buckets = l.direct && !l.tiny && key_size >= 4;
     l.count_off = off;
     if (l.direct) {
-        off += (size_t)l.ntiles * 256 * sizeof(uint16_t);
+        if (!l.buckets && !l.tiny) off += (size_t)l.ntiles * 256 * sizeof(uint16_t);
     } else {
         off += (size_t)l.ntiles * 256 * sizeof(uint32_t);
         l.chunk_rows = (l.ntiles + TS_MAX_CHUNKS - 1) / TS_MAX_CHUNKS;
@@ -875,8 +815,49 @@ static SortLayout sort_layout(size_t key_size, int64_t n, bool perm) {
         l.val_a_off = off; off += vbytes;
         l.val_b_off = off; off += vbytes;
     }
+    if (l.buckets) {
+        l.k = sb_buckets(n);
+        const auto take = [&](size_t bytes) { const size_t at = off; off += (bytes + 255) & ~(size_t)255; return at; };
+        l.compact_off = take((size_t)l.k * SB_OVER * key_size);
+        l.spl_key_off = take((size_t)l.k * key_size);
+        l.spl_pos_off = take((size_t)l.k * 4);
+        l.table_off = take((size_t)l.ntiles * l.k * 4);
+        l.tile_min_off = take((size_t)l.ntiles * key_size);
+    }
     l.total = off;
     return l;
+}
+
+// The kernels of rk_sort_buckets.hpp; the sorted tiles lie in buffer B.  A bucket that is too large for LDS is put together and
+// sorted where its keys end up (sort!, sort) or in buffer A (sortperm).
+template <typename T, bool PERM>
+static int32_t sort_buckets(const SortLayout& l, const void* keys, void* sorted_out, int64_t* perm_out, int64_t n, int rev, char* base, hipStream_t stream) {
+    typedef typename SortKey<T>::U U;
+    static_assert(SB_TILE == SORT_TILE && SB_MAX_TILES == DIRECT_TILES, "ntiles counts both");
+    SortCtl* ctl = (SortCtl*)base;
+    U* spl_key = (U*)(base + l.spl_key_off);
+    uint32_t* spl_pos = (uint32_t*)(base + l.spl_pos_off);
+    uint32_t* table = (uint32_t*)(base + l.table_off);
+    U* tile_min = (U*)(base + l.tile_min_off);
+    U* tile_key = (U*)(base + l.keys_b_off);
+    uint16_t* tile_val = PERM ? (uint16_t*)(base + l.val_b_off) : nullptr;
+    U* big_key = PERM ? (U*)(base + l.keys_a_off) : nullptr;
+    uint32_t* big_val = PERM ? (uint32_t*)(base + l.val_a_off) : nullptr;
+    const uint32_t samples = l.k * SB_OVER;
+    if (samples <= SB_DIRECT_SAMPLES) {
+        sort_splitters_kernel<T, true><<<samples / SB_SPL_EACH, SB_SPL_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, rev, ctl, l.k, nullptr, spl_key, spl_pos);
+    } else {
+        U* compact = (U*)(base + l.compact_off);
+        sort_sample_kernel<T><<<samples / 256, 256, 0, stream>>>((const T*)keys, (uint32_t)n, rev, samples, compact);
+        RK_LAUNCH_CHECK();
+        sort_splitters_kernel<T, false><<<samples / SB_SPL_EACH, SB_SPL_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, rev, ctl, l.k, compact, spl_key, spl_pos);
+    }
+    RK_LAUNCH_CHECK();
+    sort_tile_kernel<T, PERM><<<l.ntiles, SB_TILE_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, rev, l.k, spl_key, spl_pos, table, tile_min, tile_key, tile_val);
+    RK_LAUNCH_CHECK();
+    sort_bucket_kernel<T, PERM><<<l.k, SB_SORT_BLOCK, 0, stream>>>(ctl, l.k, l.ntiles, table, tile_min, rev, tile_key, tile_val, big_key, big_val, (T*)sorted_out, perm_out);
+    RK_LAUNCH_CHECK();
+    return RK_SUCCESS;
 }
 
 // sorted_out: where sort! and sort leave the sorted keys (`keys` itself for sort!)
@@ -894,7 +875,15 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
     uint32_t* val_b = PERM ? (uint32_t*)(base + l.val_b_off) : nullptr;
     const int cus = device_info().cus;
 
+    if (l.tiny) {
+        sort_tiny_kernel<T, PERM><<<1, ST_BLOCK, 0, stream>>>((const T*)keys, (T*)sorted_out, perm_out, (uint32_t)n, rev, ctl);
+        RK_LAUNCH_CHECK();
+        return RK_SUCCESS;
+    }
     constexpr bool FLOAT_KEYS = !std::is_integral<T>::value;
+    if constexpr (sizeof(T) >= 4) {
+        if (l.buckets) return sort_buckets<T, PERM>(l, keys, sorted_out, perm_out, n, rev, base, stream);
+    }
     const bool all_passes = FLOAT_KEYS && !l.direct;
     const int first_reads_b = PERM ? 1 : 0;          // sortperm: the first pass reads the caller's keys and writes buffer A
     sort_init_kernel<<<1, 256, 0, stream>>>(ctl, all_passes ? PASSES : 0, first_reads_b);
@@ -918,23 +907,28 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
     static const int xcd_map = [] { const char* e = std::getenv("RK_SORT_XCD"); return e ? std::atoi(e) : 1; }();
     const unsigned pgrid = (l.ntiles + 7u) & ~7u;
     const uint32_t xcd_chunk = xcd_map != 0 ? (l.ntiles + 7u) / 8u : 0u;
-    for (int p = 0; p < PASSES; ++p) {
-        if (l.direct) {
+    if (l.direct) {
+        if constexpr (sizeof(T) < 4) {
             uint16_t* counts = (uint16_t*)(base + l.count_off);
-            sort_upsweep_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, 1, uint16_t><<<l.ntiles, DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
-            RK_LAUNCH_CHECK();
-            sort_pass_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, PERM, true><<<l.ntiles + (sort_refines<T, true>() ? 1u : 0u), DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, nullptr, 1u, l.ntiles, 0u);
-        } else {
-            uint32_t* counts = (uint32_t*)(base + l.count_off);
-            uint32_t* chunk_total = (uint32_t*)(base + l.chunk_total_off);
-            uint32_t* chunk_prefix = (uint32_t*)(base + l.chunk_prefix_off);
+            for (int p = 0; p < PASSES; ++p) {
+                sort_upsweep_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, 1, uint16_t><<<l.ntiles, DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
+                RK_LAUNCH_CHECK();
+                sort_pass_kernel<T, DIRECT_BLOCK, DIRECT_ITEMS, PERM, true><<<l.ntiles, DIRECT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, nullptr, 1u, l.ntiles, 0u);
+                RK_LAUNCH_CHECK();
+            }
+        }
+    } else {
+        uint32_t* counts = (uint32_t*)(base + l.count_off);
+        uint32_t* chunk_total = (uint32_t*)(base + l.chunk_total_off);
+        uint32_t* chunk_prefix = (uint32_t*)(base + l.chunk_prefix_off);
+        for (int p = 0; p < PASSES; ++p) {
             sort_upsweep_kernel<T, SORT_BLOCK, SORT_ITEMS, 4, uint32_t><<<l.ntiles, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
             RK_LAUNCH_CHECK();
             sort_tilescan_kernel<<<l.nchunks, TS_BLOCK, 0, stream>>>(ctl, p, counts, l.ntiles, l.chunk_rows, chunk_total, chunk_prefix);
             RK_LAUNCH_CHECK();
             sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, chunk_prefix, l.chunk_rows, l.ntiles, xcd_chunk);
+            RK_LAUNCH_CHECK();
         }
-        RK_LAUNCH_CHECK();
     }
     if (!PERM && !(all_passes && PASSES % 2 == 0)) {
         // whole 32-bit words: buffers are 256-byte padded, the caller's array is at least element-aligned; 16-bit keys

@@ -1,0 +1,707 @@
+// Sorts of up to 2^20 keys of 4 and 8 bytes by splitters (included by rk_sort.hip).
+//
+//   sort_sample_kernel     fetches a sample of the keys (larger sorts only; smaller ones fetch it where they rank it)
+//   sort_splitters_kernel  ranks the sample by counting and keeps every SB_OVER-th of it: k - 1 splitters
+//   sort_tile_kernel       sorts every tile of 4096 keys by bucket -- between which splitters a key lies -- and leaves a table
+//                          of where the buckets start in every tile
+//   sort_bucket_kernel     a workgroup a bucket: collects its keys from all tiles, sorts them in LDS and writes the result
+//
+// A radix pass over 10^6 keys is bound by latency, and 8-byte keys take eight of them, one after the other; the four kernels
+// here are as many as two passes take and do not get more with the width of the key.  No key is moved to its bucket: a bucket
+// takes its runs out of the tiles, so nothing has to know the buckets' sizes before it writes.
+// Radix passes -> so, us a call: sortperm Int64[1000003] 136.3 -> 44.4 (kernels 3.5, 6.2, 16.2 and 20.9), Float32 66.0 -> 39.7;
+// sort Float32[1000003] 63.9 -> 33.8, Float64 132 -> 38, Int64 of 20 bits 79.7 -> 38.4; sort Float32[150000] 48.6 -> 26.0.  Each of
+// the kernels moves what it moves in a fraction of its time: what is left is their chains of dependent loads and barriers.
+//
+// Order: keys are compared together with their index -- (key, index) is a strict order -- so equal keys are split between
+// buckets like any others, a bucket's size does not depend on how the keys are distributed, and the permutation is the stable
+// one although no kernel here keeps the order of what it moves.
+//
+// Bucket sizes: a bucket holds the keys between two neighbours among k sampled quantiles, SB_OVER samples apart, so its size
+// is spread like a Gamma variable of that shape around n / k.  LDS has room for SB_CAP keys, 2.75 times n / k at 2^20 keys
+// and more below; one bucket in 2 million is larger (at 2^20 keys; the fewer the keys, the fewer) and is sorted in memory,
+// slowly.  Nothing but the time depends on a bucket's being small.
+#pragma once
+
+#include "rk_common.hpp"
+
+namespace rk {
+
+constexpr uint32_t SB_OVER = 16;                 // samples a bucket
+constexpr uint32_t SB_MAX_K = 256, SB_MAX_TILES = 256;
+constexpr int SB_SPL_BLOCK = 512, SB_SPL_EACH = 16;
+constexpr uint32_t SB_DIRECT_SAMPLES = 1024;     // up to so many samples every workgroup that ranks some fetches all of them
+constexpr int SB_TILE_BLOCK = 1024, SB_TILE_ITEMS = 4, SB_TILE = SB_TILE_BLOCK * SB_TILE_ITEMS;
+constexpr int SB_SORT_BLOCK = 1024, SB_SORT_ITEMS = 11;
+constexpr uint32_t SB_CAP = SB_SORT_BLOCK * SB_SORT_ITEMS;   // keys sorted in LDS
+constexpr uint32_t SB_BINS = 4096;               // of a bucket, in LDS
+constexpr uint32_t SB_MAX_BIN = 32;              // largest bin whose keys are ranked by comparing them with each other
+
+// Buckets of a sort of n keys: a power of two (the search among the splitters has no remainder), n / k <= 512 while that is a
+// workgroup a compute unit at most, n / k <= 4096 at 2^20 keys.
+__host__ __device__ inline uint32_t sb_buckets(int64_t n) {
+    uint32_t k = 4;
+    while ((int64_t)k * 512 < n && k < SB_MAX_K) k *= 2;
+    return k;
+}
+
+// Where the j-th of s samples is taken: somewhere in the j-th of s equal stretches (a multiplicative hash of j decides where),
+// so that samples are in index order and a step that the data repeats is not met in step.
+__device__ __forceinline__ uint32_t sb_sample_pos(uint32_t j, uint32_t s, uint32_t n) {
+    const uint32_t a = (uint32_t)((uint64_t)j * n / s), b = (uint32_t)((uint64_t)(j + 1u) * n / s);
+    uint32_t h = (j + 1u) * 0x9e3779b1u;
+    h ^= h >> 15;
+    h *= 0x85ebca77u;
+    return a + __umulhi(h, b - a);
+}
+
+// ---- splitters -------------------------------------------------------------------------------------------------
+// s = k * SB_OVER samples, all in every workgroup's LDS; a workgroup ranks SB_SPL_EACH of them against all.  s^2 comparisons
+// are 16.8 million at most, 1.3 us of the chip's vector instructions; sorting the samples in one workgroup would leave the
+// others idle for longer.  Also clears what integers record.
+// With many samples it is the fetching that counts -- a line of memory for every sample, in every workgroup -- and a kernel in
+// front packs them (compact).
+template <typename T>
+__global__ __launch_bounds__(256) void sort_sample_kernel(const T* __restrict__ keys, uint32_t n, int rev, uint32_t s, typename SortKey<T>::U* __restrict__ compact) {
+    typedef typename SortKey<T>::U U;
+    const uint32_t j = blockIdx.x * 256u + threadIdx.x;
+    if (j < s) compact[j] = enc_bits<T>(__builtin_bit_cast(U, keys[sb_sample_pos(j, s, n)]), rev, (U)0);
+}
+
+template <typename T, bool DIRECT>
+__global__ __launch_bounds__(SB_SPL_BLOCK) void sort_splitters_kernel(const T* __restrict__ keys, uint32_t n, int rev, SortCtl* ctl, uint32_t k,
+                                                                      const typename SortKey<T>::U* __restrict__ compact,
+                                                                      typename SortKey<T>::U* __restrict__ spl_key, uint32_t* __restrict__ spl_pos) {
+    typedef typename SortKey<T>::U U;
+    constexpr uint32_t PARTS = SB_SPL_BLOCK / SB_SPL_EACH, MOST = DIRECT ? SB_DIRECT_SAMPLES : SB_MAX_K * SB_OVER, UNR = MOST / SB_SPL_BLOCK;
+    __shared__ U smp[MOST];
+    __shared__ uint32_t below[SB_SPL_EACH];
+    const uint32_t tid = threadIdx.x, s = k * SB_OVER;
+    U v[UNR];
+#pragma unroll
+    for (uint32_t u = 0; u < UNR; ++u) {
+        uint32_t j = tid + u * SB_SPL_BLOCK;
+        j = j < s ? j : s - 1u;
+        v[u] = DIRECT ? __builtin_bit_cast(U, keys[sb_sample_pos(j, s, n)]) : compact[j];
+    }
+    if (blockIdx.x == 0 && tid == 0) { ctl->varying = 0ull; ctl->nexec = 0u; }
+    if (tid < SB_SPL_EACH) below[tid] = 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < UNR; ++u) {
+        const uint32_t j = tid + u * SB_SPL_BLOCK;
+        if (j < s) smp[j] = DIRECT ? enc_bits<T>(v[u], rev, (U)0) : v[u];
+    }
+    __syncthreads();
+    // of the samples in front an equal one counts as smaller
+    const uint32_t j0 = blockIdx.x * SB_SPL_EACH, j = j0 + tid % SB_SPL_EACH, i0 = tid / SB_SPL_EACH;
+    const U mine = smp[j];
+    uint32_t c = 0, i = i0;
+#pragma unroll 8
+    for (; i < j0; i += PARTS) c += smp[i] <= mine ? 1u : 0u;
+    if (i < j0 + SB_SPL_EACH) {                              // (PARTS >= SB_SPL_EACH: once at most)
+        const U x = smp[i];
+        c += (x < mine || (x == mine && i < j)) ? 1u : 0u;
+        i += PARTS;
+    }
+#pragma unroll 8
+    for (; i < s; i += PARTS) c += smp[i] < mine ? 1u : 0u;
+    atomicAdd(&below[tid % SB_SPL_EACH], c);
+    __syncthreads();
+    if (tid < SB_SPL_EACH) {
+        const uint32_t r = below[tid];
+        if (r != 0u && r % SB_OVER == 0u) {
+            spl_key[r / SB_OVER - 1u] = mine;
+            spl_pos[r / SB_OVER - 1u] = sb_sample_pos(j, s, n);
+        }
+    }
+}
+
+// ---- tiles --------------------------------------------------------------------------------------------------------
+// Every key searches the splitters in LDS, takes its place among the tile's keys of the bucket with an LDS atomic (their order
+// does not matter), and the tile is written in the order of the buckets (sortperm: with the keys' indices in the tile).
+// table[tile][bucket] = where the bucket starts in the tile | its size << 16.  Summed down the tiles that is also how many keys
+// lie in the buckets in front and how many in the bucket, so no workgroup adds to anything that others add to.
+template <typename T, bool PERM>
+__global__ __launch_bounds__(SB_TILE_BLOCK) void sort_tile_kernel(const T* __restrict__ keys, uint32_t n, int rev, uint32_t k,
+                                                                  const typename SortKey<T>::U* __restrict__ spl_key,
+                                                                  const uint32_t* __restrict__ spl_pos, uint32_t* __restrict__ table,
+                                                                  typename SortKey<T>::U* __restrict__ tile_min, typename SortKey<T>::U* __restrict__ tile_key,
+                                                                  uint16_t* __restrict__ tile_val) {
+    typedef typename SortKey<T>::U U;
+    constexpr int BLOCK = SB_TILE_BLOCK, ITEMS = SB_TILE_ITEMS;
+    constexpr bool RECORD = std::is_integral<T>::value;
+    __shared__ U lds_key[SB_TILE];
+    __shared__ uint16_t lds_val[PERM ? SB_TILE : 1];
+    __shared__ U skey[SB_MAX_K];
+    __shared__ uint32_t spos[SB_MAX_K], cnt[SB_MAX_K], wsum[SB_MAX_K / WAVE];
+    __shared__ U part[RECORD ? BLOCK / WAVE : 1];
+    const uint32_t tid = threadIdx.x, e0 = blockIdx.x * (uint32_t)SB_TILE;
+    U key[ITEMS];
+    uint32_t bucket[ITEMS], rank[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t e = e0 + tid + i * BLOCK;
+        key[i] = __builtin_bit_cast(U, keys[e < n ? e : n - 1u]);
+    }
+    if (tid < k) {
+        skey[tid] = tid < k - 1u ? spl_key[tid] : (U)0;
+        spos[tid] = tid < k - 1u ? spl_pos[tid] : 0u;
+        cnt[tid] = 0u;
+    }
+    __syncthreads();
+    bool tie = false;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) { key[i] = enc_bits<T>(key[i], rev, (U)0); bucket[i] = 0u; }
+    // splitters below the key: the searches of a lane's keys go side by side
+    for (uint32_t step = k / 2u; step != 0u; step /= 2u) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) bucket[i] += skey[bucket[i] + step - 1u] < key[i] ? step : 0u;
+    }
+    // one that equals the key: the index decides
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) tie = tie || (bucket[i] < k - 1u && skey[bucket[i]] == key[i]);
+    if (tie) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t e = e0 + tid + i * BLOCK;
+            uint32_t b = 0u;
+            for (uint32_t step = k / 2u; step != 0u; step /= 2u) {
+                const U x = skey[b + step - 1u];
+                b += (x < key[i] || (x == key[i] && spos[b + step - 1u] <= e)) ? step : 0u;
+            }
+            bucket[i] = b;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        rank[i] = 0u;
+        if (e0 + tid + i * BLOCK < n) rank[i] = atomicAdd(&cnt[bucket[i]], 1u);
+    }
+    if constexpr (RECORD) {                                  // the smallest key (those past the end are the last one again)
+        U x = key[0];
+#pragma unroll
+        for (int i = 1; i < ITEMS; ++i) x = key[i] < x ? key[i] : x;
+        x = wave_reduce(x, OpMin());
+        if (tid % WAVE == 0) part[tid / WAVE] = x;
+    }
+    __syncthreads();
+    uint32_t c = 0u, inc = 0u;
+    if (tid < SB_MAX_K) {
+        if (tid < k) c = cnt[tid];
+        inc = wave_scan_inclusive(c, OpAdd(), 0u);
+        if (tid % WAVE == WAVE - 1) wsum[tid / WAVE] = inc;
+    }
+    __syncthreads();
+    if (tid < k) {
+        uint32_t start = inc - c;
+        for (uint32_t w = 0; w < tid / WAVE; ++w) start += wsum[w];
+        cnt[tid] = start;
+        table[blockIdx.x * k + tid] = start | c << 16;
+    }
+    if constexpr (RECORD) {
+        if (tid >= BLOCK - WAVE) {
+            const U x = wave_reduce(part[tid % (BLOCK / WAVE)], OpMin());
+            if (tid == BLOCK - WAVE) tile_min[blockIdx.x] = x;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (e0 + tid + i * BLOCK < n) {
+            const uint32_t p = cnt[bucket[i]] + rank[i];
+            lds_key[p] = key[i];
+            if constexpr (PERM) lds_val[p] = (uint16_t)(tid + i * BLOCK);
+        }
+    }
+    __syncthreads();
+    const uint32_t m = n - e0 < (uint32_t)SB_TILE ? n - e0 : (uint32_t)SB_TILE;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t p = tid + i * BLOCK;
+        if (p < m) {
+            tile_key[e0 + p] = lds_key[p];
+            if constexpr (PERM) tile_val[e0 + p] = lds_val[p];
+        }
+    }
+}
+
+// ---- radix passes in LDS ------------------------------------------------------------------------------------------
+// One stable pass over m keys of a workgroup of 16 waves by an 8-bit digit: item i of lane l of wave w is element
+// (w * per + i) * 64 + l, before and after; `per` items a lane are in use.  cnt: 16 x 256 words.
+template <bool PERM, int ITEMS, typename U, typename Digit>
+__device__ __forceinline__ void sb_radix_pass(U (&key)[ITEMS], uint32_t (&val)[PERM ? ITEMS : 1], uint32_t per, uint32_t m, Digit&& digit, U* lds_key,
+                                              uint32_t* lds_val, uint32_t* cnt, uint32_t* wsum) {
+    constexpr int BLOCK = 1024, NW = BLOCK / WAVE;
+    const uint32_t tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, first = wave * per * WAVE + lane;
+    uint32_t* wcnt = cnt + wave * 256u;
+    uint32_t rank[ITEMS];
+    *(uint4*)&cnt[tid * 4u] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if ((uint32_t)i >= per) continue;
+        const bool valid = first + i * WAVE < m;
+        const uint32_t d = digit(key[i], val[PERM ? i : 0]);
+        uint32_t same_lo, same_hi;
+        match_digit_halves(d, same_lo, same_hi);
+        const uint64_t vm = __ballot(valid);
+        same_lo &= (uint32_t)vm;
+        same_hi &= (uint32_t)(vm >> 32);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
+        rank[i] = __hip_atomic_load(&wcnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) + below;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && below == 0u)
+            __hip_atomic_fetch_add(&wcnt[d], (uint32_t)__builtin_popcount(same_lo) + (uint32_t)__builtin_popcount(same_hi), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint32_t total = 0u, inc = 0u;
+    if (tid < 256u) {
+        for (int w = 0; w < NW; ++w) total += cnt[w * 256 + tid];
+        inc = wave_scan_inclusive(total, OpAdd(), 0u);
+        if (lane == WAVE - 1) wsum[wave] = inc;
+    }
+    __syncthreads();
+    if (tid < 256u) {
+        uint32_t at = inc - total;
+        for (uint32_t w = 0; w < wave; ++w) at += wsum[w];
+        for (int w = 0; w < NW; ++w) {
+            const uint32_t c = cnt[w * 256 + tid];
+            cnt[w * 256 + tid] = at;
+            at += c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if ((uint32_t)i < per && first + i * WAVE < m) {
+            const uint32_t p = wcnt[digit(key[i], val[PERM ? i : 0])] + rank[i];
+            lds_key[p] = key[i];
+            if constexpr (PERM) lds_val[p] = val[i];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if ((uint32_t)i < per && first + i * WAVE < m) {
+            key[i] = lds_key[first + i * WAVE];
+            if constexpr (PERM) val[i] = lds_val[first + i * WAVE];
+        }
+    }
+}
+
+// Integers: the digits in which the keys minus the smallest differ are counted for whoever looks at the temporary (ctl->nexec: as
+// many passes would a radix sort take).  A digit is counted by the workgroup whose bits are the first in it; most find all of
+// theirs there already.
+template <typename U> __device__ __forceinline__ void sb_record_digits(SortCtl* ctl, U bits, U* part) {
+    bits = wave_reduce(bits, OpOr());
+    if (lane_id() == 0) part[threadIdx.x / WAVE] = bits;
+    __syncthreads();
+    if (threadIdx.x >= WAVE) return;
+    bits = wave_reduce(part[lane_id() % (SB_SORT_BLOCK / WAVE)], OpOr());
+    if (threadIdx.x != 0 || (bits & ~(U)load_agent(&ctl->varying)) == (U)0) return;
+    const U old = (U)atomicOr(&ctl->varying, (unsigned long long)bits), all = old | bits;
+    uint32_t digits = 0u;
+    for (int p = 0; p < (int)sizeof(U); ++p) digits += digit_of(all, p) != 0u && digit_of(old, p) == 0u ? 1u : 0u;
+    if (digits != 0u) atomicAdd(&ctl->nexec, digits);
+}
+
+// ---- a bucket ------------------------------------------------------------------------------------------------------
+// Bitonic sort of x[0, m) (with y) by the whole workgroup, in LDS or in memory.  The variant whose comparisons all put the
+// smaller element first: elements from m on would be larger than any and never move, so they need not exist.
+template <bool PERM, typename U>
+__device__ __forceinline__ void sb_bitonic(U* x, uint32_t* y, uint32_t m) {
+    uint32_t half = 1u;
+    while (half * 2u < m) half *= 2u;
+    auto order = [&](uint32_t a, uint32_t b) {
+        if (b >= m) return;
+        const U xa = x[a], xb = x[b];
+        if constexpr (PERM) {
+            const uint32_t ya = y[a], yb = y[b];
+            if (xb < xa || (xb == xa && yb < ya)) { x[a] = xb; x[b] = xa; y[a] = yb; y[b] = ya; }
+        } else {
+            if (xb < xa) { x[a] = xb; x[b] = xa; }
+        }
+    };
+    for (uint32_t h = 1u; h <= half; h *= 2u) {              // runs of h become runs of 2 h
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < half; i += blockDim.x) {
+            const uint32_t o = i & (h - 1u), a = (i - o) * 2u;
+            order(a + o, a + 2u * h - 1u - o);
+        }
+        for (uint32_t j = h / 2u; j != 0u; j /= 2u) {
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < half; i += blockDim.x) {
+                const uint32_t o = i & (j - 1u), a = (i - o) * 2u + o;
+                order(a, a + j);
+            }
+        }
+    }
+    __syncthreads();
+}
+
+// Inside a bucket the keys are spread over SB_BINS bins by a monotone, nearly linear map of their distance from the smallest
+// (few values, many times over: with the index behind it), in no order, and a key's place in its bin is the number of smaller keys there: a
+// bin holds a key or two, and a wave compares as often as the largest bin it meets has keys.
+// Should a bin exceed SB_MAX_BIN -- a bucket around zero, where the keys of floats are far from linear; a few values many times
+// over -- every bin is divided once more into as many as it has keys, by where a key lies in it (bins of equal keys: by the
+// index; without one they need no order).  What even that does not spread is sorted by comparisons, still in LDS.
+template <typename T, bool PERM>
+__global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl, uint32_t k, uint32_t ntiles, const uint32_t* __restrict__ table,
+                                                                    const typename SortKey<T>::U* __restrict__ tile_min, int rev,
+                                                                    const typename SortKey<T>::U* __restrict__ tile_key, const uint16_t* __restrict__ tile_val,
+                                                                    typename SortKey<T>::U* big_key, uint32_t* big_val, T* sorted_out, int64_t* perm_out) {
+    typedef typename SortKey<T>::U U;
+    constexpr int BLOCK = SB_SORT_BLOCK, ITEMS = SB_SORT_ITEMS, NW = BLOCK / WAVE, PER = (int)SB_BINS / BLOCK;
+    constexpr bool RECORD = std::is_integral<T>::value;
+    static_assert(PER == 4, "a thread scans four bins");
+    // keys and indices of the bucket; while it is divided a second time, a key of every bin, its lowest and highest index, and the
+    // sizes of the new bins
+    constexpr size_t KEYS = (size_t)SB_CAP * sizeof(U), POOL = KEYS + (PERM ? (size_t)SB_CAP * 4 : 0), DIVIDE = (size_t)SB_BINS * (sizeof(U) + (PERM ? 8 : 0)) + (size_t)SB_CAP * 4;
+    __shared__ alignas(16) char pool[POOL > DIVIDE ? POOL : DIVIDE];
+    U* const lds_key = (U*)pool;
+    uint32_t* const lds_val = (uint32_t*)(pool + KEYS);      // (sortperm only)
+    U* const rep = (U*)pool;
+    uint32_t* const sub = (uint32_t*)(pool + (size_t)SB_BINS * sizeof(U));
+    uint32_t* const bin_vlo = sub + SB_CAP;                  // (sortperm only)
+    uint32_t* const bin_vhi = bin_vlo + SB_BINS;
+    __shared__ alignas(16) uint32_t bins[SB_BINS + 4];
+    __shared__ uint32_t part[4][NW];
+    __shared__ U part_key[2][NW];
+    uint32_t* const run_off = bins;                          // of a tile: keys of the bucket in the tiles in front (read before bins are)
+    uint32_t* const run_at = bins + SB_MAX_TILES;            // where the bucket starts in it
+    static_assert(2u * SB_MAX_TILES <= SB_BINS && SB_MAX_TILES <= (uint32_t)BLOCK, "a thread a tile");
+    const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, bucket = blockIdx.x;
+    uint32_t entry = 0u;
+    U smallest = (U)~(U)0;                                   // of all keys (integers)
+    if (tid < ntiles) {
+        entry = table[tid * k + bucket];
+        if (RECORD) smallest = tile_min[tid];
+    }
+    const uint32_t before = wave_reduce(entry & 0xffffu, OpAdd());
+    if constexpr (RECORD) {
+        smallest = wave_reduce(smallest, OpMin());
+        if (lane == 0) part_key[0][wave] = smallest;
+    }
+    const uint32_t run = wave_scan_inclusive(entry >> 16, OpAdd(), 0u);
+    if (lane == 0) part[0][wave] = before;
+    if (lane == WAVE - 1) part[1][wave] = run;
+    __syncthreads();
+    uint32_t start = 0u, off = run - (entry >> 16), m = 0u;
+#pragma unroll
+    for (int w = 0; w < (int)SB_MAX_TILES / WAVE; ++w) {
+        start += part[0][w];
+        if ((uint32_t)w < wave) off += part[1][w];
+        m += part[1][w];
+        if (RECORD) smallest = part_key[0][w] < smallest ? part_key[0][w] : smallest;
+    }
+    if (tid < SB_MAX_TILES) {
+        run_off[tid] = tid < ntiles ? off : ~0u;
+        run_at[tid] = entry & 0xffffu;
+    }
+    __syncthreads();
+    // the p-th key of the bucket: in the last tile with no more than p keys in front of it
+    auto find = [&](uint32_t p, uint32_t& tile) -> uint32_t {
+        tile = 0u;
+#pragma unroll
+        for (uint32_t step = SB_MAX_TILES / 2u; step != 0u; step /= 2u) tile += run_off[tile + step] <= p ? step : 0u;
+        return tile * (uint32_t)SB_TILE + run_at[tile] + (p - run_off[tile]);
+    };
+    if (m > SB_CAP) {                                        // too large for LDS: compared in memory, slowly
+        U* x = PERM ? big_key + start : (U*)sorted_out + start;
+        uint32_t* y = PERM ? big_val + start : nullptr;
+        for (uint32_t p = tid; p < m; p += BLOCK) {
+            uint32_t tile;
+            const uint32_t at = find(p, tile);
+            x[p] = tile_key[at];
+            if constexpr (PERM) y[p] = tile * (uint32_t)SB_TILE + tile_val[at];
+        }
+        sb_bitonic<PERM>(x, y, m);
+        U bits = (U)0;
+        for (uint32_t i = tid; i < m; i += BLOCK) {
+            const U u = x[i];
+            if constexpr (RECORD) bits |= (U)(u - smallest);
+            if constexpr (PERM) perm_out[start + i] = (int64_t)y[i] + 1;
+            else sorted_out[start + i] = dec_bits<T>(u, rev, (U)0);
+        }
+        if constexpr (RECORD) sb_record_digits<U>(ctl, bits, part_key[1]);
+        return;
+    }
+    U key[ITEMS], lo = (U)~(U)0, hi = (U)0;
+    uint32_t val[PERM ? ITEMS : 1], rank[ITEMS], vlo = ~0u, vhi = 0u;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if ((uint32_t)(i * BLOCK) < m) {
+            const uint32_t p = tid + i * BLOCK;
+            uint32_t tile;
+            const uint32_t at = find(p < m ? p : 0u, tile);
+            key[i] = tile_key[at];
+            if constexpr (PERM) val[i] = tile * (uint32_t)SB_TILE + tile_val[at];
+        }
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);             // searches four at a time: eleven take too many registers
+    }
+    __syncthreads();
+    *(uint4*)&bins[tid * 4] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if ((uint32_t)(i * BLOCK) < m) {
+            lo = key[i] < lo ? key[i] : lo;
+            hi = key[i] > hi ? key[i] : hi;
+            if constexpr (PERM) {
+                vlo = val[i] < vlo ? val[i] : vlo;
+                vhi = val[i] > vhi ? val[i] : vhi;
+            }
+        }
+    }
+    lo = wave_reduce(lo, OpMin());
+    hi = wave_reduce(hi, OpMax());
+    if (lane == 0) { part_key[0][wave] = lo; part_key[1][wave] = hi; }
+    if constexpr (PERM) {
+        vlo = wave_reduce(vlo, OpMin());
+        vhi = wave_reduce(vhi, OpMax());
+        if (lane == 0) { part[2][wave] = vlo; part[3][wave] = vhi; }
+    }
+    __syncthreads();
+    lo = wave_reduce(part_key[0][lane % NW], OpMin());
+    hi = wave_reduce(part_key[1][lane % NW], OpMax());
+    if constexpr (PERM) {
+        vlo = wave_reduce(part[2][lane % NW], OpMin());
+        vhi = wave_reduce(part[3][lane % NW], OpMax());
+    }
+    // distance of a key from the smallest; with its index in the low bits if that fits 32: then no two are equal
+    const uint64_t span = (uint64_t)(U)(hi - lo);
+    const uint32_t vspan = vhi - vlo, vbits = !PERM || vspan == 0u ? 0u : 32u - (uint32_t)__clz((int)vspan);
+    const bool both = PERM && (span >> (32u - vbits)) == 0ull;         // (vbits <= 20)
+    const uint64_t width = both ? span << vbits | vspan : span;
+    const uint32_t shift = width >> 32 ? 32u - (uint32_t)__clz((int)(uint32_t)(width >> 32)) : 0u;
+    const uint32_t w32 = (uint32_t)(width >> shift);
+    const bool exact = shift == 0u && w32 < SB_BINS;                   // a bin is one value
+    // w32 * scale < SB_BINS * 2^32: the last bin is SB_BINS - 1
+    const uint32_t scale = exact ? 0u : (uint32_t)((double)SB_BINS * 4294967296.0 / ((double)w32 + 1.0));
+    auto distance = [&](U x, uint32_t v) -> uint32_t {
+        asm volatile("" : "+v"(x));                // computed again at every use: kept, the bins of eleven keys spilled 20 registers
+        return both ? (uint32_t)(U)(x - lo) << vbits | (v - vlo) : (uint32_t)((uint64_t)(U)(x - lo) >> shift);
+    };
+    auto bin_of = [&](U x, uint32_t v) -> uint32_t { return exact ? distance(x, v) : __umulhi(distance(x, v), scale); };
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        rank[i] = 0u;
+        if (tid + i * BLOCK < m) rank[i] = atomicAdd(&bins[bin_of(key[i], val[PERM ? i : 0])], 1u);
+    }
+    __syncthreads();
+    const uint4 c = *(const uint4*)&bins[tid * 4];
+    const uint32_t sum = c.x + c.y + c.z + c.w, c01 = c.x > c.y ? c.x : c.y, c23 = c.z > c.w ? c.z : c.w;
+    const uint32_t inc = wave_scan_inclusive(sum, OpAdd(), 0u);
+    const uint32_t most = wave_reduce(c01 > c23 ? c01 : c23, OpMax());
+    if (lane == WAVE - 1) { part[0][wave] = inc; part[1][wave] = most; }
+    __syncthreads();
+    uint32_t first = inc - sum, largest = 0u;
+    for (int w = 0; w < NW; ++w) {
+        if ((uint32_t)w < wave) first += part[0][w];
+        largest = part[1][w] > largest ? part[1][w] : largest;
+    }
+    *(uint4*)&bins[tid * 4] = make_uint4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
+    if (tid == 0) bins[SB_BINS] = m;
+    __syncthreads();
+    const bool ordered = exact && (!PERM || both);                     // a bin holds equal keys (one index): nothing to compare
+    const bool divide = !ordered && largest > SB_MAX_BIN;
+    bool compare = false;
+    if (divide) {
+        // which bins hold different keys (bit 31), then the division
+        for (uint32_t i = tid; i < SB_CAP; i += BLOCK) sub[i] = 0u;
+        if constexpr (PERM) {
+            for (uint32_t i = tid; i < SB_BINS; i += BLOCK) { bin_vlo[i] = ~0u; bin_vhi[i] = 0u; }
+        }
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+            if (tid + i * BLOCK < m) rep[bin_of(key[i], val[PERM ? i : 0])] = key[i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (tid + i * BLOCK < m) {
+                const uint32_t b = bin_of(key[i], val[PERM ? i : 0]);
+                if (rep[b] != key[i]) atomicOr(&bins[b], 0x80000000u);
+                if constexpr (PERM) {
+                    atomicMin(&bin_vlo[b], val[PERM ? i : 0]);
+                    atomicMax(&bin_vhi[b], val[PERM ? i : 0]);
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (tid + i * BLOCK < m) {
+                const uint32_t d = distance(key[i], val[PERM ? i : 0]), b = exact ? d : __umulhi(d, scale);
+                const uint32_t q = bins[b], q0 = q & 0x7fffffffu, size = (bins[b + 1u] & 0x7fffffffu) - q0;
+                uint32_t id;
+                if (both || q >> 31) id = q0 + __umulhi(d * scale, size);
+                else if constexpr (PERM) {
+                    const uint32_t from = bin_vlo[b], spread = bin_vhi[b] - from;
+                    id = q0 + __umulhi((val[PERM ? i : 0] - from) << (spread == 0u ? 0 : __clz((int)spread)), size);
+                }
+                else id = q0 + rank[i];
+                rank[i] = id | atomicAdd(&sub[id], 1u) << 16;
+            }
+        }
+        __syncthreads();
+        uint32_t s[ITEMS], total = 0u, top = 0u;
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            s[i] = sub[tid * ITEMS + i];
+            total += s[i];
+            top = s[i] > top ? s[i] : top;
+        }
+        const uint32_t run2 = wave_scan_inclusive(total, OpAdd(), 0u);
+        top = wave_reduce(top, OpMax());
+        if (lane == WAVE - 1) { part[2][wave] = run2; part[3][wave] = top; }
+        __syncthreads();
+        uint32_t at = run2 - total;
+        largest = 0u;
+        for (int w = 0; w < NW; ++w) {
+            if ((uint32_t)w < wave) at += part[2][w];
+            largest = part[3][w] > largest ? part[3][w] : largest;
+        }
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            sub[tid * ITEMS + i] = at | s[i] << 16;
+            at += s[i];
+        }
+        __syncthreads();
+        compare = largest > SB_MAX_BIN;
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (tid + i * BLOCK < m) {                                 // place in the bucket | place in the bin << 16 | size of the bin << 22
+                const uint32_t q = sub[rank[i] & 0xffffu], r = rank[i] >> 16;
+                rank[i] = ((q & 0xffffu) + r) | (compare ? 0u : r << 16 | (q >> 16) << 22);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (tid + i * BLOCK < m) {
+            const uint32_t p = divide ? rank[i] & 0xffffu : bins[bin_of(key[i], val[PERM ? i : 0])] + rank[i];
+            lds_key[p] = key[i];
+            if constexpr (PERM) lds_val[p] = val[i];
+        }
+    }
+    __syncthreads();
+    auto smaller = [&](U x, uint32_t v, uint32_t q0, uint32_t q1) -> uint32_t {        // of the elements [q0, q1)
+        uint32_t r = 0u;
+        for (uint32_t q = q0; q < q1; ++q) {
+            const U o = lds_key[q];
+            const uint32_t ov = PERM ? lds_val[PERM ? q : 0] : q;
+            r += (o < x || (o == x && ov < v)) ? 1u : 0u;
+        }
+        return r;
+    };
+    auto store = [&](uint32_t to, U x, uint32_t v) {
+        if constexpr (PERM) perm_out[start + to] = (int64_t)v + 1;
+        else sorted_out[start + to] = dec_bits<T>(x, rev, (U)0);
+    };
+    U bits = (U)0;
+    if constexpr (RECORD) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+            if ((uint32_t)(i * BLOCK) < m) bits |= (U)(key[i] - smallest);
+    }
+    if (divide && !compare) {                                           // the keys of this thread as it holds them
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (tid + i * BLOCK < m) {
+                const uint32_t p = rank[i] & 0xffffu, q0 = p - ((rank[i] >> 16) & 0x3fu);
+                const uint32_t v = PERM ? val[PERM ? i : 0] : p;
+                store(q0 + smaller(key[i], v, q0, q0 + (rank[i] >> 22)), key[i], v);
+            }
+        }
+    } else {
+        if (compare) sb_bitonic<PERM>(lds_key, lds_val, m);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t p = tid + i * BLOCK;
+            if (p >= m) continue;
+            const U x = lds_key[p];
+            const uint32_t v = PERM ? lds_val[PERM ? p : 0] : p;
+            if (ordered || compare) {
+                store(p, x, v);
+            } else {
+                const uint32_t b = bin_of(x, v), q0 = bins[b];
+                store(q0 + smaller(x, v, q0, bins[b + 1u]), x, v);
+            }
+        }
+    }
+    if constexpr (RECORD) sb_record_digits<U>(ctl, bits, part_key[1]);
+}
+
+// ---- sorts that fit a workgroup ---------------------------------------------------------------------------------------
+// Up to 4096 keys: radix passes with everything in LDS, one kernel instead of ten or eighteen (sort Float64[1000] 63 -> 16.5 us a
+// call, Float64[4096] 66 -> 25, Float32[4096] 42 -> 16.5).  A digit in which no
+// two keys differ (integers: relative to the smallest) takes no pass.
+constexpr int ST_BLOCK = 1024, ST_ITEMS = 4, ST_MAX = ST_BLOCK * ST_ITEMS;
+
+template <typename T, bool PERM>
+__global__ __launch_bounds__(ST_BLOCK) void sort_tiny_kernel(const T* orig, T* sorted_out, int64_t* perm_out, uint32_t n, int rev, SortCtl* ctl) {
+    typedef typename SortKey<T>::U U;
+    constexpr int BLOCK = ST_BLOCK, ITEMS = ST_ITEMS, NW = BLOCK / WAVE;
+    constexpr bool RELATIVE = std::is_integral<T>::value;
+    __shared__ U lds_key[ST_MAX];
+    __shared__ uint32_t lds_val[PERM ? ST_MAX : 1];
+    __shared__ alignas(16) uint32_t cnt[NW * 256];
+    __shared__ uint32_t wsum[256 / WAVE];
+    __shared__ unsigned long long part[2][NW];
+    const uint32_t tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, per = (n + BLOCK - 1) / BLOCK, first = wave * per * WAVE + lane;
+    U key[ITEMS];
+    uint32_t val[PERM ? ITEMS : 1];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t e = first + i * WAVE;
+        key[i] = __builtin_bit_cast(U, orig[e < n ? e : n - 1u]);
+        if constexpr (PERM) val[i] = e;
+    }
+    U base = enc_bits<T>(__builtin_bit_cast(U, orig[0]), rev, (U)0);
+    unsigned long long inv = 0ull;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        key[i] = enc_bits<T>(key[i], rev, (U)0);
+        const unsigned long long v = (unsigned long long)(U)~key[i];
+        inv = v > inv ? v : inv;
+    }
+    if constexpr (RELATIVE) {
+        inv = wave_reduce(inv, OpMax());
+        if (lane == 0) part[0][wave] = inv;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) inv = part[0][w] > inv ? part[0][w] : inv;
+        base = (U)~(U)inv;
+    }
+    U mine = (U)0;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        mine |= RELATIVE ? (U)(key[i] - base) : (U)(key[i] ^ base);
+        if (RELATIVE) key[i] = (U)(key[i] - base);
+    }
+    unsigned long long bits = wave_reduce((unsigned long long)mine, OpOr());
+    if (lane == 0) part[1][wave] = bits;
+    __syncthreads();
+    bits = 0ull;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) bits |= part[1][w];
+    uint32_t ran = 0u;
+    for (int pass = 0; pass < (int)sizeof(T); ++pass) {
+        if (((bits >> (8 * pass)) & 0xffull) == 0ull) continue;
+        ++ran;
+        sb_radix_pass<PERM, ITEMS>(key, val, per, n, [&](U x, uint32_t) { return digit_of(x, pass); }, lds_key, lds_val, cnt, wsum);
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const uint32_t e = first + i * WAVE;
+        if ((uint32_t)i < per && e < n) {
+            if constexpr (PERM) perm_out[e] = (int64_t)val[i] + 1;
+            else sorted_out[e] = dec_bits<T>(key[i], rev, RELATIVE ? base : (U)0);
+        }
+    }
+    if (tid == 0) ctl->nexec = ran;
+}
+
+}  // namespace rk

@@ -290,3 +290,56 @@ def test_sort_keeps_nan_bit_patterns(rk, dtype, utype, rev):
     nan_part = perm[:nn] if rev else perm[n - nn:]
     assert np.array_equal(nan_part, np.flatnonzero(np.isnan(h)))                          # stable among the NaNs
     assert np.array_equal(np.sort(perm), np.arange(n))
+
+
+def _spread(rng, dtype, n, kind):
+    """Keys that a bucket of the sorts by splitters does not find evenly spread, and some that it does."""
+    dt = np.dtype(dtype)
+    if kind == "sorted":
+        return np.sort(_rand(rng, dtype, n))
+    if kind == "equal":
+        return np.full(n, 3, dtype=dt)
+    if kind == "few":                                   # a few values, far apart and close together
+        return rng.choice(np.array([-70000, -3, -2, 0, 1, 2, 3, 1000, 65536], dtype=dt), n)
+    if kind == "hundreds":
+        return rng.integers(-500, 500, n).astype(dt)
+    if kind == "clusters":                              # narrow clusters and far outliers: what a linear map does not spread
+        x = rng.integers(0, 200, n) * 3 + rng.choice(np.array([0, 1 << 20, (1 << 20) + 5000], dtype=np.int64), n)
+        x[:: n // 7] = 1 << 30
+        return x.astype(dt)
+    if kind == "steep":                                 # every order of magnitude, both signs
+        x = np.exp(rng.uniform(-20, 20, n)) * rng.choice([-1.0, 1.0], n)
+        return x.astype(dt)
+    return (rng.standard_normal(n) * (1 if dt.kind == "f" else 1 << 24)).astype(dt)
+
+
+@pytest.mark.parametrize("kind", ["sorted", "equal", "few", "hundreds", "clusters", "steep", "normal"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+def test_sorts_by_splitters(rk, orc, dtype, kind):
+    """4096 keys are the last that fit a workgroup, 2^20 the last that take buckets; 512 keys a bucket up to 131072 and more
+    beyond; tiles of 4096."""
+    rng = np.random.default_rng(31)
+    for n in (4095, 4096, 4097, 8193, 66_001, 131_073, (1 << 20) - 1, 1 << 20, (1 << 20) + 1):
+        x = _spread(rng, dtype, n, kind)
+        for rev in (False, True):
+            assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(x), rev=rev)), orc.sort(x, rev)), (n, rev)
+            assert np.array_equal(rk.Array(rk.sortperm(rk.ROCArray(x), rev=rev)), orc.sortperm(x, rev)), (n, rev)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
+@pytest.mark.parametrize("few", [False, True])
+def test_bucket_larger_than_lds(rk, orc, dtype, few):
+    """Every key that is sampled is larger than all the others, so these are one bucket: more keys than LDS holds."""
+    n, k = 30_000, 64
+    s = 16 * k
+    pos = []
+    for j in range(s):
+        a, b = j * n // s, (j + 1) * n // s
+        h = (j + 1) * 0x9e3779b1 & 0xffffffff
+        h ^= h >> 15
+        h = h * 0x85ebca77 & 0xffffffff
+        pos.append(a + (h * (b - a) >> 32))
+    rng = np.random.default_rng(5)
+    x = rng.integers(0, 7 if few else 1 << 20, n).astype(dtype)
+    x[pos] = (1 << 24) + rng.integers(0, 1 << 20, s)
+    _check(rk, orc, x)
