@@ -1,11 +1,13 @@
 // sort! / sortperm! of vectors (src/kernels/sorting.jl:1-3, which forwards to AcceleratedKernels' merge sort):
 // least-significant-digit radix sort, 8 bits per pass.
 //
-// Three ways by the number of keys:
+// Four ways by the number of keys:
 //   up to 4096           one workgroup does all of it in LDS (sort_tiny_kernel, rk_sort_buckets.hpp).
 //   up to 2^20           keys of 4 and 8 bytes go through splitters into buckets that are sorted in LDS (rk_sort_buckets.hpp):
 //                        such sorts are bound by the latency of their kernels, and these are four or five whatever the width.
-//   more, and keys of 2 bytes, the radix passes of this file:
+//   up to 2^26           keys of 8 bytes, and Float32 up to 2^22, go through two levels of splitters (rk_sort_split.hpp), unless they are
+//                        integers that differ in three digits at most.
+//   the others           the radix passes of this file:
 //   sort_init_kernel     clears the control block; no memset: graph-safe
 //   sort_range_kernel    one read of the keys: smallest and largest key (integers) and the bits that differ between keys;
 //                        the workgroup that finishes last decides which passes run (a digit that is the same in every key
@@ -221,6 +223,18 @@ __device__ __forceinline__ SortStep sort_step(const SortCtl* ctl, int pass) {
     return s;
 }
 
+// Sorts of 8-byte integers that take another way unless the keys differ in few digits (rk_sort_split.hpp) launch so many passes;
+// `pass` is then -1, -2, ... for the first of the digits that vary, the second ...  Returns the digit, -1: there is none to do.
+// Three: 2^24 keys in three digits, sortperm Int64 432 us so and 522 by splitters, sort 400 and 382; in four, 547 and 502, 427 and 381.
+constexpr uint32_t SORT_FEW_PASSES = 3;
+__device__ __forceinline__ int sort_pass_index(const SortCtl* ctl, int pass) {
+    if (pass >= 0) return pass;
+    if (ctl->nexec > SORT_FEW_PASSES || (uint32_t)-pass > ctl->nexec) return -1;
+    int p = -1;
+    for (int left = -pass; left != 0;) left -= ctl->skip[++p] == 0u ? 1 : 0;
+    return p;
+}
+
 // ---- init: clear the control block ----------------------------------------------------------------------------------
 // all_passes: large sorts of floats, which run every pass on keys that are not taken relative to the smallest one; their
 // plan is made here.
@@ -340,6 +354,8 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
     constexpr int VEC = 16 / (int)sizeof(T), NV = ITEMS / VEC;
     typedef typename VecOf<U, VEC>::type VU;
     __shared__ uint32_t cnt[NW * SUB][256];
+    pass = sort_pass_index(ctl, pass);
+    if (pass < 0) return;
     const SortStep step = sort_step(ctl, pass);
     if (step.skip != 0u) return;
     const bool first = (uint32_t)pass == step.first_pass;
@@ -497,7 +513,8 @@ __global__ __launch_bounds__(TS_BLOCK) void sort_tilescan_kernel(SortCtl* ctl, i
     __shared__ uint32_t gsum[2][TS_GROUPS][256];
     __shared__ uint32_t wsum[256 / WAVE];
     __shared__ uint32_t lds_ticket;
-    if (ctl->skip[pass]) return;
+    pass = sort_pass_index(ctl, pass);
+    if (pass < 0 || ctl->skip[pass]) return;
     const uint32_t d = threadIdx.x & 255u, g = threadIdx.x >> 8, chunk = blockIdx.x, nchunks = gridDim.x;
     {
         const uint32_t r0 = chunk * chunk_rows, r1 = r0 + chunk_rows < ntiles ? r0 + chunk_rows : ntiles;
@@ -552,10 +569,13 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
     __shared__ uint2 part_before[GROUPS][DIRECT ? 128 : 1], part_all[GROUPS][DIRECT ? 128 : 1];
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-    const SortStep step = sort_step(ctl, pass);
-    if (step.skip != 0u) {
+    const bool first_of_few = pass == -1;
+    pass = sort_pass_index(ctl, pass);
+    SortStep step{};
+    if (pass >= 0) step = sort_step(ctl, pass);
+    if (pass < 0 || step.skip != 0u) {
         // all keys equal: no pass ran, and the last one writes the identity permutation
-        if (PERM && pass == (int)sizeof(T) - 1 && ctl->nexec == 0u)
+        if (PERM && (first_of_few || pass == (int)sizeof(T) - 1) && ctl->nexec == 0u)
             for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < (int64_t)n; i += (int64_t)gridDim.x * BLOCK) perm_out[i] = i + 1;
         return;
     }
@@ -760,8 +780,10 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
 
 // ---- finish ------------------------------------------------------------------------------------------------------
 // sort! and sort: after an odd number of passes the result sits in buffer B, after none in the caller's keys.
+// most: passes that may have run; keys that would have taken more were sorted by splitters.
 template <typename W>
-__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, const W* orig, W* a, const W* b, int64_t nwords) {
+__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, const W* orig, W* a, const W* b, int64_t nwords, uint32_t most) {
+    if (ctl->nexec > most) return;
     const W* from = (ctl->nexec & 1u) != 0u ? b : (ctl->nexec == 0u ? orig : a);
     if (from == a) return;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords; i += (int64_t)gridDim.x * 256) a[i] = from[i];
@@ -770,6 +792,7 @@ __global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, co
 }  // namespace rk
 
 #include "rk_sort_buckets.hpp"
+#include "rk_sort_split.hpp"
 
 namespace rk {
 
@@ -788,16 +811,19 @@ struct SortLayout {
     size_t count_off, chunk_total_off, chunk_prefix_off, keys_b_off, keys_a_off, val_a_off, val_b_off, total;
     size_t compact_off, spl_key_off, spl_pos_off, table_off, tile_min_off;
     uint32_t ntiles, chunk_rows, nchunks, k;
-    bool tiny, direct, buckets;
+    bool tiny, direct, buckets, split;
+    LsLayout ls;
 };
 
-static SortLayout sort_layout(size_t key_size, int64_t n, bool perm) {
+static SortLayout sort_layout(size_t key_size, bool integers, int64_t n, bool perm) {
     SortLayout l{};
     l.ntiles = (uint32_t)((n + SORT_TILE - 1) / SORT_TILE);
     size_t off = (sizeof(SortCtl) + 255) & ~(size_t)255;
     l.tiny = n <= ST_MAX;
     l.direct = l.ntiles <= DIRECT_TILES;
     l.buckets = l.direct && !l.tiny && key_size >= 4;
+    l.split = !l.direct && (key_size == 8 ? n <= LS_MAX_KEYS : key_size == 4 && !integers && n <= LS_MAX_FLOATS);
+    const size_t ctl_end = off;
     l.count_off = off;
     if (l.direct) {
         if (!l.buckets && !l.tiny) off += (size_t)l.ntiles * 256 * sizeof(uint16_t);
@@ -807,6 +833,10 @@ static SortLayout sort_layout(size_t key_size, int64_t n, bool perm) {
         l.nchunks = (l.ntiles + l.chunk_rows - 1) / l.chunk_rows;
         l.chunk_total_off = off;  off += (size_t)TS_MAX_CHUNKS * 256 * sizeof(uint32_t);
         l.chunk_prefix_off = off; off += (size_t)TS_MAX_CHUNKS * 256 * sizeof(uint32_t);
+    }
+    if (l.split) {                                           // in the place of the counts: one of the two ways is taken
+        l.ls = ls_layout(ctl_end, key_size, n);
+        if (l.ls.total > off) off = l.ls.total;
     }
     const size_t kbytes = ((size_t)n * key_size + 255) & ~(size_t)255, vbytes = ((size_t)n * 4 + 255) & ~(size_t)255;
     l.keys_b_off = off; off += kbytes;
@@ -865,7 +895,7 @@ template <typename T, bool PERM>
 static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out, int64_t n, int rev, void* tmp, size_t tmp_bytes, hipStream_t stream) {
     typedef typename SortKey<T>::U U;
     constexpr int PASSES = (int)sizeof(T);
-    const SortLayout l = sort_layout(sizeof(T), n, PERM);
+    const SortLayout l = sort_layout(sizeof(T), std::is_integral<T>::value, n, PERM);
     if (tmp == nullptr || !is_aligned(tmp, 256) || tmp_bytes < l.total) return RK_ERR_WORKSPACE;
     char* base = (char*)tmp;
     SortCtl* ctl = (SortCtl*)base;
@@ -883,6 +913,9 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
     constexpr bool FLOAT_KEYS = !std::is_integral<T>::value;
     if constexpr (sizeof(T) >= 4) {
         if (l.buckets) return sort_buckets<T, PERM>(l, keys, sorted_out, perm_out, n, rev, base, stream);
+    }
+    if constexpr (FLOAT_KEYS && sizeof(T) >= 4) {
+        if (l.split) return sort_split<T, PERM>(l.ls, keys, sorted_out, perm_out, n, rev, base, ctl, buf_a, buf_b, val_a, val_b, stream);
     }
     const bool all_passes = FLOAT_KEYS && !l.direct;
     const int first_reads_b = PERM ? 1 : 0;          // sortperm: the first pass reads the caller's keys and writes buffer A
@@ -921,7 +954,8 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
         uint32_t* counts = (uint32_t*)(base + l.count_off);
         uint32_t* chunk_total = (uint32_t*)(base + l.chunk_total_off);
         uint32_t* chunk_prefix = (uint32_t*)(base + l.chunk_prefix_off);
-        for (int p = 0; p < PASSES; ++p) {
+        for (int i = 0; i < (l.split ? (int)SORT_FEW_PASSES : PASSES); ++i) {
+            const int p = l.split ? -1 - i : i;
             sort_upsweep_kernel<T, SORT_BLOCK, SORT_ITEMS, 4, uint32_t><<<l.ntiles, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
             RK_LAUNCH_CHECK();
             sort_tilescan_kernel<<<l.nchunks, TS_BLOCK, 0, stream>>>(ctl, p, counts, l.ntiles, l.chunk_rows, chunk_total, chunk_prefix);
@@ -929,15 +963,22 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
             sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, chunk_prefix, l.chunk_rows, l.ntiles, xcd_chunk);
             RK_LAUNCH_CHECK();
         }
+        if constexpr (sizeof(T) == 8) {
+            if (l.split) {
+                const int32_t rc = sort_split<T, PERM>(l.ls, keys, sorted_out, perm_out, n, rev, base, ctl, buf_a, buf_b, val_a, val_b, stream);
+                if (rc != RK_SUCCESS) return rc;
+            }
+        }
     }
     if (!PERM && !(all_passes && PASSES % 2 == 0)) {
+        const uint32_t most = l.split ? SORT_FEW_PASSES : (uint32_t)PASSES;
         // whole 32-bit words: buffers are 256-byte padded, the caller's array is at least element-aligned; 16-bit keys
         // with an odd count copy one element more than n only inside buffer padding on the source side -- so copy by element there
         const int64_t nwords = sizeof(T) == 2 ? n : ((int64_t)n * (int64_t)sizeof(T) + 3) / 4;
         int64_t g = (nwords + 255) / 256;
         if (g > cus * 16) g = cus * 16;
-        if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint16_t*)keys, (uint16_t*)buf_a, (const uint16_t*)buf_b, nwords);
-        else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint32_t*)keys, (uint32_t*)buf_a, (const uint32_t*)buf_b, nwords);
+        if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint16_t*)keys, (uint16_t*)buf_a, (const uint16_t*)buf_b, nwords, most);
+        else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint32_t*)keys, (uint32_t*)buf_a, (const uint32_t*)buf_b, nwords, most);
         RK_LAUNCH_CHECK();
     }
     return RK_SUCCESS;
@@ -959,7 +1000,7 @@ using namespace rk;
 extern "C" size_t rk_sort_tmp_bytes(rk_dtype dt, int64_t n, int32_t with_perm) {
     size_t ks = 0;
     if (!sort_dtype_size((int)dt, &ks) || n <= 0) return 256;
-    return sort_layout(ks, n, with_perm != 0).total;
+    return sort_layout(ks, (int)dt == RK_I16 || (int)dt == RK_I32 || (int)dt == RK_I64, n, with_perm != 0).total;
 }
 
 template <bool PERM>

@@ -84,7 +84,7 @@ __global__ __launch_bounds__(SB_SPL_BLOCK) void sort_splitters_kernel(const T* _
         j = j < s ? j : s - 1u;
         v[u] = DIRECT ? __builtin_bit_cast(U, keys[sb_sample_pos(j, s, n)]) : compact[j];
     }
-    if (blockIdx.x == 0 && tid == 0) { ctl->varying = 0ull; ctl->nexec = 0u; }
+    if (ctl != nullptr && blockIdx.x == 0 && tid == 0) { ctl->varying = 0ull; ctl->nexec = 0u; }
     if (tid < SB_SPL_EACH) below[tid] = 0u;
 #pragma unroll
     for (uint32_t u = 0; u < UNR; ++u) {
@@ -347,102 +347,53 @@ __device__ __forceinline__ void sb_bitonic(U* x, uint32_t* y, uint32_t m) {
 // Should a bin exceed SB_MAX_BIN -- a bucket around zero, where the keys of floats are far from linear; a few values many times
 // over -- every bin is divided once more into as many as it has keys, by where a key lies in it (bins of equal keys: by the
 // index; without one they need no order).  What even that does not spread is sorted by comparisons, still in LDS.
-template <typename T, bool PERM>
-__global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl, uint32_t k, uint32_t ntiles, const uint32_t* __restrict__ table,
-                                                                    const typename SortKey<T>::U* __restrict__ tile_min, int rev,
-                                                                    const typename SortKey<T>::U* __restrict__ tile_key, const uint16_t* __restrict__ tile_val,
-                                                                    typename SortKey<T>::U* big_key, uint32_t* big_val, T* sorted_out, int64_t* perm_out) {
-    typedef typename SortKey<T>::U U;
-    constexpr int BLOCK = SB_SORT_BLOCK, ITEMS = SB_SORT_ITEMS, NW = BLOCK / WAVE, PER = (int)SB_BINS / BLOCK;
-    constexpr bool RECORD = std::is_integral<T>::value;
-    static_assert(PER == 4, "a thread scans four bins");
+// LDS of a workgroup that sorts a bucket of up to ITEMS * BLOCK keys.
+template <typename U, bool PERM, int ITEMS, int BLOCK, uint32_t BINS> struct SbLds {
+    static constexpr uint32_t CAP = (uint32_t)(ITEMS * BLOCK);
     // keys and indices of the bucket; while it is divided a second time, a key of every bin, its lowest and highest index, and the
     // sizes of the new bins
-    constexpr size_t KEYS = (size_t)SB_CAP * sizeof(U), POOL = KEYS + (PERM ? (size_t)SB_CAP * 4 : 0), DIVIDE = (size_t)SB_BINS * (sizeof(U) + (PERM ? 8 : 0)) + (size_t)SB_CAP * 4;
-    __shared__ alignas(16) char pool[POOL > DIVIDE ? POOL : DIVIDE];
-    U* const lds_key = (U*)pool;
-    uint32_t* const lds_val = (uint32_t*)(pool + KEYS);      // (sortperm only)
-    U* const rep = (U*)pool;
-    uint32_t* const sub = (uint32_t*)(pool + (size_t)SB_BINS * sizeof(U));
-    uint32_t* const bin_vlo = sub + SB_CAP;                  // (sortperm only)
-    uint32_t* const bin_vhi = bin_vlo + SB_BINS;
-    __shared__ alignas(16) uint32_t bins[SB_BINS + 4];
-    __shared__ uint32_t part[4][NW];
-    __shared__ U part_key[2][NW];
-    uint32_t* const run_off = bins;                          // of a tile: keys of the bucket in the tiles in front (read before bins are)
-    uint32_t* const run_at = bins + SB_MAX_TILES;            // where the bucket starts in it
-    static_assert(2u * SB_MAX_TILES <= SB_BINS && SB_MAX_TILES <= (uint32_t)BLOCK, "a thread a tile");
-    const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, bucket = blockIdx.x;
-    uint32_t entry = 0u;
-    U smallest = (U)~(U)0;                                   // of all keys (integers)
-    if (tid < ntiles) {
-        entry = table[tid * k + bucket];
-        if (RECORD) smallest = tile_min[tid];
-    }
-    const uint32_t before = wave_reduce(entry & 0xffffu, OpAdd());
-    if constexpr (RECORD) {
-        smallest = wave_reduce(smallest, OpMin());
-        if (lane == 0) part_key[0][wave] = smallest;
-    }
-    const uint32_t run = wave_scan_inclusive(entry >> 16, OpAdd(), 0u);
-    if (lane == 0) part[0][wave] = before;
-    if (lane == WAVE - 1) part[1][wave] = run;
+    static constexpr size_t KEYS = (size_t)CAP * sizeof(U), POOL = KEYS + (PERM ? (size_t)CAP * 4 : 0), DIVIDE = (size_t)BINS * (sizeof(U) + (PERM ? 8 : 0)) + (size_t)CAP * 4;
+    alignas(16) char pool[POOL > DIVIDE ? POOL : DIVIDE];
+    alignas(16) uint32_t bins[BINS + 4];
+    uint32_t part[4][BLOCK / WAVE];
+    U part_key[2][BLOCK / WAVE];
+    U key_lo, key_hi;                                        // smallest and largest key of the bucket, lowest and highest index
+    uint32_t val_lo, val_hi;
+    // by one thread, before a barrier
+    __device__ __forceinline__ void init() { key_lo = (U)~(U)0; key_hi = (U)0; val_lo = ~0u; val_hi = 0u; }
+};
+
+template <typename U> __device__ __forceinline__ U sb_uniform(U x) {
+    if constexpr (sizeof(U) == 4) return (U)__builtin_amdgcn_readfirstlane((int)x);
+    else return (U)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) | (U)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32)) << 32;
+}
+
+// Thread t holds the elements t, t + BLOCK, ... of the m of the bucket, in any order (for those from m on, where others of the
+// thread's row exist, one that does); store(place, key, index) gets each of them.  RECORD: `smallest` is the smallest of all keys,
+// and the digits that vary are counted in ctl.
+template <bool PERM, bool RECORD, int ITEMS, int BLOCK, uint32_t BINS, typename U, typename Store>
+__device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[PERM ? ITEMS : 1], uint32_t m, SbLds<U, PERM, ITEMS, BLOCK, BINS>& lds,
+                                               SortCtl* ctl, U smallest, Store&& store) {
+    constexpr int NW = BLOCK / WAVE, PER = (int)BINS / BLOCK;
+    constexpr uint32_t CAP = (uint32_t)(ITEMS * BLOCK);
+    static_assert(PER % 4 == 0, "a thread scans PER bins, four at a time");
+    static_assert(CAP < 1u << 16, "place and size in 32 bits");
+    U* const lds_key = (U*)lds.pool;
+    uint32_t* const lds_val = (uint32_t*)(lds.pool + SbLds<U, PERM, ITEMS, BLOCK, BINS>::KEYS);      // (sortperm only)
+    U* const rep = (U*)lds.pool;
+    uint32_t* const sub = (uint32_t*)(lds.pool + (size_t)BINS * sizeof(U));
+    uint32_t* const bin_vlo = sub + CAP;                     // (sortperm only)
+    uint32_t* const bin_vhi = bin_vlo + BINS;
+    auto& bins = lds.bins;
+    auto& part = lds.part;
+    auto& part_key = lds.part_key;
+    const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    U lo = (U)~(U)0, hi = (U)0;
+    uint32_t rank[ITEMS], vlo = ~0u, vhi = 0u;
+    m = sb_uniform(m);
     __syncthreads();
-    uint32_t start = 0u, off = run - (entry >> 16), m = 0u;
 #pragma unroll
-    for (int w = 0; w < (int)SB_MAX_TILES / WAVE; ++w) {
-        start += part[0][w];
-        if ((uint32_t)w < wave) off += part[1][w];
-        m += part[1][w];
-        if (RECORD) smallest = part_key[0][w] < smallest ? part_key[0][w] : smallest;
-    }
-    if (tid < SB_MAX_TILES) {
-        run_off[tid] = tid < ntiles ? off : ~0u;
-        run_at[tid] = entry & 0xffffu;
-    }
-    __syncthreads();
-    // the p-th key of the bucket: in the last tile with no more than p keys in front of it
-    auto find = [&](uint32_t p, uint32_t& tile) -> uint32_t {
-        tile = 0u;
-#pragma unroll
-        for (uint32_t step = SB_MAX_TILES / 2u; step != 0u; step /= 2u) tile += run_off[tile + step] <= p ? step : 0u;
-        return tile * (uint32_t)SB_TILE + run_at[tile] + (p - run_off[tile]);
-    };
-    if (m > SB_CAP) {                                        // too large for LDS: compared in memory, slowly
-        U* x = PERM ? big_key + start : (U*)sorted_out + start;
-        uint32_t* y = PERM ? big_val + start : nullptr;
-        for (uint32_t p = tid; p < m; p += BLOCK) {
-            uint32_t tile;
-            const uint32_t at = find(p, tile);
-            x[p] = tile_key[at];
-            if constexpr (PERM) y[p] = tile * (uint32_t)SB_TILE + tile_val[at];
-        }
-        sb_bitonic<PERM>(x, y, m);
-        U bits = (U)0;
-        for (uint32_t i = tid; i < m; i += BLOCK) {
-            const U u = x[i];
-            if constexpr (RECORD) bits |= (U)(u - smallest);
-            if constexpr (PERM) perm_out[start + i] = (int64_t)y[i] + 1;
-            else sorted_out[start + i] = dec_bits<T>(u, rev, (U)0);
-        }
-        if constexpr (RECORD) sb_record_digits<U>(ctl, bits, part_key[1]);
-        return;
-    }
-    U key[ITEMS], lo = (U)~(U)0, hi = (U)0;
-    uint32_t val[PERM ? ITEMS : 1], rank[ITEMS], vlo = ~0u, vhi = 0u;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-        if ((uint32_t)(i * BLOCK) < m) {
-            const uint32_t p = tid + i * BLOCK;
-            uint32_t tile;
-            const uint32_t at = find(p < m ? p : 0u, tile);
-            key[i] = tile_key[at];
-            if constexpr (PERM) val[i] = tile * (uint32_t)SB_TILE + tile_val[at];
-        }
-        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);             // searches four at a time: eleven take too many registers
-    }
-    __syncthreads();
-    *(uint4*)&bins[tid * 4] = make_uint4(0u, 0u, 0u, 0u);
+    for (int c = 0; c < PER; c += 4) *(uint4*)&bins[tid * PER + c] = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         if ((uint32_t)(i * BLOCK) < m) {
@@ -456,18 +407,18 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
     }
     lo = wave_reduce(lo, OpMin());
     hi = wave_reduce(hi, OpMax());
-    if (lane == 0) { part_key[0][wave] = lo; part_key[1][wave] = hi; }
+    if (lane == 0) { atomicMin(&lds.key_lo, lo); atomicMax(&lds.key_hi, hi); }
     if constexpr (PERM) {
         vlo = wave_reduce(vlo, OpMin());
         vhi = wave_reduce(vhi, OpMax());
-        if (lane == 0) { part[2][wave] = vlo; part[3][wave] = vhi; }
+        if (lane == 0) { atomicMin(&lds.val_lo, vlo); atomicMax(&lds.val_hi, vhi); }
     }
     __syncthreads();
-    lo = wave_reduce(part_key[0][lane % NW], OpMin());
-    hi = wave_reduce(part_key[1][lane % NW], OpMax());
+    lo = sb_uniform(lds.key_lo);
+    hi = sb_uniform(lds.key_hi);
     if constexpr (PERM) {
-        vlo = wave_reduce(part[2][lane % NW], OpMin());
-        vhi = wave_reduce(part[3][lane % NW], OpMax());
+        vlo = sb_uniform(lds.val_lo);
+        vhi = sb_uniform(lds.val_hi);
     }
     // distance of a key from the smallest; with its index in the low bits if that fits 32: then no two are equal
     const uint64_t span = (uint64_t)(U)(hi - lo);
@@ -476,12 +427,14 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
     const uint64_t width = both ? span << vbits | vspan : span;
     const uint32_t shift = width >> 32 ? 32u - (uint32_t)__clz((int)(uint32_t)(width >> 32)) : 0u;
     const uint32_t w32 = (uint32_t)(width >> shift);
-    const bool exact = shift == 0u && w32 < SB_BINS;                   // a bin is one value
-    // w32 * scale < SB_BINS * 2^32: the last bin is SB_BINS - 1
-    const uint32_t scale = exact ? 0u : (uint32_t)((double)SB_BINS * 4294967296.0 / ((double)w32 + 1.0));
+    const bool exact = shift == 0u && w32 < BINS;                   // a bin is one value
+    // w32 * scale < BINS * 2^32: the last bin is BINS - 1.  (The two roundings and the reciprocal are off by 3 units of 2^-24
+    // at most, the last factor is 8 units below 1.)
+    const uint32_t scale = exact ? 0u : sb_uniform((uint32_t)((float)BINS * 4294967296.f * __builtin_amdgcn_rcpf((float)w32 + 1.f) * (1.f - 0x1p-21f)));
     auto distance = [&](U x, uint32_t v) -> uint32_t {
         asm volatile("" : "+v"(x));                // computed again at every use: kept, the bins of eleven keys spilled 20 registers
-        return both ? (uint32_t)(U)(x - lo) << vbits | (v - vlo) : (uint32_t)((uint64_t)(U)(x - lo) >> shift);
+        if constexpr (sizeof(U) == 4 && !PERM) return x - lo;
+        else return both ? (uint32_t)(U)(x - lo) << vbits | (v - vlo) : (uint32_t)((uint64_t)(U)(x - lo) >> shift);
     };
     auto bin_of = [&](U x, uint32_t v) -> uint32_t { return exact ? distance(x, v) : __umulhi(distance(x, v), scale); };
 #pragma unroll
@@ -490,10 +443,16 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
         if (tid + i * BLOCK < m) rank[i] = atomicAdd(&bins[bin_of(key[i], val[PERM ? i : 0])], 1u);
     }
     __syncthreads();
-    const uint4 c = *(const uint4*)&bins[tid * 4];
-    const uint32_t sum = c.x + c.y + c.z + c.w, c01 = c.x > c.y ? c.x : c.y, c23 = c.z > c.w ? c.z : c.w;
+    uint32_t c[PER], sum = 0u, most = 0u;
+#pragma unroll
+    for (int j = 0; j < PER; j += 4) {
+        const uint4 q = *(const uint4*)&bins[tid * PER + j];
+        c[j] = q.x; c[j + 1] = q.y; c[j + 2] = q.z; c[j + 3] = q.w;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) { sum += c[j]; most = c[j] > most ? c[j] : most; }
     const uint32_t inc = wave_scan_inclusive(sum, OpAdd(), 0u);
-    const uint32_t most = wave_reduce(c01 > c23 ? c01 : c23, OpMax());
+    most = wave_reduce(most, OpMax());
     if (lane == WAVE - 1) { part[0][wave] = inc; part[1][wave] = most; }
     __syncthreads();
     uint32_t first = inc - sum, largest = 0u;
@@ -501,17 +460,21 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
         if ((uint32_t)w < wave) first += part[0][w];
         largest = part[1][w] > largest ? part[1][w] : largest;
     }
-    *(uint4*)&bins[tid * 4] = make_uint4(first, first + c.x, first + c.x + c.y, first + c.x + c.y + c.z);
-    if (tid == 0) bins[SB_BINS] = m;
+    largest = sb_uniform(largest);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) { const uint32_t q = c[j]; c[j] = first; first += q; }
+#pragma unroll
+    for (int j = 0; j < PER; j += 4) *(uint4*)&bins[tid * PER + j] = make_uint4(c[j], c[j + 1], c[j + 2], c[j + 3]);
+    if (tid == 0) bins[BINS] = m;
     __syncthreads();
     const bool ordered = exact && (!PERM || both);                     // a bin holds equal keys (one index): nothing to compare
     const bool divide = !ordered && largest > SB_MAX_BIN;
     bool compare = false;
     if (divide) {
         // which bins hold different keys (bit 31), then the division
-        for (uint32_t i = tid; i < SB_CAP; i += BLOCK) sub[i] = 0u;
+        for (uint32_t i = tid; i < CAP; i += BLOCK) sub[i] = 0u;
         if constexpr (PERM) {
-            for (uint32_t i = tid; i < SB_BINS; i += BLOCK) { bin_vlo[i] = ~0u; bin_vhi[i] = 0u; }
+            for (uint32_t i = tid; i < BINS; i += BLOCK) { bin_vlo[i] = ~0u; bin_vhi[i] = 0u; }
         }
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
@@ -568,7 +531,7 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
             at += s[i];
         }
         __syncthreads();
-        compare = largest > SB_MAX_BIN;
+        compare = sb_uniform(largest) > SB_MAX_BIN;
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             if (tid + i * BLOCK < m) {                                 // place in the bucket | place in the bin << 16 | size of the bin << 22
@@ -596,10 +559,6 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
         }
         return r;
     };
-    auto store = [&](uint32_t to, U x, uint32_t v) {
-        if constexpr (PERM) perm_out[start + to] = (int64_t)v + 1;
-        else sorted_out[start + to] = dec_bits<T>(x, rev, (U)0);
-    };
     U bits = (U)0;
     if constexpr (RECORD) {
 #pragma unroll
@@ -619,7 +578,7 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
         if (compare) sb_bitonic<PERM>(lds_key, lds_val, m);
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t p = tid + i * BLOCK;
+                const uint32_t p = tid + i * BLOCK;
             if (p >= m) continue;
             const U x = lds_key[p];
             const uint32_t v = PERM ? lds_val[PERM ? p : 0] : p;
@@ -632,6 +591,98 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
         }
     }
     if constexpr (RECORD) sb_record_digits<U>(ctl, bits, part_key[1]);
+}
+
+template <typename T, bool PERM>
+__global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl, uint32_t k, uint32_t ntiles, const uint32_t* __restrict__ table,
+                                                                    const typename SortKey<T>::U* __restrict__ tile_min, int rev,
+                                                                    const typename SortKey<T>::U* __restrict__ tile_key, const uint16_t* __restrict__ tile_val,
+                                                                    typename SortKey<T>::U* big_key, uint32_t* big_val, T* sorted_out, int64_t* perm_out) {
+    typedef typename SortKey<T>::U U;
+    constexpr int BLOCK = SB_SORT_BLOCK, ITEMS = SB_SORT_ITEMS;
+    constexpr bool RECORD = std::is_integral<T>::value;
+    __shared__ SbLds<U, PERM, ITEMS, BLOCK, SB_BINS> lds;
+    auto& bins = lds.bins;
+    auto& part = lds.part;
+    auto& part_key = lds.part_key;
+    uint32_t* const run_off = bins;                          // of a tile: keys of the bucket in the tiles in front (read before bins are)
+    uint32_t* const run_at = bins + SB_MAX_TILES;            // where the bucket starts in it
+    static_assert(2u * SB_MAX_TILES <= SB_BINS && SB_MAX_TILES <= (uint32_t)BLOCK, "a thread a tile");
+    const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, bucket = blockIdx.x;
+    uint32_t entry = 0u;
+    U smallest = (U)~(U)0;                                   // of all keys (integers)
+    if (tid == 0u) lds.init();
+    if (tid < ntiles) {
+        entry = table[tid * k + bucket];
+        if (RECORD) smallest = tile_min[tid];
+    }
+    const uint32_t before = wave_reduce(entry & 0xffffu, OpAdd());
+    if constexpr (RECORD) {
+        smallest = wave_reduce(smallest, OpMin());
+        if (lane == 0) part_key[0][wave] = smallest;
+    }
+    const uint32_t run = wave_scan_inclusive(entry >> 16, OpAdd(), 0u);
+    if (lane == 0) part[0][wave] = before;
+    if (lane == WAVE - 1) part[1][wave] = run;
+    __syncthreads();
+    uint32_t start = 0u, off = run - (entry >> 16), m = 0u;
+#pragma unroll
+    for (int w = 0; w < (int)SB_MAX_TILES / WAVE; ++w) {
+        start += part[0][w];
+        if ((uint32_t)w < wave) off += part[1][w];
+        m += part[1][w];
+        if (RECORD) smallest = part_key[0][w] < smallest ? part_key[0][w] : smallest;
+    }
+    if (tid < SB_MAX_TILES) {
+        run_off[tid] = tid < ntiles ? off : ~0u;
+        run_at[tid] = entry & 0xffffu;
+    }
+    __syncthreads();
+    // the p-th key of the bucket: in the last tile with no more than p keys in front of it
+    auto find = [&](uint32_t p, uint32_t& tile) -> uint32_t {
+        tile = 0u;
+#pragma unroll
+        for (uint32_t step = SB_MAX_TILES / 2u; step != 0u; step /= 2u) tile += run_off[tile + step] <= p ? step : 0u;
+        return tile * (uint32_t)SB_TILE + run_at[tile] + (p - run_off[tile]);
+    };
+    if (m > SB_CAP) {                                        // too large for LDS: compared in memory, slowly
+        U* x = PERM ? big_key + start : (U*)sorted_out + start;
+        uint32_t* y = PERM ? big_val + start : nullptr;
+        for (uint32_t p = tid; p < m; p += BLOCK) {
+            uint32_t tile;
+            const uint32_t at = find(p, tile);
+            x[p] = tile_key[at];
+            if constexpr (PERM) y[p] = tile * (uint32_t)SB_TILE + tile_val[at];
+        }
+        sb_bitonic<PERM>(x, y, m);
+        U bits = (U)0;
+        for (uint32_t i = tid; i < m; i += BLOCK) {
+            const U u = x[i];
+            if constexpr (RECORD) bits |= (U)(u - smallest);
+            if constexpr (PERM) perm_out[start + i] = (int64_t)y[i] + 1;
+            else sorted_out[start + i] = dec_bits<T>(u, rev, (U)0);
+        }
+        if constexpr (RECORD) sb_record_digits<U>(ctl, bits, part_key[1]);
+        return;
+    }
+    U key[ITEMS];
+    uint32_t val[PERM ? ITEMS : 1];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if ((uint32_t)(i * BLOCK) < m) {
+            const uint32_t p = tid + i * BLOCK;
+            uint32_t tile;
+            const uint32_t at = find(p < m ? p : 0u, tile);
+            key[i] = tile_key[at];
+            if constexpr (PERM) val[i] = tile * (uint32_t)SB_TILE + tile_val[at];
+        }
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);             // searches four at a time: eleven take too many registers
+    }
+    start = sb_uniform(start);
+    sb_sort_bucket<PERM, RECORD, ITEMS, BLOCK, SB_BINS>(key, val, m, lds, ctl, smallest, [&](uint32_t to, U x, uint32_t v) {
+        if constexpr (PERM) perm_out[start + to] = (int64_t)v + 1;
+        else sorted_out[start + to] = dec_bits<T>(x, rev, (U)0);
+    });
 }
 
 // ---- sorts that fit a workgroup ---------------------------------------------------------------------------------------

@@ -343,3 +343,49 @@ def test_bucket_larger_than_lds(rk, orc, dtype, few):
     x = rng.integers(0, 7 if few else 1 << 20, n).astype(dtype)
     x[pos] = (1 << 24) + rng.integers(0, 1 << 20, s)
     _check(rk, orc, x)
+
+
+@pytest.mark.parametrize("kind", ["sorted", "equal", "few", "hundreds", "clusters", "steep", "normal"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+def test_sorts_by_two_levels_of_splitters(rk, orc, dtype, kind):
+    """More than 2^20 keys; tiles of 4096 keys below 2^22 and of 8192 from there on, of which the last is full, or holds one key."""
+    rng = np.random.default_rng(32)
+    for n, rev in (((1 << 20) + 1, False), ((1 << 21) - 5, True), ((1 << 22) - 1, False), (1 << 22, True), ((1 << 22) + 8193, False)):
+        x = _spread(rng, dtype, n, kind)
+        assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(x), rev=rev)), orc.sort(x, rev)), (n, rev)
+        assert np.array_equal(rk.Array(rk.sortperm(rk.ROCArray(x), rev=rev)), orc.sortperm(x, rev)), (n, rev)
+
+
+@pytest.mark.parametrize("digits", [(), (2,), (0, 7), (1, 3, 6), (0, 2, 3, 5), (0, 1, 2, 3, 4, 5, 6, 7)])
+def test_large_int64_by_varying_digits(rk, orc, digits):
+    """Keys that differ in three digits at most take radix passes, others splitters; sort! in place and into another array."""
+    rng = np.random.default_rng(33)
+    n = (1 << 20) + 4097
+    x = np.full(n, 1 << 40, dtype=np.int64)
+    for d in digits:
+        x ^= rng.integers(0, 256, n).astype(np.int64) << (8 * d)
+    _check(rk, orc, x)
+    y = rk.ROCArray(x)
+    rk.sort_(y)
+    assert np.array_equal(rk.Array(y), orc.sort(x, False))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
+@pytest.mark.parametrize("few", [False, True])
+def test_part_and_buckets_larger_than_lds(rk, orc, dtype, few):
+    """Every key that is sampled first is larger than all the others: these are one part of more tiles than a bucket's workgroup
+    holds the runs of, and its 256 buckets are larger than LDS."""
+    n, s = (1 << 20) + 300_000, 4096
+    j = np.arange(s, dtype=np.uint64)
+    a, b = j * n // s, (j + 1) * n // s
+    m = np.uint64(0xffffffff)
+    h = (j + 1) * np.uint64(0x9e3779b1) & m
+    h ^= h >> np.uint64(15)
+    h = h * np.uint64(0x85ebca77) & m
+    pos = (a + (h * (b - a) >> np.uint64(32))).astype(np.int64)
+    rng = np.random.default_rng(6)
+    x = (rng.integers(0, 7, n) if few else rng.integers(0, 1 << 20, n)).astype(dtype)
+    if dtype == np.int64:
+        x += rng.integers(0, 7, n) << 40                     # (four digits and more)
+    x[pos] = (1 << 50) + rng.integers(0, 1 << 20, s)
+    _check(rk, orc, x)
