@@ -383,7 +383,8 @@ extern "C" int32_t rk_gather_slices(const void* x, const int64_t* idx, void* y, 
 // the count leaves behind makes the second read a plain streaming kernel:
 //   mask_count_kernel    set bytes of every tile of 4096 Bools (one wave), as exclusive prefixes inside groups of tiles,
 //                        and the exclusive prefixes of the groups (the workgroup that finishes last scans them)
-//   mask_select_kernel   a wave per tile: its first output slot is two loads away, so there is no look-back, no barrier
+//   mask_select_kernel, mask_select_dense_kernel
+//                        a wave per tile: its first output slot is two loads away, so there is no look-back, no barrier
 //                        and nothing to wait for; selected elements go from x to y without an index in between
 // Bound by memory: the mask (the second read comes from the Infinity Cache up to 2^27 Bools), the lines of x that hold a
 // selected element, and the result.  Before, this was a u8 -> Int64 reduction, the one-pass findall and a gather by its
@@ -585,6 +586,80 @@ __global__ __launch_bounds__(256) void mask_select_kernel(const uint8_t* __restr
     if (fill > 0) flush();
 }
 
+// Where most lines of x hold a selected element anyway (4- and 8-byte elements): x is read whole, 16 bytes a lane beside the mask bytes
+// of the same elements, so that no load waits for another, and the selected ones are put together in LDS.  A step is four such
+// loads; those of the next are issued before a step is worked on.  Bound by memory.
+// The whole call, by list of hits -> so, us: Float32[2^26] 10 % 91 -> 88, 25 % 108.5 -> 95, 50 % 131 -> 107, 90 % 170 -> 131; Int64[2^26] 25 %
+// 178 -> 150, 90 % 268 -> 250.  (Loads that stay in the caches instead of nontemporal ones: Float32[2^26] 25 % 106.5, 90 % 143.)
+template <typename E>
+__global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* __restrict__ mask, int64_t n, const E* __restrict__ x, E* __restrict__ y,
+                                                                int64_t nsel, int64_t ntiles, const uint32_t* __restrict__ tile_prefix,
+                                                                const int64_t* __restrict__ group_prefix, int group_shift) {
+    constexpr int V = 16 / (int)sizeof(E), LOADS = 4, STEP = LOADS * WAVE * V, STEPS = MSK_TILE / STEP;
+    typedef E vec __attribute__((ext_vector_type(V)));
+    struct Loaded { vec x[LOADS]; uint32_t m[LOADS]; };     // m: a byte an element
+    __shared__ E lds_strip[256 / WAVE][STEP];
+    const int wave = threadIdx.x / WAVE, lane = lane_id();
+    const int64_t tile = (int64_t)blockIdx.x * (256 / WAVE) + wave;
+    if (tile >= ntiles) return;
+    const int64_t e0 = tile * MSK_TILE;
+    E* const strip = lds_strip[wave];
+    auto load = [&](Loaded& l, int64_t at) {
+#pragma unroll
+        for (int g = 0; g < LOADS; ++g) {
+            const int64_t i = at + g * (WAVE * V) + lane * V;
+            l.m[g] = 0u;
+            if (i + V <= n) {
+                if constexpr (V == 4) l.m[g] = load_nt((const uint32_t*)(mask + i));
+                else l.m[g] = load_nt((const uint16_t*)(mask + i));
+                l.x[g] = load_nt((const vec*)(x + i));
+            } else {
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    l.x[g][j] = (E)0;
+                    if (i + j < n) { l.m[g] |= (uint32_t)mask[i + j] << (8 * j); l.x[g][j] = x[i + j]; }
+                }
+            }
+        }
+    };
+    Loaded cur;
+    load(cur, e0);
+    int64_t base = group_prefix[tile >> group_shift] + (int64_t)tile_prefix[tile];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+        Loaded next;
+        if (s + 1 < STEPS) load(next, e0 + (s + 1) * STEP);
+        // hits of a lane, a byte a load; of the lanes in front they are 252 at most, so the bytes of the sum do not meet
+        uint32_t c = 0u;
+#pragma unroll
+        for (int g = 0; g < LOADS; ++g) {
+            cur.m[g] &= 0x01010101u;
+            c |= (uint32_t)__popc(cur.m[g]) << (8 * g);
+        }
+        const uint32_t exc = wave_scan_inclusive(c, OpAdd(), 0u) - c;
+        const uint32_t front = (uint32_t)read_lane((int32_t)exc, WAVE - 1), own = (uint32_t)read_lane((int32_t)c, WAVE - 1);
+        uint32_t fill = 0u;
+#pragma unroll
+        for (int g = 0; g < LOADS; ++g) {
+            uint32_t p = fill + ((exc >> (8 * g)) & 0xffu);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                if ((cur.m[g] >> (8 * j)) & 1u) strip[p++] = cur.x[g][j];
+            }
+            fill += ((front >> (8 * g)) & 0xffu) + ((own >> (8 * g)) & 0xffu);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (uint32_t i = lane; i < fill; i += WAVE)
+            if (base + i < nsel) y[base + i] = strip[i];    // nsel: a mask that changed since the count stays in bounds
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        base += fill;
+        if (s + 1 < STEPS) cur = next;
+    }
+}
+
 }  // namespace rk
 
 extern "C" size_t rk_mask_tmp_bytes(int64_t n) { return n <= 0 ? 256 : mask_tmp(n).bytes; }
@@ -630,6 +705,16 @@ extern "C" int32_t rk_mask_select(const uint8_t* mask, int64_t n, const void* x,
     const uint32_t* tp = (const uint32_t*)((const char*)tmp + t.tile_off);
     hipStream_t st = (hipStream_t)stream;
 #define RK_MSEL(E) rk::mask_select_kernel<E><<<(unsigned)blocks, 256, 0, st>>>(mask, n, aligned, (const E*)x, (E*)y, nsel, t.ntiles, tp, gp, msk_group_shift(n))
+    // Elements of x that sit in the Infinity Cache cost the list of hits little: Float32[2^24] 10 % 36.7 us by list and 40.4 whole, 25 % 39.0 and
+    // 41.3, 50 % 45.0 and 44.5; Int64[2^24] (128 MiB) 43.9 and 52.7, 56.1 and 55.6, 62.8 and 61.2.  Beyond, an eighth of the elements is the line
+    // (7 %: Float32[2^26] 86.7 and 86.3, Int64[2^26] 118 and 136; 10 %: 91 and 88, 139 and 139).
+    const bool cached = (uint64_t)n * elsize <= ((uint64_t)1 << 27);
+    if ((elsize == 4 || elsize == 8) && nsel >= (cached ? n / 4 * 3 : n / 8) && is_aligned(x, 16) && is_aligned(mask, 4)) {
+        if (elsize == 4) mask_select_dense_kernel<uint32_t><<<(unsigned)blocks, 256, 0, st>>>(mask, n, (const uint32_t*)x, (uint32_t*)y, nsel, t.ntiles, tp, gp, msk_group_shift(n));
+        else mask_select_dense_kernel<uint64_t><<<(unsigned)blocks, 256, 0, st>>>(mask, n, (const uint64_t*)x, (uint64_t*)y, nsel, t.ntiles, tp, gp, msk_group_shift(n));
+        RK_LAUNCH_CHECK();
+        return RK_SUCCESS;
+    }
     switch (elsize) {
         case 1: RK_MSEL(uint8_t); break;
         case 2: RK_MSEL(uint16_t); break;

@@ -172,6 +172,33 @@ def test_mask_bytes_and_the_bound_of_the_result(rk, n):
     assert (dy.cpu().numpy()[len(want):] == -7).all()
 
 
+@pytest.mark.parametrize("n", [1, 3, 255, 1023, 1025, 4095, 4097, 70_003, 16 * 4096 + 2])
+@pytest.mark.parametrize("elsize", [4, 8])
+@pytest.mark.parametrize("xoff,moff", [(0, 0), (0, 4), (0, 1), (8, 0)])
+def test_mask_select_of_most_elements(rk, n, elsize, xoff, moff):
+    """Masks that select three quarters and more read x whole when x is aligned to 16 bytes and the mask to 4: ends of steps and
+    tiles, elements in front of the result and behind it, a result that ends early and a mask that grows."""
+    import torch
+    rng = np.random.default_rng(n + elsize + moff)
+    dt = np.int32 if elsize == 4 else np.int64
+    x, m = rng.integers(0, 1 << 30, n).astype(dt), rng.random(n) < 0.85
+    m[: n // 2] |= rng.random() < 0.5                              # now and then lanes whose every element is selected
+    m[0] = True
+    dx = torch.zeros(elsize * n + 64, dtype=torch.uint8, device="cuda")
+    dx[xoff:xoff + elsize * n] = torch.from_numpy(x.view(np.uint8).copy()).cuda()
+    dm = torch.zeros(n + 64, dtype=torch.uint8, device="cuda")
+    dm[moff:moff + n] = torch.from_numpy(m.view(np.uint8).copy()).cuda()
+    want = x[m]
+    for nsel in (len(want), len(want) - len(want) // 50):
+        dy = torch.from_numpy(np.full(len(want) + 16, -7, dtype=dt)).cuda()
+        assert _mask_calls(rk, dm.data_ptr() + moff, dx.data_ptr() + xoff, dy.data_ptr(), elsize, n, nsel) == len(want)
+        got = dy.cpu().numpy()
+        assert np.array_equal(got[:nsel], want[:nsel]) and (got[nsel:] == -7).all()
+    dy = torch.from_numpy(np.full(len(want) + 16, -7, dtype=dt)).cuda()
+    _mask_calls(rk, dm.data_ptr() + moff, dx.data_ptr() + xoff, dy.data_ptr(), elsize, n, between=lambda: dm.fill_(1))
+    assert (dy.cpu().numpy()[len(want):] == -7).all()
+
+
 def test_the_paths_the_tunables_select():
     """RK_SELECT_ORDERED=0 (persistent workgroups fed by a tile counter) and RK_SCAN_DYNAMIC_IDS=1 (the same for the
     long scans) are read once per process, so they are exercised in a child process: findall and a long cumsum against
