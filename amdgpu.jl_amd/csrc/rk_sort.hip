@@ -858,6 +858,19 @@ static SortLayout sort_layout(size_t key_size, bool integers, int64_t n, bool pe
     return l;
 }
 
+// What a temporary needs that serves every sort of up to n keys of a size, floats and integers: a caller may keep the one of its
+// largest sort.  A way's own need grows with the number of keys, but falls where another way, or larger tiles, take over.
+static size_t sort_tmp_need(size_t key_size, int64_t n, bool perm) {
+    const int64_t last[] = {ST_MAX, DIRECT_TILES * SORT_TILE, LS_SMALL_TILES, LS_MAX_FLOATS, LS_MAX_KEYS, n};     // of a way
+    size_t need = 0;
+    for (int64_t m : last)
+        for (int integers = 0; integers < 2; ++integers) {
+            const size_t total = sort_layout(key_size, integers != 0, m < n ? m : n, perm).total;
+            need = total > need ? total : need;
+        }
+    return need;
+}
+
 // The kernels of rk_sort_buckets.hpp; the sorted tiles lie in buffer B.  A bucket that is too large for LDS is put together and
 // sorted where its keys end up (sort!, sort) or in buffer A (sortperm).
 template <typename T, bool PERM>
@@ -1000,7 +1013,7 @@ using namespace rk;
 extern "C" size_t rk_sort_tmp_bytes(rk_dtype dt, int64_t n, int32_t with_perm) {
     size_t ks = 0;
     if (!sort_dtype_size((int)dt, &ks) || n <= 0) return 256;
-    return sort_layout(ks, (int)dt == RK_I16 || (int)dt == RK_I32 || (int)dt == RK_I64, n, with_perm != 0).total;
+    return sort_tmp_need(ks, n, with_perm != 0);
 }
 
 template <bool PERM>

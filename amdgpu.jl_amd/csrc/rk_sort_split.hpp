@@ -503,7 +503,8 @@ constexpr int64_t LS_MAX_KEYS = (int64_t)1 << 26;          // LS_BUCKETS buckets
 constexpr int64_t LS_MAX_FLOATS = (int64_t)1 << 22;        // Float32: figures above
 
 // Keys a tile, of both levels: runs as long as two workgroups a compute unit in LDS allow, but hundreds of tiles.
-static inline uint32_t ls_tile_shift(int64_t n) { return n < ((int64_t)1 << 22) ? 12 : 13; }
+constexpr int64_t LS_SMALL_TILES = ((int64_t)1 << 22) - 1;  // keys up to which the tiles are the smaller ones
+static inline uint32_t ls_tile_shift(int64_t n) { return n <= LS_SMALL_TILES ? 12 : 13; }
 
 struct LsLayout {
     size_t compact_off, spl_key_off, spl_index_off, table_off, sizes_off, runs_off, part_key_off, part_index_off, tiles_off, buckets_off, table2_off, total;

@@ -431,7 +431,8 @@ RK_API int32_t rk_permutedims(const void* src, void* dst, size_t elsize, int ndi
  *                `perm_out`; unlike `sortperm!(ix, x)` it does not read an initial `ix`
  *                (the reference always passes 1:n, src/kernels/sorting.jl:3).
  * `tmp`: caller-owned, 256-byte aligned, at least rk_sort_tmp_bytes(dt, n, with_perm) bytes, any
- * contents; it is the ping-pong buffer plus bookkeeping, cleared by the call itself.  n < 2^31. */
+ * contents; it is the ping-pong buffer plus bookkeeping, cleared by the call itself.  n < 2^31.
+ * What suffices for n keys suffices for fewer of the same size: a temporary may be kept for the largest sort. */
 RK_API size_t  rk_sort_tmp_bytes(rk_dtype dt, int64_t n, int32_t with_perm);
 RK_API int32_t rk_sort(rk_dtype dt, void* keys, int64_t n, int32_t rev, void* tmp, size_t tmp_bytes,
                 void* stream);

@@ -249,6 +249,18 @@ def test_volumerhs_and_scatter_validation(L):
     assert f(None, 1, L.shape_array((0,)), None, None, None, 0, None) == L.RK_SUCCESS
 
 
+def test_a_sort_temporary_serves_every_smaller_sort(L):
+    """What rk_sort_tmp_bytes asks for never falls as n grows, whichever way a sort of n keys takes, and is the same for the
+    floats and the integers of a size."""
+    tb = L.lib.rk_sort_tmp_bytes
+    edges = [4096, 1 << 17, 1 << 20, (1 << 22) - 8192, 1 << 22, (1 << 22) + 8192, 1 << 24, 1 << 26, (1 << 26) + (1 << 22)]
+    sizes = sorted({e + d for e in edges for d in (-4097, -1, 0, 1, 4097) if e + d > 0})
+    for kinds in ((L.RK_F16, L.RK_I16), (L.RK_F32, L.RK_I32), (L.RK_F64, L.RK_I64)):
+        for perm in (0, 1):
+            need = [tb(kinds[0], n, perm) for n in sizes]
+            assert need == sorted(need) and need == [tb(kinds[1], n, perm) for n in sizes]
+
+
 def test_workspace_queries(L):
     wb = L.lib.rk_workspace_bytes
     base = wb(L.RK_KIND_MAPREDUCE, L.RK_F32, 1, L.shape_array((1 << 20,)), 1)
