@@ -586,56 +586,83 @@ __global__ __launch_bounds__(256) void mask_select_kernel(const uint8_t* __restr
     if (fill > 0) flush();
 }
 
-// Where most lines of x hold a selected element anyway (4- and 8-byte elements): x is read whole, 16 bytes a lane beside the mask bytes
-// of the same elements, so that no load waits for another, and the selected ones are put together in LDS.  A step is four such
-// loads; those of the next are issued before a step is worked on.  Bound by memory.
-// The whole call, by list of hits -> so, us: Float32[2^26] 10 % 91 -> 88, 25 % 108.5 -> 95, 50 % 131 -> 107, 90 % 170 -> 131; Int64[2^26] 25 %
-// 178 -> 150, 90 % 268 -> 250.  (Loads that stay in the caches instead of nontemporal ones: Float32[2^26] 25 % 106.5, 90 % 143.)
+// Where most lines of x hold a selected element anyway (4- and 8-byte elements): x is read 16 bytes a lane, where the mask bytes of the
+// same elements have a hit, so that no load waits for a list, and the selected ones are put together in LDS.  A step is four such
+// loads; those of the next are issued before a step is worked on (two steps ahead: no faster).  The mask is read first, all of the tile's:
+// where hits are clustered, most lines of x hold none.  Bound by memory.
+// The whole call, by list of hits -> so, us: Float32[2^26] 10 % 91 -> 88, 25 % 108.5 -> 95, 50 % 129 -> 105, 90 % 170 -> 131; Int64[2^26] 25 %
+// 178 -> 149, 90 % 268 -> 250; every hit of Int64[2^26] in the first quarter 85.2 -> 84.3, in runs of 13 of 100 tiles 80.2 -> 75.5 (x read
+// whole, beside its mask bytes: 150 and 145).  (Loads that stay in the caches instead of nontemporal ones: Float32[2^26] 25 % 106.5, 90 % 143.)
 template <typename E>
 __global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* __restrict__ mask, int64_t n, const E* __restrict__ x, E* __restrict__ y,
                                                                 int64_t nsel, int64_t ntiles, const uint32_t* __restrict__ tile_prefix,
                                                                 const int64_t* __restrict__ group_prefix, int group_shift) {
     constexpr int V = 16 / (int)sizeof(E), LOADS = 4, STEP = LOADS * WAVE * V, STEPS = MSK_TILE / STEP;
     typedef E vec __attribute__((ext_vector_type(V)));
-    struct Loaded { vec x[LOADS]; uint32_t m[LOADS]; };     // m: a byte an element
-    __shared__ E lds_strip[256 / WAVE][STEP];
+    struct Loaded { vec x[LOADS]; };
+    __shared__ alignas(16) E lds_strip[256 / WAVE][STEP];
     const int wave = threadIdx.x / WAVE, lane = lane_id();
     const int64_t tile = (int64_t)blockIdx.x * (256 / WAVE) + wave;
     if (tile >= ntiles) return;
     const int64_t e0 = tile * MSK_TILE;
     E* const strip = lds_strip[wave];
-    auto load = [&](Loaded& l, int64_t at) {
+    static_assert(sizeof(lds_strip[0]) == MSK_TILE, "the strip holds the mask of a tile");
+    auto wave_sync = [] {                                   // what the lanes of the wave wrote to LDS is there for all of them
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // the mask bytes of the tile, 16 a lane and load, change lanes in the strip
+    typedef uint32_t mask_vec_at4 __attribute__((ext_vector_type(4), aligned(4)));
+    mask_vec bytes[MSK_LOADS];
+    uint32_t any = 0u;
+#pragma unroll
+    for (int k = 0; k < MSK_LOADS; ++k) {
+        const int64_t i = e0 + k * SEL_CHUNK + lane * 16;
+        bytes[k] = i + 16 <= n ? (mask_vec)load_nt((const mask_vec_at4*)(mask + i)) : mask_load16(mask, i, n, 0);
+    }
+    int64_t base = group_prefix[tile >> group_shift] + (int64_t)tile_prefix[tile];
+#pragma unroll
+    for (int k = 0; k < MSK_LOADS; ++k) {
+        bytes[k] &= 0x01010101u;
+        any |= bytes[k][0] | bytes[k][1] | bytes[k][2] | bytes[k][3];
+        *(mask_vec*)((char*)strip + k * SEL_CHUNK + lane * 16) = bytes[k];
+    }
+    if (__ballot(any != 0u) == 0ull) return;
+    wave_sync();
+    uint32_t m[STEPS * LOADS];                              // a byte an element
+#pragma unroll
+    for (int k = 0; k < STEPS * LOADS; ++k) {
+        const char* from = (const char*)strip + (k * WAVE + lane) * V;
+        if constexpr (V == 4) m[k] = *(const uint32_t*)from;
+        else m[k] = *(const uint16_t*)from;
+    }
+    wave_sync();
+    auto load = [&](Loaded& l, int s) {
 #pragma unroll
         for (int g = 0; g < LOADS; ++g) {
-            const int64_t i = at + g * (WAVE * V) + lane * V;
-            l.m[g] = 0u;
+            const int k = s * LOADS + g;
+            const int64_t i = e0 + k * (WAVE * V) + lane * V;
+            if (m[k] == 0u) continue;
             if (i + V <= n) {
-                if constexpr (V == 4) l.m[g] = load_nt((const uint32_t*)(mask + i));
-                else l.m[g] = load_nt((const uint16_t*)(mask + i));
                 l.x[g] = load_nt((const vec*)(x + i));
             } else {
 #pragma unroll
-                for (int j = 0; j < V; ++j) {
-                    l.x[g][j] = (E)0;
-                    if (i + j < n) { l.m[g] |= (uint32_t)mask[i + j] << (8 * j); l.x[g][j] = x[i + j]; }
-                }
+                for (int j = 0; j < V; ++j)
+                    if (i + j < n) l.x[g][j] = x[i + j];
             }
         }
     };
     Loaded cur;
-    load(cur, e0);
-    int64_t base = group_prefix[tile >> group_shift] + (int64_t)tile_prefix[tile];
+    load(cur, 0);
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
         Loaded next;
-        if (s + 1 < STEPS) load(next, e0 + (s + 1) * STEP);
+        if (s + 1 < STEPS) load(next, s + 1);
         // hits of a lane, a byte a load; of the lanes in front they are 252 at most, so the bytes of the sum do not meet
         uint32_t c = 0u;
 #pragma unroll
-        for (int g = 0; g < LOADS; ++g) {
-            cur.m[g] &= 0x01010101u;
-            c |= (uint32_t)__popc(cur.m[g]) << (8 * g);
-        }
+        for (int g = 0; g < LOADS; ++g) c |= (uint32_t)__popc(m[s * LOADS + g]) << (8 * g);
         const uint32_t exc = wave_scan_inclusive(c, OpAdd(), 0u) - c;
         const uint32_t front = (uint32_t)read_lane((int32_t)exc, WAVE - 1), own = (uint32_t)read_lane((int32_t)c, WAVE - 1);
         uint32_t fill = 0u;
@@ -644,17 +671,14 @@ __global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* _
             uint32_t p = fill + ((exc >> (8 * g)) & 0xffu);
 #pragma unroll
             for (int j = 0; j < V; ++j) {
-                if ((cur.m[g] >> (8 * j)) & 1u) strip[p++] = cur.x[g][j];
+                if ((m[s * LOADS + g] >> (8 * j)) & 1u) strip[p++] = cur.x[g][j];
             }
             fill += ((front >> (8 * g)) & 0xffu) + ((own >> (8 * g)) & 0xffu);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
         for (uint32_t i = lane; i < fill; i += WAVE)
             if (base + i < nsel) y[base + i] = strip[i];    // nsel: a mask that changed since the count stays in bounds
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         base += fill;
         if (s + 1 < STEPS) cur = next;
     }

@@ -199,6 +199,27 @@ def test_mask_select_of_most_elements(rk, n, elsize, xoff, moff):
     assert (dy.cpu().numpy()[len(want):] == -7).all()
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.int64])
+@pytest.mark.parametrize("hits", ["random", "runs of 10", "first quarter", "every second tile", "last element"])
+def test_mask_select_beyond_the_cache(rk, dtype, hits):
+    """x beyond 128 MiB is read 16 bytes a lane from an eighth of the elements on, lanes and tiles without a hit left out: hits
+    evenly spread, in runs that begin and end inside a lane's elements, in tiles that are full beside empty ones; mask bytes
+    other than 0 and 1, of which bit 0 counts."""
+    import torch
+    rng = np.random.default_rng(5)
+    n = (1 << 27) // np.dtype(dtype).itemsize + 4099
+    x, i = rng.integers(-1000, 1000, n).astype(dtype), np.arange(n)
+    m = {"random": lambda: rng.random(n) < 0.25, "runs of 10": lambda: i % 37 < 10, "first quarter": lambda: i < n // 4,
+         "every second tile": lambda: i // 4096 % 2 == 1, "last element": lambda: (i < n // 8 + 1) | (i == n - 1)}[hits]()
+    mask = (m + 2 * rng.integers(0, 128, n)).astype(np.uint8)
+    dx, dm, want = torch.from_numpy(x).cuda(), torch.from_numpy(mask).cuda(), x[m]
+    assert len(want) >= n // 8
+    dy = torch.full((len(want) + 16,), -7, dtype=dx.dtype, device="cuda")
+    assert _mask_calls(rk, dm.data_ptr(), dx.data_ptr(), dy.data_ptr(), x.itemsize, n) == len(want)
+    got = dy.cpu().numpy()
+    assert np.array_equal(got[:len(want)], want) and (got[len(want):] == -7).all()
+
+
 def test_the_paths_the_tunables_select():
     """RK_SELECT_ORDERED=0 (persistent workgroups fed by a tile counter) and RK_SCAN_DYNAMIC_IDS=1 (the same for the
     long scans) are read once per process, so they are exercised in a child process: findall and a long cumsum against
