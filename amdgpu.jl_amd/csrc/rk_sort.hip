@@ -809,7 +809,7 @@ constexpr uint32_t DIRECT_TILES = 256;
 
 struct SortLayout {
     size_t count_off, chunk_total_off, chunk_prefix_off, keys_b_off, keys_a_off, val_a_off, val_b_off, total;
-    size_t compact_off, spl_key_off, spl_pos_off, table_off, tile_min_off;
+    size_t compact_off, spl_key_off, spl_pos_off, table_off;
     uint32_t ntiles, chunk_rows, nchunks, k;
     bool tiny, direct, buckets, split;
     LsLayout ls;
@@ -852,7 +852,6 @@ static SortLayout sort_layout(size_t key_size, bool integers, int64_t n, bool pe
         l.spl_key_off = take((size_t)l.k * key_size);
         l.spl_pos_off = take((size_t)l.k * 4);
         l.table_off = take((size_t)l.ntiles * l.k * 4);
-        l.tile_min_off = take((size_t)l.ntiles * key_size);
     }
     l.total = off;
     return l;
@@ -881,7 +880,6 @@ static int32_t sort_buckets(const SortLayout& l, const void* keys, void* sorted_
     U* spl_key = (U*)(base + l.spl_key_off);
     uint32_t* spl_pos = (uint32_t*)(base + l.spl_pos_off);
     uint32_t* table = (uint32_t*)(base + l.table_off);
-    U* tile_min = (U*)(base + l.tile_min_off);
     U* tile_key = (U*)(base + l.keys_b_off);
     uint16_t* tile_val = PERM ? (uint16_t*)(base + l.val_b_off) : nullptr;
     U* big_key = PERM ? (U*)(base + l.keys_a_off) : nullptr;
@@ -896,9 +894,9 @@ static int32_t sort_buckets(const SortLayout& l, const void* keys, void* sorted_
         sort_splitters_kernel<T, false><<<samples / SB_SPL_EACH, SB_SPL_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, rev, ctl, l.k, compact, spl_key, spl_pos);
     }
     RK_LAUNCH_CHECK();
-    sort_tile_kernel<T, PERM><<<l.ntiles, SB_TILE_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, rev, l.k, spl_key, spl_pos, table, tile_min, tile_key, tile_val);
+    sort_tile_kernel<T, PERM><<<l.ntiles, SB_TILE_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, rev, l.k, spl_key, spl_pos, table, tile_key, tile_val);
     RK_LAUNCH_CHECK();
-    sort_bucket_kernel<T, PERM><<<l.k, SB_SORT_BLOCK, 0, stream>>>(ctl, l.k, l.ntiles, table, tile_min, rev, tile_key, tile_val, big_key, big_val, (T*)sorted_out, perm_out);
+    sort_bucket_kernel<T, PERM><<<l.k, SB_SORT_BLOCK, 0, stream>>>(l.k, l.ntiles, table, rev, tile_key, tile_val, big_key, big_val, (T*)sorted_out, perm_out);
     RK_LAUNCH_CHECK();
     return RK_SUCCESS;
 }

@@ -58,7 +58,7 @@ __device__ __forceinline__ uint32_t sb_sample_pos(uint32_t j, uint32_t s, uint32
 // ---- splitters -------------------------------------------------------------------------------------------------
 // s = k * SB_OVER samples, all in every workgroup's LDS; a workgroup ranks SB_SPL_EACH of them against all.  s^2 comparisons
 // are 16.8 million at most, 1.3 us of the chip's vector instructions; sorting the samples in one workgroup would leave the
-// others idle for longer.  Also clears what integers record.
+// others idle for longer.  ctl: of sorts that run no radix pass.
 // With many samples it is the fetching that counts -- a line of memory for every sample, in every workgroup -- and a kernel in
 // front packs them (compact).
 template <typename T>
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(SB_SPL_BLOCK) void sort_splitters_kernel(const T* _
         j = j < s ? j : s - 1u;
         v[u] = DIRECT ? __builtin_bit_cast(U, keys[sb_sample_pos(j, s, n)]) : compact[j];
     }
-    if (ctl != nullptr && blockIdx.x == 0 && tid == 0) { ctl->varying = 0ull; ctl->nexec = 0u; }
+    if (ctl != nullptr && blockIdx.x == 0 && tid == 0) ctl->nexec = 0u;
     if (tid < SB_SPL_EACH) below[tid] = 0u;
 #pragma unroll
     for (uint32_t u = 0; u < UNR; ++u) {
@@ -125,16 +125,13 @@ template <typename T, bool PERM>
 __global__ __launch_bounds__(SB_TILE_BLOCK) void sort_tile_kernel(const T* __restrict__ keys, uint32_t n, int rev, uint32_t k,
                                                                   const typename SortKey<T>::U* __restrict__ spl_key,
                                                                   const uint32_t* __restrict__ spl_pos, uint32_t* __restrict__ table,
-                                                                  typename SortKey<T>::U* __restrict__ tile_min, typename SortKey<T>::U* __restrict__ tile_key,
-                                                                  uint16_t* __restrict__ tile_val) {
+                                                                  typename SortKey<T>::U* __restrict__ tile_key, uint16_t* __restrict__ tile_val) {
     typedef typename SortKey<T>::U U;
     constexpr int BLOCK = SB_TILE_BLOCK, ITEMS = SB_TILE_ITEMS;
-    constexpr bool RECORD = std::is_integral<T>::value;
     __shared__ U lds_key[SB_TILE];
     __shared__ uint16_t lds_val[PERM ? SB_TILE : 1];
     __shared__ U skey[SB_MAX_K];
     __shared__ uint32_t spos[SB_MAX_K], cnt[SB_MAX_K], wsum[SB_MAX_K / WAVE];
-    __shared__ U part[RECORD ? BLOCK / WAVE : 1];
     const uint32_t tid = threadIdx.x, e0 = blockIdx.x * (uint32_t)SB_TILE;
     U key[ITEMS];
     uint32_t bucket[ITEMS], rank[ITEMS];
@@ -177,13 +174,6 @@ __global__ __launch_bounds__(SB_TILE_BLOCK) void sort_tile_kernel(const T* __res
         rank[i] = 0u;
         if (e0 + tid + i * BLOCK < n) rank[i] = atomicAdd(&cnt[bucket[i]], 1u);
     }
-    if constexpr (RECORD) {                                  // the smallest key (those past the end are the last one again)
-        U x = key[0];
-#pragma unroll
-        for (int i = 1; i < ITEMS; ++i) x = key[i] < x ? key[i] : x;
-        x = wave_reduce(x, OpMin());
-        if (tid % WAVE == 0) part[tid / WAVE] = x;
-    }
     __syncthreads();
     uint32_t c = 0u, inc = 0u;
     if (tid < SB_MAX_K) {
@@ -197,12 +187,6 @@ __global__ __launch_bounds__(SB_TILE_BLOCK) void sort_tile_kernel(const T* __res
         for (uint32_t w = 0; w < tid / WAVE; ++w) start += wsum[w];
         cnt[tid] = start;
         table[blockIdx.x * k + tid] = start | c << 16;
-    }
-    if constexpr (RECORD) {
-        if (tid >= BLOCK - WAVE) {
-            const U x = wave_reduce(part[tid % (BLOCK / WAVE)], OpMin());
-            if (tid == BLOCK - WAVE) tile_min[blockIdx.x] = x;
-        }
     }
     __syncthreads();
 #pragma unroll
@@ -291,22 +275,6 @@ __device__ __forceinline__ void sb_radix_pass(U (&key)[ITEMS], uint32_t (&val)[P
     }
 }
 
-// Integers: the digits in which the keys minus the smallest differ are counted for whoever looks at the temporary (ctl->nexec: as
-// many passes would a radix sort take).  A digit is counted by the workgroup whose bits are the first in it; most find all of
-// theirs there already.
-template <typename U> __device__ __forceinline__ void sb_record_digits(SortCtl* ctl, U bits, U* part) {
-    bits = wave_reduce(bits, OpOr());
-    if (lane_id() == 0) part[threadIdx.x / WAVE] = bits;
-    __syncthreads();
-    if (threadIdx.x >= WAVE) return;
-    bits = wave_reduce(part[lane_id() % (SB_SORT_BLOCK / WAVE)], OpOr());
-    if (threadIdx.x != 0 || (bits & ~(U)load_agent(&ctl->varying)) == (U)0) return;
-    const U old = (U)atomicOr(&ctl->varying, (unsigned long long)bits), all = old | bits;
-    uint32_t digits = 0u;
-    for (int p = 0; p < (int)sizeof(U); ++p) digits += digit_of(all, p) != 0u && digit_of(old, p) == 0u ? 1u : 0u;
-    if (digits != 0u) atomicAdd(&ctl->nexec, digits);
-}
-
 // ---- a bucket ------------------------------------------------------------------------------------------------------
 // Bitonic sort of x[0, m) (with y) by the whole workgroup, in LDS or in memory.  The variant whose comparisons all put the
 // smaller element first: elements from m on would be larger than any and never move, so they need not exist.
@@ -356,7 +324,6 @@ template <typename U, bool PERM, int ITEMS, int BLOCK, uint32_t BINS> struct SbL
     alignas(16) char pool[POOL > DIVIDE ? POOL : DIVIDE];
     alignas(16) uint32_t bins[BINS + 4];
     uint32_t part[4][BLOCK / WAVE];
-    U part_key[2][BLOCK / WAVE];
     U key_lo, key_hi;                                        // smallest and largest key of the bucket, lowest and highest index
     uint32_t val_lo, val_hi;
     // by one thread, before a barrier
@@ -369,11 +336,10 @@ template <typename U> __device__ __forceinline__ U sb_uniform(U x) {
 }
 
 // Thread t holds the elements t, t + BLOCK, ... of the m of the bucket, in any order (for those from m on, where others of the
-// thread's row exist, one that does); store(place, key, index) gets each of them.  RECORD: `smallest` is the smallest of all keys,
-// and the digits that vary are counted in ctl.
-template <bool PERM, bool RECORD, int ITEMS, int BLOCK, uint32_t BINS, typename U, typename Store>
+// thread's row exist, one that does); store(place, key, index) gets each of them.
+template <bool PERM, int ITEMS, int BLOCK, uint32_t BINS, typename U, typename Store>
 __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[PERM ? ITEMS : 1], uint32_t m, SbLds<U, PERM, ITEMS, BLOCK, BINS>& lds,
-                                               SortCtl* ctl, U smallest, Store&& store) {
+                                               Store&& store) {
     constexpr int NW = BLOCK / WAVE, PER = (int)BINS / BLOCK;
     constexpr uint32_t CAP = (uint32_t)(ITEMS * BLOCK);
     static_assert(PER % 4 == 0, "a thread scans PER bins, four at a time");
@@ -386,7 +352,6 @@ __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[
     uint32_t* const bin_vhi = bin_vlo + BINS;
     auto& bins = lds.bins;
     auto& part = lds.part;
-    auto& part_key = lds.part_key;
     const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     U lo = (U)~(U)0, hi = (U)0;
     uint32_t rank[ITEMS], vlo = ~0u, vhi = 0u;
@@ -559,12 +524,6 @@ __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[
         }
         return r;
     };
-    U bits = (U)0;
-    if constexpr (RECORD) {
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-            if ((uint32_t)(i * BLOCK) < m) bits |= (U)(key[i] - smallest);
-    }
     if (divide && !compare) {                                           // the keys of this thread as it holds them
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
@@ -590,37 +549,25 @@ __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[
             }
         }
     }
-    if constexpr (RECORD) sb_record_digits<U>(ctl, bits, part_key[1]);
 }
 
 template <typename T, bool PERM>
-__global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl, uint32_t k, uint32_t ntiles, const uint32_t* __restrict__ table,
-                                                                    const typename SortKey<T>::U* __restrict__ tile_min, int rev,
+__global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(uint32_t k, uint32_t ntiles, const uint32_t* __restrict__ table, int rev,
                                                                     const typename SortKey<T>::U* __restrict__ tile_key, const uint16_t* __restrict__ tile_val,
                                                                     typename SortKey<T>::U* big_key, uint32_t* big_val, T* sorted_out, int64_t* perm_out) {
     typedef typename SortKey<T>::U U;
     constexpr int BLOCK = SB_SORT_BLOCK, ITEMS = SB_SORT_ITEMS;
-    constexpr bool RECORD = std::is_integral<T>::value;
     __shared__ SbLds<U, PERM, ITEMS, BLOCK, SB_BINS> lds;
     auto& bins = lds.bins;
     auto& part = lds.part;
-    auto& part_key = lds.part_key;
     uint32_t* const run_off = bins;                          // of a tile: keys of the bucket in the tiles in front (read before bins are)
     uint32_t* const run_at = bins + SB_MAX_TILES;            // where the bucket starts in it
     static_assert(2u * SB_MAX_TILES <= SB_BINS && SB_MAX_TILES <= (uint32_t)BLOCK, "a thread a tile");
     const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, bucket = blockIdx.x;
     uint32_t entry = 0u;
-    U smallest = (U)~(U)0;                                   // of all keys (integers)
     if (tid == 0u) lds.init();
-    if (tid < ntiles) {
-        entry = table[tid * k + bucket];
-        if (RECORD) smallest = tile_min[tid];
-    }
+    if (tid < ntiles) entry = table[tid * k + bucket];
     const uint32_t before = wave_reduce(entry & 0xffffu, OpAdd());
-    if constexpr (RECORD) {
-        smallest = wave_reduce(smallest, OpMin());
-        if (lane == 0) part_key[0][wave] = smallest;
-    }
     const uint32_t run = wave_scan_inclusive(entry >> 16, OpAdd(), 0u);
     if (lane == 0) part[0][wave] = before;
     if (lane == WAVE - 1) part[1][wave] = run;
@@ -631,7 +578,6 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
         start += part[0][w];
         if ((uint32_t)w < wave) off += part[1][w];
         m += part[1][w];
-        if (RECORD) smallest = part_key[0][w] < smallest ? part_key[0][w] : smallest;
     }
     if (tid < SB_MAX_TILES) {
         run_off[tid] = tid < ntiles ? off : ~0u;
@@ -655,14 +601,10 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
             if constexpr (PERM) y[p] = tile * (uint32_t)SB_TILE + tile_val[at];
         }
         sb_bitonic<PERM>(x, y, m);
-        U bits = (U)0;
         for (uint32_t i = tid; i < m; i += BLOCK) {
-            const U u = x[i];
-            if constexpr (RECORD) bits |= (U)(u - smallest);
             if constexpr (PERM) perm_out[start + i] = (int64_t)y[i] + 1;
-            else sorted_out[start + i] = dec_bits<T>(u, rev, (U)0);
+            else sorted_out[start + i] = dec_bits<T>(x[i], rev, (U)0);
         }
-        if constexpr (RECORD) sb_record_digits<U>(ctl, bits, part_key[1]);
         return;
     }
     U key[ITEMS];
@@ -679,7 +621,7 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(SortCtl* ctl
         if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);             // searches four at a time: eleven take too many registers
     }
     start = sb_uniform(start);
-    sb_sort_bucket<PERM, RECORD, ITEMS, BLOCK, SB_BINS>(key, val, m, lds, ctl, smallest, [&](uint32_t to, U x, uint32_t v) {
+    sb_sort_bucket<PERM, ITEMS, BLOCK, SB_BINS>(key, val, m, lds, [&](uint32_t to, U x, uint32_t v) {
         if constexpr (PERM) perm_out[start + to] = (int64_t)v + 1;
         else sorted_out[start + to] = dec_bits<T>(x, rev, (U)0);
     });

@@ -333,7 +333,7 @@ __global__ __launch_bounds__(LS_BLOCK) void sort_parts_kernel(const SortCtl* ctl
             index[i] = PERM ? (from >> shift << shift) + tile_val[from] : sample(j);
         }
     }
-    sb_sort_bucket<true, false, ITEMS, LS_BLOCK, SB_BINS>(key, index, s, lds, nullptr, (U)0, [&](uint32_t to, U x, uint32_t v) {
+    sb_sort_bucket<true, ITEMS, LS_BLOCK, SB_BINS>(key, index, s, lds, [&](uint32_t to, U x, uint32_t v) {
         if (to == 0u || to % LS_OVER != 0u) return;
         spl_key[part * LS_BUCKETS + to / LS_OVER - 1u] = x;
         spl_index[part * LS_BUCKETS + to / LS_OVER - 1u] = v;
@@ -492,7 +492,7 @@ __global__ __launch_bounds__(LS_LAST_BLOCK, (ls_last_waves<typename SortKey<T>::
         if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     start = sb_uniform(start);
-    sb_sort_bucket<PERM, false, ITEMS, BLOCK, LS_BINS>(key, val, m, lds, nullptr, (U)0, [&](uint32_t to, U x, uint32_t v) {
+    sb_sort_bucket<PERM, ITEMS, BLOCK, LS_BINS>(key, val, m, lds, [&](uint32_t to, U x, uint32_t v) {
         if constexpr (PERM) perm_out[start + to] = (int64_t)v + 1;
         else sorted_out[start + to] = dec_bits<T>(x, rev, (U)0);
     });

@@ -150,7 +150,8 @@ def _passes_run(rk, x, perm):
 @pytest.mark.parametrize("n", [2, 4096, 4097, 300_000, 1 << 20])
 def test_digits_that_no_two_relative_keys_differ_in_run_no_pass(rk, orc, dtype, n, perm):
     """Small integer sorts: a pass for every digit in which keys minus the smallest one differ, wherever it stands (an id in
-    the high digits and a small number, perhaps negative, in the low one; a step; a range that carries), and no other."""
+    the high digits and a small number, perhaps negative, in the low one; a step; a range that carries), and no other.  More
+    than 4096 keys of 4 and 8 bytes are sorted by splitters, in no pass at all."""
     rng = np.random.default_rng(n)
     bits = 8 * np.dtype(dtype).itemsize
     ids, small = rng.integers(0, 100, n).astype(np.int64), rng.integers(-100, 101, n).astype(np.int64)
@@ -162,7 +163,7 @@ def test_digits_that_no_two_relative_keys_differ_in_run_no_pass(rk, orc, dtype, 
     for k in cases:
         x = k.astype(dtype)
         rel = np.bitwise_or.reduce(x.astype(np.int64).view(np.uint64) - np.uint64(int(x.min()) & (2 ** 64 - 1)))
-        want = sum(1 for p in range(bits // 8) if (int(rel) >> (8 * p)) & 255)
+        want = sum(1 for p in range(bits // 8) if (int(rel) >> (8 * p)) & 255) if bits == 16 or n <= 4096 else 0
         ran, got = _passes_run(rk, x, perm)
         assert np.array_equal(got, orc.sortperm(x) if perm else orc.sort(x))
         assert ran == want, (ran, want, hex(int(rel)))
