@@ -36,6 +36,8 @@ constexpr int SB_SORT_BLOCK = 1024, SB_SORT_ITEMS = 11;
 constexpr uint32_t SB_CAP = SB_SORT_BLOCK * SB_SORT_ITEMS;   // keys sorted in LDS
 constexpr uint32_t SB_BINS = 4096;               // of a bucket, in LDS
 constexpr uint32_t SB_MAX_BIN = 32;              // largest bin whose keys are ranked by comparing them with each other
+constexpr uint32_t SB_DIVIDE_BIN = 16;           // if there is a larger one: largest that is not divided
+constexpr uint32_t SB_TOGETHER = 24;             // lanes of a wave that go to the bin of the first: from here on they add to it once
 
 // Buckets of a sort of n keys: a power of two (the search among the splitters has no remainder), n / k <= 512 while that is a
 // workgroup a compute unit at most, n / k <= 4096 at 2^20 keys.
@@ -159,14 +161,13 @@ __global__ __launch_bounds__(SB_TILE_BLOCK) void sort_tile_kernel(const T* __res
     for (int i = 0; i < ITEMS; ++i) tie = tie || (bucket[i] < k - 1u && skey[bucket[i]] == key[i]);
     if (tie) {
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t e = e0 + tid + i * BLOCK;
-            uint32_t b = 0u;
-            for (uint32_t step = k / 2u; step != 0u; step /= 2u) {
-                const U x = skey[b + step - 1u];
-                b += (x < key[i] || (x == key[i] && spos[b + step - 1u] <= e)) ? step : 0u;
+        for (int i = 0; i < ITEMS; ++i) bucket[i] = 0u;
+        for (uint32_t step = k / 2u; step != 0u; step /= 2u) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                const U x = skey[bucket[i] + step - 1u];
+                bucket[i] += (x < key[i] || (x == key[i] && spos[bucket[i] + step - 1u] <= e0 + tid + i * BLOCK)) ? step : 0u;
             }
-            bucket[i] = b;
         }
     }
 #pragma unroll
@@ -309,22 +310,32 @@ __device__ __forceinline__ void sb_bitonic(U* x, uint32_t* y, uint32_t m) {
     __syncthreads();
 }
 
-// Inside a bucket the keys are spread over SB_BINS bins by a monotone, nearly linear map of their distance from the smallest
-// (few values, many times over: with the index behind it), in no order, and a key's place in its bin is the number of smaller keys there: a
-// bin holds a key or two, and a wave compares as often as the largest bin it meets has keys.
-// Should a bin exceed SB_MAX_BIN -- a bucket around zero, where the keys of floats are far from linear; a few values many times
-// over -- every bin is divided once more into as many as it has keys, by where a key lies in it (bins of equal keys: by the
-// index; without one they need no order).  What even that does not spread is sorted by comparisons, still in LDS.
+// Inside a bucket the keys are spread over bins by a monotone, nearly linear map of their distance from the smallest, in no order, and a
+// key's place in its bin is the number of smaller keys there: a bin holds a key or two, and a wave compares as often as the largest bin
+// it meets has keys.
+// sortperm: what is spread are the highest 32 bits that vary of the distance and, behind it, the index, so that few values, many times
+// over, are spread as well.
+// Should a bin exceed SB_MAX_BIN -- a bucket around zero, where the keys of floats are far from linear; values in clusters, or few of
+// them, far apart -- every such bin is divided once more, into as many as it has keys (bins of equal keys: by the index; without one they
+// need no order), and those again, SB_LEVELS times.  What even that does not spread is sorted by comparisons, still in LDS.
+// A division takes 3 to 5 us, most of it fetching code that nothing else runs; comparing 4096 keys 50.  2^20 keys, us a call, four radix passes or
+// fewer / comparing what one division by the bucket's range does not spread / so: sort Int32 (id << 16) + small number 45 / 86 / 48, Float64 of
+// whole numbers below 16384 86 / 76 / 51, Float32 of them 56 / 70 / 50; sortperm Int64 (id << 32) + small number 68 / 168 / 59, Float32 of 256
+// values in order 45 / 100 / 43, at random 45 / 58 / 53, of 16 46 / 62 / 52, Int32 of 256 42 / 46 / 42, of 16 42 / 50 / 46.
+constexpr int SB_LEVELS = 6;
+
 // LDS of a workgroup that sorts a bucket of up to ITEMS * BLOCK keys.
 template <typename U, bool PERM, int ITEMS, int BLOCK, uint32_t BINS> struct SbLds {
     static constexpr uint32_t CAP = (uint32_t)(ITEMS * BLOCK);
-    // keys and indices of the bucket; while it is divided a second time, a key of every bin, its lowest and highest index, and the
-    // sizes of the new bins
-    static constexpr size_t KEYS = (size_t)CAP * sizeof(U), POOL = KEYS + (PERM ? (size_t)CAP * 4 : 0), DIVIDE = (size_t)BINS * (sizeof(U) + (PERM ? 8 : 0)) + (size_t)CAP * 4;
+    // keys and indices of the bucket; while bins are divided, the sizes of the new ones and, for a bin that starts at q, smallest and largest
+    // key and index at q / SB_DIVIDE_BIN
+    static constexpr uint32_t LARGE = CAP / SB_DIVIDE_BIN;
+    static constexpr size_t KEYS = (size_t)CAP * sizeof(U), POOL = KEYS + (PERM ? (size_t)CAP * 4 : 0);
+    static constexpr size_t DIVIDE = (size_t)CAP * 4 + (size_t)LARGE * (2 * sizeof(U) + (PERM ? 12 : 4));
     alignas(16) char pool[POOL > DIVIDE ? POOL : DIVIDE];
     alignas(16) uint32_t bins[BINS + 4];
     uint32_t part[4][BLOCK / WAVE];
-    U key_lo, key_hi;                                        // smallest and largest key of the bucket, lowest and highest index
+    U key_lo, key_hi;                                        // smallest and largest key of the bucket, and index
     uint32_t val_lo, val_hi;
     // by one thread, before a barrier
     __device__ __forceinline__ void init() { key_lo = (U)~(U)0; key_hi = (U)0; val_lo = ~0u; val_hi = 0u; }
@@ -335,26 +346,43 @@ template <typename U> __device__ __forceinline__ U sb_uniform(U x) {
     else return (U)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) | (U)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32)) << 32;
 }
 
+// Bits of x.
+template <typename U> __device__ __forceinline__ uint32_t sb_bits(U x) {
+    if constexpr (sizeof(U) == 4) return x == 0u ? 0u : 32u - (uint32_t)__clz((int)x);
+    else return x == 0ull ? 0u : 64u - (uint32_t)__clzll((long long)x);
+}
+
+// Words of LDS that other threads write at the same time.
+template <typename U> __device__ __forceinline__ void sb_put(U* p, U x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+template <typename U> __device__ __forceinline__ U sb_get(const U* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+
+// The highest 32 bits of d, a distance of up to `bits` bits, with `word` behind it (sortperm).
+template <bool PERM, typename U> __device__ __forceinline__ uint32_t sb_code(U d, uint32_t bits, uint32_t word) {
+    const uint32_t top = sizeof(U) == 4 || bits <= 32u ? (uint32_t)d : (uint32_t)((uint64_t)d >> (bits - 32u));
+    if constexpr (PERM) return bits >= 32u ? top : (uint32_t)__builtin_amdgcn_alignbit(top, word, bits);
+    else return bits >= 32u || bits == 0u ? top : top << (32u - bits);
+}
+
 // Thread t holds the elements t, t + BLOCK, ... of the m of the bucket, in any order (for those from m on, where others of the
-// thread's row exist, one that does); store(place, key, index) gets each of them.
-template <bool PERM, int ITEMS, int BLOCK, uint32_t BINS, typename U, typename Store>
+// thread's row exist, one that does); store(place, key, index) gets each of them.  KNOWN: the indices lie in [vlo, vhi]; otherwise
+// the smallest and the largest are looked for.
+template <bool PERM, bool KNOWN, int ITEMS, int BLOCK, uint32_t BINS, typename U, typename Store>
 __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[PERM ? ITEMS : 1], uint32_t m, SbLds<U, PERM, ITEMS, BLOCK, BINS>& lds,
-                                               Store&& store) {
+                                               uint32_t vlo, uint32_t vhi, Store&& store) {
+    typedef SbLds<U, PERM, ITEMS, BLOCK, BINS> Lds;
     constexpr int NW = BLOCK / WAVE, PER = (int)BINS / BLOCK;
-    constexpr uint32_t CAP = (uint32_t)(ITEMS * BLOCK);
+    constexpr uint32_t CAP = Lds::CAP;
+    constexpr bool RANGE = PERM && !KNOWN;
     static_assert(PER % 4 == 0, "a thread scans PER bins, four at a time");
     static_assert(CAP < 1u << 16, "place and size in 32 bits");
     U* const lds_key = (U*)lds.pool;
-    uint32_t* const lds_val = (uint32_t*)(lds.pool + SbLds<U, PERM, ITEMS, BLOCK, BINS>::KEYS);      // (sortperm only)
-    U* const rep = (U*)lds.pool;
-    uint32_t* const sub = (uint32_t*)(lds.pool + (size_t)BINS * sizeof(U));
-    uint32_t* const bin_vlo = sub + CAP;                     // (sortperm only)
-    uint32_t* const bin_vhi = bin_vlo + BINS;
+    uint32_t* const lds_val = (uint32_t*)(lds.pool + Lds::KEYS);        // (sortperm only)
     auto& bins = lds.bins;
     auto& part = lds.part;
     const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     U lo = (U)~(U)0, hi = (U)0;
-    uint32_t rank[ITEMS], vlo = ~0u, vhi = 0u;
+    uint32_t rank[ITEMS];
+    if constexpr (RANGE) { vlo = ~0u; vhi = 0u; }
     m = sb_uniform(m);
     __syncthreads();
 #pragma unroll
@@ -364,7 +392,7 @@ __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[
         if ((uint32_t)(i * BLOCK) < m) {
             lo = key[i] < lo ? key[i] : lo;
             hi = key[i] > hi ? key[i] : hi;
-            if constexpr (PERM) {
+            if constexpr (RANGE) {
                 vlo = val[i] < vlo ? val[i] : vlo;
                 vhi = val[i] > vhi ? val[i] : vhi;
             }
@@ -373,7 +401,7 @@ __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[
     lo = wave_reduce(lo, OpMin());
     hi = wave_reduce(hi, OpMax());
     if (lane == 0) { atomicMin(&lds.key_lo, lo); atomicMax(&lds.key_hi, hi); }
-    if constexpr (PERM) {
+    if constexpr (RANGE) {
         vlo = wave_reduce(vlo, OpMin());
         vhi = wave_reduce(vhi, OpMax());
         if (lane == 0) { atomicMin(&lds.val_lo, vlo); atomicMax(&lds.val_hi, vhi); }
@@ -381,31 +409,43 @@ __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[
     __syncthreads();
     lo = sb_uniform(lds.key_lo);
     hi = sb_uniform(lds.key_hi);
-    if constexpr (PERM) {
+    const U span = hi - lo;
+    const uint32_t bits = sb_bits(span);
+    if constexpr (RANGE) {
         vlo = sb_uniform(lds.val_lo);
         vhi = sb_uniform(lds.val_hi);
     }
-    // distance of a key from the smallest; with its index in the low bits if that fits 32: then no two are equal
-    const uint64_t span = (uint64_t)(U)(hi - lo);
-    const uint32_t vspan = vhi - vlo, vbits = !PERM || vspan == 0u ? 0u : 32u - (uint32_t)__clz((int)vspan);
-    const bool both = PERM && (span >> (32u - vbits)) == 0ull;         // (vbits <= 20)
-    const uint64_t width = both ? span << vbits | vspan : span;
-    const uint32_t shift = width >> 32 ? 32u - (uint32_t)__clz((int)(uint32_t)(width >> 32)) : 0u;
-    const uint32_t w32 = (uint32_t)(width >> shift);
-    const bool exact = shift == 0u && w32 < BINS;                   // a bin is one value
-    // w32 * scale < BINS * 2^32: the last bin is BINS - 1.  (The two roundings and the reciprocal are off by 3 units of 2^-24
+    const uint32_t vspan = vhi - vlo, vshift = vspan == 0u ? 0u : 32u - sb_bits(vspan);
+    const auto word_of = [&](uint32_t v) -> uint32_t { return PERM ? (v - vlo) << vshift : 0u; };
+    // a bin is one value; sortperm: of equal keys, one index
+    const bool exact = PERM ? bits == 0u && vspan < BINS : span < (U)BINS;
+    // code * scale < BINS * 2^32: the last bin is BINS - 1.  (The two roundings and the reciprocal are off by 3 units of 2^-24
     // at most, the last factor is 8 units below 1.)
-    const uint32_t scale = exact ? 0u : sb_uniform((uint32_t)((float)BINS * 4294967296.f * __builtin_amdgcn_rcpf((float)w32 + 1.f) * (1.f - 0x1p-21f)));
-    auto distance = [&](U x, uint32_t v) -> uint32_t {
+    const uint32_t most_code = sb_code<PERM>(span, bits, vspan << vshift);
+    const uint32_t scale = exact ? 0u : sb_uniform((uint32_t)((float)BINS * 4294967296.f * __builtin_amdgcn_rcpf((float)most_code + 1.f) * (1.f - 0x1p-21f)));
+    auto code_of = [&](U x, uint32_t v) -> uint32_t {
         asm volatile("" : "+v"(x));                // computed again at every use: kept, the bins of eleven keys spilled 20 registers
-        if constexpr (sizeof(U) == 4 && !PERM) return x - lo;
-        else return both ? (uint32_t)(U)(x - lo) << vbits | (v - vlo) : (uint32_t)((uint64_t)(U)(x - lo) >> shift);
+        return sb_code<PERM>((U)(x - lo), bits, word_of(v));
     };
-    auto bin_of = [&](U x, uint32_t v) -> uint32_t { return exact ? distance(x, v) : __umulhi(distance(x, v), scale); };
+    auto bin_of = [&](U x, uint32_t v) -> uint32_t {
+        if (exact) return PERM ? v - vlo : (uint32_t)(x - lo);
+        return __umulhi(code_of(x, v), scale);
+    };
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
         rank[i] = 0u;
-        if (tid + i * BLOCK < m) rank[i] = atomicAdd(&bins[bin_of(key[i], val[PERM ? i : 0])], 1u);
+        if ((uint32_t)(i * BLOCK) >= m) continue;
+        const bool valid = tid + i * BLOCK < m;
+        const uint32_t b = bin_of(key[i], val[PERM ? i : 0]), b0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+        const uint64_t same = __ballot(valid && b == b0);
+        const uint32_t together = (uint32_t)__popcll(same);
+        if (together >= SB_TOGETHER) {                          // (lane 0 is one of them)
+            if (lane == 0u) rank[i] = atomicAdd(&bins[b0], together);
+            rank[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)rank[i]) + __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+            if (valid && b != b0) rank[i] = atomicAdd(&bins[b], 1u);
+        } else if (valid) {
+            rank[i] = atomicAdd(&bins[b], 1u);
+        }
     }
     __syncthreads();
     uint32_t c[PER], sum = 0u, most = 0u;
@@ -432,121 +472,294 @@ __device__ __forceinline__ void sb_sort_bucket(U (&key)[ITEMS], uint32_t (&val)[
     for (int j = 0; j < PER; j += 4) *(uint4*)&bins[tid * PER + j] = make_uint4(c[j], c[j + 1], c[j + 2], c[j + 3]);
     if (tid == 0) bins[BINS] = m;
     __syncthreads();
-    const bool ordered = exact && (!PERM || both);                     // a bin holds equal keys (one index): nothing to compare
-    const bool divide = !ordered && largest > SB_MAX_BIN;
-    bool compare = false;
-    if (divide) {
-        // which bins hold different keys (bit 31), then the division
-        for (uint32_t i = tid; i < CAP; i += BLOCK) sub[i] = 0u;
-        if constexpr (PERM) {
-            for (uint32_t i = tid; i < BINS; i += BLOCK) { bin_vlo[i] = ~0u; bin_vhi[i] = 0u; }
-        }
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-            if (tid + i * BLOCK < m) rep[bin_of(key[i], val[PERM ? i : 0])] = key[i];
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            if (tid + i * BLOCK < m) {
-                const uint32_t b = bin_of(key[i], val[PERM ? i : 0]);
-                if (rep[b] != key[i]) atomicOr(&bins[b], 0x80000000u);
-                if constexpr (PERM) {
-                    atomicMin(&bin_vlo[b], val[PERM ? i : 0]);
-                    atomicMax(&bin_vhi[b], val[PERM ? i : 0]);
-                }
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            if (tid + i * BLOCK < m) {
-                const uint32_t d = distance(key[i], val[PERM ? i : 0]), b = exact ? d : __umulhi(d, scale);
-                const uint32_t q = bins[b], q0 = q & 0x7fffffffu, size = (bins[b + 1u] & 0x7fffffffu) - q0;
-                uint32_t id;
-                if (both || q >> 31) id = q0 + __umulhi(d * scale, size);
-                else if constexpr (PERM) {
-                    const uint32_t from = bin_vlo[b], spread = bin_vhi[b] - from;
-                    id = q0 + __umulhi((val[PERM ? i : 0] - from) << (spread == 0u ? 0 : __clz((int)spread)), size);
-                }
-                else id = q0 + rank[i];
-                rank[i] = id | atomicAdd(&sub[id], 1u) << 16;
-            }
-        }
-        __syncthreads();
-        uint32_t s[ITEMS], total = 0u, top = 0u;
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            s[i] = sub[tid * ITEMS + i];
-            total += s[i];
-            top = s[i] > top ? s[i] : top;
-        }
-        const uint32_t run2 = wave_scan_inclusive(total, OpAdd(), 0u);
-        top = wave_reduce(top, OpMax());
-        if (lane == WAVE - 1) { part[2][wave] = run2; part[3][wave] = top; }
-        __syncthreads();
-        uint32_t at = run2 - total;
-        largest = 0u;
-        for (int w = 0; w < NW; ++w) {
-            if ((uint32_t)w < wave) at += part[2][w];
-            largest = part[3][w] > largest ? part[3][w] : largest;
-        }
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            sub[tid * ITEMS + i] = at | s[i] << 16;
-            at += s[i];
-        }
-        __syncthreads();
-        compare = sb_uniform(largest) > SB_MAX_BIN;
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            if (tid + i * BLOCK < m) {                                 // place in the bucket | place in the bin << 16 | size of the bin << 22
-                const uint32_t q = sub[rank[i] & 0xffffu], r = rank[i] >> 16;
-                rank[i] = ((q & 0xffffu) + r) | (compare ? 0u : r << 16 | (q >> 16) << 22);
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-        if (tid + i * BLOCK < m) {
-            const uint32_t p = divide ? rank[i] & 0xffffu : bins[bin_of(key[i], val[PERM ? i : 0])] + rank[i];
-            lds_key[p] = key[i];
-            if constexpr (PERM) lds_val[p] = val[i];
-        }
-    }
-    __syncthreads();
-    auto smaller = [&](U x, uint32_t v, uint32_t q0, uint32_t q1) -> uint32_t {        // of the elements [q0, q1)
+    // elements [q0, q1) that come before one, which stands at p
+    auto smaller = [&](U x, uint32_t v, uint32_t q0, uint32_t q1) -> uint32_t {
         uint32_t r = 0u;
-        for (uint32_t q = q0; q < q1; ++q) {
-            const U o = lds_key[q];
-            const uint32_t ov = PERM ? lds_val[PERM ? q : 0] : q;
-            r += (o < x || (o == x && ov < v)) ? 1u : 0u;
+        constexpr uint32_t FLIGHT = PERM ? 4u : 2u;
+        for (uint32_t q = q0; q < q1; q += FLIGHT) {
+            U o[FLIGHT];
+            uint32_t ov[FLIGHT];
+#pragma unroll
+            for (uint32_t j = 0; j < FLIGHT; ++j) {
+                const uint32_t at = q + j < q1 ? q + j : q;
+                o[j] = lds_key[at];
+                ov[j] = PERM ? lds_val[PERM ? at : 0] : at;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < FLIGHT; ++j) r += q + j < q1 && (o[j] < x || (o[j] == x && ov[j] < v)) ? 1u : 0u;
         }
         return r;
     };
-    if (divide && !compare) {                                           // the keys of this thread as it holds them
+    if (exact || largest <= SB_MAX_BIN) {
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
             if (tid + i * BLOCK < m) {
-                const uint32_t p = rank[i] & 0xffffu, q0 = p - ((rank[i] >> 16) & 0x3fu);
-                const uint32_t v = PERM ? val[PERM ? i : 0] : p;
-                store(q0 + smaller(key[i], v, q0, q0 + (rank[i] >> 22)), key[i], v);
+                const uint32_t p = bins[bin_of(key[i], val[PERM ? i : 0])] + rank[i];
+                lds_key[p] = key[i];
+                if constexpr (PERM) lds_val[p] = val[i];
             }
         }
-    } else {
-        if (compare) sb_bitonic<PERM>(lds_key, lds_val, m);
+        __syncthreads();
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) {
-                const uint32_t p = tid + i * BLOCK;
+            const uint32_t p = tid + i * BLOCK;
             if (p >= m) continue;
             const U x = lds_key[p];
             const uint32_t v = PERM ? lds_val[PERM ? p : 0] : p;
-            if (ordered || compare) {
+            if (exact) {                                                // nothing to compare
                 store(p, x, v);
             } else {
                 const uint32_t b = bin_of(x, v), q0 = bins[b];
                 store(q0 + smaller(x, v, q0, bins[b + 1u]), x, v);
             }
+        }
+        return;
+    }
+    // rank: from here on, where the element's bin starts, and of a bin that can be compared its size << 16 and the element's place in
+    // it << 24, of others the element's place << 16
+    constexpr uint32_t LARGE = 0x80000000u;
+    constexpr int ROWS = ITEMS > 8 ? 4 : 2;                             // whose reads are in flight together
+    static_assert(SB_MAX_BIN <= 64u && CAP < 1u << 14, "start, size and place in 31 bits");
+    uint32_t* const sub = (uint32_t*)lds.pool;
+    U* const bin_lo = (U*)(lds.pool + (size_t)CAP * 4);
+    U* const bin_hi = bin_lo + Lds::LARGE;
+    uint32_t* const bin_size = (uint32_t*)(bin_hi + Lds::LARGE);
+    uint32_t* const bin_vlo = bin_size + Lds::LARGE;                    // (sortperm only)
+    uint32_t* const bin_vhi = bin_vlo + Lds::LARGE;
+    const auto entry = [](uint32_t r) { return (r & 0xffffu) / SB_DIVIDE_BIN % Lds::LARGE; };
+    const auto place_in_bin = [](uint32_t r) { return (r & LARGE) != 0u ? (r & ~LARGE) >> 16 : r >> 24; };
+    const auto divides = [](uint32_t r) { return (r & LARGE) != 0u || (r >> 16 & 0xffu) > SB_DIVIDE_BIN; };
+    // Of the lanes side by side that go to one entry, the first: 64 that write to one word of LDS take 70 cycles.  (All lanes call.)
+    const auto first_of_run = [](uint32_t at) { return (uint32_t)__builtin_amdgcn_update_dpp((int)~at, (int)at, 0x138, 0xf, 0xf, false) != at; };
+    const auto enter = [&](bool valid, uint32_t q0, uint32_t size, uint32_t place) -> uint32_t {
+        const bool writes = valid && size > SB_DIVIDE_BIN;
+        if (first_of_run(writes ? q0 : ~0u) && writes) sb_put(&bin_size[q0 / SB_DIVIDE_BIN], size);
+        return size <= SB_MAX_BIN ? q0 | size << 16 | place << 24 : LARGE | q0 | place << 16;
+    };
+#pragma unroll
+    for (int i0 = 0; i0 < ITEMS; i0 += ROWS) {
+        uint32_t q0[ROWS], q1[ROWS];
+#pragma unroll
+        for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+            if ((uint32_t)((i0 + j) * BLOCK) >= m) continue;
+            const uint32_t b = bin_of(key[i0 + j], val[PERM ? i0 + j : 0]);
+            q0[j] = bins[b];
+            q1[j] = bins[b + 1u];
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+            if ((uint32_t)((i0 + j) * BLOCK) >= m) continue;
+            rank[i0 + j] = enter(tid + (i0 + j) * BLOCK < m, q0[j], q1[j] - q0[j], rank[i0 + j]);
+        }
+    }
+    // How bins are first divided: as though their keys were spread evenly in them, with less than 2/5 of the bucket in the largest (around
+    // zero, floats have up to 1/20 in a bin, Float64 1/4; two values would have half), otherwise from their smallest to their largest key.
+    // Evenly, bins of equal keys are told from others first, unless 4-byte keys have less than 1/8 in the largest: the float buckets
+    // around zero of sorts up to 2^20 keys are what those sorts wait for (sort Float32[2^20] 35.8 -> 34.7 us; 64 equal keys a bin 44 -> 51).
+    constexpr bool UNSEEN = sizeof(U) == 4 && ITEMS > 8;
+    bool any_mixed = true;                                              // there is a bin of different keys
+    for (int level = 0; level < SB_LEVELS && largest > SB_MAX_BIN; ++level) {
+        const bool evenly = level == 0 && largest * 5u <= m * 2u, unseen = UNSEEN && evenly && largest * 8u <= m;
+        if (level != 0) __syncthreads();
+        for (uint32_t i = tid; i < m; i += BLOCK) sub[i] = 0u;
+        // the range of every bin: from any of its elements, then those outside what is known move it, a few of them first: of a few keys
+        // many times over, all 64 lanes of a wave would move the same range, one after the other
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (unseen || (uint32_t)(i * BLOCK) >= m) continue;
+            const bool writes = tid + i * BLOCK < m && divides(rank[i]);
+            const uint32_t at = entry(rank[i]);
+            if (first_of_run(writes ? at : ~0u) && writes) {
+                sb_put(&bin_lo[at], key[i]);
+                sb_put(&bin_hi[at], key[i]);
+                if (PERM && !evenly) { sb_put(&bin_vlo[at], val[PERM ? i : 0]); sb_put(&bin_vhi[at], val[PERM ? i : 0]); }
+            }
+        }
+        __syncthreads();
+        bool mixed = false;
+        if (evenly && !unseen) {
+#pragma unroll
+            for (int i0 = 0; i0 < ITEMS; i0 += ROWS) {
+                if ((uint32_t)(i0 * BLOCK) >= m) continue;
+                U from[ROWS], to[ROWS];
+#pragma unroll
+                for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+                    const uint32_t at = entry(rank[i0 + j]);
+                    from[j] = sb_get(&bin_lo[at]);
+                    to[j] = sb_get(&bin_hi[at]);
+                }
+#pragma unroll
+                for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+                    const int i = i0 + j;
+                    if (tid + i * BLOCK < m && divides(rank[i]) && key[i] != from[j]) {
+                        mixed = true;
+                        if (to[j] == from[j]) sb_put(&bin_hi[entry(rank[i])], key[i]);
+                    }
+                }
+            }
+        } else if (!unseen) {
+            const auto move = [&](int i, U from, U to, uint32_t vfrom, uint32_t vto) {
+                if (tid + i * BLOCK < m && divides(rank[i])) {
+                    const uint32_t at = entry(rank[i]);
+                    mixed = mixed || key[i] != from || key[i] != to;
+                    if (key[i] < from) atomicMin(&bin_lo[at], key[i]);
+                    if (key[i] > to) atomicMax(&bin_hi[at], key[i]);
+                    if constexpr (PERM) {
+                        if (val[i] < vfrom) atomicMin(&bin_vlo[at], val[i]);
+                        if (val[i] > vto) atomicMax(&bin_vhi[at], val[i]);
+                    }
+                }
+            };
+            if (lane % 16u == 0u) {
+                const uint32_t at = entry(rank[0]);
+                move(0, sb_get(&bin_lo[at]), sb_get(&bin_hi[at]), PERM ? sb_get(&bin_vlo[at]) : 0u, PERM ? sb_get(&bin_vhi[at]) : 0u);
+            }
+#pragma unroll
+            for (int i0 = 0; i0 < ITEMS; i0 += ROWS) {
+                if ((uint32_t)(i0 * BLOCK) >= m) continue;
+                U from[ROWS], to[ROWS];
+                uint32_t vfrom[ROWS], vto[ROWS];
+#pragma unroll
+                for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+                    const uint32_t at = entry(rank[i0 + j]);
+                    from[j] = sb_get(&bin_lo[at]);
+                    to[j] = sb_get(&bin_hi[at]);
+                    vfrom[j] = PERM ? sb_get(&bin_vlo[at]) : 0u;
+                    vto[j] = PERM ? sb_get(&bin_vhi[at]) : 0u;
+                }
+#pragma unroll
+                for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) move(i0 + j, from[j], to[j], vfrom[j], vto[j]);
+            }
+        }
+        if (PERM && !unseen) {
+            __syncthreads();
+        } else if (!unseen) {
+            any_mixed = __syncthreads_or(mixed ? 1 : 0) != 0;
+            if (!any_mixed) break;                                      // equal keys need no order
+        }
+#pragma unroll
+        for (int i0 = 0; i0 < ITEMS; i0 += ROWS) {
+            if ((uint32_t)(i0 * BLOCK) >= m) continue;
+            U from[ROWS], wide[ROWS];
+            uint32_t size[ROWS], vfrom[PERM ? ROWS : 1], vwide[PERM ? ROWS : 1];
+#pragma unroll
+            for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+                const uint32_t at = entry(rank[i0 + j]);
+                from[j] = bin_lo[at];
+                wide[j] = (U)(bin_hi[at] - from[j]);
+                size[j] = bin_size[at];
+                if constexpr (PERM) {
+                    vfrom[j] = evenly ? vlo : bin_vlo[at];
+                    vwide[j] = evenly ? vspan : bin_vhi[at] - vfrom[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+                const int i = i0 + j;
+                if (tid + i * BLOCK < m) {
+                    uint32_t id = rank[i] & 0xffffu;
+                    const bool large = divides(rank[i]);
+                    const uint32_t bw = sb_bits(wide[j]);
+                    if (level != 0 && !large) {
+                        atomicAdd(&sub[id], 1u);
+                        continue;
+                    }
+                    if (!large || unseen || (evenly && bw != 0u)) {     // by where in its bin the element lies
+                        const uint32_t in_bin = code_of(key[i], val[PERM ? i : 0]) * scale;
+                        id += __umulhi(in_bin, large ? size[j] : rank[i] >> 16 & 0xffu);
+                    } else if (!PERM && bw == 0u) {
+                        id += place_in_bin(rank[i]);
+                    } else {
+                        uint32_t word = 0u, most_word = 0u;
+                        if constexpr (PERM) {
+                            const int vs = vwide[j] == 0u ? 0 : __clz((int)vwide[j]);
+                            word = (val[i] - vfrom[j]) << vs;
+                            most_word = vwide[j] << vs;
+                        }
+                        // as above: below `size` for all of the bin
+                        const uint32_t most_of_bin = sb_code<PERM>(wide[j], bw, most_word);
+                        const uint32_t per = (uint32_t)((float)size[j] * 4294967296.f * __builtin_amdgcn_rcpf((float)most_of_bin + 1.f) * (1.f - 0x1p-21f));
+                        id += __umulhi(sb_code<PERM>((U)(key[i] - from[j]), bw, word), per);
+                    }
+                    rank[i] = LARGE | id | atomicAdd(&sub[id], 1u) << 16;
+                }
+            }
+        }
+        __syncthreads();
+        uint32_t s[ITEMS], total = 0u, top = 0u;
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) s[i] = sub[tid * ITEMS + i];
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (tid * ITEMS + i >= m) s[i] = 0u;
+            total += s[i];
+            top = s[i] > top ? s[i] : top;
+        }
+        const uint32_t run = wave_scan_inclusive(total, OpAdd(), 0u);
+        top = wave_reduce(top, OpMax());
+        if (lane == WAVE - 1) { part[2][wave] = run; part[3][wave] = top; }
+        __syncthreads();
+        uint32_t at = run - total;
+        largest = 0u;
+        for (int w = 0; w < NW; ++w) {
+            if ((uint32_t)w < wave) at += part[2][w];
+            largest = part[3][w] > largest ? part[3][w] : largest;
+        }
+        largest = sb_uniform(largest);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            if (tid * ITEMS + i < m) sub[tid * ITEMS + i] = at | s[i] << 16;
+            at += s[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i0 = 0; i0 < ITEMS; i0 += ROWS) {
+            if ((uint32_t)(i0 * BLOCK) >= m) continue;
+            uint32_t q[ROWS];
+#pragma unroll
+            for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) q[j] = sub[rank[i0 + j] & 0xffffu];
+#pragma unroll
+            for (int j = 0; j < ROWS && i0 + j < ITEMS; ++j) {
+                const int i = i0 + j;
+                const bool valid = tid + i * BLOCK < m && (level == 0 || divides(rank[i]));
+                const uint32_t r = enter(valid, q[j] & 0xffffu, q[j] >> 16, place_in_bin(rank[i]));
+                if (valid) rank[i] = r;
+            }
+        }
+    }
+    __syncthreads();
+    if (any_mixed && largest > SB_MAX_BIN) {                            // in any order
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t p = tid + i * BLOCK;
+            if (p < m) {
+                lds_key[p] = key[i];
+                if constexpr (PERM) lds_val[p] = val[i];
+            }
+        }
+        sb_bitonic<PERM>(lds_key, lds_val, m);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const uint32_t p = tid + i * BLOCK;
+            if (p < m) store(p, lds_key[p], PERM ? lds_val[PERM ? p : 0] : p);
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        if (tid + i * BLOCK < m) {
+            const uint32_t p = (rank[i] & 0xffffu) + place_in_bin(rank[i]);
+            lds_key[p] = key[i];
+            if constexpr (PERM) lds_val[p] = val[i];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {                                   // the elements of this thread as it holds them
+        if (tid + i * BLOCK < m) {
+            const uint32_t q0 = rank[i] & 0xffffu, p = q0 + place_in_bin(rank[i]), v = PERM ? val[PERM ? i : 0] : p;
+            if (!PERM && (rank[i] & LARGE) != 0u) store(p, key[i], v);
+            else store(q0 + smaller(key[i], v, q0, q0 + (rank[i] >> 16 & 0xffu)), key[i], v);
         }
     }
 }
@@ -569,13 +782,20 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(uint32_t k, 
     if (tid < ntiles) entry = table[tid * k + bucket];
     const uint32_t before = wave_reduce(entry & 0xffffu, OpAdd());
     const uint32_t run = wave_scan_inclusive(entry >> 16, OpAdd(), 0u);
-    if (lane == 0) part[0][wave] = before;
+    const uint64_t there = __ballot((entry >> 16) != 0u);     // tiles that hold keys of the bucket
+    if (lane == 0) {
+        part[0][wave] = before;
+        part[2][wave] = there == 0ull ? ~0u : wave * WAVE + (uint32_t)__builtin_ctzll(there);
+        part[3][wave] = there == 0ull ? 0u : wave * WAVE + (WAVE - 1) - (uint32_t)__builtin_clzll(there);
+    }
     if (lane == WAVE - 1) part[1][wave] = run;
     __syncthreads();
-    uint32_t start = 0u, off = run - (entry >> 16), m = 0u;
+    uint32_t start = 0u, off = run - (entry >> 16), m = 0u, first_tile = ~0u, last_tile = 0u;
 #pragma unroll
     for (int w = 0; w < (int)SB_MAX_TILES / WAVE; ++w) {
         start += part[0][w];
+        first_tile = part[2][w] < first_tile ? part[2][w] : first_tile;
+        last_tile = part[3][w] > last_tile ? part[3][w] : last_tile;
         if ((uint32_t)w < wave) off += part[1][w];
         m += part[1][w];
     }
@@ -621,7 +841,7 @@ __global__ __launch_bounds__(SB_SORT_BLOCK) void sort_bucket_kernel(uint32_t k, 
         if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);             // searches four at a time: eleven take too many registers
     }
     start = sb_uniform(start);
-    sb_sort_bucket<PERM, ITEMS, BLOCK, SB_BINS>(key, val, m, lds, [&](uint32_t to, U x, uint32_t v) {
+    sb_sort_bucket<PERM, true, ITEMS, BLOCK, SB_BINS>(key, val, m, lds, sb_uniform(first_tile) * (uint32_t)SB_TILE, sb_uniform(last_tile) * (uint32_t)SB_TILE + (SB_TILE - 1), [&](uint32_t to, U x, uint32_t v) {
         if constexpr (PERM) perm_out[start + to] = (int64_t)v + 1;
         else sorted_out[start + to] = dec_bits<T>(x, rev, (U)0);
     });

@@ -87,14 +87,13 @@ __device__ __forceinline__ void ls_split_tile(U (&key)[ITEMS], const V (&val)[PE
     }
     if (tie) {
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t e = index(i);
-            uint32_t b = 0u;
-            for (uint32_t step = leaves / 2u; step != 0u; step /= 2u) {
-                const U x = s.ordered[b + step - 1u];
-                b += (x < key[i] || (x == key[i] && s.index[b + step - 1u] <= e)) ? step : 0u;
+        for (int i = 0; i < ITEMS; ++i) place[i] = 0u;
+        for (uint32_t step = leaves / 2u; step != 0u; step /= 2u) {
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                const U x = s.ordered[place[i] + step - 1u];
+                place[i] += (x < key[i] || (x == key[i] && s.index[place[i] + step - 1u] <= index(i))) ? step : 0u;
             }
-            place[i] = b;
         }
     }
 #pragma unroll
@@ -333,7 +332,7 @@ __global__ __launch_bounds__(LS_BLOCK) void sort_parts_kernel(const SortCtl* ctl
             index[i] = PERM ? (from >> shift << shift) + tile_val[from] : sample(j);
         }
     }
-    sb_sort_bucket<true, ITEMS, LS_BLOCK, SB_BINS>(key, index, s, lds, [&](uint32_t to, U x, uint32_t v) {
+    sb_sort_bucket<true, false, ITEMS, LS_BLOCK, SB_BINS>(key, index, s, lds, 0u, 0u, [&](uint32_t to, U x, uint32_t v) {
         if (to == 0u || to % LS_OVER != 0u) return;
         spl_key[part * LS_BUCKETS + to / LS_OVER - 1u] = x;
         spl_index[part * LS_BUCKETS + to / LS_OVER - 1u] = v;
@@ -406,7 +405,7 @@ __global__ __launch_bounds__(LS_BLOCK, (ls_split_waves<typename SortKey<T>::U, P
     if (d.count == TILE) split(std::true_type{}); else split(std::false_type{});
 }
 
-template <typename U, bool PERM> constexpr int ls_last_waves() { return PERM ? 4 : sizeof(U) == 8 ? 6 : 8; }
+template <typename U, bool PERM> constexpr int ls_last_waves() { return PERM && sizeof(U) == 8 ? 4 : PERM || sizeof(U) == 8 ? 6 : 8; }
 
 // A workgroup a bucket.  xcd_chunk: each XCD takes neighbouring buckets (0: as they come), which share the lines where their runs meet.
 template <typename T, bool PERM>
@@ -492,7 +491,7 @@ __global__ __launch_bounds__(LS_LAST_BLOCK, (ls_last_waves<typename SortKey<T>::
         if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     start = sb_uniform(start);
-    sb_sort_bucket<PERM, ITEMS, BLOCK, LS_BINS>(key, val, m, lds, [&](uint32_t to, U x, uint32_t v) {
+    sb_sort_bucket<PERM, false, ITEMS, BLOCK, LS_BINS>(key, val, m, lds, 0u, 0u, [&](uint32_t to, U x, uint32_t v) {
         if constexpr (PERM) perm_out[start + to] = (int64_t)v + 1;
         else sorted_out[start + to] = dec_bits<T>(x, rev, (U)0);
     });

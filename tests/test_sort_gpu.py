@@ -308,13 +308,16 @@ def _spread(rng, dtype, n, kind):
         x = rng.integers(0, 200, n) * 3 + rng.choice(np.array([0, 1 << 20, (1 << 20) + 5000], dtype=np.int64), n)
         x[:: n // 7] = 1 << 30
         return x.astype(dt)
+    if kind == "gaps":                                  # a few small numbers, again and again far apart, and those once more: what several
+        far, near = (1 << 40, 1 << 20) if dt.itemsize == 8 else (1 << 20, 1 << 10)           # divisions of a bucket take apart
+        return (rng.integers(0, 50, n) * far + rng.integers(0, 3, n) * near + rng.integers(0, 3, n)).astype(dt)
     if kind == "steep":                                 # every order of magnitude, both signs
         x = np.exp(rng.uniform(-20, 20, n)) * rng.choice([-1.0, 1.0], n)
         return x.astype(dt)
     return (rng.standard_normal(n) * (1 if dt.kind == "f" else 1 << 24)).astype(dt)
 
 
-@pytest.mark.parametrize("kind", ["sorted", "equal", "few", "hundreds", "clusters", "steep", "normal"])
+@pytest.mark.parametrize("kind", ["sorted", "equal", "few", "hundreds", "clusters", "gaps", "steep", "normal"])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
 def test_sorts_by_splitters(rk, orc, dtype, kind):
     """4096 keys are the last that fit a workgroup, 2^20 the last that take buckets; 512 keys a bucket up to 131072 and more
@@ -346,7 +349,7 @@ def test_bucket_larger_than_lds(rk, orc, dtype, few):
     _check(rk, orc, x)
 
 
-@pytest.mark.parametrize("kind", ["sorted", "equal", "few", "hundreds", "clusters", "steep", "normal"])
+@pytest.mark.parametrize("kind", ["sorted", "equal", "few", "hundreds", "clusters", "gaps", "steep", "normal"])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
 def test_sorts_by_two_levels_of_splitters(rk, orc, dtype, kind):
     """More than 2^20 keys; tiles of 4096 keys below 2^22 and of 8192 from there on, of which the last is full, or holds one key."""
