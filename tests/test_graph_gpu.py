@@ -125,3 +125,40 @@ def test_graph_replays_of_findall_reverse_permutedims_sort(rk, orc):
         assert np.array_equal(rk.Array(keys), orc.sort(hk, rev=True)), replay
         assert np.array_equal(rk.Array(rev), h2[::-1, :]), replay
         assert np.array_equal(rk.Array(tr), h2.T), replay
+
+
+def test_graph_replays_of_sorts_by_two_levels_of_splitters(rk, orc):
+    """Of Int64 keys the device decides by their digits, in every replay anew, whether radix passes or splitters sort them."""
+    from amdgpu_jl_amd import _lib as L
+    from amdgpu_jl_amd.array import stream_ptr
+
+    n = (1 << 20) + 4099
+    rng = np.random.default_rng(44)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        f, i = rk.ROCArray(dims=(n,), dtype=np.float64), rk.ROCArray(dims=(n,), dtype=np.int64)
+        fs, perm = rk.ROCArray(dims=(n,), dtype=np.float64), rk.ROCArray(dims=(n,), dtype=np.int64)
+        tmp = torch.empty(int(L.lib.rk_sort_tmp_bytes(L.RK_I64, n, 1)), dtype=torch.uint8, device="cuda")
+
+        def calls():
+            s = stream_ptr()
+            L.check(L.lib.rk_sort_to(L.RK_F64, f.ptr, fs.ptr, n, 1, tmp.data_ptr(), tmp.numel(), s), "rk_sort_to")
+            L.check(L.lib.rk_sortperm(L.RK_I64, i.ptr, perm.ptr, n, 0, tmp.data_ptr(), tmp.numel(), s), "rk_sortperm")
+            L.check(L.lib.rk_sort(L.RK_I64, i.ptr, n, 0, tmp.data_ptr(), tmp.numel(), s), "rk_sort")
+        f.buf.zero_(); i.buf.zero_()
+        calls()
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        calls()
+    for replay in range(4):
+        hf = rng.standard_normal(n)
+        hi = rng.integers(-2**62, 2**62, n) if replay % 2 == 0 else rng.integers(-1000, 1000, n)
+        _upload(f, hf); _upload(i, hi)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(rk.Array(fs), orc.sort(hf, rev=True)), replay
+        assert np.array_equal(rk.Array(perm), orc.sortperm(hi)), replay
+        assert np.array_equal(rk.Array(i), orc.sort(hi)), replay
+        assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(hi))), orc.sort(hi))         # eager work between the replays

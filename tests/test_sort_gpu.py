@@ -107,10 +107,11 @@ def test_full_size_sort(rk, orc):
 
 
 @pytest.mark.parametrize("tiles", [1, 2, 7, 8, 9, 127, 128, 129, 255, 256, 257])
-@pytest.mark.parametrize("dtype", [np.int16, np.float32, np.int64])
+@pytest.mark.parametrize("dtype", [np.int16, np.float16, np.float32, np.int64])
 def test_table_of_counts_edges(rk, orc, dtype, tiles):
-    # up to 256 tiles of 4096 keys every workgroup sums the columns of the table of counts itself (8 groups of rows, 16 rows
-    # a round): one key more and less than whole tiles around the edges of the groups and of the dispatch
+    # up to 256 tiles of 4096 keys every workgroup of a pass over 2-byte keys sums the columns of the table of counts itself (8
+    # groups of rows, 16 rows a round): one key more and less than whole tiles around the edges of the groups and of the dispatch;
+    # 4- and 8-byte keys have the edges of the tiles that splitters sort there
     rng = np.random.default_rng(tiles)
     for n in (tiles * 4096 - 1, tiles * 4096, tiles * 4096 + 1):
         x = _rand(rng, dtype, n)
@@ -330,22 +331,28 @@ def test_sorts_by_splitters(rk, orc, dtype, kind):
             assert np.array_equal(rk.Array(rk.sortperm(rk.ROCArray(x), rev=rev)), orc.sortperm(x, rev)), (n, rev)
 
 
+def _sampled(n, s):
+    """Where a sort of n keys takes its s samples; the constants are those of the source, so that a change there shows here."""
+    import pathlib
+    text = (pathlib.Path(__file__).parent.parent / "amdgpu.jl_amd" / "csrc" / "rk_sort_buckets.hpp").read_text()
+    for line in ("constexpr uint32_t SB_OVER = 16;", "uint32_t h = (j + 1u) * 0x9e3779b1u;", "h ^= h >> 15;", "h *= 0x85ebca77u;", "return a + __umulhi(h, b - a);"):
+        assert line in text, line
+    j, m = np.arange(s, dtype=np.uint64), np.uint64(0xffffffff)
+    a, b = j * np.uint64(n) // np.uint64(s), (j + np.uint64(1)) * np.uint64(n) // np.uint64(s)
+    h = (j + np.uint64(1)) * np.uint64(0x9e3779b1) & m
+    h ^= h >> np.uint64(15)
+    h = h * np.uint64(0x85ebca77) & m
+    return (a + (h * (b - a) >> np.uint64(32))).astype(np.int64)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int32, np.int64])
 @pytest.mark.parametrize("few", [False, True])
 def test_bucket_larger_than_lds(rk, orc, dtype, few):
     """Every key that is sampled is larger than all the others, so these are one bucket: more keys than LDS holds."""
-    n, k = 30_000, 64
-    s = 16 * k
-    pos = []
-    for j in range(s):
-        a, b = j * n // s, (j + 1) * n // s
-        h = (j + 1) * 0x9e3779b1 & 0xffffffff
-        h ^= h >> 15
-        h = h * 0x85ebca77 & 0xffffffff
-        pos.append(a + (h * (b - a) >> 32))
+    n, s = 30_000, 16 * 64
     rng = np.random.default_rng(5)
     x = rng.integers(0, 7 if few else 1 << 20, n).astype(dtype)
-    x[pos] = (1 << 24) + rng.integers(0, 1 << 20, s)
+    x[_sampled(n, s)] = (1 << 24) + rng.integers(0, 1 << 20, s)
     _check(rk, orc, x)
 
 
@@ -360,9 +367,10 @@ def test_sorts_by_two_levels_of_splitters(rk, orc, dtype, kind):
         assert np.array_equal(rk.Array(rk.sortperm(rk.ROCArray(x), rev=rev)), orc.sortperm(x, rev)), (n, rev)
 
 
-@pytest.mark.parametrize("digits", [(), (2,), (0, 7), (1, 3, 6), (0, 2, 3, 5), (0, 1, 2, 3, 4, 5, 6, 7)])
+@pytest.mark.parametrize("digits", [(), (2,), (3, 4), (2, 3, 4), (0, 7), (1, 3, 6), (0, 2, 3, 5), (0, 1, 2, 3, 4, 5, 6, 7)])
 def test_large_int64_by_varying_digits(rk, orc, digits):
-    """Keys that differ in three digits at most take radix passes, others splitters; sort! in place and into another array."""
+    """Keys take radix passes if there are three digits at most from the lowest that varies to the top of their range, others
+    splitters; sort! in place and into another array."""
     rng = np.random.default_rng(33)
     n = (1 << 20) + 4097
     x = np.full(n, 1 << 40, dtype=np.int64)
@@ -372,6 +380,42 @@ def test_large_int64_by_varying_digits(rk, orc, digits):
     y = rk.ROCArray(x)
     rk.sort_(y)
     assert np.array_equal(rk.Array(y), orc.sort(x, False))
+    for perm in (False, True):
+        planned, got = _passes_run(rk, x, perm)
+        assert np.array_equal(got, orc.sortperm(x) if perm else orc.sort(x))
+        assert planned == (max(digits) - min(digits) + 1 if digits else 0)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.int64])
+@pytest.mark.parametrize("n", [(1 << 23) - 1, 1 << 23, (1 << 24) + 1, 1 << 26])
+def test_long_sorts_by_two_levels_of_splitters(rk, dtype, n):
+    """From 2^23 keys on an XCD takes neighbouring buckets; 2^26 keys are the most that are sorted this way.  Against torch's sort."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    x = torch.randn(n, device="cuda", generator=g, dtype=torch.float64) if dtype == np.float64 else \
+        torch.randint(-2**62, 2**62, (n,), device="cuda", generator=g, dtype=torch.int64)
+    xd = rk.ROCArray(buf=x.view(torch.uint8), dims=(n,), dtype=dtype)
+    want = torch.sort(x, stable=True)
+    assert torch.equal(rk.sort(xd).buf[:8 * n].view(x.dtype), want.values)
+    assert torch.equal(rk.sortperm(xd).buf[:8 * n].view(torch.int64) - 1, want.indices)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.int64])
+def test_part_whose_keys_lie_far_apart(rk, dtype):
+    """The smallest keys stand in the first and the last six tiles of 2048: a tile of their part collects runs on both sides of
+    more empty ones than LDS holds at a time."""
+    import torch
+    rng = np.random.default_rng(34)
+    n, tile = 1 << 24, 8192
+    x = (1 << 50) + rng.integers(0, 1 << 40, n)
+    for part in (slice(0, 6 * tile), slice(n - 6 * tile, n)):
+        x[part] = rng.integers(0, 1 << 40, 6 * tile)
+    x = torch.from_numpy(x.astype(dtype)).cuda()
+    xd = rk.ROCArray(buf=x.view(torch.uint8), dims=(n,), dtype=dtype)
+    want = torch.sort(x, stable=True)
+    assert torch.equal(rk.sort(xd).buf[:8 * n].view(x.dtype), want.values)
+    assert torch.equal(rk.sortperm(xd).buf[:8 * n].view(torch.int64) - 1, want.indices)
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64, np.int64])
@@ -380,16 +424,9 @@ def test_part_and_buckets_larger_than_lds(rk, orc, dtype, few):
     """Every key that is sampled first is larger than all the others: these are one part of more tiles than a bucket's workgroup
     holds the runs of, and its 256 buckets are larger than LDS."""
     n, s = (1 << 20) + 300_000, 4096
-    j = np.arange(s, dtype=np.uint64)
-    a, b = j * n // s, (j + 1) * n // s
-    m = np.uint64(0xffffffff)
-    h = (j + 1) * np.uint64(0x9e3779b1) & m
-    h ^= h >> np.uint64(15)
-    h = h * np.uint64(0x85ebca77) & m
-    pos = (a + (h * (b - a) >> np.uint64(32))).astype(np.int64)
     rng = np.random.default_rng(6)
     x = (rng.integers(0, 7, n) if few else rng.integers(0, 1 << 20, n)).astype(dtype)
     if dtype == np.int64:
         x += rng.integers(0, 7, n) << 40                     # (four digits and more)
-    x[pos] = (1 << 50) + rng.integers(0, 1 << 20, s)
+    x[_sampled(n, s)] = (1 << 50) + rng.integers(0, 1 << 20, s)
     _check(rk, orc, x)
