@@ -6,7 +6,7 @@
 //   up to 2^20           keys of 4 and 8 bytes go through splitters into buckets that are sorted in LDS (rk_sort_buckets.hpp):
 //                        such sorts are bound by the latency of their kernels, and these are four or five whatever the width.
 //   up to 2^26           keys of 8 bytes, and Float32 up to 2^22, go through two levels of splitters (rk_sort_split.hpp), unless they are
-//                        integers that differ in three digits at most.
+//                        integers with three digits at most from the lowest that varies to the top of their range.
 //   the others           the radix passes of this file:
 //   sort_init_kernel     clears the control block; no memset: graph-safe
 //   sort_range_kernel    one read of the keys: smallest and largest key (integers) and the bits that differ between keys;
@@ -19,8 +19,8 @@
 //                        (58 a key, 32 of them the match), not by memory.
 //
 // How a tile learns where its digits go:
-//   up to 256 tiles (2^20 keys)  every workgroup of the pass sums the columns of the table of counts itself (256 rows of
-//                        512 bytes out of L2, one or two rounds of loads): nothing waits for anything.  A tile or less per
+//   up to 256 tiles (2^20 keys of 2 bytes)  every workgroup of the pass sums the columns of the table of counts itself (256 rows
+//                        of 512 bytes out of L2, one or two rounds of loads): nothing waits for anything.  A tile or less per
 //                        compute unit: it is 16 waves with 4 keys a lane, not 4 waves with 16.
 //   beyond               sort_tilescan_kernel: exclusive scan of the counts down the tiles in one launch (chunks of tiles; the
 //                        workgroup that finishes last scans the chunk totals and the digit totals); the pass kernel gives
@@ -212,7 +212,7 @@ __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool re
 }
 
 // What the plan says about one pass.  All words are asked for together: read where they are used, each waits for the branch
-// that the one before decides, round trips to memory in front of the keys (sortperm(Int64[1000003]) 138.6 against 136.6 us).
+// that the one before decides, round trips to memory in front of the keys (eight passes over 10^6 keys 138.6 against 136.6 us).
 struct SortStep {
     uint32_t skip, src_b, first_pass, last_pass;
     unsigned long long inv_min;
@@ -223,7 +223,7 @@ __device__ __forceinline__ SortStep sort_step(const SortCtl* ctl, int pass) {
     return s;
 }
 
-// Sorts of 8-byte integers that take another way unless the keys differ in few digits (rk_sort_split.hpp) launch so many passes;
+// Sorts of 8-byte integers that take another way unless the plan has few passes (rk_sort_split.hpp) launch so many;
 // `pass` is then -1, -2, ... for the first of the digits that vary, the second ...  Returns the digit, -1: there is none to do.
 // Three: 2^24 keys in three digits, sortperm Int64 432 us so and 522 by splitters, sort 400 and 382; in four, 547 and 502, 427 and 381.
 constexpr uint32_t SORT_FEW_PASSES = 3;
@@ -802,9 +802,9 @@ namespace rk {
 constexpr int64_t SORT_TILE = 4096;
 constexpr int SORT_ITEMS = (int)SORT_TILE / SORT_BLOCK;
 constexpr int DIRECT_BLOCK = 1024, DIRECT_ITEMS = (int)SORT_TILE / DIRECT_BLOCK;
-// Up to here a pass sums the columns of the table of counts itself.  Every tile reads the counts of all tiles, so that traffic
-// grows with their square: sort!(Float32), summed here / by the tile scan, 0.75 x 2^20 keys 61.4 / 102 us, 2^20 64.6 / 112, 1.5 x
-// 2^20 98 / 117, 2^21 112 / 131, 2^22 267 / 136.  256 tiles are a workgroup a compute unit.
+// Up to here a pass (over 2-byte keys) sums the columns of the table of counts itself.  Every tile reads the counts of all tiles, so that
+// traffic grows with their square: four passes over Float32 keys, which no longer come here, summed here / by the tile scan, 0.75 x 2^20
+// keys 61.4 / 102 us, 2^20 64.6 / 112, 1.5 x 2^20 98 / 117, 2^21 112 / 131, 2^22 267 / 136.  256 tiles are a workgroup a compute unit.
 constexpr uint32_t DIRECT_TILES = 256;
 
 struct SortLayout {

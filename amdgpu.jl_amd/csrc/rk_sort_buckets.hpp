@@ -9,8 +9,8 @@
 // A radix pass over 10^6 keys is bound by latency, and 8-byte keys take eight of them, one after the other; the four kernels
 // here are as many as two passes take and do not get more with the width of the key.  No key is moved to its bucket: a bucket
 // takes its runs out of the tiles, so nothing has to know the buckets' sizes before it writes.
-// Radix passes -> so, us a call: sortperm Int64[1000003] 136.3 -> 44.4 (kernels 3.5, 6.2, 16.2 and 20.9), Float32 66.0 -> 39.7;
-// sort Float32[1000003] 63.9 -> 33.8, Float64 132 -> 38, Int64 of 20 bits 79.7 -> 38.4; sort Float32[150000] 48.6 -> 26.0.  Each of
+// Radix passes -> so, us a call: sortperm Int64[1000003] 136.3 -> 42.3 (kernels 2.9, 5.7, 15.9 and 19.1), Float32 66.0 -> 39;
+// sort Float32[1000003] 63.9 -> 33.8, Float64 132 -> 38, Int64 of 20 bits 79.7 -> 38; sort Float32[150000] 48.6 -> 26.0.  Each of
 // the kernels moves what it moves in a fraction of its time: what is left is their chains of dependent loads and barriers.
 //
 // Order: keys are compared together with their index -- (key, index) is a strict order -- so equal keys are split between
@@ -19,8 +19,9 @@
 //
 // Bucket sizes: a bucket holds the keys between two neighbours among k sampled quantiles, SB_OVER samples apart, so its size
 // is spread like a Gamma variable of that shape around n / k.  LDS has room for SB_CAP keys, 2.75 times n / k at 2^20 keys
-// and more below; one bucket in 2 million is larger (at 2^20 keys; the fewer the keys, the fewer) and is sorted in memory,
-// slowly.  Nothing but the time depends on a bucket's being small.
+// and more below; one bucket in 2 million is larger (at 2^20 keys; the fewer the keys, the fewer) and is sorted in memory: such
+// a call takes 0.4 to 1 ms.  Where samples are taken depends on the number of keys alone, so for an input it always happens or
+// never does.  Nothing but the time depends on a bucket's being small.
 #pragma once
 
 #include "rk_common.hpp"

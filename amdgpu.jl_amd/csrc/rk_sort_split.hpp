@@ -14,16 +14,18 @@
 // ballots.  Nothing is scattered over memory: a tile is written where it was read, and the next kernel collects its runs.
 //
 // Radix passes -> so, us a call: sort Float64[2^21] 248 -> 75, [2^24] 718 -> 315, [2^26] 3093 -> 1162; sort Int64 of 64 bits 262 -> 110,
-// 760 -> 357; sortperm Int64 288 -> 120, 1026 -> 484; sort Float32[1500000] 113 -> 58, [2^22] 136 -> 95, few values many times over
-// 140 -> 140.  For Float32 beyond, such input is faster in four radix passes (2^24 keys of two values 241 against 345; of 2^26 normal ones 764
-// against 984); so is Int32 at once, which needs a read for the digits that vary, and launches for the passes that then do not
-// run (2^21 keys of 20 bits).
-// The kernels of sort Float64[2^24]: 64 first, 5 runs, 21 parts, 91 second, 128 last; 256 MiB read and written are 41.  They are bound by
-// vector instructions (sort Float32[2^26], a key: 60 first, 84 second, 213 last; 110, 150 and 380 us at one a cycle).
+// 760 -> 357; sortperm Int64 288 -> 120, 1026 -> 484; sort Float32[1500000] 113 -> 58, [2^22] 136 -> 92, two values 135 -> 128, 256 values
+// 136 -> 109; sortperm Float32[2^22] 148 -> 106, two values 143 -> 145, 256 values 145 -> 130.  For Float32 beyond, radix passes are faster (2^24
+// keys of two values 241 against 345, of 2^26 normal ones 764 against 984, both before large bins were divided more than once); so is Int32 at
+// once, which needs a read for the digits that vary, and launches for the passes that then do not run (2^21 keys of 20 bits).
+// The kernels of sort Float64[2^24]: 61 first, 5 runs, 23 parts, 82 second, 129 last; 256 MiB read and written are 41.  They are bound by
+// vector instructions (sort Float32[2^22], a key: 58 first, 85 second, 204 last).
 //
 // Order, and the sizes of buckets: as in rk_sort_buckets.hpp, (key, index) is a strict order.  Within a part the index is a key's place in
 // the part (sort) or its index in the array (sortperm).  A part gets as many buckets as its size asks for, with LS_OVER samples a
-// bucket, so one bucket in 10^9 does not fit LDS; it is sorted in memory, slowly.
+// bucket, so up to 2^25 keys one bucket in 10^11 does not fit LDS and is sorted in memory, as in rk_sort_buckets.hpp.  LS_BUCKETS are the
+// most that a part gets: at 2^26 keys 3 % of the parts are larger than that is meant for, and one bucket in 10^7 does not fit, in one
+// sort of 250.
 #pragma once
 
 #include "rk_sort_buckets.hpp"
