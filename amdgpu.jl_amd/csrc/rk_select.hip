@@ -619,7 +619,7 @@ __global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* _
 #pragma unroll
     for (int k = 0; k < MSK_LOADS; ++k) {
         const int64_t i = e0 + k * SEL_CHUNK + lane * 16;
-        bytes[k] = i + 16 <= n ? (mask_vec)load_nt((const mask_vec_at4*)(mask + i)) : mask_load16(mask, i, n, 0);
+        bytes[k] = i + 16 <= n ? (mask_vec)__builtin_nontemporal_load((const mask_vec_at4*)(mask + i)) : mask_load16(mask, i, n, 0);
     }
     int64_t base = group_prefix[tile >> group_shift] + (int64_t)tile_prefix[tile];
 #pragma unroll
