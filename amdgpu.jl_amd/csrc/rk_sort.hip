@@ -1,12 +1,14 @@
 // sort! / sortperm! of vectors (src/kernels/sorting.jl:1-3, which forwards to AcceleratedKernels' merge sort):
 // least-significant-digit radix sort, 8 bits per pass.
 //
-// Four ways by the number of keys:
+// Five ways by the number of keys:
 //   up to 4096           one workgroup does all of it in LDS (sort_tiny_kernel, rk_sort_buckets.hpp).
 //   up to 2^20           keys of 4 and 8 bytes go through splitters into buckets that are sorted in LDS (rk_sort_buckets.hpp):
 //                        such sorts are bound by the latency of their kernels, and these are four or five whatever the width.
 //   up to 2^26           keys of 8 bytes, and Float32 up to 2^22, go through two levels of splitters (rk_sort_split.hpp), unless they are
 //                        integers with three digits at most from the lowest that varies to the top of their range.
+//   up to 2^26           sort of more Float32, and of more than 2^23 Int32, moves the keys into buckets once (rk_sort_quantiles.hpp), unless a bucket
+//                        gets too large for that, or integers differ in one digit.
 //   the others           the radix passes of this file:
 //   sort_init_kernel     clears the control block; no memset: graph-safe
 //   sort_range_kernel    one read of the keys: smallest and largest key (integers) and the bits that differ between keys;
@@ -26,7 +28,7 @@
 //                        workgroup that finishes last scans the chunk totals and the digit totals); the pass kernel gives
 //                        each XCD a contiguous eighth of the tiles.
 // Large sorts of floats run every pass (their digits are hardly ever constant) and do without the range read.
-//   sort_finish_kernel   moves the result of sort! into the caller's array when an odd number of passes ran
+//   sort_finish_kernel   moves the result of sort! into the caller's array when an odd number of passes ran, and a copy of the keys when none did
 //
 // Keys are mapped to unsigned integers that sort like Base.isless (-0.0 < 0.0, NaN last; sortperm makes every NaN the
 // canonical one so that they are equal keys, sort! keeps their bit patterns), complemented for rev=true; the mapping is
@@ -192,12 +194,20 @@ __device__ __forceinline__ bool digits_skewed(uint32_t d, bool valid) {
 // so are low digits in which the keys do not differ.
 // Otherwise (floats) a digit in which no two keys differ is skipped: their exponent bytes are constant or not whatever is
 // subtracted.
+// first: what the first pass says of its source, SORT_A or SORT_B (it reads the caller's keys either way, and writes the other one);
+// SORT_ENDS_IN_A: whichever lets the last pass write buffer A.
+constexpr int SORT_A = 0, SORT_B = 1, SORT_ENDS_IN_A = 2;
 __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool relative, unsigned long long range, unsigned long long varying,
-                                               int first_reads_b) {
-    uint32_t src_b = first_reads_b ? 1u : 0u, nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
-    for (int p = 0; p < passes; ++p) {
+                                               int first_source) {
+    const auto skipped = [&](int p) {
         const unsigned long long upto = p == 7 ? ~0ull : (1ull << (8 * (p + 1))) - 1ull;
-        const bool skip = relative ? (range >> (8 * p)) == 0ull || (varying & upto) == 0ull : ((varying >> (8 * p)) & 0xffull) == 0ull;
+        return relative ? (range >> (8 * p)) == 0ull || (varying & upto) == 0ull : ((varying >> (8 * p)) & 0xffull) == 0ull;
+    };
+    uint32_t src_b = first_source == SORT_B ? 1u : 0u, nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
+    if (first_source == SORT_ENDS_IN_A)
+        for (int p = 0; p < passes; ++p) src_b ^= skipped(p) ? 0u : 1u;
+    for (int p = 0; p < passes; ++p) {
+        const bool skip = skipped(p);
         ctl->skip[p] = skip ? 1u : 0u;
         if (skip) continue;
         ctl->src_is_b[p] = src_b;
@@ -238,13 +248,13 @@ __device__ __forceinline__ int sort_pass_index(const SortCtl* ctl, int pass) {
 // ---- init: clear the control block ----------------------------------------------------------------------------------
 // all_passes: large sorts of floats, which run every pass on keys that are not taken relative to the smallest one; their
 // plan is made here.
-__global__ __launch_bounds__(256) void sort_init_kernel(SortCtl* ctl, int all_passes, int first_reads_b) {
+__global__ __launch_bounds__(256) void sort_init_kernel(SortCtl* ctl, int all_passes, int first_source) {
     for (int i = threadIdx.x; i < SORT_CTL_CLEAR; i += 256) ctl->skip[i] = 0u;
     if (all_passes == 0) return;
     __syncthreads();
     if (threadIdx.x == 0) {
         ctl->inv_min = ~0ull;
-        sort_make_plan(ctl, all_passes, false, 0ull, ~0ull, first_reads_b);
+        sort_make_plan(ctl, all_passes, false, 0ull, ~0ull, first_source);
     }
 }
 
@@ -295,7 +305,7 @@ __device__ __forceinline__ void for_each_key(const T* __restrict__ keys, int64_t
 constexpr int RANGE_BLOCK = 1024;       // few, large workgroups: each ends with device-wide atomics on shared words
 template <typename T>
 __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __restrict__ keys, int64_t n, int64_t head, int64_t nvec, int rev,
-                                                                 int first_reads_b, SortCtl* ctl) {
+                                                                 int first_source, SortCtl* ctl) {
     typedef typename SortKey<T>::U U;
     typedef unsigned long long W;
     constexpr int VEC = 16 / sizeof(T);
@@ -336,7 +346,7 @@ __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __rest
     if (__builtin_amdgcn_readfirstlane(finishes_last) == 0) return;
     const U smallest = (U)~(U)load_agent(&ctl->inv_min);
     if (threadIdx.x == 0)
-        sort_make_plan(ctl, (int)sizeof(T), RELATIVE, RELATIVE ? load_agent(&ctl->key_max) - (W)smallest : 0ull, load_agent(&ctl->varying), first_reads_b);
+        sort_make_plan(ctl, (int)sizeof(T), RELATIVE, RELATIVE ? load_agent(&ctl->key_max) - (W)smallest : 0ull, load_agent(&ctl->varying), first_source);
 }
 
 // ---- digit counts of every tile -----------------------------------------------------------------------------------
@@ -362,72 +372,75 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
     const U* in = first ? (const U*)orig : (step.src_b != 0u ? buf_b : buf_a);
     const U umin = (U)~step.inv_min;
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-    for (int i = tid; i < NW * SUB * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
-    const uint32_t tile = blockIdx.x;
-    const uint32_t e0 = tile * (uint32_t)TILE;
-    const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
-    uint32_t* row = cnt[wave * SUB + (lane & (SUB - 1))];
-    // When many lanes hold the same digit (judged on every fourth key) the two most frequent values -- as seen from the
-    // first lane still in play -- are taken out with a ballot each and added by that lane alone; uniform floats have
-    // 50% and 37% of their keys in two values of the exponent digit.
-    bool skewed = false;
-    auto count = [&](uint32_t d, bool valid, int i) {
-        if ((i & 3) == 0) skewed = digits_skewed(d, valid);
-        if (skewed) {
+    for (uint32_t tile = blockIdx.x; tile * (uint32_t)TILE < n; tile += gridDim.x) {
+        if (tile != blockIdx.x) __syncthreads();
+        for (int i = tid; i < NW * SUB * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
+        const uint32_t e0 = tile * (uint32_t)TILE;
+        const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
+        uint32_t* row = cnt[wave * SUB + (lane & (SUB - 1))];
+        // When many lanes hold the same digit (judged on every fourth key) the two most frequent values -- as seen from the
+        // first lane still in play -- are taken out with a ballot each and added by that lane alone; uniform floats have
+        // 50% and 37% of their keys in two values of the exponent digit.
+        bool skewed = false;
+        auto count = [&](uint32_t d, bool valid, int i) {
+            if ((i & 3) == 0) skewed = digits_skewed(d, valid);
+            if (skewed) {
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const uint64_t active = __ballot(valid);
-                if (active != 0ull) {
-                    const int head = __ffsll((unsigned long long)active) - 1;
-                    const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, head);
-                    const uint64_t same = __ballot(valid && d == d0);
-                    if (lane == head) atomicAdd(&row[d0], (uint32_t)__popcll(same));
-                    valid = valid && d != d0;
+                for (int r = 0; r < 2; ++r) {
+                    const uint64_t active = __ballot(valid);
+                    if (active != 0ull) {
+                        const int head = __ffsll((unsigned long long)active) - 1;
+                        const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)d, head);
+                        const uint64_t same = __ballot(valid && d == d0);
+                        if (lane == head) atomicAdd(&row[d0], (uint32_t)__popcll(same));
+                        valid = valid && d != d0;
+                    }
                 }
             }
-        }
-        if (valid) atomicAdd(&row[d], 1u);
-    };
-    // (the two read paths share no variables: merged into one key array they made the compiler shuffle it through
-    // private memory)
-    bool vectors = false;
-    if constexpr (NV > 0) vectors = e0 + (uint32_t)TILE <= n && (((uintptr_t)(in + e0)) & 15) == 0;
-    if (vectors) {
-        const VU* vin = (const VU*)(in + e0);
-        VU v[NV > 0 ? NV : 1];
+            if (valid) atomicAdd(&row[d], 1u);
+        };
+        // (the two read paths share no variables: merged into one key array they made the compiler shuffle it through
+        // private memory)
+        bool vectors = false;
+        if constexpr (NV > 0) vectors = e0 + (uint32_t)TILE <= n && (((uintptr_t)(in + e0)) & 15) == 0;
+        if (vectors) {
+            const VU* vin = (const VU*)(in + e0);
+            VU v[NV > 0 ? NV : 1];
 #pragma unroll
-        for (int r = 0; r < NV; ++r) v[r] = vin[r * BLOCK + tid];
-        __syncthreads();
+            for (int r = 0; r < NV; ++r) v[r] = vin[r * BLOCK + tid];
+            __syncthreads();
 #pragma unroll
-        for (int r = 0; r < NV; ++r) {
+            for (int r = 0; r < NV; ++r) {
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                U k = (U)v[r][j];
-                if (first) k = enc_bits<T>(k, rev, umin);
-                count(digit_of(k, pass), true, r * VEC + j);
+                for (int j = 0; j < VEC; ++j) {
+                    U k = (U)v[r][j];
+                    if (first) k = enc_bits<T>(k, rev, umin);
+                    count(digit_of(k, pass), true, r * VEC + j);
+                }
+            }
+        } else {
+            U key[ITEMS];
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                const uint32_t e = woff + i * WAVE;
+                key[i] = (U)0;
+                if (e < n) key[i] = in[e];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i) {
+                const U k = first ? enc_bits<T>(key[i], rev, umin) : key[i];
+                count(digit_of(k, pass), woff + i * WAVE < n, i);
             }
         }
-    } else {
-        U key[ITEMS];
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t e = woff + i * WAVE;
-            key[i] = (U)0;
-            if (e < n) key[i] = in[e];
-        }
         __syncthreads();
+        if (BLOCK == 256 || tid < 256) {
+            uint32_t c = 0;
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const U k = first ? enc_bits<T>(key[i], rev, umin) : key[i];
-            count(digit_of(k, pass), woff + i * WAVE < n, i);
+            for (int w = 0; w < NW * SUB; ++w) c += cnt[w][tid];
+            tile_count[(uint64_t)tile * 256 + tid] = (C)c;
         }
     }
-    __syncthreads();
-    if (BLOCK > 256 && tid >= 256) return;
-    uint32_t c = 0;
-#pragma unroll
-    for (int w = 0; w < NW * SUB; ++w) c += cnt[w][tid];
-    tile_count[(uint64_t)tile * 256 + tid] = (C)c;
 }
 
 // ---- where every tile's keys go (large sorts) --------------------------------------------------------------------------
@@ -551,7 +564,8 @@ __global__ __launch_bounds__(TS_BLOCK) void sort_tilescan_kernel(SortCtl* ctl, i
 // waves hide the latencies (measured: 4 against 6 workgroups a CU differ by 4%)
 template <typename T, bool PERM, bool DIRECT> constexpr int sort_pass_waves() { return (DIRECT || (!PERM && sizeof(T) <= 4)) ? 4 : 3; }
 
-template <typename T, int BLOCK, int ITEMS, bool PERM, bool DIRECT>
+// SEVERAL: tiles a workgroup, in turn (as a loop, every pass takes 4 % longer).
+template <typename T, int BLOCK, int ITEMS, bool PERM, bool DIRECT, bool SEVERAL = false>
 __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void sort_pass_kernel(const T* __restrict__ orig, typename SortKey<T>::U* buf_a,
                                                                typename SortKey<T>::U* buf_b, uint32_t* val_a, uint32_t* val_b,
                                                                int64_t* __restrict__ perm_out, uint32_t n, int pass, int rev, SortCtl* ctl,
@@ -586,205 +600,208 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
     U* dst = src_b ? buf_a : buf_b;
     const uint32_t* vsrc = src_b ? val_b : val_a;
     uint32_t* vdst = src_b ? val_a : val_b;
-    for (int i = tid; i < NW * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
-    __syncthreads();
-    uint32_t tile = blockIdx.x;
-    if (!DIRECT && xcd_chunk != 0u) {
-        const uint32_t i = blockIdx.x >> 3;
-        tile = i < xcd_chunk ? (blockIdx.x & 7u) * xcd_chunk + i : ntiles;
-    }
-    if (tile >= ntiles) return;
-    const uint32_t e0 = tile * (uint32_t)TILE;
-    const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
+    for (uint32_t at = blockIdx.x;;) {
+        for (int i = tid; i < NW * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
+        __syncthreads();
+        const uint32_t tile = !DIRECT && xcd_chunk != 0u ? (at & 7u) * xcd_chunk + (at >> 3) : at;
+        if (tile < ntiles) {
+            const uint32_t e0 = tile * (uint32_t)TILE;
+            const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
 
-    // Every tile but the last is full: its code carries no bounds checks (they cost an exec-mask save and a
-    // branch per key and round).
-    auto sort_tile = [&](auto full_tile) {
-        constexpr bool FULL = decltype(full_tile)::value;
-        // load (and map on the first pass)
-        U key[ITEMS];
-        uint32_t val[PERM ? ITEMS : 1];
-        uint32_t rank[ITEMS];
+            // Every tile but the last is full: its code carries no bounds checks (they cost an exec-mask save and a
+            // branch per key and round).
+            auto sort_tile = [&](auto full_tile) {
+                constexpr bool FULL = decltype(full_tile)::value;
+                // load (and map on the first pass)
+                U key[ITEMS];
+                uint32_t val[PERM ? ITEMS : 1];
+                uint32_t rank[ITEMS];
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t e = woff + i * WAVE;
-            key[i] = (U)~(U)0;
-            if (FULL || e < n) key[i] = in[e];
-        }
-        if constexpr (PERM) {
+                for (int i = 0; i < ITEMS; ++i) {
+                    const uint32_t e = woff + i * WAVE;
+                    key[i] = (U)~(U)0;
+                    if (FULL || e < n) key[i] = in[e];
+                }
+                if constexpr (PERM) {
 #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) val[i] = woff + i * WAVE;              // first pass: the key's own index
-            if (!first) {
+                    for (int i = 0; i < ITEMS; ++i) val[i] = woff + i * WAVE;              // first pass: the key's own index
+                    if (!first) {
 #pragma unroll
-                for (int i = 0; i < ITEMS; ++i)
-                    if (FULL || woff + i * WAVE < n) val[i] = vsrc[woff + i * WAVE];
-            }
-        }
-        if constexpr (DIRECT) {
-            // columns of the table of counts: all rows, and the rows of the tiles in front.  At most 256 rows, 16 in flight.
-            const uint32_t c = (uint32_t)tid & 127u, g = (uint32_t)tid >> 7;
-            const uint32_t* col = (const uint32_t*)counts + c;
-            uint2 bef = {0u, 0u}, sum = {0u, 0u};
-            constexpr uint32_t UNR = 16;
-            for (uint32_t r0 = g; r0 < ntiles; r0 += GROUPS * UNR) {
-                uint32_t w[UNR];
+                        for (int i = 0; i < ITEMS; ++i)
+                            if (FULL || woff + i * WAVE < n) val[i] = vsrc[woff + i * WAVE];
+                    }
+                }
+                if constexpr (DIRECT) {
+                    // columns of the table of counts: all rows, and the rows of the tiles in front.  At most 256 rows, 16 in flight.
+                    const uint32_t c = (uint32_t)tid & 127u, g = (uint32_t)tid >> 7;
+                    const uint32_t* col = (const uint32_t*)counts + c;
+                    uint2 bef = {0u, 0u}, sum = {0u, 0u};
+                    constexpr uint32_t UNR = 16;
+                    for (uint32_t r0 = g; r0 < ntiles; r0 += GROUPS * UNR) {
+                        uint32_t w[UNR];
 #pragma unroll
-                for (uint32_t u = 0; u < UNR; ++u) {
-                    const uint32_t r = r0 + u * GROUPS;
-                    w[u] = col[(uint64_t)(r < ntiles ? r : ntiles - 1u) * 128];
+                        for (uint32_t u = 0; u < UNR; ++u) {
+                            const uint32_t r = r0 + u * GROUPS;
+                            w[u] = col[(uint64_t)(r < ntiles ? r : ntiles - 1u) * 128];
+                        }
+#pragma unroll
+                        for (uint32_t u = 0; u < UNR; ++u) {
+                            const uint32_t r = r0 + u * GROUPS;
+                            const uint32_t lo = r < ntiles ? w[u] & 0xffffu : 0u, hi = r < ntiles ? w[u] >> 16 : 0u;
+                            sum.x += lo;
+                            sum.y += hi;
+                            bef.x += r < tile ? lo : 0u;
+                            bef.y += r < tile ? hi : 0u;
+                        }
+                    }
+                    part_before[g][c] = bef;
+                    part_all[g][c] = sum;
+                }
+                if (first) {
+#pragma unroll
+                    for (int i = 0; i < ITEMS; ++i) key[i] = enc_bits<T>(key[i], rev, umin);    // padding keys are never counted
+                }
+                // rank inside the wave: lanes with the same digit find each other with 8 ballots; every lane reads the
+                // wave's counter of its digit -- the rank of the group's first key -- and then the lowest lane of the group
+                // adds the size of the group to it.  LDS executes the instructions of one wave in order, so the read of
+                // the next round sees this add, and the 16 rounds queue up back to back; a result is used two rounds later.
+                uint32_t* wcnt = cnt[wave];
+                constexpr int DEPTH = 2;                       // counter reads in flight before their result is used
+                uint32_t pend_before[DEPTH], pend_below[DEPTH];
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) {
+                    const bool valid = FULL || woff + i * WAVE < n;
+                    const uint32_t d = digit_of(key[i], pass);
+                    uint32_t same_lo, same_hi;
+                    match_digit_halves(d, same_lo, same_hi);
+                    if (!FULL) {
+                        const uint64_t vm = __ballot(valid);
+                        same_lo &= (uint32_t)vm;
+                        same_hi &= (uint32_t)(vm >> 32);
+                    }
+                    const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
+                    const uint32_t before = __hip_atomic_load(&wcnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                    __builtin_amdgcn_wave_barrier();
+                    if (valid && below == 0u) {
+                        const uint32_t total = (uint32_t)__builtin_popcount(same_lo) + (uint32_t)__builtin_popcount(same_hi);
+                        __hip_atomic_fetch_add(&wcnt[d], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                    }
+                    if (i >= DEPTH) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
+                    pend_before[i % DEPTH] = before;
+                    pend_below[i % DEPTH] = below;
+                    __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (uint32_t u = 0; u < UNR; ++u) {
-                    const uint32_t r = r0 + u * GROUPS;
-                    const uint32_t lo = r < ntiles ? w[u] & 0xffffu : 0u, hi = r < ntiles ? w[u] >> 16 : 0u;
-                    sum.x += lo;
-                    sum.y += hi;
-                    bef.x += r < tile ? lo : 0u;
-                    bef.y += r < tile ? hi : 0u;
+                for (int i = ITEMS; i < ITEMS + DEPTH; ++i) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
+                __syncthreads();
+                // digit d = tid (the first 256 threads): count of the tile and of each wave, first slot inside the sorted tile
+                // (exclusive scan over the digits) and in the whole output
+                uint32_t wave_count[NW];
+                uint32_t count = 0, excl = 0, all = 0, inc = 0, inc_all = 0;
+                const bool has_digit = BLOCK == 256 || tid < 256;
+                if (has_digit) {
+#pragma unroll
+                    for (int w = 0; w < NW; ++w) {
+                        wave_count[w] = cnt[w][tid];
+                        count += wave_count[w];
+                    }
+                    if constexpr (DIRECT) {
+#pragma unroll
+                        for (int g = 0; g < GROUPS; ++g) {
+                            const uint2 b = part_before[g][tid >> 1], a = part_all[g][tid >> 1];
+                            excl += (tid & 1) ? b.y : b.x;
+                            all += (tid & 1) ? a.y : a.x;
+                        }
+                        inc_all = wave_scan_inclusive(all, OpAdd(), 0u);
+                        if (lane == WAVE - 1) wsum[1][wave] = inc_all;
+                    } else {
+                        excl = ((const uint32_t*)counts)[(uint64_t)tile * 256 + tid] + chunk_prefix[(uint64_t)(tile / chunk_rows) * 256 + tid];
+                    }
+                    inc = wave_scan_inclusive(count, OpAdd(), 0u);
+                    if (lane == WAVE - 1) wsum[0][wave] = inc;
                 }
-            }
-            part_before[g][c] = bef;
-            part_all[g][c] = sum;
-        }
-        if (first) {
+                __syncthreads();
+                if (has_digit) {
+                    uint32_t start = inc - count, base = DIRECT ? inc_all - all : ctl->hist[pass][tid];
+                    for (int w = 0; w < wave; ++w) {
+                        start += wsum[0][w];
+                        if (DIRECT) base += wsum[1][w];
+                    }
+                    goff[tid] = base + excl - start;
 #pragma unroll
-            for (int i = 0; i < ITEMS; ++i) key[i] = enc_bits<T>(key[i], rev, umin);    // padding keys are never counted
-        }
-        // rank inside the wave: lanes with the same digit find each other with 8 ballots; every lane reads the
-        // wave's counter of its digit -- the rank of the group's first key -- and then the lowest lane of the group
-        // adds the size of the group to it.  LDS executes the instructions of one wave in order, so the read of
-        // the next round sees this add, and the 16 rounds queue up back to back; a result is used two rounds later.
-        uint32_t* wcnt = cnt[wave];
-        constexpr int DEPTH = 2;                       // counter reads in flight before their result is used
-        uint32_t pend_before[DEPTH], pend_below[DEPTH];
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const bool valid = FULL || woff + i * WAVE < n;
-            const uint32_t d = digit_of(key[i], pass);
-            uint32_t same_lo, same_hi;
-            match_digit_halves(d, same_lo, same_hi);
-            if (!FULL) {
-                const uint64_t vm = __ballot(valid);
-                same_lo &= (uint32_t)vm;
-                same_hi &= (uint32_t)(vm >> 32);
-            }
-            const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
-            const uint32_t before = __hip_atomic_load(&wcnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            __builtin_amdgcn_wave_barrier();
-            if (valid && below == 0u) {
-                const uint32_t total = (uint32_t)__builtin_popcount(same_lo) + (uint32_t)__builtin_popcount(same_hi);
-                __hip_atomic_fetch_add(&wcnt[d], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            }
-            if (i >= DEPTH) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
-            pend_before[i % DEPTH] = before;
-            pend_below[i % DEPTH] = below;
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int i = ITEMS; i < ITEMS + DEPTH; ++i) rank[i - DEPTH] = pend_before[i % DEPTH] + pend_below[i % DEPTH];
-        __syncthreads();
-        // digit d = tid (the first 256 threads): count of the tile and of each wave, first slot inside the sorted tile
-        // (exclusive scan over the digits) and in the whole output
-        uint32_t wave_count[NW];
-        uint32_t count = 0, excl = 0, all = 0, inc = 0, inc_all = 0;
-        const bool has_digit = BLOCK == 256 || tid < 256;
-        if (has_digit) {
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                wave_count[w] = cnt[w][tid];
-                count += wave_count[w];
-            }
-            if constexpr (DIRECT) {
-#pragma unroll
-                for (int g = 0; g < GROUPS; ++g) {
-                    const uint2 b = part_before[g][tid >> 1], a = part_all[g][tid >> 1];
-                    excl += (tid & 1) ? b.y : b.x;
-                    all += (tid & 1) ? a.y : a.x;
+                    for (int w = 0; w < NW; ++w) {
+                        cnt[w][tid] = start;
+                        start += wave_count[w];
+                    }
                 }
-                inc_all = wave_scan_inclusive(all, OpAdd(), 0u);
-                if (lane == WAVE - 1) wsum[1][wave] = inc_all;
-            } else {
-                excl = ((const uint32_t*)counts)[(uint64_t)tile * 256 + tid] + chunk_prefix[(uint64_t)(tile / chunk_rows) * 256 + tid];
-            }
-            inc = wave_scan_inclusive(count, OpAdd(), 0u);
-            if (lane == WAVE - 1) wsum[0][wave] = inc;
+                __syncthreads();
+                // reorder the tile in LDS.  Reads first, writes after, so that the 16 table reads are in flight together.
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) {
+                    uint32_t d = digit_of(key[i], pass);
+                    asm volatile("" : "+v"(d));            // computed again here: 16 LDS addresses kept from the ranking cost a wave of occupancy
+                    rank[i] += wcnt[d];
+                }
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) {
+                    if (FULL || woff + i * WAVE < n) {
+                        lds_keys[rank[i]] = key[i];
+                        if constexpr (PERM) lds_vals[rank[i]] = val[i];
+                    }
+                }
+                __syncthreads();
+                // write runs of equal digits: thread q takes the q-th key of the sorted tile.  Again all reads of a kind
+                // together; `last` is decided once, not per key.
+                const uint32_t valid_n = n - e0 < (uint32_t)TILE ? n - e0 : (uint32_t)TILE;
+                U out_key[ITEMS];
+                uint32_t slot[ITEMS];
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) {
+                    const uint32_t q = (uint32_t)tid + i * BLOCK;
+                    out_key[i] = (U)0;
+                    if (FULL || q < valid_n) out_key[i] = lds_keys[q];
+                }
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i) slot[i] = goff[digit_of(out_key[i], pass)] + (uint32_t)tid + i * BLOCK;
+                auto writable = [&](int i) { return FULL || (uint32_t)tid + i * BLOCK < valid_n; };
+                if constexpr (PERM) {
+                    uint32_t out_val[ITEMS];
+#pragma unroll
+                    for (int i = 0; i < ITEMS; ++i) {
+                        out_val[i] = 0;
+                        if (FULL || (uint32_t)tid + i * BLOCK < valid_n) out_val[i] = lds_vals[(uint32_t)tid + i * BLOCK];
+                    }
+                    if (last) {
+#pragma unroll
+                        for (int i = 0; i < ITEMS; ++i) if (writable(i)) perm_out[slot[i]] = (int64_t)out_val[i] + 1;
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < ITEMS; ++i) if (writable(i)) { dst[slot[i]] = out_key[i]; vdst[slot[i]] = out_val[i]; }
+                    }
+                } else if (last) {
+#pragma unroll
+                    for (int i = 0; i < ITEMS; ++i) if (writable(i)) ((T*)dst)[slot[i]] = dec_bits<T>(out_key[i], rev, umin);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < ITEMS; ++i) if (writable(i)) dst[slot[i]] = out_key[i];
+                }
+            };
+            if (e0 + (uint32_t)TILE <= n) sort_tile(std::true_type{}); else sort_tile(std::false_type{});
         }
+        if (!SEVERAL) break;
+        at += gridDim.x;
+        if (at >= (xcd_chunk != 0u ? xcd_chunk * 8u : ntiles)) break;
         __syncthreads();
-        if (has_digit) {
-            uint32_t start = inc - count, base = DIRECT ? inc_all - all : ctl->hist[pass][tid];
-            for (int w = 0; w < wave; ++w) {
-                start += wsum[0][w];
-                if (DIRECT) base += wsum[1][w];
-            }
-            goff[tid] = base + excl - start;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                cnt[w][tid] = start;
-                start += wave_count[w];
-            }
-        }
-        __syncthreads();
-        // reorder the tile in LDS.  Reads first, writes after, so that the 16 table reads are in flight together.
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            uint32_t d = digit_of(key[i], pass);
-            asm volatile("" : "+v"(d));            // computed again here: 16 LDS addresses kept from the ranking cost a wave of occupancy
-            rank[i] += wcnt[d];
-        }
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            if (FULL || woff + i * WAVE < n) {
-                lds_keys[rank[i]] = key[i];
-                if constexpr (PERM) lds_vals[rank[i]] = val[i];
-            }
-        }
-        __syncthreads();
-        // write runs of equal digits: thread q takes the q-th key of the sorted tile.  Again all reads of a kind
-        // together; `last` is decided once, not per key.
-        const uint32_t valid_n = n - e0 < (uint32_t)TILE ? n - e0 : (uint32_t)TILE;
-        U out_key[ITEMS];
-        uint32_t slot[ITEMS];
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t q = (uint32_t)tid + i * BLOCK;
-            out_key[i] = (U)0;
-            if (FULL || q < valid_n) out_key[i] = lds_keys[q];
-        }
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) slot[i] = goff[digit_of(out_key[i], pass)] + (uint32_t)tid + i * BLOCK;
-        auto writable = [&](int i) { return FULL || (uint32_t)tid + i * BLOCK < valid_n; };
-        if constexpr (PERM) {
-            uint32_t out_val[ITEMS];
-#pragma unroll
-            for (int i = 0; i < ITEMS; ++i) {
-                out_val[i] = 0;
-                if (FULL || (uint32_t)tid + i * BLOCK < valid_n) out_val[i] = lds_vals[(uint32_t)tid + i * BLOCK];
-            }
-            if (last) {
-#pragma unroll
-                for (int i = 0; i < ITEMS; ++i) if (writable(i)) perm_out[slot[i]] = (int64_t)out_val[i] + 1;
-            } else {
-#pragma unroll
-                for (int i = 0; i < ITEMS; ++i) if (writable(i)) { dst[slot[i]] = out_key[i]; vdst[slot[i]] = out_val[i]; }
-            }
-        } else if (last) {
-#pragma unroll
-            for (int i = 0; i < ITEMS; ++i) if (writable(i)) ((T*)dst)[slot[i]] = dec_bits<T>(out_key[i], rev, umin);
-        } else {
-#pragma unroll
-            for (int i = 0; i < ITEMS; ++i) if (writable(i)) dst[slot[i]] = out_key[i];
-        }
-    };
-    if (e0 + (uint32_t)TILE <= n) sort_tile(std::true_type{}); else sort_tile(std::false_type{});
+    }
 }
 
 // ---- finish ------------------------------------------------------------------------------------------------------
-// sort! and sort: after an odd number of passes the result sits in buffer B, after none in the caller's keys.
-// most: passes that may have run; keys that would have taken more were sorted by splitters.
+// sort! and sort: after an odd number of passes the result of sort! sits in buffer B, after none that of both in the caller's keys.
+// most: passes that may have run; keys that would have taken more were sorted in another way.  ends_in_a: the plan was made so.
 template <typename W>
-__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, const W* orig, W* a, const W* b, int64_t nwords, uint32_t most) {
+__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, const W* orig, W* a, const W* b, int64_t nwords, uint32_t most, int ends_in_a) {
     if (ctl->nexec > most) return;
-    const W* from = (ctl->nexec & 1u) != 0u ? b : (ctl->nexec == 0u ? orig : a);
+    const W* from = ctl->nexec == 0u ? orig : (ctl->nexec & 1u) != 0u && !ends_in_a ? b : a;
     if (from == a) return;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords; i += (int64_t)gridDim.x * 256) a[i] = from[i];
 }
@@ -793,6 +810,7 @@ __global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, co
 
 #include "rk_sort_buckets.hpp"
 #include "rk_sort_split.hpp"
+#include "rk_sort_quantiles.hpp"
 
 namespace rk {
 
@@ -811,8 +829,9 @@ struct SortLayout {
     size_t count_off, chunk_total_off, chunk_prefix_off, keys_b_off, keys_a_off, val_a_off, val_b_off, total;
     size_t compact_off, spl_key_off, spl_pos_off, table_off;
     uint32_t ntiles, chunk_rows, nchunks, k;
-    bool tiny, direct, buckets, split;
+    bool tiny, direct, buckets, quantiles, split;
     LsLayout ls;
+    SqLayout sq;
 };
 
 static SortLayout sort_layout(size_t key_size, bool integers, int64_t n, bool perm) {
@@ -822,7 +841,8 @@ static SortLayout sort_layout(size_t key_size, bool integers, int64_t n, bool pe
     l.tiny = n <= ST_MAX;
     l.direct = l.ntiles <= DIRECT_TILES;
     l.buckets = l.direct && !l.tiny && key_size >= 4;
-    l.split = !l.direct && (key_size == 8 ? n <= LS_MAX_KEYS : key_size == 4 && !integers && n <= LS_MAX_FLOATS);
+    l.quantiles = key_size == 4 && !perm && n > (integers ? SQ_MIN_INTEGERS : LS_MAX_FLOATS) && n <= SQ_MAX_KEYS;
+    l.split = !l.direct && !l.quantiles && (key_size == 8 ? n <= LS_MAX_KEYS : key_size == 4 && !integers && n <= LS_MAX_FLOATS);
     const size_t ctl_end = off;
     l.count_off = off;
     if (l.direct) {
@@ -837,6 +857,10 @@ static SortLayout sort_layout(size_t key_size, bool integers, int64_t n, bool pe
     if (l.split) {                                           // in the place of the counts: one of the two ways is taken
         l.ls = ls_layout(ctl_end, key_size, n);
         if (l.ls.total > off) off = l.ls.total;
+    }
+    if (l.quantiles) {                                       // (as above)
+        l.sq = sq_layout(ctl_end, n);
+        if (l.sq.total > off) off = l.sq.total;
     }
     const size_t kbytes = ((size_t)n * key_size + 255) & ~(size_t)255, vbytes = ((size_t)n * 4 + 255) & ~(size_t)255;
     l.keys_b_off = off; off += kbytes;
@@ -860,7 +884,7 @@ static SortLayout sort_layout(size_t key_size, bool integers, int64_t n, bool pe
 // What a temporary needs that serves every sort of up to n keys of a size, floats and integers: a caller may keep the one of its
 // largest sort.  A way's own need grows with the number of keys, but falls where another way, or larger tiles, take over.
 static size_t sort_tmp_need(size_t key_size, int64_t n, bool perm) {
-    const int64_t last[] = {ST_MAX, DIRECT_TILES * SORT_TILE, LS_SMALL_TILES, LS_MAX_FLOATS, LS_MAX_KEYS, n};     // of a way
+    const int64_t last[] = {ST_MAX, DIRECT_TILES * SORT_TILE, LS_SMALL_TILES, LS_MAX_FLOATS, SQ_MIN_INTEGERS, SQ_MAX_KEYS, LS_MAX_KEYS, n};     // of a way
     size_t need = 0;
     for (int64_t m : last)
         for (int integers = 0; integers < 2; ++integers) {
@@ -929,8 +953,10 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
         if (l.split) return sort_split<T, PERM>(l.ls, keys, sorted_out, perm_out, n, rev, base, ctl, buf_a, buf_b, val_a, val_b, stream);
     }
     const bool all_passes = FLOAT_KEYS && !l.direct;
-    const int first_reads_b = PERM ? 1 : 0;          // sortperm: the first pass reads the caller's keys and writes buffer A
-    sort_init_kernel<<<1, 256, 0, stream>>>(ctl, all_passes ? PASSES : 0, first_reads_b);
+    // sortperm: the first pass reads the caller's keys and writes buffer A.  sort: the last one writes the result, whatever their number
+    // (a copy behind an odd number of them 85 us for 2^26 Float32); sort!: the keys lie where the result goes, so the first cannot.
+    const int first_source = PERM ? SORT_B : keys != sorted_out ? SORT_ENDS_IN_A : SORT_A;
+    sort_init_kernel<<<1, 256, 0, stream>>>(ctl, all_passes ? PASSES : 0, first_source);
     RK_LAUNCH_CHECK();
     if (!all_passes) {
         constexpr int KVEC = 16 / (int)sizeof(T);
@@ -941,15 +967,24 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
         int64_t g = (nvec + RANGE_BLOCK * 4 - 1) / (RANGE_BLOCK * 4);
         if (g > cus * 2) g = cus * 2;
         if (g < 1) g = 1;
-        sort_range_kernel<T><<<(unsigned)g, RANGE_BLOCK, 0, stream>>>((const T*)keys, n, head, nvec, rev, first_reads_b, ctl);
+        sort_range_kernel<T><<<(unsigned)g, RANGE_BLOCK, 0, stream>>>((const T*)keys, n, head, nvec, rev, first_source, ctl);
         RK_LAUNCH_CHECK();
+    }
+    if constexpr (sizeof(T) == 4 && !PERM) {
+        if (l.quantiles) {
+            const int32_t rc = sort_quantiles<T>(l.sq, keys, sorted_out, n, rev, base, ctl, first_source, buf_b, stream);
+            if (rc != RK_SUCCESS) return rc;
+        }
     }
     // tunable, read once: XCD-contiguous tiles (RK_SORT_XCD=0: off).  Large sorts launch one workgroup per tile: the
     // hardware's dispatcher balances the load better than a fixed share of tiles per resident workgroup (2^26 Float32:
     // 866 against 986 us with 4 a CU), and each XCD takes a contiguous eighth of the tiles, so the runs that neighbouring
     // tiles write next to each other meet in one L2 (workgroups go to the XCDs round-robin by their index).
     static const int xcd_map = [] { const char* e = std::getenv("RK_SORT_XCD"); return e ? std::atoi(e) : 1; }();
-    const unsigned pgrid = (l.ntiles + 7u) & ~7u;
+    // Behind sort_quantiles, whose buckets nearly always fit, these kernels end at once, and sooner the fewer their workgroups.
+    unsigned pgrid = (l.ntiles + 7u) & ~7u;
+    if (l.quantiles && pgrid > (unsigned)cus * 16u) pgrid = (unsigned)cus * 16u;
+    const unsigned ugrid = pgrid < l.ntiles ? pgrid : l.ntiles;
     const uint32_t xcd_chunk = xcd_map != 0 ? (l.ntiles + 7u) / 8u : 0u;
     if (l.direct) {
         if constexpr (sizeof(T) < 4) {
@@ -967,11 +1002,19 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
         uint32_t* chunk_prefix = (uint32_t*)(base + l.chunk_prefix_off);
         for (int i = 0; i < (l.split ? (int)SORT_FEW_PASSES : PASSES); ++i) {
             const int p = l.split ? -1 - i : i;
-            sort_upsweep_kernel<T, SORT_BLOCK, SORT_ITEMS, 4, uint32_t><<<l.ntiles, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
+            sort_upsweep_kernel<T, SORT_BLOCK, SORT_ITEMS, 4, uint32_t><<<ugrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
             RK_LAUNCH_CHECK();
             sort_tilescan_kernel<<<l.nchunks, TS_BLOCK, 0, stream>>>(ctl, p, counts, l.ntiles, l.chunk_rows, chunk_total, chunk_prefix);
             RK_LAUNCH_CHECK();
-            sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, chunk_prefix, l.chunk_rows, l.ntiles, xcd_chunk);
+            const auto run = [&](auto kernel) {
+                kernel<<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, chunk_prefix, l.chunk_rows, l.ntiles, xcd_chunk);
+            };
+            if constexpr (sizeof(T) == 4 && !PERM) {
+                if (l.quantiles) run(sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false, true>);
+                else run(sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false>);
+            } else {
+                run(sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false>);
+            }
             RK_LAUNCH_CHECK();
         }
         if constexpr (sizeof(T) == 8) {
@@ -981,15 +1024,15 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
             }
         }
     }
-    if (!PERM && !(all_passes && PASSES % 2 == 0)) {
+    if (!PERM && (l.quantiles || !(all_passes && PASSES % 2 == 0))) {
         const uint32_t most = l.split ? SORT_FEW_PASSES : (uint32_t)PASSES;
         // whole 32-bit words: buffers are 256-byte padded, the caller's array is at least element-aligned; 16-bit keys
         // with an odd count copy one element more than n only inside buffer padding on the source side -- so copy by element there
         const int64_t nwords = sizeof(T) == 2 ? n : ((int64_t)n * (int64_t)sizeof(T) + 3) / 4;
         int64_t g = (nwords + 255) / 256;
         if (g > cus * 16) g = cus * 16;
-        if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint16_t*)keys, (uint16_t*)buf_a, (const uint16_t*)buf_b, nwords, most);
-        else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint32_t*)keys, (uint32_t*)buf_a, (const uint32_t*)buf_b, nwords, most);
+        if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint16_t*)keys, (uint16_t*)buf_a, (const uint16_t*)buf_b, nwords, most, first_source == SORT_ENDS_IN_A ? 1 : 0);
+        else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint32_t*)keys, (uint32_t*)buf_a, (const uint32_t*)buf_b, nwords, most, first_source == SORT_ENDS_IN_A ? 1 : 0);
         RK_LAUNCH_CHECK();
     }
     return RK_SUCCESS;

@@ -15,9 +15,9 @@
 //
 // Radix passes -> so, us a call: sort Float64[2^21] 248 -> 75, [2^24] 718 -> 315, [2^26] 3093 -> 1162; sort Int64 of 64 bits 262 -> 110,
 // 760 -> 357; sortperm Int64 288 -> 120, 1026 -> 484; sort Float32[1500000] 113 -> 58, [2^22] 136 -> 92, two values 135 -> 128, 256 values
-// 136 -> 109; sortperm Float32[2^22] 148 -> 106, two values 143 -> 145, 256 values 145 -> 130.  For Float32 beyond, radix passes are faster (2^24
-// keys of two values 241 against 345, of 2^26 normal ones 764 against 984, both before large bins were divided more than once); so is Int32 at
-// once, which needs a read for the digits that vary, and launches for the passes that then do not run (2^21 keys of 20 bits).
+// 136 -> 109; sortperm Float32[2^22] 148 -> 106, two values 143 -> 145, 256 values 145 -> 130.  For Float32 beyond, sort takes one move into
+// buckets (rk_sort_quantiles.hpp), and sortperm radix passes; so does Int32 at once, which needs a read for the digits that vary, and launches for the
+// passes that then do not run (2^21 keys of 20 bits).
 // The kernels of sort Float64[2^24]: 61 first, 5 runs, 23 parts, 82 second, 129 last; 256 MiB read and written are 41.  They are bound by
 // vector instructions (sort Float32[2^22], a key: 58 first, 85 second, 204 last).
 //

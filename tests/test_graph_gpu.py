@@ -162,3 +162,40 @@ def test_graph_replays_of_sorts_by_two_levels_of_splitters(rk, orc):
         assert np.array_equal(rk.Array(perm), orc.sortperm(hi)), replay
         assert np.array_equal(rk.Array(i), orc.sort(hi)), replay
         assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(hi))), orc.sort(hi))         # eager work between the replays
+
+
+def test_graph_replays_of_sorts_by_quantiles(rk, orc):
+    """In every replay anew the device decides whether buckets or radix passes sort the keys."""
+    from amdgpu_jl_amd import _lib as L
+    from amdgpu_jl_amd.array import stream_ptr
+
+    nf, ni = (1 << 22) + 4099, (1 << 23) + 5
+    rng = np.random.default_rng(45)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        f, i = rk.ROCArray(dims=(nf,), dtype=np.float32), rk.ROCArray(dims=(ni,), dtype=np.int32)
+        fs, si = rk.ROCArray(dims=(nf,), dtype=np.float32), rk.ROCArray(dims=(ni,), dtype=np.int32)
+        tmp = torch.empty(int(L.lib.rk_sort_tmp_bytes(L.RK_I32, ni, 0)), dtype=torch.uint8, device="cuda")
+
+        def calls():
+            s = stream_ptr()
+            L.check(L.lib.rk_sort_to(L.RK_F32, f.ptr, fs.ptr, nf, 1, tmp.data_ptr(), tmp.numel(), s), "rk_sort_to")
+            L.check(L.lib.rk_sort_to(L.RK_I32, i.ptr, si.ptr, ni, 0, tmp.data_ptr(), tmp.numel(), s), "rk_sort_to")
+            L.check(L.lib.rk_sort(L.RK_I32, i.ptr, ni, 1, tmp.data_ptr(), tmp.numel(), s), "rk_sort")
+        f.buf.zero_(); i.buf.zero_()
+        calls()
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        calls()
+    for replay in range(5):
+        hf = (rng.standard_normal(nf) if replay % 2 == 0 else rng.integers(0, 2 + replay, nf)).astype(np.float32)
+        hi = rng.integers(-2**31, 2**31 if replay % 3 == 0 else -2**31 + (3 if replay % 3 == 1 else 1), ni).astype(np.int32)
+        _upload(f, hf); _upload(i, hi)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(rk.Array(fs), np.sort(hf)[::-1]), replay
+        assert np.array_equal(rk.Array(si), np.sort(hi)), replay
+        assert np.array_equal(rk.Array(i), np.sort(hi)[::-1]), replay
+        assert np.array_equal(rk.Array(rk.sort(rk.ROCArray(hf))), np.sort(hf))         # eager work between the replays

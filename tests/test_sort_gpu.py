@@ -430,3 +430,85 @@ def test_part_and_buckets_larger_than_lds(rk, orc, dtype, few):
         x += rng.integers(0, 7, n) << 40                     # (four digits and more)
     x[_sampled(n, s)] = (1 << 50) + rng.integers(0, 1 << 20, s)
     _check(rk, orc, x)
+
+
+def _device_sort_check(rk, x, revs=(False, True)):
+    """sort and sort! of a vector against torch's sort, bit for bit (no -0.0 beside 0.0 and no NaN among the keys)."""
+    import torch
+    xt = torch.from_numpy(x).cuda()
+    want = torch.sort(xt).values.view(torch.int32)
+    for rev in revs:
+        xd = rk.ROCArray(buf=xt.clone().view(torch.uint8), dims=(x.size,), dtype=x.dtype.type)
+        assert torch.equal(rk.sort(xd, rev=rev).buf[:4 * x.size].view(torch.int32), want.flip(0) if rev else want), rev
+        assert torch.equal(xd.buf[:4 * x.size].view(torch.int32), xt.view(torch.int32))
+        rk.sort_(xd, rev=rev)
+        assert torch.equal(xd.buf[:4 * x.size].view(torch.int32), want.flip(0) if rev else want), rev
+
+
+QUANTILES = {np.float32: (1 << 22) + 1, np.int32: (1 << 23) + 1}         # from so many keys on sorts of 4-byte keys move them into buckets once
+
+
+@pytest.mark.parametrize("kind", ["sorted", "equal", "few", "hundreds", "clusters", "gaps", "steep", "normal", "zeros", "quantized", "two in a bin"])
+@pytest.mark.parametrize("dtype", [np.float32, np.int32])
+def test_sorts_by_quantiles(rk, dtype, kind):
+    """One key more than sorts by other ways take, and tiles of 24576 keys of which the last is full, lacks a key or holds one; keys
+    that the buckets hold, and that send the call to the radix passes, over all digits or some, or none at all."""
+    rng = np.random.default_rng(41)
+    n0 = QUANTILES[dtype]
+    for n in (n0, 24576 * 343, 24576 * 343 + 1, 24576 * 344 - 1):
+        if n < n0:
+            continue
+        if kind == "zeros":
+            x = np.maximum(rng.standard_normal(n) - 1.3, 0) * (1 if dtype == np.float32 else 1 << 24)
+        elif kind == "quantized":
+            x = rng.standard_normal(n).astype(np.float16).astype(np.float32) * (1 if dtype == np.float32 else 1 << 24)
+            x[x == 0] = 0
+        elif kind == "two in a bin":                     # 3000 values, many times over, each with its neighbour
+            v = rng.standard_normal(1500).astype(np.float32) * (1 if dtype == np.float32 else 1 << 24)
+            x = rng.choice(np.concatenate([v, np.nextafter(v, np.float32(np.inf)) if dtype == np.float32 else v + 1]), n)
+        else:
+            x = _spread(rng, dtype, n, kind)
+        _device_sort_check(rk, np.ascontiguousarray(x.astype(dtype)), (False, True) if n == n0 else (False,))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int32])
+@pytest.mark.parametrize("near,width", [(1000, 1), (9000, 1), (15000, 64), (20000, 1), (18000, 8192), (60000, 1)])
+def test_bucket_with_a_cluster(rk, dtype, near, width):
+    """`near` keys among `width` times the values of a bin, in one bucket: many rounds of merges, bins that are sorted in memory, keys that lie
+    in LDS half a bucket at a time, and more than a bucket may have."""
+    rng = np.random.default_rng(near)
+    n = QUANTILES[dtype] + 12345
+    span = 1 << 30 if dtype == np.int32 else 1 << 22     # of Float32: of the bits of one binade, so that cells are lines of equal slope
+    x = rng.integers(0, span, n)
+    bucket = span // 256 if dtype == np.float32 else span // 512
+    at = span // 3
+    x[rng.choice(n, near, replace=False)] = at + rng.integers(0, max(2, min(bucket // 8192 * width, bucket)), near)
+    x = (x + (127 << 23)).astype(np.uint32).view(np.float32) if dtype == np.float32 else x.astype(np.int32)
+    _device_sort_check(rk, x, (False,))
+
+
+@pytest.mark.parametrize("n", [1 << 24, 1 << 25, (1 << 26) - 24575, 1 << 26, (1 << 26) + 1])
+def test_long_sorts_of_floats(rk, n):
+    """2^26 keys are the most that go into buckets; the next length takes radix passes."""
+    x = np.random.default_rng(n).standard_normal(n, dtype=np.float32)
+    x[x == 0] = 0                                        # (some are -0.0)
+    _device_sort_check(rk, x, (False,))
+
+
+def test_sorts_by_quantiles_keep_special_floats_and_neighbours(rk, orc):
+    """NaNs of every bit pattern, infinities, zeros of both signs, at both ends of a view that starts at an odd element."""
+    n = QUANTILES[np.float32] + 77
+    rng = np.random.default_rng(42)
+    x = rng.standard_normal(n + 8).astype(np.float32)
+    u = x.view(np.uint32)
+    bits = np.array([0xffc00001, 0x7fc12345, 0x7f800001, 0xff800001, 0x7fffffff, 0x7f800000, 0xff800000, 0x80000000, 0, 1, 0x80000001, 0x7f7fffff], dtype=np.uint32)
+    u[rng.choice(n, 6000, replace=False)] = rng.choice(bits, 6000)
+    for rev in (False, True):
+        d = rk.ROCArray(x.copy())
+        rk.sort_(d.view_range(4, n + 3), rev=rev)
+        whole = rk.Array(d)
+        got, src = whole[3:n + 3], x[3:n + 3]
+        assert np.array_equal(whole[:3].view(np.uint32), u[:3]) and np.array_equal(whole[n + 3:].view(np.uint32), u[n + 3:])
+        assert np.array_equal(np.sort(got.view(np.uint32)), np.sort(src.view(np.uint32)))
+        want = orc.sort(src, rev)
+        assert np.array_equal(got, want, equal_nan=True) and np.array_equal(np.signbit(got[~np.isnan(got)]), np.signbit(want[~np.isnan(want)]))
