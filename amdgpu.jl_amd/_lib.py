@@ -95,6 +95,7 @@ PROTOTYPES = {
     "rk_workspace_init": (C.c_int32, [C.c_void_p, C.c_size_t, C.c_void_p]),
     "rk_set_wait_budget": (C.c_int64, [C.c_int64]),
     "rk_workspace_status": (C.c_int32, [C.c_void_p, C.c_size_t, C.c_void_p]),
+    "rk_wait_words": (C.c_int32, [C.c_void_p, C.c_uint32, C.c_uint64, C.c_int64]),
     "rk_sort_status": (C.c_int32, [C.c_void_p, C.c_size_t, C.c_void_p]),
     "rk_accumulate_static_status": (C.c_int32, [C.c_void_p]),
     "rk_mapreduce": (C.c_int32, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_int, _I64P, C.c_uint32,

@@ -1,6 +1,7 @@
 // C ABI entry points of librk.so: argument validation (runs without a GPU), dispatch on the
 // element types, workspace management.  The kernels live in rk_*_impl.hpp / rk_*.hip.
 #include <atomic>
+#include <chrono>
 #include <mutex>
 #include <cstdlib>
 #include <cstddef>
@@ -296,6 +297,20 @@ int64_t rk_set_wait_budget(int64_t rounds) {
     const long long prev = wait_budget();
     g_wait_budget.store(rounds > 0 ? (long long)rounds : WAIT_BUDGET_DEFAULT, std::memory_order_relaxed);
     return (int64_t)prev;
+}
+
+int32_t rk_wait_words(const void* base, uint32_t mask, uint64_t unset, int64_t us) {
+    const uint64_t* const w = (const uint64_t*)base;
+    const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(us > 0 ? us : 0);
+    for (uint32_t missing = base != nullptr ? mask : 0u; missing != 0u;) {
+        for (int look = 0; look < 64 && missing != 0u; ++look) {
+            const int i = __builtin_ctz(missing);
+            if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) != unset) missing &= missing - 1u;
+            else __builtin_ia32_pause();
+        }
+        if (missing != 0u && std::chrono::steady_clock::now() >= end) return 0;
+    }
+    return 1;
 }
 
 int32_t rk_workspace_status(const void* ws, size_t ws_bytes, void* stream) {

@@ -69,7 +69,7 @@ def _select(x: ROCArray, mask: ROCArray) -> ROCArray:
     tmp = torch.empty(nbytes, dtype=torch.uint8, device=device())
     ws, ws_bytes = workspace()
     slot = take_slot()
-    fill_slot(slot, L.lib.rk_mask_count, "rk_mask_count", (mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes))
+    fill_slot(slot, L.lib.rk_mask_count, "rk_mask_count", (mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes), words=1)
     total = int(slot[1][:8].view(np.int64)[0])
     give_slot(slot)
     y = ROCArray(dims=(total,), dtype=x.dtype)

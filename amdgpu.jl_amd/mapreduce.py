@@ -222,7 +222,7 @@ def mapreduce(f, op: str, A: ROCArray, dims=None, init=None):
         # the kernel writes the value to pinned host memory: no result array, no copy
         slot = take_slot()
         fn, name, args = _dense_args(f, prog, op, A, dtype_code(out_dt), slot[0], init, out_dt, mask)
-        fill_slot(slot, fn, name, args)
+        fill_slot(slot, fn, name, args, words=1)
         value = slot[1][:out_dt.itemsize].view(out_dt)[0].copy()
         give_slot(slot)
         return value
@@ -362,7 +362,8 @@ def _findminmax(A, want_max: bool, dims):
         ws, ws_bytes = workspace()
         slot = take_slot()
         fill_slot(slot, L.lib.rk_findminmax, "rk_findminmax",
-                  (1 if want_max else 0, A.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, slot[0], slot[0] + 16, ws, ws_bytes))
+                  (1 if want_max else 0, A.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, slot[0], slot[0] + 16, ws, ws_bytes),
+                  words=1 | ((1 << A.ndim) - 1) << 2)
         value = slot[1][:A.dtype.itemsize].view(A.dtype)[0].copy()
         c = tuple(int(v) for v in slot[1][16:16 + 8 * A.ndim].view(np.int64))
         give_slot(slot)

@@ -142,6 +142,15 @@ RK_API int32_t rk_workspace_status(const void* ws, size_t ws_bytes, void* stream
 RK_API int32_t rk_sort_status(const void* tmp, size_t tmp_bytes, void* stream);
 RK_API int32_t rk_accumulate_static_status(void* stream);
 
+/* ---- scalar results in host memory ------------------------------------------------
+ * Results of rk_mapreduce, rk_findminmax and rk_mask_count may lie in pinned host memory.  Such a result is written once, a
+ * 64-bit word or less at a time, when the call has read all that it reads; the host can have it before the stream's
+ * end is reported to it (no counterpart in the reference, which copies the result back).
+ *   rk_wait_words   waits until every word i of `base` with bit i of `mask` set differs from `unset`, which the caller has
+ *                   put there before the call whose results they are; 1, or 0 if that takes longer than `us` microseconds
+ *                   (then a word may also be `unset` as a result: wait for the stream).  Starts nothing and needs no device. */
+RK_API int32_t rk_wait_words(const void* base, uint32_t mask, uint64_t unset, int64_t us);
+
 /* ---- mapreduce ------------------------------------------------------------------
  * Replaces GPUArrays.mapreducedim!(f, op, R, A; init)      src/kernels/mapreduce.jl:86-173
  * and its device kernels partial_mapreduce_device / reduce_group        :43-82, :8-34.

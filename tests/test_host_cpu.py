@@ -84,3 +84,31 @@ def test_reshape_counts_the_elements_of_the_dims_it_makes(rk):
             x.reshape(*dims)
     y = rk.ROCArray(buf=torch.zeros(16, dtype=torch.uint8), dims=(4,), dtype=np.float32)
     assert y.reshape(2.5, 2).dims == (2, 2)
+
+
+@pytest.mark.parametrize("words,written,waits", [(1, [0], 0), (0b1101, [0, 2, 3], 0), (0b1101, [0, 3], 1), (1, [], 1), (0, [0], 1)])
+def test_a_slot_is_read_when_its_words_are_there(slots, monkeypatch, words, written, waits):
+    """The stream is waited for only if a word of the result is missing after the time that the words are waited for; words
+    that are no part of the result, and what an earlier call has left, do not count."""
+    array, slot, state = slots
+    monkeypatch.setattr(array, "_WAIT_US", 50)
+    slot[1][:] = 9
+
+    def call(*args):
+        for i in written:
+            slot[1][8 * i] ^= 0xff                       # a byte of a word is enough
+        return 0
+    array.fill_slot(array.take_slot(), call, "call", (), words=words)
+    assert state["stream"].waits == waits
+
+
+def test_wait_words_sees_what_another_thread_writes(rk):
+    import threading
+    from amdgpu_jl_amd import _lib as L
+    w = np.full(4, 5, dtype=np.uint64)
+    later = threading.Timer(0.05, lambda: w.__setitem__(2, 6))
+    later.start()
+    assert L.lib.rk_wait_words(w.ctypes.data, 0b100, 5, 20_000_000) == 1          # (the interpreter is not held meanwhile)
+    later.join()
+    assert L.lib.rk_wait_words(w.ctypes.data, 0b110, 5, 1000) == 0
+    assert L.lib.rk_wait_words(w.ctypes.data, 0, 5, 0) == 1 and L.lib.rk_wait_words(None, 1, 5, 0) == 1
