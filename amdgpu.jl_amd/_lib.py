@@ -121,6 +121,9 @@ PROTOTYPES = {
     "rk_findall_scatter": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, _I64P, C.c_void_p]),
     "rk_gather_slices": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
     "rk_mask_tmp_bytes": (C.c_size_t, [C.c_int64]),
+    "rk_mask_bits_tmp_bytes": (C.c_size_t, [C.c_int64]),
+    "rk_mask_count_bits": (C.c_int32, [C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p, C.c_size_t, C.c_void_p]),
+    "rk_mask_select_bits": (C.c_int32, [C.c_int64, C.c_void_p, C.c_void_p, C.c_size_t, C.c_int64, C.c_void_p, C.c_size_t, C.c_void_p]),
     "rk_mask_count": (C.c_int32, [C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p, C.c_size_t, C.c_void_p]),
     "rk_mask_select": (C.c_int32, [C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_size_t, C.c_int64, C.c_void_p, C.c_size_t,
                                    C.c_void_p]),

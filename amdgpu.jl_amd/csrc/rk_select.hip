@@ -379,34 +379,42 @@ extern "C" int32_t rk_gather_slices(const void* x, const int64_t* idx, void* y, 
 }
 
 // ---- x[mask] ------------------------------------------------------------------------------------------------------
-// The length of the result has to be known before it can be allocated, so the mask is read twice whatever is done; what
-// the count leaves behind makes the second read a plain streaming kernel:
+// The length of the result has to be known before it can be allocated; what the count leaves behind makes the rest a plain
+// streaming kernel, which does not read the mask again (rk_mask_count_bits, rk_mask_select_bits; the entry points with the smaller
+// temporary read it twice):
 //   mask_count_kernel    set bytes of every tile of 4096 Bools (one wave), as exclusive prefixes inside groups of tiles,
-//                        and the exclusive prefixes of the groups (the workgroup that finishes last scans them)
+//                        the exclusive prefixes of the groups (the workgroup that finishes last scans them), and the mask, a bit a Bool
 //   mask_select_kernel, mask_select_dense_kernel
 //                        a wave per tile: its first output slot is two loads away, so there is no look-back, no barrier
 //                        and nothing to wait for; selected elements go from x to y without an index in between
-// Bound by memory: the mask (the second read comes from the Infinity Cache up to 2^27 Bools), the lines of x that hold a
-// selected element, and the result.  Before, this was a u8 -> Int64 reduction, the one-pass findall and a gather by its
-// Int64 indices (16 bytes of index traffic per selected element): Float32[2^26], 25 % set, the whole call 193 -> 113 us.
+// Bound by memory: the mask, the lines of x that hold a selected element, and the result.  Before, this was a u8 -> Int64 reduction,
+// the one-pass findall and a gather by its Int64 indices (16 bytes of index traffic per selected element): Float32[2^26], 25 %
+// set, the whole call 193 -> 113 us.  Bits instead of the mask bytes for the second kernel, and a count whose loads do not stay in
+// the caches (where they push out what the call before has written), us a call of 2^26 at 1, 25, 50 and 90 %:
+//   bytes twice       Float32 53 95 105 130, Int64 54 149 184 250     (5 us of these the wait for the stream instead of the count)
+//   bits              Float32 46 84  96 127, Int64 47 141 190 239
+//   and so            Float32 42 84  95 111, Int64 43 140 162 240
 namespace rk {
 
 constexpr int MSK_TILE = 4096, MSK_LOADS = MSK_TILE / SEL_CHUNK;
 constexpr int MSK_BLOCK = 1024, MSK_WAVES = MSK_BLOCK / WAVE;
 
 // Tiles per group, i.e. per workgroup of the count: 16 (one a wave) keeps the chip busy down to short masks, 64 keeps the
-// number of group totals that one workgroup scans at the end small.
-inline int msk_group_shift(int64_t n) { return n <= ((int64_t)1 << 24) ? 4 : 6; }
+// number of group totals that one workgroup scans at the end small.  Float32, 16 / 32 / 64, us a call at 25 %: 2^24 32.9 / 33.1 / 33.1,
+// 2^25 58.1 / 56.0 / 57.2, 2^26 88.7 / 85.8 / 84.3.
+inline int msk_group_shift(int64_t n) { return n <= ((int64_t)1 << 24) ? 4 : n <= ((int64_t)1 << 25) ? 5 : 6; }
 struct MaskTmp {
     int64_t ntiles, ngroups;
-    size_t tile_off, bytes;          // [group prefixes: Int64][tile prefixes: UInt32]
+    size_t tile_off, bits_off, bytes, bits_bytes;          // [group prefixes: Int64][tile prefixes: UInt32][a bit a Bool: 64 words of 64 a tile]
 };
 inline MaskTmp mask_tmp(int64_t n) {
     MaskTmp m;
     m.ntiles = (n + MSK_TILE - 1) / MSK_TILE;
     m.ngroups = (m.ntiles + (1 << msk_group_shift(n)) - 1) >> msk_group_shift(n);
     m.tile_off = ((size_t)m.ngroups * sizeof(int64_t) + 255) & ~(size_t)255;
-    m.bytes = m.tile_off + (((size_t)m.ntiles * sizeof(uint32_t) + 255) & ~(size_t)255);
+    m.bits_off = m.tile_off + (((size_t)m.ntiles * sizeof(uint32_t) + 255) & ~(size_t)255);
+    m.bytes = m.bits_off;                                               // (without the bits)
+    m.bits_bytes = (size_t)m.ntiles * (MSK_TILE / 8);
     return m;
 }
 
@@ -426,9 +434,24 @@ __device__ __forceinline__ mask_vec mask_load16(const uint8_t* __restrict__ mask
     return v;
 }
 
-template <int TPW>                   // tiles per wave
+// Bit 0 of 16 bytes, in order.
+__device__ __forceinline__ uint32_t mask_bits16(const mask_vec& v) {
+    const mask_vec b = v & 0x01010101u;
+    const uint32_t lo = __builtin_amdgcn_udot4(b[1], 0x80402010u, __builtin_amdgcn_udot4(b[0], 0x08040201u, 0u, false), false);
+    const uint32_t hi = __builtin_amdgcn_udot4(b[3], 0x80402010u, __builtin_amdgcn_udot4(b[2], 0x08040201u, 0u, false), false);
+    return lo | (hi << 8);
+}
+
+// What lane l reads of a tile by its four loads, Bools k * 1024 + 16 l ... of the tile, 16 bits each: word l of the tile's bits.
+__device__ __forceinline__ uint64_t mask_word(const mask_vec (&x)[MSK_LOADS]) {
+    static_assert(MSK_LOADS == 4, "");
+    return (uint64_t)(mask_bits16(x[2]) | mask_bits16(x[3]) << 16) << 32 | (mask_bits16(x[0]) | mask_bits16(x[1]) << 16);
+}
+
+// BITS: the words stay behind, and nothing reads the mask again.
+template <int TPW, bool BITS>        // TPW: tiles per wave
 __global__ __launch_bounds__(MSK_BLOCK) void mask_count_kernel(const uint8_t* __restrict__ mask, int64_t n, int aligned, int64_t ntiles,
-                                                               uint32_t* __restrict__ tile_prefix, int64_t* group_prefix,
+                                                               uint32_t* __restrict__ tile_prefix, uint64_t* __restrict__ bits, int64_t* group_prefix,
                                                                int64_t* count_out, uint32_t* tickets, int ticket_group) {
     __shared__ uint32_t lds_count[MSK_WAVES * TPW];
     __shared__ int64_t lds_wave[MSK_WAVES];
@@ -443,7 +466,10 @@ __global__ __launch_bounds__(MSK_BLOCK) void mask_count_kernel(const uint8_t* __
         for (int t = 0; t < TPW; ++t)
 #pragma unroll
             for (int k = 0; k < MSK_LOADS; ++k)
-                x[t][k] = *(const mask_vec*)(mask + (first + wave * TPW + t) * MSK_TILE + k * SEL_CHUNK + lane * 16);
+            {
+                const mask_vec* const from = (const mask_vec*)(mask + (first + wave * TPW + t) * MSK_TILE + k * SEL_CHUNK + lane * 16);
+                x[t][k] = BITS ? load_nt(from) : *from;
+            }
     } else {
 #pragma unroll
         for (int t = 0; t < TPW; ++t)
@@ -453,12 +479,10 @@ __global__ __launch_bounds__(MSK_BLOCK) void mask_count_kernel(const uint8_t* __
     }
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
-        c[t] = 0;
-#pragma unroll
-        for (int k = 0; k < MSK_LOADS; ++k) {
-            const mask_vec b = x[t][k] & 0x01010101u;
-            c[t] += (uint32_t)(__popc(b[0]) + __popc(b[1]) + __popc(b[2]) + __popc(b[3]));
-        }
+        const uint64_t b = mask_word(x[t]);
+        const int64_t tile = first + wave * TPW + t;
+        c[t] = (uint32_t)__popcll(b);
+        if (BITS && tile < ntiles) bits[tile * WAVE + lane] = b;
     }
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
@@ -511,11 +535,31 @@ __global__ __launch_bounds__(MSK_BLOCK) void mask_count_kernel(const uint8_t* __
     if (tid == 0) *count_out = carry;
 }
 
+// The lane's word of a tile, from the bits of the count or from the mask.
+template <bool BITS> __device__ __forceinline__ uint64_t mask_tile_word(const void* __restrict__ mask, int64_t n, int aligned, int64_t tile, int lane) {
+    if constexpr (BITS) return ((const uint64_t*)mask)[tile * WAVE + lane];
+    const uint8_t* const bytes = (const uint8_t*)mask;
+    const int64_t e0 = tile * MSK_TILE + lane * 16;
+    typedef uint32_t mask_vec_at4 __attribute__((ext_vector_type(4), aligned(4)));
+    mask_vec m[MSK_LOADS];
+    if (aligned && tile * MSK_TILE + MSK_TILE <= n) {       // (to 4 bytes)
+#pragma unroll
+        for (int k = 0; k < MSK_LOADS; ++k) m[k] = (mask_vec)__builtin_nontemporal_load((const mask_vec_at4*)(bytes + e0 + k * SEL_CHUNK));
+    } else {
+#pragma unroll
+        for (int k = 0; k < MSK_LOADS; ++k) {
+            const int64_t i = e0 + k * SEL_CHUNK;
+            m[k] = aligned && i + 16 <= n ? (mask_vec)__builtin_nontemporal_load((const mask_vec_at4*)(bytes + i)) : mask_load16(bytes, i, n, 0);
+        }
+    }
+    return mask_word(m);
+}
+
 // A wave per tile.  The set positions of the tile are listed in LDS (strip; the lanes' hits are ranked by one scan for every
 // two loads), then every lane takes every 64th of them: loads of x walk forward over the tile, stores are whole lines.
 // A list of the tile's hits and not a masked store per 64 elements: at 25 % set that is a quarter of the loads and stores.
-template <typename E>
-__global__ __launch_bounds__(256) void mask_select_kernel(const uint8_t* __restrict__ mask, int64_t n, int aligned, const E* __restrict__ x,
+template <typename E, bool BITS>
+__global__ __launch_bounds__(256) void mask_select_kernel(const void* __restrict__ mask, int64_t n, int aligned, const E* __restrict__ x,
                                                           E* __restrict__ y, int64_t nsel, int64_t ntiles,
                                                           const uint32_t* __restrict__ tile_prefix, const int64_t* __restrict__ group_prefix,
                                                           int group_shift) {
@@ -526,14 +570,7 @@ __global__ __launch_bounds__(256) void mask_select_kernel(const uint8_t* __restr
     const int64_t tile = (int64_t)blockIdx.x * (256 / WAVE) + wave;
     if (tile >= ntiles) return;
     const int64_t e0 = tile * MSK_TILE;
-    mask_vec m[MSK_LOADS];
-    if (aligned && e0 + MSK_TILE <= n) {
-#pragma unroll
-        for (int k = 0; k < MSK_LOADS; ++k) m[k] = load_nt((const mask_vec*)(mask + e0 + k * SEL_CHUNK + lane * 16));
-    } else {
-#pragma unroll
-        for (int k = 0; k < MSK_LOADS; ++k) m[k] = mask_load16(mask, e0 + k * SEL_CHUNK + lane * 16, n, aligned);
-    }
+    const uint64_t m = mask_tile_word<BITS>(mask, n, aligned, tile, lane);
     int64_t base = group_prefix[tile >> group_shift] + (int64_t)tile_prefix[tile];
     const E* src = x + e0;
     uint16_t* strip = lds_strip[wave];
@@ -562,14 +599,7 @@ __global__ __launch_bounds__(256) void mask_select_kernel(const uint8_t* __restr
     };
 #pragma unroll
     for (int k0 = 0; k0 < MSK_LOADS; k0 += 2) {
-        uint32_t hits[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const mask_vec b = m[k0 + h] & 0x01010101u;
-            const uint32_t lo = __builtin_amdgcn_udot4(b[1], 0x80402010u, __builtin_amdgcn_udot4(b[0], 0x08040201u, 0u, false), false);
-            const uint32_t hi = __builtin_amdgcn_udot4(b[3], 0x80402010u, __builtin_amdgcn_udot4(b[2], 0x08040201u, 0u, false), false);
-            hits[h] = lo | (hi << 8);
-        }
+        const uint32_t hits[2] = {(uint32_t)(m >> (16 * k0)) & 0xffffu, (uint32_t)(m >> (16 * k0 + 16)) & 0xffffu};
         const int32_t c = (int32_t)(__popc(hits[0]) | ((uint32_t)__popc(hits[1]) << 16));
         const int32_t inc = wave_scan_inclusive(c, op, 0);
         const uint32_t exc = (uint32_t)(inc - c), tot = (uint32_t)read_lane(inc, WAVE - 1);
@@ -586,15 +616,16 @@ __global__ __launch_bounds__(256) void mask_select_kernel(const uint8_t* __restr
     if (fill > 0) flush();
 }
 
-// Where most lines of x hold a selected element anyway (4- and 8-byte elements): x is read 16 bytes a lane, where the mask bytes of the
+// Where most lines of x hold a selected element anyway (4- and 8-byte elements): x is read 16 bytes a lane, where the bits of the
 // same elements have a hit, so that no load waits for a list, and the selected ones are put together in LDS.  A step is four such
-// loads; those of the next are issued before a step is worked on (two steps ahead: no faster).  The mask is read first, all of the tile's:
-// where hits are clustered, most lines of x hold none.  Bound by memory.
-// The whole call, by list of hits -> so, us: Float32[2^26] 10 % 91 -> 88, 25 % 108.5 -> 95, 50 % 129 -> 105, 90 % 170 -> 131; Int64[2^26] 25 %
+// loads; those of the next are issued before a step is worked on (two steps ahead: no faster).  The bits are read first, all of the tile's:
+// where hits are clustered, most lines of x hold none.  Bound by memory.  (The result 16 bytes a lane instead of one element: Float32[2^26]
+// 90 % 111.6 -> 108.9, else the same; nontemporal as well: 25 % 84.7 -> 89.2, 90 % 128.)
+// The whole call, by list of hits -> so, both reading mask bytes instead of bits, us: Float32[2^26] 10 % 91 -> 88, 25 % 108.5 -> 95, 50 % 129 -> 105, 90 % 170 -> 131; Int64[2^26] 25 %
 // 178 -> 149, 90 % 268 -> 250; every hit of Int64[2^26] in the first quarter 85.2 -> 84.3, in runs of 13 of 100 tiles 80.2 -> 75.5 (x read
 // whole, beside its mask bytes: 150 and 145).  (Loads that stay in the caches instead of nontemporal ones: Float32[2^26] 25 % 106.5, 90 % 143.)
-template <typename E>
-__global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* __restrict__ mask, int64_t n, const E* __restrict__ x, E* __restrict__ y,
+template <typename E, bool BITS>
+__global__ __launch_bounds__(256) void mask_select_dense_kernel(const void* __restrict__ mask, int64_t n, const E* __restrict__ x, E* __restrict__ y,
                                                                 int64_t nsel, int64_t ntiles, const uint32_t* __restrict__ tile_prefix,
                                                                 const int64_t* __restrict__ group_prefix, int group_shift) {
     constexpr int V = 16 / (int)sizeof(E), LOADS = 4, STEP = LOADS * WAVE * V, STEPS = MSK_TILE / STEP;
@@ -606,44 +637,40 @@ __global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* _
     if (tile >= ntiles) return;
     const int64_t e0 = tile * MSK_TILE;
     E* const strip = lds_strip[wave];
-    static_assert(sizeof(lds_strip[0]) == MSK_TILE, "the strip holds the mask of a tile");
     auto wave_sync = [] {                                   // what the lanes of the wave wrote to LDS is there for all of them
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    // the mask bytes of the tile, 16 a lane and load, change lanes in the strip
-    typedef uint32_t mask_vec_at4 __attribute__((ext_vector_type(4), aligned(4)));
-    mask_vec bytes[MSK_LOADS];
-    uint32_t any = 0u;
+    // Load k of a lane is elements (k * 64 + lane) * V ...: their bits are the lowest V of a 16 of one of the words that it takes.
+    constexpr int WORDS = 16 / V;
+    static_assert(WORDS * WAVE * V == SEL_CHUNK, "as many loads of x for the 1024 Bools of a load as words");
+    uint64_t w[WORDS];
 #pragma unroll
-    for (int k = 0; k < MSK_LOADS; ++k) {
-        const int64_t i = e0 + k * SEL_CHUNK + lane * 16;
-        bytes[k] = i + 16 <= n ? (mask_vec)__builtin_nontemporal_load((const mask_vec_at4*)(mask + i)) : mask_load16(mask, i, n, 0);
-    }
+    for (int q = 0; q < WORDS; ++q) w[q] = BITS ? ((const uint64_t*)mask)[tile * WAVE + q * (WAVE / WORDS) + lane / WORDS] : 0ull;
     int64_t base = group_prefix[tile >> group_shift] + (int64_t)tile_prefix[tile];
+    if constexpr (!BITS) {                                  // the words change lanes in the strip
+        uint64_t* const words = (uint64_t*)strip;
+        words[lane] = mask_tile_word<false>(mask, n, 1, tile, lane);
+        wave_sync();
 #pragma unroll
-    for (int k = 0; k < MSK_LOADS; ++k) {
-        bytes[k] &= 0x01010101u;
-        any |= bytes[k][0] | bytes[k][1] | bytes[k][2] | bytes[k][3];
-        *(mask_vec*)((char*)strip + k * SEL_CHUNK + lane * 16) = bytes[k];
+        for (int q = 0; q < WORDS; ++q) w[q] = words[q * (WAVE / WORDS) + lane / WORDS];
+        wave_sync();
     }
+#pragma unroll
+    for (int q = 0; q < WORDS; ++q) w[q] >>= lane % WORDS * V;
+    uint64_t any = 0u;
+#pragma unroll
+    for (int q = 0; q < WORDS; ++q) any |= w[q];
+    any &= 0x0001000100010001ull * ((1u << V) - 1u);
     if (__ballot(any != 0u) == 0ull) return;
-    wave_sync();
-    uint32_t m[STEPS * LOADS];                              // a byte an element
-#pragma unroll
-    for (int k = 0; k < STEPS * LOADS; ++k) {
-        const char* from = (const char*)strip + (k * WAVE + lane) * V;
-        if constexpr (V == 4) m[k] = *(const uint32_t*)from;
-        else m[k] = *(const uint16_t*)from;
-    }
-    wave_sync();
+    auto m = [&](int k) { return (uint32_t)(w[k % WORDS] >> (k / WORDS * 16)) & ((1u << V) - 1u); };
     auto load = [&](Loaded& l, int s) {
 #pragma unroll
         for (int g = 0; g < LOADS; ++g) {
             const int k = s * LOADS + g;
             const int64_t i = e0 + k * (WAVE * V) + lane * V;
-            if (m[k] == 0u) continue;
+            if (m(k) == 0u) continue;
             if (i + V <= n) {
                 l.x[g] = load_nt((const vec*)(x + i));
             } else {
@@ -662,7 +689,7 @@ __global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* _
         // hits of a lane, a byte a load; of the lanes in front they are 252 at most, so the bytes of the sum do not meet
         uint32_t c = 0u;
 #pragma unroll
-        for (int g = 0; g < LOADS; ++g) c |= (uint32_t)__popc(m[s * LOADS + g]) << (8 * g);
+        for (int g = 0; g < LOADS; ++g) c |= (uint32_t)__popc(m(s * LOADS + g)) << (8 * g);
         const uint32_t exc = wave_scan_inclusive(c, OpAdd(), 0u) - c;
         const uint32_t front = (uint32_t)read_lane((int32_t)exc, WAVE - 1), own = (uint32_t)read_lane((int32_t)c, WAVE - 1);
         uint32_t fill = 0u;
@@ -671,7 +698,7 @@ __global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* _
             uint32_t p = fill + ((exc >> (8 * g)) & 0xffu);
 #pragma unroll
             for (int j = 0; j < V; ++j) {
-                if ((m[s * LOADS + g] >> (8 * j)) & 1u) strip[p++] = cur.x[g][j];
+                if ((m(s * LOADS + g) >> j) & 1u) strip[p++] = cur.x[g][j];
             }
             fill += ((front >> (8 * g)) & 0xffu) + ((own >> (8 * g)) & 0xffu);
         }
@@ -686,12 +713,11 @@ __global__ __launch_bounds__(256) void mask_select_dense_kernel(const uint8_t* _
 
 }  // namespace rk
 
-extern "C" size_t rk_mask_tmp_bytes(int64_t n) { return n <= 0 ? 256 : mask_tmp(n).bytes; }
+namespace rk {
 
-extern "C" int32_t rk_mask_count(const uint8_t* mask, int64_t n, int64_t* count_out, void* tmp, size_t tmp_bytes, void* ws, size_t ws_bytes,
-                                 void* stream) {
+template <bool BITS>
+static int32_t mask_count(const uint8_t* mask, int64_t n, int64_t* count_out, void* tmp, size_t tmp_bytes, void* ws, size_t ws_bytes, hipStream_t st) {
     if (n < 0 || count_out == nullptr) return RK_ERR_INVALID_ARGUMENT;
-    hipStream_t st = (hipStream_t)stream;
     if (n == 0) {
         store_count_kernel<<<1, 1, 0, st>>>(count_out, 0);
         RK_LAUNCH_CHECK();
@@ -700,53 +726,90 @@ extern "C" int32_t rk_mask_count(const uint8_t* mask, int64_t n, int64_t* count_
     if (mask == nullptr) return RK_ERR_INVALID_ARGUMENT;
     const MaskTmp t = mask_tmp(n);
     Workspace w{};
-    if (tmp == nullptr || !is_aligned(tmp, 256) || tmp_bytes < t.bytes || !carve_workspace(ws, ws_bytes, 0, &w)) return RK_ERR_WORKSPACE;
+    if (tmp == nullptr || !is_aligned(tmp, 256) || tmp_bytes < t.bytes + (BITS ? t.bits_bytes : 0) || !carve_workspace(ws, ws_bytes, 0, &w)) return RK_ERR_WORKSPACE;
     const int tg = ordered_ticket_group(t.ngroups);
     if (t.ngroups > 0x7fffffff) return RK_ERR_TOO_LARGE;
     const int aligned = is_aligned(mask, 16) ? 1 : 0;
     int64_t* gp = (int64_t*)tmp;
     uint32_t* tp = (uint32_t*)((char*)tmp + t.tile_off);
-    if (msk_group_shift(n) == 4) mask_count_kernel<1><<<(unsigned)t.ngroups, MSK_BLOCK, 0, st>>>(mask, n, aligned, t.ntiles, tp, gp, count_out, w.tickets, tg);
-    else mask_count_kernel<4><<<(unsigned)t.ngroups, MSK_BLOCK, 0, st>>>(mask, n, aligned, t.ntiles, tp, gp, count_out, w.tickets, tg);
+    uint64_t* bits = (uint64_t*)((char*)tmp + t.bits_off);
+#define RK_MCOUNT(TPW) mask_count_kernel<TPW, BITS><<<(unsigned)t.ngroups, MSK_BLOCK, 0, st>>>(mask, n, aligned, t.ntiles, tp, bits, gp, count_out, w.tickets, tg)
+    switch (msk_group_shift(n)) {
+        case 4: RK_MCOUNT(1); break;
+        case 5: RK_MCOUNT(2); break;
+        default: RK_MCOUNT(4); break;
+    }
+#undef RK_MCOUNT
     RK_LAUNCH_CHECK();
     return RK_SUCCESS;
 }
 
-extern "C" int32_t rk_mask_select(const uint8_t* mask, int64_t n, const void* x, void* y, size_t elsize, int64_t nsel, const void* tmp,
-                                  size_t tmp_bytes, void* stream) {
+template <bool BITS>
+static int32_t mask_select(const uint8_t* mask, int64_t n, const void* x, void* y, size_t elsize, int64_t nsel, const void* tmp, size_t tmp_bytes, hipStream_t st) {
     if (n < 0 || nsel < 0) return RK_ERR_INVALID_ARGUMENT;
     if (elsize != 1 && elsize != 2 && elsize != 4 && elsize != 8 && elsize != 16) return RK_ERR_UNSUPPORTED;
     if (n == 0 || nsel == 0) return RK_SUCCESS;
-    if (mask == nullptr || x == nullptr || y == nullptr) return RK_ERR_INVALID_ARGUMENT;
+    if ((!BITS && mask == nullptr) || x == nullptr || y == nullptr) return RK_ERR_INVALID_ARGUMENT;
     const size_t align = elsize < 16 ? elsize : 8;
     if (!is_aligned(x, align) || !is_aligned(y, align)) return RK_ERR_INVALID_ARGUMENT;
     const MaskTmp t = mask_tmp(n);
-    if (tmp == nullptr || !is_aligned(tmp, 256) || tmp_bytes < t.bytes) return RK_ERR_WORKSPACE;
+    if (tmp == nullptr || !is_aligned(tmp, 256) || tmp_bytes < t.bytes + (BITS ? t.bits_bytes : 0)) return RK_ERR_WORKSPACE;
     const int64_t blocks = (t.ntiles + 3) / 4;
     if (blocks > 0x7fffffff) return RK_ERR_TOO_LARGE;
-    const int aligned = is_aligned(mask, 16) ? 1 : 0;
     const int64_t* gp = (const int64_t*)tmp;
     const uint32_t* tp = (const uint32_t*)((const char*)tmp + t.tile_off);
-    hipStream_t st = (hipStream_t)stream;
-#define RK_MSEL(E) rk::mask_select_kernel<E><<<(unsigned)blocks, 256, 0, st>>>(mask, n, aligned, (const E*)x, (E*)y, nsel, t.ntiles, tp, gp, msk_group_shift(n))
-    // Elements of x that sit in the Infinity Cache cost the list of hits little: Float32[2^24] 10 % 36.7 us by list and 40.4 whole, 25 % 39.0 and
-    // 41.3, 50 % 45.0 and 44.5; Int64[2^24] (128 MiB) 43.9 and 52.7, 56.1 and 55.6, 62.8 and 61.2.  Beyond, an eighth of the elements is the line
-    // (7 %: Float32[2^26] 86.7 and 86.3, Int64[2^26] 118 and 136; 10 %: 91 and 88, 139 and 139).
-    const bool cached = (uint64_t)n * elsize <= ((uint64_t)1 << 27);
-    if ((elsize == 4 || elsize == 8) && nsel >= (cached ? n / 4 * 3 : n / 8) && is_aligned(x, 16) && is_aligned(mask, 4)) {
-        if (elsize == 4) mask_select_dense_kernel<uint32_t><<<(unsigned)blocks, 256, 0, st>>>(mask, n, (const uint32_t*)x, (uint32_t*)y, nsel, t.ntiles, tp, gp, msk_group_shift(n));
-        else mask_select_dense_kernel<uint64_t><<<(unsigned)blocks, 256, 0, st>>>(mask, n, (const uint64_t*)x, (uint64_t*)y, nsel, t.ntiles, tp, gp, msk_group_shift(n));
+    const void* from = BITS ? (const void*)((const char*)tmp + t.bits_off) : mask;
+    const int aligned = is_aligned(mask, 4) ? 1 : 0;         // (of a mask that is read)
+    const int shift = msk_group_shift(n);
+    // The less of x comes from the Infinity Cache, the earlier reading it 16 bytes a lane pays.  By list of hits / so, us a call at 3, 6, 10, 25, 40
+    // and 60 % at random, from bits: Float32[2^26] 62/61 76/71 83/78 96/85 107/91 123/99, Int64[2^26] 69/75 100/94 126/113 167/141 184/150 210/204;
+    // 128 MiB: Float32[2^25] 35/39 46/44 49/48 55/51 58/54 64/58, Int64[2^24] 29/32 34/36 41/42 53/51 56/53 58/57; 64 MiB: Float32[2^24] 27/27 29/29
+    // 30/32 33/34 35/35 44/38; Float32[2^22] and less the same until 40 %, at 90 % 33 and 29.
+    // From mask bytes: Float32[2^24] 10 % 36.7 by list and 40.4, 25 % 39.0 and 41.3, 50 % 45.0 and 44.5; Int64[2^24] 43.9 and 52.7, 56.1 and 55.6,
+    // 62.8 and 61.2; beyond 128 MiB an eighth is the line (7 %: Float32[2^26] 86.7 and 86.3, Int64[2^26] 118 and 136; 10 %: 91 and 88, 139 and 139).
+    const uint64_t x_bytes = (uint64_t)n * elsize, mib128 = (uint64_t)1 << 27;
+    const int64_t line = BITS ? (x_bytes > mib128 ? n / 16 : x_bytes > mib128 / 2 ? n / 8 : n / 2) : x_bytes > mib128 ? n / 8 : n / 4 * 3;
+    if ((elsize == 4 || elsize == 8) && nsel >= line && is_aligned(x, 16) && (BITS || aligned)) {
+        if (elsize == 4) mask_select_dense_kernel<uint32_t, BITS><<<(unsigned)blocks, 256, 0, st>>>(from, n, (const uint32_t*)x, (uint32_t*)y, nsel, t.ntiles, tp, gp, shift);
+        else mask_select_dense_kernel<uint64_t, BITS><<<(unsigned)blocks, 256, 0, st>>>(from, n, (const uint64_t*)x, (uint64_t*)y, nsel, t.ntiles, tp, gp, shift);
         RK_LAUNCH_CHECK();
         return RK_SUCCESS;
     }
+#define RK_MSEL(E) mask_select_kernel<E, BITS><<<(unsigned)blocks, 256, 0, st>>>(from, n, aligned, (const E*)x, (E*)y, nsel, t.ntiles, tp, gp, shift)
     switch (elsize) {
         case 1: RK_MSEL(uint8_t); break;
         case 2: RK_MSEL(uint16_t); break;
         case 4: RK_MSEL(uint32_t); break;
         case 8: RK_MSEL(uint64_t); break;
-        default: RK_MSEL(rk::Bytes16); break;
+        default: RK_MSEL(Bytes16); break;
     }
 #undef RK_MSEL
     RK_LAUNCH_CHECK();
     return RK_SUCCESS;
+}
+
+}  // namespace rk
+
+extern "C" size_t rk_mask_tmp_bytes(int64_t n) { return n <= 0 ? 256 : mask_tmp(n).bytes; }
+
+extern "C" int32_t rk_mask_count(const uint8_t* mask, int64_t n, int64_t* count_out, void* tmp, size_t tmp_bytes, void* ws, size_t ws_bytes,
+                                 void* stream) {
+    return mask_count<false>(mask, n, count_out, tmp, tmp_bytes, ws, ws_bytes, (hipStream_t)stream);
+}
+
+extern "C" int32_t rk_mask_select(const uint8_t* mask, int64_t n, const void* x, void* y, size_t elsize, int64_t nsel, const void* tmp,
+                                  size_t tmp_bytes, void* stream) {
+    return mask_select<false>(mask, n, x, y, elsize, nsel, tmp, tmp_bytes, (hipStream_t)stream);
+}
+
+extern "C" size_t rk_mask_bits_tmp_bytes(int64_t n) { return n <= 0 ? 256 : mask_tmp(n).bytes + mask_tmp(n).bits_bytes; }
+
+extern "C" int32_t rk_mask_count_bits(const uint8_t* mask, int64_t n, int64_t* count_out, void* tmp, size_t tmp_bytes, void* ws, size_t ws_bytes,
+                                      void* stream) {
+    return mask_count<true>(mask, n, count_out, tmp, tmp_bytes, ws, ws_bytes, (hipStream_t)stream);
+}
+
+extern "C" int32_t rk_mask_select_bits(int64_t n, const void* x, void* y, size_t elsize, int64_t nsel, const void* tmp, size_t tmp_bytes,
+                                       void* stream) {
+    return mask_select<true>(nullptr, n, x, y, elsize, nsel, tmp, tmp_bytes, (hipStream_t)stream);
 }

@@ -65,17 +65,16 @@ def _select(x: ROCArray, mask: ROCArray) -> ROCArray:
     n = len(x)
     if n == 0:
         return ROCArray(dims=(0,), dtype=x.dtype)
-    nbytes = int(L.lib.rk_mask_tmp_bytes(n))
+    nbytes = int(L.lib.rk_mask_bits_tmp_bytes(n))
     tmp = torch.empty(nbytes, dtype=torch.uint8, device=device())
     ws, ws_bytes = workspace()
     slot = take_slot()
-    fill_slot(slot, L.lib.rk_mask_count, "rk_mask_count", (mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes), words=1)
+    fill_slot(slot, L.lib.rk_mask_count_bits, "rk_mask_count_bits", (mask.ptr, n, slot[0], tmp.data_ptr(), nbytes, ws, ws_bytes), words=1)
     total = int(slot[1][:8].view(np.int64)[0])
     give_slot(slot)
     y = ROCArray(dims=(total,), dtype=x.dtype)
     if total > 0:
-        L.check(L.lib.rk_mask_select(mask.ptr, n, x.ptr, y.ptr, x.dtype.itemsize, total, tmp.data_ptr(), nbytes, stream_ptr()),
-                "rk_mask_select")
+        L.check(L.lib.rk_mask_select_bits(n, x.ptr, y.ptr, x.dtype.itemsize, total, tmp.data_ptr(), nbytes, stream_ptr()), "rk_mask_select_bits")
     return y
 
 

@@ -143,7 +143,7 @@ RK_API int32_t rk_sort_status(const void* tmp, size_t tmp_bytes, void* stream);
 RK_API int32_t rk_accumulate_static_status(void* stream);
 
 /* ---- scalar results in host memory ------------------------------------------------
- * Results of rk_mapreduce, rk_findminmax and rk_mask_count may lie in pinned host memory.  Such a result is written once, a
+ * Results of rk_mapreduce, rk_findminmax, rk_mask_count and rk_mask_count_bits may lie in pinned host memory.  Such a result is written once, a
  * 64-bit word or less at a time, when the call has read all that it reads; the host can have it before the stream's
  * end is reported to it (no counterpart in the reference, which copies the result back).
  *   rk_wait_words   waits until every word i of `base` with bit i of `mask` set differs from `unset`, which the caller has
@@ -404,6 +404,14 @@ RK_API int32_t rk_mask_count(const uint8_t* mask, int64_t n, int64_t* count_out,
                       void* ws, size_t ws_bytes, void* stream);
 RK_API int32_t rk_mask_select(const uint8_t* mask, int64_t n, const void* x, void* y, size_t elsize, int64_t nsel,
                        const void* tmp, size_t tmp_bytes, void* stream);
+/* The same with a `tmp` of rk_mask_bits_tmp_bytes(n) bytes (n / 8 more): the count also leaves the mask
+ * there, a bit a Bool, and the select does not read the mask again.  The two belong together: a
+ * temporary that rk_mask_count filled is not one for rk_mask_select_bits. */
+RK_API size_t  rk_mask_bits_tmp_bytes(int64_t n);
+RK_API int32_t rk_mask_count_bits(const uint8_t* mask, int64_t n, int64_t* count_out, void* tmp, size_t tmp_bytes,
+                           void* ws, size_t ws_bytes, void* stream);
+RK_API int32_t rk_mask_select_bits(int64_t n, const void* x, void* y, size_t elsize, int64_t nsel, const void* tmp,
+                            size_t tmp_bytes, void* stream);
 
 /* ---- reverse / reverse! -------------------------------------------------------------------
  * Replaces both `_reverse!` kernels of src/kernels/reverse.jl: out of place (`:59-88`, y != x)

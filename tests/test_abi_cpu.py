@@ -249,6 +249,24 @@ def test_volumerhs_and_scatter_validation(L):
     assert f(None, 1, L.shape_array((0,)), None, None, None, 0, None) == L.RK_SUCCESS
 
 
+def test_mask_bits_validation(L):
+    one, big = C.c_void_p(0x1000), C.c_void_p(0x100000)
+    mb, mc, ms = L.lib.rk_mask_bits_tmp_bytes, L.lib.rk_mask_count_bits, L.lib.rk_mask_select_bits
+    for n in (1, 4096, 4097, 1 << 24, (1 << 24) + 1, 1 << 26):
+        assert mb(n) - L.lib.rk_mask_tmp_bytes(n) == (n + 4095) // 4096 * 512
+    need = mb(5)
+    assert mb(0) == 256
+    assert mc(None, 5, one, big, need, big, 16 << 20, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert mc(one, 5, None, big, need, big, 16 << 20, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert mc(one, -1, one, big, need, big, 16 << 20, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert mc(one, 5, one, big, need - 1, big, 16 << 20, None) == L.RK_ERR_WORKSPACE
+    assert mc(one, 5, one, big, need, None, 0, None) == L.RK_ERR_WORKSPACE
+    assert ms(5, None, one, 4, 3, big, need, None) == L.RK_ERR_INVALID_ARGUMENT
+    assert ms(5, one, one, 3, 3, big, need, None) == L.RK_ERR_UNSUPPORTED
+    assert ms(5, one, one, 4, 3, big, need - 1, None) == L.RK_ERR_WORKSPACE
+    assert ms(5, None, None, 4, 0, None, 0, None) == L.RK_SUCCESS
+
+
 def test_a_sort_temporary_serves_every_smaller_sort(L):
     """What rk_sort_tmp_bytes asks for never falls as n grows, whichever way a sort of n keys takes, and is the same for the
     floats and the integers of a size."""

@@ -199,6 +199,36 @@ def test_mask_select_of_most_elements(rk, n, elsize, xoff, moff):
     assert (dy.cpu().numpy()[len(want):] == -7).all()
 
 
+@pytest.mark.parametrize("n", [1, 63, 4095, 4096, 4097, (1 << 24) - 1, (1 << 24) + 4097, (1 << 25) + 1])
+@pytest.mark.parametrize("elsize", [1, 4, 8])
+@pytest.mark.parametrize("share", [0.05, 0.45, 0.55])
+def test_mask_bits_of_the_count(rk, n, elsize, share):
+    """What the count leaves of a mask at an odd address with bytes other than 0 and 1, one, two and four tiles a wave, shares
+    around the lines between the two kernels, and the first and last element of every tile."""
+    import torch
+    from amdgpu_jl_amd import _lib as L
+    from amdgpu_jl_amd.array import stream_ptr, workspace
+    gen = torch.Generator(device="cuda").manual_seed(n + elsize)
+    dx = torch.randint(0, 256, (n * elsize,), dtype=torch.uint8, device="cuda", generator=gen)
+    mask = torch.randint(0, 128, (n + 1,), dtype=torch.uint8, device="cuda", generator=gen) * 2
+    m = torch.rand(n, device="cuda", generator=gen) < share
+    m[::4096] = True
+    m[4095::4096] = True
+    mask[1:] += m.to(torch.uint8)
+    want = dx.view(n, elsize)[m].reshape(-1)
+    tmp = torch.randint(0, 256, (int(L.lib.rk_mask_bits_tmp_bytes(n)),), dtype=torch.uint8, device="cuda", generator=gen)
+    total = torch.full((1,), -1, dtype=torch.int64, device="cuda")
+    ws, ws_bytes = workspace()
+    L.check(L.lib.rk_mask_count_bits(mask.data_ptr() + 1, n, total.data_ptr(), tmp.data_ptr(), tmp.numel(), ws, ws_bytes, stream_ptr()), "count")
+    nsel = int(total.item())
+    assert nsel * elsize == want.numel()
+    for short in (0, nsel // 3):                                   # a result that ends early
+        dy = torch.full((want.numel() + 16,), 0xA5, dtype=torch.uint8, device="cuda")
+        L.check(L.lib.rk_mask_select_bits(n, dx.data_ptr(), dy.data_ptr(), elsize, nsel - short, tmp.data_ptr(), tmp.numel(), stream_ptr()), "select")
+        end = (nsel - short) * elsize
+        assert torch.equal(dy[:end], want[:end]) and bool((dy[end:] == 0xA5).all())
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.int64])
 @pytest.mark.parametrize("hits", ["random", "runs of 10", "first quarter", "every second tile", "last element"])
 def test_mask_select_beyond_the_cache(rk, dtype, hits):
