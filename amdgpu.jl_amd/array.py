@@ -241,11 +241,18 @@ def _rescue_slot(slot) -> None:
     give_slot(slot)
 
 
-# What the words of a slot hold before a kernel writes them: no result that is met in practice, and one that it is all the same
-# only costs the wait for the stream.
+# What the words of a slot hold before a kernel writes them.  A result of 4 bytes or more that is the same all the same only costs the
+# wait for the stream; of 1 or 2 bytes it would be met every day, and the host does not look for these (scalar_words).
 _UNSET = 0x7ff4c0de5e1f1e55
 _UNSET_BYTES = np.full(SLOT_BYTES // 8, _UNSET, dtype=np.uint64).view(np.uint8)
 _WAIT_US = 200
+
+
+def scalar_words(dtype, more: int = 0) -> int:
+    """``words`` of ``fill_slot`` for a result of ``dtype`` in word 0, and the words ``more``.  None for results that a kernel writes as 1
+    or 2 bytes, every pattern of which is an ordinary value (of Bool two are): maximum of UInt8 that is 85 would wait 200 us in vain."""
+    dt = np.dtype(dtype)
+    return 1 | more if dt.itemsize >= 4 or dt == np.bool_ else 0
 
 
 def fill_slot(slot, fn, name, args, words: int = 0) -> None:

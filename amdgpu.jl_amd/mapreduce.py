@@ -14,7 +14,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib as L
-from .array import ROCArray, dtype_code, fill_slot, give_slot, stream_ptr, take_slot, workspace
+from .array import ROCArray, dtype_code, fill_slot, give_slot, scalar_words, stream_ptr, take_slot, workspace
 from .views import ROCView
 
 # f of mapreduce(f, op, A): enumerated, like the C ABI
@@ -222,7 +222,7 @@ def mapreduce(f, op: str, A: ROCArray, dims=None, init=None):
         # the kernel writes the value to pinned host memory: no result array, no copy
         slot = take_slot()
         fn, name, args = _dense_args(f, prog, op, A, dtype_code(out_dt), slot[0], init, out_dt, mask)
-        fill_slot(slot, fn, name, args, words=1)
+        fill_slot(slot, fn, name, args, words=scalar_words(out_dt))
         value = slot[1][:out_dt.itemsize].view(out_dt)[0].copy()
         give_slot(slot)
         return value
@@ -363,7 +363,7 @@ def _findminmax(A, want_max: bool, dims):
         slot = take_slot()
         fill_slot(slot, L.lib.rk_findminmax, "rk_findminmax",
                   (1 if want_max else 0, A.code, A.ptr, A.ndim, L.shape_array(A.dims), mask, slot[0], slot[0] + 16, ws, ws_bytes),
-                  words=1 | ((1 << A.ndim) - 1) << 2)
+                  words=scalar_words(A.dtype, ((1 << A.ndim) - 1) << 2))
         value = slot[1][:A.dtype.itemsize].view(A.dtype)[0].copy()
         c = tuple(int(v) for v in slot[1][16:16 + 8 * A.ndim].view(np.int64))
         give_slot(slot)
