@@ -143,12 +143,17 @@ RK_API int32_t rk_sort_status(const void* tmp, size_t tmp_bytes, void* stream);
 RK_API int32_t rk_accumulate_static_status(void* stream);
 
 /* ---- scalar results in host memory ------------------------------------------------
- * Results of rk_mapreduce, rk_findminmax, rk_mask_count and rk_mask_count_bits may lie in pinned host memory.  Such a result is written once, a
- * 64-bit word or less at a time, when the call has read all that it reads; the host can have it before the stream's
- * end is reported to it (no counterpart in the reference, which copies the result back).
+ * A call of rk_mapreduce, rk_findminmax, rk_mask_count or rk_mask_count_bits that has a single result may write it to pinned host
+ * memory.  It is written once, a 64-bit word or less at a time (of a result of 1, 2 or 4 bytes only these).  When all of its words are
+ * there -- of rk_findminmax the value and every coordinate: a coordinate alone says nothing -- the call has read its operand for the last
+ * time, and the host can have the result before the stream's end is reported to it (no counterpart in the reference, which
+ * copies the result back).  Nothing else has ended by then: ws, tmp and what the call left in them are in use until the stream
+ * gets past it.  Hand them on in stream order only; another stream, or memory that is freed outside of the stream's order, has to wait for the stream.
+ * Words of a call with several results say nothing about each other.
  *   rk_wait_words   waits until every word i of `base` with bit i of `mask` set differs from `unset`, which the caller has
  *                   put there before the call whose results they are; 1, or 0 if that takes longer than `us` microseconds
- *                   (then a word may also be `unset` as a result: wait for the stream).  Starts nothing and needs no device. */
+ *                   (then a word may also be `unset` as a result: wait for the stream.  Results of 1 and 2 bytes will be, now and then).
+ *                   Starts nothing and needs no device. */
 RK_API int32_t rk_wait_words(const void* base, uint32_t mask, uint64_t unset, int64_t us);
 
 /* ---- mapreduce ------------------------------------------------------------------
