@@ -28,7 +28,7 @@
 //                        workgroup that finishes last scans the chunk totals and the digit totals); the pass kernel gives
 //                        each XCD a contiguous eighth of the tiles.
 // Large sorts of floats run every pass (their digits are hardly ever constant) and do without the range read.
-//   sort_finish_kernel   moves the result of sort! into the caller's array when an odd number of passes ran, and a copy of the keys when none did
+//   sort_finish_kernel   moves the result of sort! into the caller's array when an odd number of passes ran
 //
 // Keys are mapped to unsigned integers that sort like Base.isless (-0.0 < 0.0, NaN last; sortperm makes every NaN the
 // canonical one so that they are equal keys, sort! keeps their bit patterns), complemented for rev=true; the mapping is
@@ -199,15 +199,16 @@ __device__ __forceinline__ bool digits_skewed(uint32_t d, bool valid) {
 constexpr int SORT_A = 0, SORT_B = 1, SORT_ENDS_IN_A = 2;
 __device__ __forceinline__ void sort_make_plan(SortCtl* ctl, int passes, bool relative, unsigned long long range, unsigned long long varying,
                                                int first_source) {
-    const auto skipped = [&](int p) {
-        const unsigned long long upto = p == 7 ? ~0ull : (1ull << (8 * (p + 1))) - 1ull;
-        return relative ? (range >> (8 * p)) == 0ull || (varying & upto) == 0ull : ((varying >> (8 * p)) & 0xffull) == 0ull;
-    };
-    uint32_t src_b = first_source == SORT_B ? 1u : 0u, nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
-    if (first_source == SORT_ENDS_IN_A)
-        for (int p = 0; p < passes; ++p) src_b ^= skipped(p) ? 0u : 1u;
+    uint32_t runs = 0u;                                      // a bit a pass
     for (int p = 0; p < passes; ++p) {
-        const bool skip = skipped(p);
+        const unsigned long long upto = p == 7 ? ~0ull : (1ull << (8 * (p + 1))) - 1ull;
+        const bool skip = relative ? (range >> (8 * p)) == 0ull || (varying & upto) == 0ull : ((varying >> (8 * p)) & 0xffull) == 0ull;
+        runs |= skip ? 0u : 1u << p;
+    }
+    uint32_t src_b = first_source == SORT_ENDS_IN_A ? (uint32_t)__popc(runs) & 1u : first_source == SORT_B ? 1u : 0u;
+    uint32_t nexec = 0, first = 0xffffffffu, last = 0xffffffffu;
+    for (int p = 0; p < passes; ++p) {
+        const bool skip = (runs >> p & 1u) == 0u;
         ctl->skip[p] = skip ? 1u : 0u;
         if (skip) continue;
         ctl->src_is_b[p] = src_b;
@@ -354,7 +355,8 @@ __global__ __launch_bounds__(RANGE_BLOCK) void sort_range_kernel(const T* __rest
 // aligned full tiles are read as 16-byte vectors.  One LDS atomic per key into one of SUB histograms per wave,
 // chosen by the lane: skewed digits (exponent bytes, the high bytes of small integers) then queue up 16 deep on a
 // counter instead of 64 deep, and no lane has to find out who else holds its digit.
-template <typename T, int BLOCK, int ITEMS, int SUB, typename C>
+// SEVERAL: tiles a workgroup, in turn.
+template <typename T, int BLOCK, int ITEMS, int SUB, typename C, bool SEVERAL = false>
 __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restrict__ orig, const typename SortKey<T>::U* buf_a,
                                                                 const typename SortKey<T>::U* buf_b, uint32_t n, int pass, int rev,
                                                                 SortCtl* ctl, C* __restrict__ tile_count) {
@@ -372,8 +374,7 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
     const U* in = first ? (const U*)orig : (step.src_b != 0u ? buf_b : buf_a);
     const U umin = (U)~step.inv_min;
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-    for (uint32_t tile = blockIdx.x; tile * (uint32_t)TILE < n; tile += gridDim.x) {
-        if (tile != blockIdx.x) __syncthreads();
+    for (uint32_t tile = blockIdx.x;;) {
         for (int i = tid; i < NW * SUB * 256; i += BLOCK) (&cnt[0][0])[i] = 0;
         const uint32_t e0 = tile * (uint32_t)TILE;
         const uint32_t woff = e0 + (uint32_t)wave * (WAVE * ITEMS) + lane;
@@ -440,6 +441,10 @@ __global__ __launch_bounds__(BLOCK, 8) void sort_upsweep_kernel(const T* __restr
             for (int w = 0; w < NW * SUB; ++w) c += cnt[w][tid];
             tile_count[(uint64_t)tile * 256 + tid] = (C)c;
         }
+        if (!SEVERAL) break;
+        tile += gridDim.x;
+        if (tile * (uint32_t)TILE >= n) break;
+        __syncthreads();
     }
 }
 
@@ -588,9 +593,12 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
     SortStep step{};
     if (pass >= 0) step = sort_step(ctl, pass);
     if (pass < 0 || step.skip != 0u) {
-        // all keys equal: no pass ran, and the last one writes the identity permutation
-        if (PERM && (first_of_few || pass == (int)sizeof(T) - 1) && ctl->nexec == 0u)
-            for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < (int64_t)n; i += (int64_t)gridDim.x * BLOCK) perm_out[i] = i + 1;
+        // all keys equal: no pass ran, and the last one writes the identity permutation, or the copy of the keys
+        if ((first_of_few || pass == (int)sizeof(T) - 1) && ctl->nexec == 0u && (PERM || (const void*)orig != (const void*)buf_a))
+            for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < (int64_t)n; i += (int64_t)gridDim.x * BLOCK) {
+                if (PERM) perm_out[i] = i + 1;
+                else ((T*)buf_a)[i] = orig[i];
+            }
         return;
     }
     const bool first = (uint32_t)pass == step.first_pass, last = (uint32_t)pass == step.last_pass;
@@ -796,14 +804,12 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
 }
 
 // ---- finish ------------------------------------------------------------------------------------------------------
-// sort! and sort: after an odd number of passes the result of sort! sits in buffer B, after none that of both in the caller's keys.
-// most: passes that may have run; keys that would have taken more were sorted in another way.  ends_in_a: the plan was made so.
+// sort!: after an odd number of passes the result sits in buffer B.
+// most: passes that may have run; keys that would have taken more were sorted in another way.
 template <typename W>
-__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, const W* orig, W* a, const W* b, int64_t nwords, uint32_t most, int ends_in_a) {
-    if (ctl->nexec > most) return;
-    const W* from = ctl->nexec == 0u ? orig : (ctl->nexec & 1u) != 0u && !ends_in_a ? b : a;
-    if (from == a) return;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords; i += (int64_t)gridDim.x * 256) a[i] = from[i];
+__global__ __launch_bounds__(256) void sort_finish_kernel(const SortCtl* ctl, W* a, const W* b, int64_t nwords, uint32_t most) {
+    if (ctl->nexec > most || (ctl->nexec & 1u) == 0u) return;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nwords; i += (int64_t)gridDim.x * 256) a[i] = b[i];
 }
 
 }  // namespace rk
@@ -1002,19 +1008,20 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
         uint32_t* chunk_prefix = (uint32_t*)(base + l.chunk_prefix_off);
         for (int i = 0; i < (l.split ? (int)SORT_FEW_PASSES : PASSES); ++i) {
             const int p = l.split ? -1 - i : i;
-            sort_upsweep_kernel<T, SORT_BLOCK, SORT_ITEMS, 4, uint32_t><<<ugrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
+            const auto count = [&](auto several) {
+                sort_upsweep_kernel<T, SORT_BLOCK, SORT_ITEMS, 4, uint32_t, decltype(several)::value><<<ugrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, (uint32_t)n, p, rev, ctl, counts);
+            };
+            const auto pass = [&](auto several) {
+                sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false, decltype(several)::value><<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, chunk_prefix, l.chunk_rows, l.ntiles, xcd_chunk);
+            };
+            constexpr bool MAY = sizeof(T) == 4 && !PERM;    // (l.quantiles needs)
+            if (MAY && l.quantiles) count(std::integral_constant<bool, MAY>{});
+            else count(std::false_type{});
             RK_LAUNCH_CHECK();
             sort_tilescan_kernel<<<l.nchunks, TS_BLOCK, 0, stream>>>(ctl, p, counts, l.ntiles, l.chunk_rows, chunk_total, chunk_prefix);
             RK_LAUNCH_CHECK();
-            const auto run = [&](auto kernel) {
-                kernel<<<pgrid, SORT_BLOCK, 0, stream>>>((const T*)keys, buf_a, buf_b, val_a, val_b, perm_out, (uint32_t)n, p, rev, ctl, counts, chunk_prefix, l.chunk_rows, l.ntiles, xcd_chunk);
-            };
-            if constexpr (sizeof(T) == 4 && !PERM) {
-                if (l.quantiles) run(sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false, true>);
-                else run(sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false>);
-            } else {
-                run(sort_pass_kernel<T, SORT_BLOCK, SORT_ITEMS, PERM, false>);
-            }
+            if (MAY && l.quantiles) pass(std::integral_constant<bool, MAY>{});
+            else pass(std::false_type{});
             RK_LAUNCH_CHECK();
         }
         if constexpr (sizeof(T) == 8) {
@@ -1024,15 +1031,15 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
             }
         }
     }
-    if (!PERM && (l.quantiles || !(all_passes && PASSES % 2 == 0))) {
+    if (!PERM && keys == sorted_out && (l.quantiles || !(all_passes && PASSES % 2 == 0))) {
         const uint32_t most = l.split ? SORT_FEW_PASSES : (uint32_t)PASSES;
         // whole 32-bit words: buffers are 256-byte padded, the caller's array is at least element-aligned; 16-bit keys
         // with an odd count copy one element more than n only inside buffer padding on the source side -- so copy by element there
         const int64_t nwords = sizeof(T) == 2 ? n : ((int64_t)n * (int64_t)sizeof(T) + 3) / 4;
         int64_t g = (nwords + 255) / 256;
         if (g > cus * 16) g = cus * 16;
-        if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint16_t*)keys, (uint16_t*)buf_a, (const uint16_t*)buf_b, nwords, most, first_source == SORT_ENDS_IN_A ? 1 : 0);
-        else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (const uint32_t*)keys, (uint32_t*)buf_a, (const uint32_t*)buf_b, nwords, most, first_source == SORT_ENDS_IN_A ? 1 : 0);
+        if (sizeof(T) == 2) sort_finish_kernel<uint16_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (uint16_t*)buf_a, (const uint16_t*)buf_b, nwords, most);
+        else sort_finish_kernel<uint32_t><<<(unsigned)g, 256, 0, stream>>>(ctl, (uint32_t*)buf_a, (const uint32_t*)buf_b, nwords, most);
         RK_LAUNCH_CHECK();
     }
     return RK_SUCCESS;
