@@ -8,7 +8,7 @@
 //   up to 2^26           keys of 8 bytes, and Float32 up to 2^22, go through two levels of splitters (rk_sort_split.hpp), unless they are
 //                        integers with three digits at most from the lowest that varies to the top of their range.
 //   up to 2^26           sort of more Float32, and of more than 2^23 Int32, moves the keys into buckets once (rk_sort_quantiles.hpp), unless a bucket
-//                        gets too large for that, or integers differ in one digit.
+//                        gets too large for that or has few values, or integers differ in one digit (two up to 2^25 keys).
 //   the others           the radix passes of this file:
 //   sort_init_kernel     clears the control block; no memset: graph-safe
 //   sort_range_kernel    one read of the keys: smallest and largest key (integers) and the bits that differ between keys;
@@ -962,8 +962,10 @@ static int32_t sort_typed(const void* keys, void* sorted_out, int64_t* perm_out,
     // sortperm: the first pass reads the caller's keys and writes buffer A.  sort: the last one writes the result, whatever their number
     // (a copy behind an odd number of them 85 us for 2^26 Float32); sort!: the keys lie where the result goes, so the first cannot.
     const int first_source = PERM ? SORT_B : keys != sorted_out ? SORT_ENDS_IN_A : SORT_A;
-    sort_init_kernel<<<1, 256, 0, stream>>>(ctl, all_passes ? PASSES : 0, first_source);
-    RK_LAUNCH_CHECK();
+    if (!(all_passes && l.quantiles)) {                      // (of those sq_sample_kernel does it)
+        sort_init_kernel<<<1, 256, 0, stream>>>(ctl, all_passes ? PASSES : 0, first_source);
+        RK_LAUNCH_CHECK();
+    }
     if (!all_passes) {
         constexpr int KVEC = 16 / (int)sizeof(T);
         int64_t head = (int64_t)(((16 - ((uintptr_t)keys & 15)) & 15) / sizeof(T));

@@ -3,29 +3,37 @@
 //
 //   sq_sample_kernel    fetches a sample of the keys, and its smallest and largest
 //   sq_table_kernel     counts the samples in SQ_CELLS equal cells between these; from there on, a key's bucket is the straight line
-//                       that its cell has for the share of smaller samples, in units of a bucket
+//                       that its cell has for the share of smaller samples, in units of a bucket.  Values in large numbers, and keys far from
+//                       all the others, get buckets of their own, and the cells cover the rest: a second launch, which else ends at once
 //   sq_count_kernel     the sizes of the buckets, by tile; of floats, which bits vary
 //   sq_offsets_kernel   where the buckets lie, and where the keys of each chunk of tiles go; decides
 //   sq_scatter_kernel   sorts every tile in LDS by bucket and writes its runs where they belong
 //   sq_bucket_kernel    a workgroup a bucket: its keys in registers, spread over bins, put in order in LDS, written once
 //
-// Every key is read three times and written twice, whatever its bits; four radix passes read it eight times and write it four times,
-// and match digits by ballots because they have to keep the order of what they move.  Here nothing has to: equal keys of sort are the
-// same bits, so a key's place is one LDS atomic.
+// Every key is read three times and written twice, of integers read once more in front (sort_range_kernel, 50 us of 2^26 keys), whatever its bits; four
+// radix passes read it eight times and write it four times, and match digits by ballots because they have to keep the order of what they
+// move.  Here nothing has to: equal keys of sort are the same bits, so a key's place is one LDS atomic.
 //
-// Radix passes -> so, us a call: sort Float32[2^23] 171 -> 126, [2^24] 241 -> 171, [2^26] 761 -> 447; Int32 of 32 bits [2^24] 263 -> 194,
-// [2^26] 810 -> 488, of 20 bits [2^24] 232 -> 187, [2^26] 738 -> 464.  The kernels of Float32[2^26]: 11 sample, 12 table, 50 count, 9 offsets, 147
-// scatter, 185 buckets; 512 MiB read and written are 81.  The scatter is bound by its writes, runs of ten keys on the average (with tiles
-// of 12288 keys and twice as many workgroups 181, 87 if nothing is written), the buckets by LDS and vector instructions in phases that one
-// workgroup a compute unit does not overlap.  The fewer bytes a key, the shorter the runs' lines: keys of 8 bytes, and sortperm, whose index
-// would travel along, take two levels of splitters (rk_sort_split.hpp).
-// Below 2^22 keys the launches count: Float32[2^22] 91 in rk_sort_split.hpp, 95 so.  Int32[2^22] of 8 bits, one radix pass and seven launches
-// for nothing more, 69 -> 76, [2^23] 94 -> 97, [2^24] 132 -> 127; of 32 bits [2^22] 147 -> 108, which the others would pay for.
+// Radix passes -> so, us a call: sort Float32[2^23] 172 -> 128, [2^24] 248 -> 171, [2^26] 758 -> 449; Int32 of 32 bits [2^24] 265 -> 196,
+// [2^26] 811 -> 489, of 20 bits [2^24] 234 -> 188, [2^26] 740 -> 460.  The kernels of Float32[2^26]: 8 sample, 18 table, 50 count, 8 offsets, 155
+// scatter, 190 buckets; 512 MiB read and written are 81.  By counters (profiles/sort_quantiles_sq_counters.txt) the count is bound by its vector
+// instructions, 20 a key.  The scatter and the buckets are neither: vector units busy 43 and 59 %, LDS 35 and 40 % of the time (half of that bank
+// conflicts), and over two fifths of a wave's time is waiting, in phases that one workgroup a compute unit does not overlap; the scatter also writes 367 MiB
+// for 256, runs of ten keys on the average (with tiles of 12288 keys and twice as many workgroups 181, 87 if nothing is written).  The fewer bytes a
+// key, the shorter the runs' lines: keys of 8 bytes, and sortperm, whose index would travel along, take two levels of splitters (rk_sort_split.hpp).
+// Below 2^22 keys the launches count: Float32[2^22] 91 in rk_sort_split.hpp, 95 so.  Int32[2^22] of 8 bits, one radix pass and eight launches
+// for nothing more, 69 -> 76, [2^23] 94 -> 96, [2^24] 132 -> 124; of 32 bits [2^22] 147 -> 108, which the others would pay for.
 //
-// If a bucket exceeds what its workgroup holds (SQ_CAP), as values in large numbers or narrow clusters make one, that is known before a
-// key is moved, mostly from the sample, and the radix passes run instead: their plan is there, or the plan says that none runs, and the
-// kernels of the other way end at once.  That costs them: Float32[2^26] of which nine in ten are zero 724 -> 852, of two values 711 -> 528 (digits
-// that do not vary are skipped now); Int32[2^26] of 100 ids with a number 735 -> 718.
+// Float32 around a number or with one in large numbers, radix passes / cells over the whole sampled range / so, us a call of 2^24 and of 2^26 keys: N(1000, 1) with
+// 0.1 % zeros 239 / 277 / 237 and 727 / 864 / 602; N(1013, 10) with 0.1 % NaN 241 / 282 / 225 and 734 / 878 / 542; N(20, 5) with 0.1 % -9999 239 / 209 / 225 and
+// 742 / 948 / 528; half zeros 248 / 289 / 212 and 743 / 885 / 505; nine in ten zeros 245 / 285 / 185 and 723 / 849 / 437.  Int32 ids with 0.01 % typemax
+// 265 / 741 / 217 and 777 / 1025 / 522.
+//
+// If a bucket exceeds what its workgroup holds (SQ_CAP) all the same, that is known before a key is moved, mostly from the sample, and the radix passes run
+// instead: their plan is there, or the plan says that none runs, and the kernels of the other way end at once.  So they do where the sample says that a bucket has
+// few values.  That costs them sample, table and launches, and above 2^24 keys passes whose workgroups take several tiles: Float32 of N(0, 1) rounded to 0.001
+// [2^24] 258 -> 294, [2^26] 776 -> 897; of 256 levels 242 -> 279, 719 -> 836; Int32 of a power law [2^24] 238 -> 284, of 16 bits [2^23] 120 -> 145,
+// [2^24] 164 -> 183, [2^26] 463 -> 497.
 #pragma once
 
 #include <cmath>
@@ -39,28 +47,48 @@ constexpr int64_t SQ_TILE = 6 * 4 * SQ_BLOCK;        // keys a tile: what LDS ho
 constexpr uint32_t SQ_CELLS = 4096;              // of the sampled range
 constexpr uint32_t SQ_MAX_K = 2560;              // buckets, a multiple of 64
 constexpr uint32_t SQ_GROUP = 16;                // neighbouring keys that are sampled together: a line of memory is fetched anyway
+// Samples a bucket: 512 take 3.5 + 2 us more of Float32[2^26] and make the buckets more alike, 186 for 190.
+constexpr uint32_t SQ_SAMPLES = 256;
 constexpr uint32_t SQ_SAMPLES_EACH = 4;          // samples a thread fetches
 constexpr uint32_t SQ_TABLE_GRID = 64;
 constexpr uint32_t SQ_CHUNKS = 512;              // of tiles, at most
 constexpr uint32_t SQ_CHUNK_TILES = 6;
 constexpr uint32_t SQ_COLUMNS = 64;              // buckets that a workgroup of sq_offsets_kernel takes
+constexpr uint32_t SQ_FREQUENT = 4;              // values in large numbers, at most: zeros, NaNs, a number that stands for a missing one
+constexpr uint32_t SQ_HEAVY = SQ_FREQUENT + 2u;  // and the two beyond which keys are few and far
 
 struct SqCtl {
     uint32_t lo, range, up;                      // a key's cell: the highest 12 bits of its distance from lo, at most range, << up
     uint32_t way;                                // SQ_BUCKETS ...
     uint32_t ok;                                 // the buckets fit
-    uint32_t ticket[2];
+    uint32_t ticket[3];
+    uint32_t heavies, heavy[SQ_HEAVY], heavy_bucket[SQ_HEAVY], heavy_size[SQ_HEAVY];       // values with a bucket of their own
 };
 // SQ_PLANNED: the radix passes run as they are planned: over all digits (floats), or over those that a read of all keys in front has found to
-// vary (integers); SQ_SOME_DIGITS: one bucket holds far too many of the samples, and floats get a plan after such a read.
+// vary (integers); SQ_SOME_DIGITS: one bucket holds far too many of the samples, or buckets hold few values, and floats get a plan after such a read.
 constexpr uint32_t SQ_BUCKETS = 0, SQ_PLANNED = 1, SQ_SOME_DIGITS = 2;
 constexpr uint32_t SQ_CHECKED = 16384;           // samples that are looked at for that
-constexpr uint32_t SQ_FEW_PASSES = 1;            // integers that differ in so few digits are sorted by radix passes
+// Values a bucket, on the average: with fewer the lanes of a wave meet on few counters in LDS (N(0, 1) rounded to 0.001, three values a bucket of 2^24
+// keys: the bucket kernel 281 us for 54, the call 404 for 294 by radix passes; five of 2^23: 288 and 212).
+constexpr uint32_t SQ_FEW_VALUES = 8;
+// Integers that differ in so few digits are sorted by radix passes, and those of fewer values than there are cells.  Two passes / buckets, 16 bits, us a
+// call: 2^24 keys 183 / 199, 2^25 285 / 287, 2^26 534 / 498; 1000 values 191 / 366, 296 / 484, 515 / 538.
+constexpr int64_t SQ_TWO_PASSES = (int64_t)1 << 25;
+inline uint32_t sq_few_passes(int64_t n) { return n <= SQ_TWO_PASSES ? 2u : 1u; }
 
 // What a cell holds: the share of the samples in front of it, in 65535ths, << 16, and its own.  With the place in the cell as a 16-bit
 // fraction that is one product, at most where the next cell starts: a key's share of the k buckets, in 2^-32.
-struct SqMap { uint32_t lo, range, up, k; };
-__device__ __forceinline__ SqMap sq_map(const SqCtl* ctl, uint32_t k) { return SqMap{ctl->lo, ctl->range, ctl->up, k << 8}; }
+// Keys beyond the ends count as these.  A heavy value stands in a bucket of its own, between those of the smaller and of the larger keys
+// of its place, which are two apart then; its keys are counted, not moved, and written by sq_bucket_kernel.
+struct SqMap { uint32_t lo, range, up, k, heavies, heavy[SQ_HEAVY]; };
+__device__ __forceinline__ uint32_t sq_lines(uint32_t k, uint32_t heavies) { return (heavies != 0u ? k - 2u * SQ_HEAVY : k) << 8; }
+__device__ __forceinline__ SqMap sq_map(const SqCtl* ctl, uint32_t k) {
+    const uint32_t heavies = sb_uniform(ctl->heavies);
+    SqMap m{ctl->lo, ctl->range, ctl->up, sq_lines(k, heavies), heavies, {}};
+#pragma unroll
+    for (uint32_t h = 0; h < SQ_HEAVY; ++h) m.heavy[h] = sb_uniform(ctl->heavy[h]);
+    return m;
+}
 
 __device__ __forceinline__ uint32_t sq_bucket(const uint32_t* cells, const SqMap& m, uint32_t key) {
     uint32_t t = __builtin_elementwise_sub_sat(key, m.lo);
@@ -69,6 +97,31 @@ __device__ __forceinline__ uint32_t sq_bucket(const uint32_t* cells, const SqMap
     uint32_t share;
     asm("v_mad_u32_u16 %0, %1, %2, %2" : "=v"(share) : "v"(t >> 4), "v"(cell));
     return (uint32_t)((uint64_t)(share >> 8) * (uint64_t)(m.k & 0xffffffu) >> 32);
+}
+
+// f(h, value) for every heavy value.
+template <typename F> __device__ __forceinline__ void sq_heavies(const SqMap& m, F&& f) {
+    static_assert(SQ_HEAVY == 6u, "");
+    if (m.heavies == 0u) return;
+    f(0, m.heavy[0]);
+    if (m.heavies == 1u) return;
+    f(1, m.heavy[1]);
+    if (m.heavies == 2u) return;
+    f(2, m.heavy[2]);
+    if (m.heavies == 3u) return;
+    f(3, m.heavy[3]);
+    if (m.heavies == 4u) return;
+    f(4, m.heavy[4]);
+    if (m.heavies == 5u) return;
+    f(5, m.heavy[5]);
+}
+
+// The buckets b[i] of the keys, as sq_bucket gives them, with those of the heavy values among them.
+template <int N> __device__ __forceinline__ void sq_around(const SqMap& m, const uint32_t (&key)[N], uint32_t (&b)[N]) {
+    sq_heavies(m, [&](int, uint32_t v) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) b[i] += (key[i] >= v ? 1u : 0u) + (key[i] > v ? 1u : 0u);
+    });
 }
 
 // enc_bits / dec_bits of sort and sort!, which keep the bit patterns of NaNs, without branches.  flip: all ones for rev=true.
@@ -94,11 +147,11 @@ template <typename T> __device__ __forceinline__ T& sq_at(T* p, uint32_t i) {
 // ---- sample -------------------------------------------------------------------------------------------------------
 // Groups of neighbouring keys from somewhere in each of equal stretches of the array.
 template <typename T>
-__global__ __launch_bounds__(SQ_BLOCK) void sq_sample_kernel(const T* __restrict__ keys, uint32_t n, uint32_t flip, const SortCtl* ctl, uint32_t* __restrict__ sample,
+__global__ __launch_bounds__(SQ_BLOCK) void sq_sample_kernel(const T* __restrict__ keys, uint32_t n, uint32_t flip, SortCtl* ctl, int first_source, uint32_t few_passes, uint32_t* __restrict__ sample,
                                                              uint2* __restrict__ ends, uint32_t* __restrict__ hist, SqCtl* sq) {
     __shared__ uint32_t part[2][SQ_BLOCK / WAVE];
     const uint32_t tid = threadIdx.x, groups = gridDim.x * (SQ_BLOCK * SQ_SAMPLES_EACH / SQ_GROUP);
-    const bool few = std::is_integral<T>::value && ctl->nexec <= SQ_FEW_PASSES;
+    const bool few = std::is_integral<T>::value && (ctl->nexec <= few_passes || (uint32_t)ctl->key_max - ~(uint32_t)ctl->inv_min < SQ_CELLS);
     if (blockIdx.x == 0u && tid == 0u) {
         SqCtl c{};
         c.way = few ? SQ_PLANNED : SQ_BUCKETS;
@@ -134,6 +187,14 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_sample_kernel(const T* __restrict
         }
         ends[blockIdx.x] = make_uint2(lo, hi);
     }
+    if (!std::is_integral<T>::value && blockIdx.x == 0u) {               // as sort_init_kernel
+        for (uint32_t i = tid; i < SORT_CTL_CLEAR; i += SQ_BLOCK) ctl->skip[i] = 0u;
+        __syncthreads();
+        if (tid == 0u) {
+            ctl->inv_min = ~0ull;
+            sort_make_plan(ctl, 4, false, 0ull, ~0ull, first_source);
+        }
+    }
 }
 
 // Adds one to the counter of each lane; lanes that go where the first one goes add together if they are many (values in large numbers).
@@ -150,40 +211,63 @@ __device__ __forceinline__ void sq_add(uint32_t* cnt, uint32_t c) {
 }
 
 // ---- the buckets' bounds ----------------------------------------------------------------------------------------------
+// Counts the samples in cells.  If a few values stand for many of the samples, or nearly all lie in few of the cells -- one NaN or zero among a
+// thousand values around 1000 leaves them two -- it says so, and the kernel runs again (REFINE) with these values apart and the cells where the keys
+// are: of 2^26 keys of N(1000, 1) 0.1 % zeros, or of N(1013, 10) 0.1 % NaN, are sorted by buckets then.
+template <bool REFINE>
 __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __restrict__ sample, uint32_t samples, const uint2* __restrict__ ends,
                                                             uint32_t nends, uint32_t offset, uint32_t k, uint32_t too_many, int floats, uint32_t* hist, uint32_t* __restrict__ cells, SqCtl* sq) {
     constexpr uint32_t PER = SQ_CELLS / SQ_BLOCK;
     __shared__ uint32_t h[SQ_CELLS], cnt[SQ_MAX_K];
-    __shared__ uint32_t part[3][SQ_BLOCK / WAVE], lds_ticket;
+    __shared__ uint32_t part[4][SQ_BLOCK / WAVE], lds_ticket;
+    constexpr uint32_t SQ_PICKS = 8;
+    __shared__ uint32_t found, end_cell[2], heavy_cell[SQ_FREQUENT], picked[SQ_FREQUENT], best[SQ_FREQUENT], pick[SQ_FREQUENT][SQ_PICKS];
     const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
-    if (sq->way == SQ_PLANNED) return;
-    uint32_t lo = ~0u, hi = 0u;
-    for (uint32_t i = tid; i < nends; i += SQ_BLOCK) {
-        const uint2 e = ends[i];
-        lo = e.x < lo ? e.x : lo;
-        hi = e.y > hi ? e.y : hi;
+    if (sq->way == SQ_PLANNED || (REFINE && sq->heavies == 0u)) return;
+    uint32_t lo = ~0u, hi = 0u, up = 0u;
+    SqMap map{};
+    if (REFINE) {
+        map = sq_map(sq, k);
+        lo = map.lo;
+        hi = lo + map.range;
+        up = map.up;
+    } else {
+        for (uint32_t i = tid; i < nends; i += SQ_BLOCK) {
+            const uint2 e = ends[i];
+            lo = e.x < lo ? e.x : lo;
+            hi = e.y > hi ? e.y : hi;
+        }
+        lo = wave_reduce(lo, OpMin());
+        hi = wave_reduce(hi, OpMax());
+        if (lane == 0u) { part[0][wave] = lo; part[1][wave] = hi; }
     }
-    lo = wave_reduce(lo, OpMin());
-    hi = wave_reduce(hi, OpMax());
-    if (lane == 0u) { part[0][wave] = lo; part[1][wave] = hi; }
 #pragma unroll
     for (uint32_t c = 0; c < PER; ++c) h[tid + c * SQ_BLOCK] = 0u;
     __syncthreads();
-    for (int w = 0; w < SQ_BLOCK / WAVE; ++w) {
-        lo = part[0][w] < lo ? part[0][w] : lo;
-        hi = part[1][w] > hi ? part[1][w] : hi;
-    }
     // Cells start where binades do: the density of floats halves or doubles there, which a line in the middle of a cell would not follow.
-    const auto bits_up = [](uint32_t range) { return range == 0u ? 31u : (uint32_t)__clz((int)range); };
-    uint32_t up = bits_up(hi - lo);
-    for (;; --up) {
-        const uint32_t most = up < 20u ? (1u << (20u - up)) - 1u : 0u, down = (lo + offset) & most;
-        const uint32_t from = down < lo ? lo - down : 0u;
-        if (bits_up(hi - from) >= up) { lo = from; break; }
+    const auto divide = [&]() {
+        const auto bits_up = [](uint32_t range) { return range == 0u ? 31u : (uint32_t)__clz((int)range); };
+        for (up = bits_up(hi - lo);; --up) {
+            const uint32_t most = up < 20u ? (1u << (20u - up)) - 1u : 0u, down = (lo + offset) & most;
+            const uint32_t from = down < lo ? lo - down : 0u;
+            if (bits_up(hi - from) >= up) { lo = from; break; }
+        }
+    };
+    if (!REFINE) {
+        for (int w = 0; w < SQ_BLOCK / WAVE; ++w) {
+            lo = part[0][w] < lo ? part[0][w] : lo;
+            hi = part[1][w] > hi ? part[1][w] : hi;
+        }
+        divide();
     }
     const uint32_t range = hi - lo;
+    const auto is_heavy = [&](uint32_t x) {
+        bool heavy = false;
+        sq_heavies(map, [&](int, uint32_t w) { heavy = heavy || x == w; });
+        return heavy;
+    };
     // The lanes of a wave are far apart in the array: of keys in order, neighbours would all add to one cell.
-    const uint32_t quads = samples / 4u / SQ_TABLE_GRID;                // (a multiple of 128)
+    const uint32_t quads = samples / 4u / SQ_TABLE_GRID;                // (a multiple of WAVE)
     const uint4* const mine = (const uint4*)sample + (size_t)blockIdx.x * quads + lane * (quads / WAVE);
     constexpr uint32_t UNR = 4;
     for (uint32_t i = wave; i < quads / WAVE; i += SQ_BLOCK / WAVE * UNR) {
@@ -193,10 +277,19 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __re
 #pragma unroll
         for (uint32_t u = 0; u < UNR; ++u) {
             if (i + u * (SQ_BLOCK / WAVE) >= quads / WAVE) continue;
-            sq_add(h, (v[u].x - lo) << up >> 20);
-            sq_add(h, (v[u].y - lo) << up >> 20);
-            sq_add(h, (v[u].z - lo) << up >> 20);
-            sq_add(h, (v[u].w - lo) << up >> 20);
+            if (!REFINE) {
+                sq_add(h, (v[u].x - lo) << up >> 20);
+                sq_add(h, (v[u].y - lo) << up >> 20);
+                sq_add(h, (v[u].z - lo) << up >> 20);
+                sq_add(h, (v[u].w - lo) << up >> 20);
+            } else {
+                const uint32_t x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t d = __builtin_elementwise_sub_sat(x[j], lo);
+                    if (!is_heavy(x[j])) atomicAdd(&h[(d < range ? d : range) << up >> 20], 1u);
+                }
+            }
         }
     }
     __syncthreads();
@@ -207,21 +300,136 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __re
     }
     publish_barrier();
     __syncthreads();
-    if (tid == 0u) lds_ticket = atomicAdd(&sq->ticket[0], 1u);
+    if (tid == 0u) lds_ticket = atomicAdd(&sq->ticket[REFINE ? 2 : 0], 1u);
     __syncthreads();
     if (lds_ticket != SQ_TABLE_GRID - 1u) return;
     // the last one
-    uint32_t c[PER], sum = 0u;
+    const auto scan = [&](const uint32_t (&c)[PER], uint32_t& all) {        // how many are in front of the thread's cells, and all of them
+        uint32_t sum = 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < PER; ++j) sum += c[j];
+        const uint32_t inc = wave_scan_inclusive(sum, OpAdd(), 0u);
+        __syncthreads();
+        if (lane == WAVE - 1) part[2][wave] = inc;
+        __syncthreads();
+        uint32_t before = inc - sum;
+        all = 0u;
+        for (uint32_t w = 0; w < SQ_BLOCK / WAVE; ++w) {
+            before += w < wave ? part[2][w] : 0u;
+            all += part[2][w];
+        }
+        return before;
+    };
+    uint32_t c[PER], all;
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) c[j] = load_agent(&hist[tid * PER + j]);
 #pragma unroll
-    for (uint32_t j = 0; j < PER; ++j) sum += c[j];
-    const uint32_t inc = wave_scan_inclusive(sum, OpAdd(), 0u);
-    if (lane == WAVE - 1) part[2][wave] = inc;
-    __syncthreads();
-    uint32_t before = inc - sum;
-    for (uint32_t w = 0; w < wave; ++w) before += part[2][w];
-    const auto share = [&](uint32_t x) { return (uint32_t)((uint64_t)x * 65535ull / samples); };
+    for (uint32_t j = 0; j < PER; ++j) h[tid * PER + j] = c[j];
+    uint32_t before = scan(c, all);
+    if constexpr (!REFINE) {
+        // the cells beyond which half a bucket's share of the samples lies
+        const auto find_ends = [&](uint32_t before, uint32_t all) {
+#pragma unroll
+            for (uint32_t j = 0; j < PER; ++j) {
+                const uint32_t behind = all - before - c[j];
+                if (before <= SQ_SAMPLES / 2u && before + c[j] > SQ_SAMPLES / 2u) end_cell[0] = tid * PER + j;
+                if (behind <= SQ_SAMPLES / 2u && behind + c[j] > SQ_SAMPLES / 2u) end_cell[1] = tid * PER + j;
+                before += c[j];
+            }
+        };
+        // whether these leave an eighth of the range or less
+        const auto few_cells = [&]() { return up < 20u && end_cell[0] <= end_cell[1] && end_cell[1] - end_cell[0] < SQ_CELLS / 8u; };
+        if (tid < SQ_FREQUENT) { picked[tid] = 0u; best[tid] = 0u; }
+        if (tid == 0u) { found = 0u; end_cell[0] = 0u; end_cell[1] = SQ_CELLS - 1u; }
+        __syncthreads();
+        find_ends(before, all);
+        // a cell far above its neighbours may hold such a value
+#pragma unroll
+        for (uint32_t j = 0; j < PER; ++j) {
+            const uint32_t at = tid * PER + j, beside = (at != 0u ? h[at - 1u] : 0u) + (at + 1u < SQ_CELLS ? h[at + 1u] : 0u);
+            if (c[j] >= beside + beside / 8u + SQ_SAMPLES / 2u) {
+                const uint32_t s = atomicAdd(&found, 1u);
+                if (s < SQ_FREQUENT) heavy_cell[s] = at;
+            }
+        }
+        __syncthreads();
+        const uint32_t heavy_cells = found <= SQ_FREQUENT ? found : 0u;
+        if (heavy_cells != 0u || few_cells()) {
+            const auto add_heavy = [&](uint32_t v) {
+                if (is_heavy(v)) return;
+#pragma unroll
+                for (uint32_t q = 0; q < SQ_HEAVY; ++q) map.heavy[q] = q == map.heavies ? v : map.heavy[q];
+                ++map.heavies;
+            };
+            if (heavy_cells != 0u) {
+                // it is what a third of up to eight of the cell's samples are, and more than one
+                constexpr uint32_t FROM = 4u * SQ_CHECKED, EACH = FROM / 4u / SQ_BLOCK;
+#pragma unroll 4
+                for (uint32_t u = 0; u < EACH; ++u) {
+                    const uint4 v = ((const uint4*)sample)[(lane * (FROM / 4u / WAVE) + u * (SQ_BLOCK / WAVE) + wave) * (samples / FROM)];
+                    const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        for (uint32_t s = 0; s < heavy_cells; ++s)
+                            if ((x[i] - lo) << up >> 20 == heavy_cell[s] && picked[s] < SQ_PICKS) {
+                                const uint32_t p = atomicAdd(&picked[s], 1u);
+                                if (p < SQ_PICKS) pick[s][p] = x[i];
+                            }
+                }
+                __syncthreads();
+                if (tid < heavy_cells && picked[tid] > SQ_PICKS) picked[tid] = SQ_PICKS;
+                __syncthreads();
+                const uint32_t s = tid / SQ_PICKS, p = tid % SQ_PICKS;
+                if (s < heavy_cells && p < picked[s]) {
+                    uint32_t same = 0u;
+                    for (uint32_t q = 0; q < SQ_PICKS; ++q) same += q < picked[s] && pick[s][q] == pick[s][p] ? 1u : 0u;
+                    atomicMax(&best[s], same << 8 | p);
+                }
+                __syncthreads();
+                if (tid < heavy_cells && (best[tid] >> 8 < 2u || (best[tid] >> 8) * 3u < picked[tid])) best[tid] = 0u;
+                if (tid == 0u) { end_cell[0] = 0u; end_cell[1] = SQ_CELLS - 1u; }
+                __syncthreads();
+                for (uint32_t t = 0; t < heavy_cells; ++t) {
+                    if (best[t] == 0u) continue;
+                    add_heavy(pick[t][best[t] & 0xffu]);
+#pragma unroll
+                    for (uint32_t j = 0; j < PER; ++j)           // what remains
+                        if (heavy_cell[t] == tid * PER + j) c[j] = (uint32_t)((uint64_t)c[j] * (picked[t] - (best[t] >> 8)) / picked[t]);
+                }
+                uint32_t all_of = all;
+                const uint32_t before_of = scan(c, all_of);
+                find_ends(before_of, all_of);
+                __syncthreads();
+            }
+            if (few_cells()) {
+                const uint32_t new_lo = lo + (end_cell[0] << (20u - up));
+                const uint64_t end = (uint64_t)lo + ((uint64_t)(end_cell[1] + 1u) << (20u - up)) - 1u;
+                const uint32_t new_hi = end < (uint64_t)hi ? (uint32_t)end : hi;
+                if (new_lo != 0u) add_heavy(new_lo - 1u);       // keys beyond are no neighbours of those in front: a bucket of both would not be spread
+                if (new_hi != ~0u) add_heavy(new_hi + 1u);
+                lo = new_lo;
+                hi = new_hi;
+                divide();
+            }
+            if (map.heavies != 0u) {
+#pragma unroll
+                for (uint32_t j = 0; j < PER; ++j) hist[tid * PER + j] = 0u;
+                if (tid != 0u) return;
+                sq->lo = lo;
+                sq->range = hi - lo;
+                sq->up = up;
+                sq->heavies = map.heavies;
+                for (uint32_t q = 0; q < SQ_HEAVY; ++q) sq->heavy[q] = map.heavy[q];
+                return;
+            }
+            // (c may be less by now)
+#pragma unroll
+            for (uint32_t j = 0; j < PER; ++j) c[j] = h[tid * PER + j];
+        }
+        map = SqMap{lo, range, up, sq_lines(k, 0u), 0u, {}};
+    }
+    const float per_sample = 65535.f / (float)(all != 0u ? all : 1u);
+    const auto share = [&](uint32_t x) { const uint32_t s = (uint32_t)((float)x * per_sample); return s < 65535u ? s : 65535u; };
     uint32_t at = share(before);
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) {
@@ -234,34 +442,70 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __re
     for (uint32_t b = tid; b < k; b += SQ_BLOCK) cnt[b] = 0u;
     constexpr uint32_t QUADS = SQ_CHECKED / 4u / SQ_BLOCK;
     const uint32_t stride = samples / 4u / (SQ_CHECKED / 4u), key0 = sample[0];
-    const SqMap map{lo, range, up, k << 8};
-    uint32_t varying = 0u, most = 0u;
+    uint32_t varying = 0u, most = 0u, others = 0u, first[QUADS], first_bucket[QUADS];
     __syncthreads();
 #pragma unroll
     for (uint32_t u = 0; u < QUADS; ++u) {
         const uint4 v = ((const uint4*)sample)[(lane * (SQ_CHECKED / 4u / WAVE) + u * (SQ_BLOCK / WAVE) + wave) * stride];
-        varying |= (v.x ^ key0) | (v.y ^ key0) | (v.z ^ key0) | (v.w ^ key0);
-        sq_add(cnt, sq_bucket(h, map, v.x));
-        sq_add(cnt, sq_bucket(h, map, v.y));
-        sq_add(cnt, sq_bucket(h, map, v.z));
-        sq_add(cnt, sq_bucket(h, map, v.w));
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+        uint32_t b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            varying |= x[i] ^ key0;
+            b[i] = sq_bucket(h, map, x[i]);
+        }
+        if constexpr (REFINE) sq_around(map, x, b);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (!REFINE) sq_add(cnt, b[i]);
+            else if (!is_heavy(x[i])) atomicAdd(&cnt[b[i]], 1u);
+            else b[i] = ~0u;
+        }
+        first[u] = x[0];
+        first_bucket[u] = b[0];
     }
     __syncthreads();
     for (uint32_t b = tid; b < k; b += SQ_BLOCK) most = cnt[b] > most ? cnt[b] : most;
+    // how many samples, of those that are not neighbours, equal one of their bucket; low half: how many are not that one
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < QUADS; ++u)
+        if (first_bucket[u] != ~0u) cnt[first_bucket[u]] = first[u];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < QUADS; ++u) others += first_bucket[u] != ~0u && cnt[first_bucket[u]] == first[u] ? 1u << 16 : 0u;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < QUADS; ++u)
+        if (first_bucket[u] != ~0u) cnt[first_bucket[u]] = u * SQ_BLOCK + tid;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t u = 0; u < QUADS; ++u)
+        if (first_bucket[u] != ~0u) others += cnt[first_bucket[u]] == u * SQ_BLOCK + tid ? 0u - (1u << 16) : 1u;
     most = wave_reduce(most, OpMax());
     varying = wave_reduce(varying, OpOr());
-    if (lane == 0u) { part[0][wave] = most; part[1][wave] = varying; }
+    others = wave_reduce(others, OpAdd());
+    if (lane == 0u) { part[0][wave] = most; part[1][wave] = varying; part[3][wave] = others; }
     __syncthreads();
     if (tid != 0u) return;
     for (int w = 1; w < SQ_BLOCK / WAVE; ++w) {
         most = part[0][w] > most ? part[0][w] : most;
         varying |= part[1][w];
+        others += part[3][w];
     }
     const bool all_vary = (varying & 0xffu) != 0u && (varying >> 8 & 0xffu) != 0u && (varying >> 16 & 0xffu) != 0u && varying >> 24 != 0u;
-    sq->lo = lo;
-    sq->range = range;
-    sq->up = up;
-    sq->way = most <= too_many ? SQ_BUCKETS : floats != 0 && !all_vary ? SQ_SOME_DIGITS : SQ_PLANNED;
+    const bool few_values = (others >> 16) * SQ_FEW_VALUES > (others & 0xffffu);
+    sq->lo = map.lo;
+    sq->range = map.range;
+    sq->up = map.up;
+    if constexpr (REFINE) {
+        for (uint32_t q = 0; q < SQ_HEAVY; ++q) {
+            uint32_t x[1] = {map.heavy[q]}, b[1] = {sq_bucket(h, map, x[0])};
+            sq_around(map, x, b);
+            sq->heavy_bucket[q] = q < map.heavies ? b[0] : ~0u;
+        }
+    }
+    sq->way = most <= too_many && !few_values ? SQ_BUCKETS : floats != 0 && !all_vary ? SQ_SOME_DIGITS : SQ_PLANNED;
 }
 
 // ---- tiles ----------------------------------------------------------------------------------------------------------
@@ -343,21 +587,34 @@ __global__ __launch_bounds__(SQ_BLOCK, 8) void sq_count_kernel(const T* __restri
     for (uint32_t b = tid; b < k; b += SQ_BLOCK) cnt[b] = 0u;
     for (uint32_t b = tid; b < k / 2u; b += SQ_BLOCK) row[0][b] = 0u;
     const uint32_t key0 = sq_enc<T>(__builtin_bit_cast(uint32_t, keys[0]), flip);
-    uint32_t varying = 0u;
+    uint32_t varying = 0u, heavy_count[SQ_HEAVY] = {};              // (of the wave)
     const auto add = [&](const SqTile<2>& t, auto&& has) {
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-            uint32_t b[4], r[4];
+            uint32_t x[4], b[4], r[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const uint32_t x = sq_enc<T>(t.key[4 * v + i], flip);       // (where there is none, the tile's first)
-                if (!INTEGERS) varying |= x ^ key0;
-                b[i] = x;
+                x[i] = sq_enc<T>(t.key[4 * v + i], flip);                   // (where there is none, the tile's first)
+                if (!INTEGERS) varying |= x[i] ^ key0;
             }
             if (way != SQ_BUCKETS) continue;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) b[i] = sq_bucket(table, map, b[i]);
-            sq_take(cnt, b, r, [&](int i) { return has(4 * v + i); });
+            for (int i = 0; i < 4; ++i) b[i] = sq_bucket(table, map, x[i]);
+            if (map.heavies == 0u) {
+                sq_take(cnt, b, r, [&](int i) { return has(4 * v + i); });
+                continue;
+            }
+            uint32_t gone = 0u;
+            sq_heavies(map, [&](int h, uint32_t w) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bool is = x[i] == w && has(4 * v + i);
+                    heavy_count[h] += (uint32_t)__popcll(__ballot(is));
+                    gone |= is ? 1u << i : 0u;
+                    b[i] += (x[i] >= w ? 1u : 0u) + (x[i] > w ? 1u : 0u);
+                }
+            });
+            sq_take(cnt, b, r, [&](int i) { return has(4 * v + i) && (gone >> i & 1u) == 0u; });
         }
     };
     __syncthreads();
@@ -384,6 +641,12 @@ __global__ __launch_bounds__(SQ_BLOCK, 8) void sq_count_kernel(const T* __restri
         }
     }
     __syncthreads();
+    if (map.heavies != 0u) {
+        sq_heavies(map, [&](int h, uint32_t) {
+            if (tid % WAVE == 0u) atomicAdd(&cnt[sq->heavy_bucket[h]], heavy_count[h]);
+        });
+        __syncthreads();
+    }
     for (uint32_t b = tid; b < k; b += SQ_BLOCK) totals[(size_t)blockIdx.x * k + b] = cnt[b];
     for (uint32_t b = tid; b < k / 2u; b += SQ_BLOCK) {
         for (uint32_t tile = t0; tile < t1; ++tile) rows[(size_t)tile * (k / 2u) + b] = row[tile - t0][b];
@@ -443,11 +706,22 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_offsets_kernel(uint32_t* totals, 
     if (way == SQ_BUCKETS && lds_ticket != gridDim.x - 1u) return;
     // the last one
     constexpr uint32_t PER = (SQ_MAX_K + SQ_BLOCK - 1u) / SQ_BLOCK;
+    const uint32_t heavies = sb_uniform(sq->heavies);
     uint32_t c[PER], total = 0u, most = 0u;
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) c[j] = tid * PER + j < k ? load_agent(&sizes[tid * PER + j]) : 0u;
 #pragma unroll
-    for (uint32_t j = 0; j < PER; ++j) { total += c[j]; most = c[j] > most ? c[j] : most; }
+    for (uint32_t j = 0; j < PER; ++j) {
+        total += c[j];
+        uint32_t size = c[j];
+        for (uint32_t h = 0; h < heavies; ++h)
+            if (tid * PER + j == sq->heavy_bucket[h]) {
+                sq->heavy_size[h] = size;
+                size = 0u;
+                sizes[tid * PER + j] = 0u;                   // (nothing to sort)
+            }
+        most = size > most ? size : most;
+    }
     uint32_t varying = 0u;
     for (uint32_t i = tid; floats != 0 && i < nchunks; i += SQ_BLOCK) varying |= seen[i];
     const uint32_t inc = wave_scan_inclusive(total, OpAdd(), 0u);
@@ -479,19 +753,14 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_offsets_kernel(uint32_t* totals, 
 // The sizes of a tile's buckets are known, so a key's place in the sorted tile is one addition in LDS.
 // Every workgroup takes a tile of every round of gridDim.x, neighbours on one XCD, whose runs meet in its L2; the keys of its next tile are
 // asked for when those of this one lie in LDS, before it is written.
-template <typename T>
-__global__ __launch_bounds__(SQ_BLOCK, 4) void sq_scatter_kernel(const T* keys, uint32_t n, uint32_t flip, uint32_t k, const uint32_t* __restrict__ cells,
-                                                                 uint32_t ntiles, uint32_t chunk_tiles, const uint16_t* __restrict__ rows,
-                                                                 const uint32_t* __restrict__ totals, const uint32_t* __restrict__ starts, const SqCtl* sq,
-                                                                 uint32_t* __restrict__ out) {
+// HEAVY: there are heavy values.
+template <typename T, bool HEAVY>
+__device__ __forceinline__ void sq_scatter_tiles(const T* keys, uint32_t n, uint32_t flip, uint32_t k, const uint32_t* __restrict__ cells, uint32_t ntiles, uint32_t chunk_tiles,
+                                                 const uint16_t* __restrict__ rows, const uint32_t* __restrict__ totals, const uint32_t* __restrict__ starts,
+                                                 const SqCtl* sq, uint32_t* __restrict__ out, uint32_t* lds_key, uint32_t* table, uint32_t* cnt, uint32_t* to) {
     constexpr uint32_t TILE = SQ_TILE, PER = (SQ_MAX_K + SQ_BLOCK - 1u) / SQ_BLOCK;
     constexpr int NV = SQ_TILE / (4 * SQ_BLOCK), ITEMS = 4 * NV;
-    __shared__ uint32_t lds_key[TILE];
-    __shared__ alignas(16) uint32_t table[SQ_CELLS];
-    __shared__ uint32_t cnt[SQ_MAX_K];           // of a bucket: where its next key goes in the tile
-    __shared__ uint32_t to[SQ_MAX_K];            // where its keys go, less where it starts in the tile
-    if (sq->ok == 0u) return;
-    const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const uint32_t tid = sq_again(threadIdx.x), lane = tid % WAVE, wave = tid / WAVE;
     const uint32_t tile0 = (blockIdx.x & 7u) * (gridDim.x / 8u) + (blockIdx.x >> 3), whole = n / TILE;
     if (tile0 >= ntiles) return;
     uint32_t* const part = lds_key;
@@ -509,16 +778,23 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_scatter_kernel(const T* keys, 
             before[j] = sq_at(total, b) + sq_at(row, b);
             with[j] = sq_at(total1, b) + sq_at(row, b + k);
         }
+        if (HEAVY) {                                         // (none of a heavy value's are moved)
+#pragma unroll
+            for (uint32_t h = 0; h < SQ_HEAVY; ++h)
+#pragma unroll
+                for (uint32_t j = 0; j < PER; ++j)
+                    if (tid * per + j == sq->heavy_bucket[h]) with[j] = before[j];
+        }
     };
     fetch_counts(tile0);
     if (tile0 < whole) t.template load<true>((const uint32_t*)keys + (size_t)tile0 * TILE, TILE);
-    const SqMap map = sq_map(sq, k);
+    const SqMap map = HEAVY ? sq_map(sq, k) : SqMap{sq->lo, sq->range, sq->up, k << 8, 0u, {}};
     for (uint32_t c = 4u * tid; c < SQ_CELLS; c += 4u * SQ_BLOCK) *(uint4*)&table[c] = *(const uint4*)&cells[c];
     uint32_t first[PER];
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) first[j] = sq_at(starts, tid * per + j < k ? tid * per + j : k - 1u);
     const auto scatter = [&](uint32_t count, uint32_t next, auto full) {
-        constexpr bool FULL = decltype(full)::value;
+        constexpr bool FULL = decltype(full)::value, ALL = FULL && !HEAVY;
         uint32_t sum = 0u;
 #pragma unroll
         for (uint32_t j = 0; j < PER; ++j) sum += j < per && tid * per + j < k ? with[j] - before[j] : 0u;
@@ -527,6 +803,11 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_scatter_kernel(const T* keys, 
         __syncthreads();
         uint32_t start = inc - sum;
         for (uint32_t w = 0; w < wave; ++w) start += part[w];
+        uint32_t moved = count;
+        if constexpr (HEAVY) {
+            moved = 0u;
+            for (uint32_t w = 0; w < SQ_BLOCK / WAVE; ++w) moved += part[w];
+        }
 #pragma unroll
         for (uint32_t j = 0; j < PER; ++j) {
             const uint32_t b = tid * per + j;
@@ -537,15 +818,25 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_scatter_kernel(const T* keys, 
 #pragma unroll
         for (int i0 = 0; i0 < ITEMS; i0 += 4) {
             uint32_t b[4], place[4];
+            [[maybe_unused]] bool gone[4] = {};              // of a heavy value
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 t.key[i0 + i] = sq_enc<T>(t.key[i0 + i], flip);
                 b[i] = sq_bucket(table, map, t.key[i0 + i]);
             }
-            sq_take(cnt, b, place, [&](int i) { return t.template has<FULL>(i0 + i, count); });
+            if constexpr (HEAVY) {
+                const uint32_t x[4] = {t.key[i0], t.key[i0 + 1], t.key[i0 + 2], t.key[i0 + 3]};
+                sq_around(map, x, b);
+                sq_heavies(map, [&](int, uint32_t w) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) gone[i] = gone[i] || x[i] == w;
+                });
+            }
+            const auto moves = [&](int i) { return t.template has<FULL>(i0 + i, count) && (!HEAVY || !gone[i]); };
+            sq_take(cnt, b, place, moves);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (t.template has<FULL>(i0 + i, count)) lds_key[place[i]] = t.key[i0 + i];
+                if (moves(i)) lds_key[place[i]] = t.key[i0 + i];
         }
         if (FULL) {
             t.template load<true>((const uint32_t*)keys + (size_t)(next < whole ? next : 0u) * TILE, TILE);
@@ -557,12 +848,20 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_scatter_kernel(const T* keys, 
         for (int i0 = 0; i0 < ITEMS; i0 += 4) {
             uint32_t x[4], at[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = lds_key[FULL || tid + (i0 + i) * SQ_BLOCK < count ? tid + (i0 + i) * SQ_BLOCK : 0u];
+            for (int i = 0; i < 4; ++i) x[i] = lds_key[ALL || tid + (i0 + i) * SQ_BLOCK < moved ? tid + (i0 + i) * SQ_BLOCK : 0u];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) at[i] = to[sq_bucket(table, map, x[i])] + tid + (i0 + i) * SQ_BLOCK;
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (HEAVY) at[i] = sq_bucket(table, map, x[i]);
+                else at[i] = to[sq_bucket(table, map, x[i])] + tid + (i0 + i) * SQ_BLOCK;
+            }
+            if constexpr (HEAVY) {
+                sq_around(map, x, at);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) at[i] = to[at[i]] + tid + (i0 + i) * SQ_BLOCK;
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (FULL || tid + (i0 + i) * SQ_BLOCK < count) sq_at(out, at[i]) = x[i];
+                if (ALL || tid + (i0 + i) * SQ_BLOCK < moved) sq_at(out, at[i]) = x[i];
         }
         __syncthreads();
     };
@@ -572,6 +871,20 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_scatter_kernel(const T* keys, 
         t.template load<false>((const uint32_t*)keys + (size_t)tile * TILE, n - tile * TILE);
         scatter(n - tile * TILE, 0u, std::false_type{});
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(SQ_BLOCK, 4) void sq_scatter_kernel(const T* keys, uint32_t n, uint32_t flip, uint32_t k, const uint32_t* __restrict__ cells,
+                                                                 uint32_t ntiles, uint32_t chunk_tiles, const uint16_t* __restrict__ rows,
+                                                                 const uint32_t* __restrict__ totals, const uint32_t* __restrict__ starts, const SqCtl* sq,
+                                                                 uint32_t* __restrict__ out) {
+    __shared__ uint32_t lds_key[SQ_TILE];
+    __shared__ alignas(16) uint32_t table[SQ_CELLS];
+    __shared__ uint32_t cnt[SQ_MAX_K];           // of a bucket: where its next key goes in the tile
+    __shared__ uint32_t to[SQ_MAX_K];            // where its keys go, less where it starts in the tile
+    if (sq->ok == 0u) return;
+    if (sq->heavies == 0u) sq_scatter_tiles<T, false>(keys, n, flip, k, cells, ntiles, chunk_tiles, rows, totals, starts, sq, out, lds_key, table, cnt, to);
+    else sq_scatter_tiles<T, true>(keys, n, flip, k, cells, ntiles, chunk_tiles, rows, totals, starts, sq, out, lds_key, table, cnt, to);
 }
 
 // ---- a bucket ---------------------------------------------------------------------------------------------------------
@@ -597,7 +910,8 @@ template <int FROM> __device__ __forceinline__ void sq_network(uint32_t (&x)[16]
     }
 }
 
-// In memory, by one workgroup: radix passes of 8 bits over the distance from the smallest key.  Of a bucket that bins do not spread.
+// In memory, by one workgroup: radix passes of 8 bits over the distance from the smallest key.  Of a bucket that bins do not spread: a step of
+// a wave is four loads that are asked for while the step in front is worked on.
 // a: the keys; b: as much room.  Returns whether the sorted keys are in b.
 __device__ bool sq_radix(uint32_t* a, uint32_t* b, uint32_t m, uint32_t lo, uint32_t bits, uint32_t* cnt, uint32_t* wsum) {
     constexpr uint32_t NW = SQ_BLOCK / WAVE;
@@ -612,22 +926,43 @@ __device__ bool sq_radix(uint32_t* a, uint32_t* b, uint32_t m, uint32_t lo, uint
         for (uint32_t i = tid; i < NW * 256u; i += SQ_BLOCK) cnt[i] = 0u;
         __syncthreads();
         for (int move = 0; move < 2; ++move) {
-            for (uint32_t e0 = first; e0 < end; e0 += WAVE) {
-                const bool valid = e0 + lane < end;
-                const uint32_t x = valid ? src[e0 + lane] : 0u, d = (x - lo) >> shift & 0xffu;
-                uint32_t same_lo, same_hi;
-                match_digit_halves(d, same_lo, same_hi);
-                const uint64_t vm = __ballot(valid);
-                same_lo &= (uint32_t)vm;
-                same_hi &= (uint32_t)(vm >> 32);
-                const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
-                const uint32_t at = __hip_atomic_load(&wcnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) + below;
-                __builtin_amdgcn_wave_barrier();
-                if (valid && below == 0u)
-                    __hip_atomic_fetch_add(&wcnt[d], (uint32_t)__builtin_popcount(same_lo) + (uint32_t)__builtin_popcount(same_hi), __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WAVEFRONT);
-                __builtin_amdgcn_wave_barrier();
-                if (move != 0 && valid) dst[at] = x;
+            constexpr int U = 4;
+            uint32_t next[U];
+            const auto fetch = [&](uint32_t e0) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) next[u] = e0 + u * WAVE + lane < end ? src[e0 + u * WAVE + lane] : 0u;
+            };
+            fetch(first);
+            for (uint32_t e0 = first; e0 < end; e0 += U * WAVE) {
+                uint32_t x[U], at[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) x[u] = next[u];
+                fetch(e0 + U * WAVE);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const bool valid = e0 + u * WAVE + lane < end;
+                    const uint32_t d = (x[u] - lo) >> shift & 0xffu;
+                    if (move == 0) {
+                        if (valid) atomicAdd(&wcnt[d], 1u);
+                        continue;
+                    }
+                    uint32_t same_lo, same_hi;
+                    match_digit_halves(d, same_lo, same_hi);
+                    const uint64_t vm = __ballot(valid);
+                    same_lo &= (uint32_t)vm;
+                    same_hi &= (uint32_t)(vm >> 32);
+                    const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
+                    at[u] = __hip_atomic_load(&wcnt[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) + below;
+                    __builtin_amdgcn_wave_barrier();
+                    if (valid && below == 0u)
+                        __hip_atomic_fetch_add(&wcnt[d], (uint32_t)__builtin_popcount(same_lo) + (uint32_t)__builtin_popcount(same_hi), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WAVEFRONT);
+                    __builtin_amdgcn_wave_barrier();
+                }
+                if (move == 0) continue;
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (e0 + u * WAVE + lane < end) dst[at[u]] = x[u];
             }
             __syncthreads();
             if (move != 0) continue;
@@ -656,7 +991,7 @@ __device__ bool sq_radix(uint32_t* a, uint32_t* b, uint32_t m, uint32_t lo, uint
 
 constexpr int SQ_VECTORS = 12;
 constexpr uint32_t SQ_CAP = 4u * SQ_VECTORS * SQ_BLOCK, SQ_BINS = 8192, SQ_SLOTS = 31936;
-constexpr uint32_t SQ_ROUNDS = 320;
+constexpr uint32_t SQ_ROUNDS = 64;             // of merges, at most: sq_radix takes about as long
 
 // Where the 4 slots q lie, and slot s: lanes that each read 16 neighbours, 4 at a time, read different banks.  (Slots stay among their 16.)
 __device__ __forceinline__ uint32_t sq_quad(uint32_t q) { return q ^ (q >> 4 & 3u); }
@@ -754,16 +1089,26 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_bucket_kernel(uint32_t* in, co
             const float width = __builtin_bit_cast(float, sq_dec<T>(hi, flip)) - value_lo;
             per_value = (float)BINS * (1.f - 0x1p-20f) / width;
             if (span > 3u << 23 && __builtin_fabsf(width) < __builtin_inff() && __builtin_fabsf(per_value) < __builtin_inff()) {
-                // which of the two spreads the first row better, over 64 bins
+                // which of the two spreads the first row better, over an eighth of the bins (over 64 of them a few keys at one place do not show: of 2^24
+                // keys of N(0, 1) 1 % of which are a million times as large, one bucket made the call 379 us for 176)
                 uint32_t* const coarse = slot;
-                if (tid < 128u) coarse[tid] = 0u;
+                coarse[tid] = coarse[SQ_BLOCK + tid] = 0u;
                 __syncthreads();
                 if (has(0)) {
-                    atomicAdd(&coarse[(uint32_t)((float)(t.key[0] - lo) * per_key) / (BINS / 64u)], 1u);
-                    atomicAdd(&coarse[64u + (uint32_t)((__builtin_bit_cast(float, sq_dec<T>(t.key[0], flip)) - value_lo) * per_value) / (BINS / 64u)], 1u);
+                    atomicAdd(&coarse[(uint32_t)((float)(t.key[0] - lo) * per_key) / (BINS / SQ_BLOCK)], 1u);
+                    atomicAdd(&coarse[SQ_BLOCK + (uint32_t)((__builtin_bit_cast(float, sq_dec<T>(t.key[0], flip)) - value_lo) * per_value) / (BINS / SQ_BLOCK)], 1u);
                 }
                 __syncthreads();
-                by_value = sb_uniform(wave_reduce(coarse[64u + lane], OpMax())) < sb_uniform(wave_reduce(coarse[lane], OpMax()));
+                const uint32_t by_bits = wave_reduce(coarse[tid], OpMax()), by_val = wave_reduce(coarse[SQ_BLOCK + tid], OpMax());
+                if (lane == 0u) { part[2][wave] = by_bits; part[3][wave] = by_val; }
+                __syncthreads();
+                uint32_t most_bits = 0u, most_val = 0u;
+#pragma unroll 4
+                for (int w = 0; w < NW; ++w) {
+                    most_bits = part[2][w] > most_bits ? part[2][w] : most_bits;
+                    most_val = part[3][w] > most_val ? part[3][w] : most_val;
+                }
+                by_value = sb_uniform(most_val) < sb_uniform(most_bits);
             }
         }
         const auto with_bins = [&](auto&& run) {
@@ -935,12 +1280,26 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_bucket_kernel(uint32_t* in, co
         }
         uint32_t* const mine = in + start;
         uint32_t* const other = (uint32_t*)out + start;
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) t.key[i] = 0u;      // (needs their registers)
         const bool there = sq_radix(mine, other, m, lo, sb_bits(span), bins, part[0]);
         for (uint32_t i = tid; i < m; i += SQ_BLOCK) out[start + i] = __builtin_bit_cast(T, sq_dec<T>(there ? other[i] : mine[i], flip));
         __syncthreads();
         clear_bins();
         return false;
     };
+    const uint32_t heavies = sq->heavies;
+    for (uint32_t h = 0; h < heavies; ++h) {
+        const uint32_t b = sq->heavy_bucket[h], m = sq->heavy_size[h], v = sq_dec<T>(sq->heavy[h], flip);
+        uint32_t* const to = (uint32_t*)out + starts[b];
+        const uint32_t to_line = (0u - (uint32_t)((uintptr_t)to >> 2)) & 3u, head = to_line < m ? to_line : m, quads = (m - head) / 4u;
+        typename VecOf<uint32_t, 4>::type o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = v;
+        for (uint32_t q = blockIdx.x * SQ_BLOCK + tid; q < quads; q += gridDim.x * SQ_BLOCK) store_nt((typename VecOf<uint32_t, 4>::type*)(to + head + 4u * q), o);
+        if (blockIdx.x == h && tid < head) to[tid] = v;
+        if (blockIdx.x == h && tid < m - head - 4u * quads) to[head + 4u * quads + tid] = v;
+    }
     uint32_t bucket = blockIdx.x, start = sb_uniform(starts[bucket]), m = sb_uniform(sizes[bucket]);
     fetch(start, m);
     clear_bins();
@@ -957,6 +1316,8 @@ __global__ __launch_bounds__(SQ_BLOCK, 4) void sq_bucket_kernel(uint32_t* in, co
 }
 
 // ---- host --------------------------------------------------------------------------------------------------------
+// The most keys: 2560 buckets and a tile are what fits LDS with the cells here (132 of 160 KiB in the scatter; the count keeps the counters of six tiles), and their runs
+// are ten keys.  One more takes the radix passes, 758 us for 449; larger tiles or buckets were not tried.
 constexpr int64_t SQ_MIN_INTEGERS = (int64_t)1 << 23, SQ_MAX_KEYS = (int64_t)1 << 26;
 constexpr int64_t SQ_MEAN = 26624;                         // keys a bucket, at most: 1.2 times as many lie in LDS at a time
 constexpr int64_t SQ_ROUND = 256;                          // buckets: a multiple of a workgroup a compute unit
@@ -975,7 +1336,7 @@ static SqLayout sq_layout(size_t off, int64_t n) {
     l.nchunks = (l.ntiles + l.chunk_tiles - 1u) / l.chunk_tiles;
     const float fit = (float)SQ_CAP * (float)SQ_CHECKED / (float)n;            // of the samples that are looked at, those of a bucket that just fits
     l.too_many = (uint32_t)(fit + 4.f * std::sqrt(fit));
-    l.sample_grid = l.k / 8u;                                // 512 samples a bucket
+    l.sample_grid = l.k / (SQ_BLOCK * SQ_SAMPLES_EACH / SQ_SAMPLES);
     const uint32_t k = l.k;
     const auto take = [&](size_t bytes) { const size_t at = off; off += (bytes + 255) & ~(size_t)255; return at; };
     l.sq_off = take(sizeof(SqCtl));
@@ -1008,11 +1369,14 @@ static int32_t sort_quantiles(const SqLayout& l, const void* keys, void* sorted_
     const uint32_t k = l.k;
     const uint32_t cus = (uint32_t)device_info().cus, resident = cus / 8u * 8u;
     const int floats = std::is_integral<T>::value ? 0 : 1;
-    sq_sample_kernel<T><<<l.sample_grid, SQ_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, flip, ctl, moved, ends, hist, sq);
+    sq_sample_kernel<T><<<l.sample_grid, SQ_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, flip, ctl, first_source, sq_few_passes(n), moved, ends, hist, sq);
     RK_LAUNCH_CHECK();
     // from a key to the number whose multiples of 2^23 are binades
     const uint32_t offset = std::is_integral<T>::value ? 0u : flip != 0u ? 1u - 0x007fffffu : 0x007fffffu;
-    sq_table_kernel<<<SQ_TABLE_GRID, SQ_BLOCK, 0, stream>>>(moved, l.sample_grid * SQ_BLOCK * SQ_SAMPLES_EACH, ends, l.sample_grid, offset, k, l.too_many, floats, hist, cells, sq);
+    const uint32_t samples = l.sample_grid * SQ_BLOCK * SQ_SAMPLES_EACH;
+    sq_table_kernel<false><<<SQ_TABLE_GRID, SQ_BLOCK, 0, stream>>>(moved, samples, ends, l.sample_grid, offset, k, l.too_many, floats, hist, cells, sq);
+    RK_LAUNCH_CHECK();
+    sq_table_kernel<true><<<SQ_TABLE_GRID, SQ_BLOCK, 0, stream>>>(moved, samples, ends, l.sample_grid, offset, k, l.too_many, floats, hist, cells, sq);
     RK_LAUNCH_CHECK();
     sq_count_kernel<T><<<l.nchunks, SQ_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, flip, k, cells, l.ntiles, l.chunk_tiles, (uint32_t*)rows, totals, seen, sq);
     RK_LAUNCH_CHECK();

@@ -471,11 +471,16 @@ def test_sorts_by_quantiles(rk, dtype, kind):
         _device_sort_check(rk, np.ascontiguousarray(x.astype(dtype)), (False, True) if n == n0 else (False,))
 
 
+def _moved_into_buckets(rk, x):
+    """Whether a sort of the keys went through buckets: it leaves a number of passes that none has."""
+    return _passes_run(rk, x, False)[0] == 0xffffffff
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.int32])
 @pytest.mark.parametrize("near,width", [(1000, 1), (9000, 1), (15000, 64), (20000, 1), (18000, 8192), (60000, 1)])
 def test_bucket_with_a_cluster(rk, dtype, near, width):
-    """`near` keys among `width` times the values of a bin, in one bucket: many rounds of merges, bins that are sorted in memory, keys that lie
-    in LDS half a bucket at a time, and more than a bucket may have."""
+    """`near` keys among `width` times the values of a bin: many rounds of merges, bins that are sorted in memory, and a cluster that is larger than
+    a bucket may be, which a value of its own or the radix passes take."""
     rng = np.random.default_rng(near)
     n = QUANTILES[dtype] + 12345
     span = 1 << 30 if dtype == np.int32 else 1 << 22     # of Float32: of the bits of one binade, so that cells are lines of equal slope
@@ -485,6 +490,37 @@ def test_bucket_with_a_cluster(rk, dtype, near, width):
     x[rng.choice(n, near, replace=False)] = at + rng.integers(0, max(2, min(bucket // 8192 * width, bucket)), near)
     x = (x + (127 << 23)).astype(np.uint32).view(np.float32) if dtype == np.float32 else x.astype(np.int32)
     _device_sort_check(rk, x, (False,))
+
+
+SENTINELS = {                                            # keys around a number, a share of them replaced
+    "zeros": (1000, 1, 0.001, (0,)), "few zeros": (300, 10, 0.0001, (0,)), "missing": (20, 5, 0.03, (-9999,)), "nine in ten": (0, 1, 0.9, (0,)),
+    "four": (20, 5, 0.3, (-9999, 0, 1e6, 2e6)), "half": (0, 1, 0.5, (0.25,)), "nothing else": (0, 1, 1.0, (7, 70_000, 1 << 20))}
+
+
+@pytest.mark.parametrize("dtype,kind", [(t, k) for t in (np.float32, np.int32) for k in SENTINELS] + [(np.float32, "NaN"), (np.float32, "infinities")])
+def test_sorts_of_keys_with_a_value_in_large_numbers(rk, orc, dtype, kind):
+    """A few values that stand for many keys, or that lie far from all the others: they have buckets of their own, the table covers the rest, and
+    the keys are moved once."""
+    rng = np.random.default_rng(43)
+    for n in (QUANTILES[dtype], 24576 * 344 + 1):
+        mean, width, share, values = SENTINELS.get(kind, (1013, 10, 0.03, (np.nan,) if kind == "NaN" else (np.inf, -np.inf, np.nan)))
+        x = mean + width * rng.standard_normal(n)
+        if dtype == np.int32:
+            x *= 100_000                                 # (three digits and more)
+        at = rng.random(n) < share
+        x[at] = rng.choice(np.array(values), int(at.sum()))
+        x = x.astype(dtype)
+        x[x == 0] = 0
+        assert _moved_into_buckets(rk, x), n
+        if kind not in ("NaN", "infinities"):
+            _device_sort_check(rk, x, (False, True))
+            continue
+        for rev in (False, True):
+            want = orc.sort(x, rev)
+            y = rk.ROCArray(x)
+            assert np.array_equal(rk.Array(rk.sort(y, rev=rev)).view(np.uint32), want.view(np.uint32))
+            rk.sort_(y, rev=rev)
+            assert np.array_equal(rk.Array(y).view(np.uint32), want.view(np.uint32))
 
 
 @pytest.mark.parametrize("n", [1 << 24, 1 << 25, (1 << 26) - 24575, 1 << 26, (1 << 26) + 1])
