@@ -492,6 +492,23 @@ def test_bucket_with_a_cluster(rk, dtype, near, width):
     _device_sort_check(rk, x, (False,))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.int32])
+@pytest.mark.parametrize("near,values", [(36000, 40), (40000, 40), (36000, 20000), (40000, 200)])
+def test_bucket_that_does_not_fit_one_window(rk, dtype, near, values):
+    """A cluster inside one cell, of more keys than lie in LDS at a time (31920) and fewer than a bucket's workgroup holds (49152), none of its values
+    frequent: 20000 neighbours spread over many bins are sorted a window after the other; of 40 in one bin or two, or 200 in few, a bin exceeds half a window,
+    and the bucket is sorted in memory."""
+    rng = np.random.default_rng(near + values)
+    n = QUANTILES[dtype] + 12345
+    span = 1 << 30 if dtype == np.int32 else 1 << 27     # (of Float32: of their bits, 16 binades)
+    x = rng.integers(0, span, n)
+    at = span // 4096 * 1365 + span // 16384             # in the middle of a cell, away from a bucket's end
+    x[rng.choice(n, near, replace=False)] = at + rng.integers(0, values, near)
+    x = (x + (120 << 23)).astype(np.uint32).view(np.float32) if dtype == np.float32 else x.astype(np.int32)
+    assert _moved_into_buckets(rk, x)
+    _device_sort_check(rk, x)
+
+
 SENTINELS = {                                            # keys around a number, a share of them replaced
     "zeros": (1000, 1, 0.001, (0,)), "few zeros": (300, 10, 0.0001, (0,)), "missing": (20, 5, 0.03, (-9999,)), "nine in ten": (0, 1, 0.9, (0,)),
     "four": (20, 5, 0.3, (-9999, 0, 1e6, 2e6)), "half": (0, 1, 0.5, (0.25,)), "nothing else": (0, 1, 1.0, (7, 70_000, 1 << 20))}
@@ -521,6 +538,31 @@ def test_sorts_of_keys_with_a_value_in_large_numbers(rk, orc, dtype, kind):
             assert np.array_equal(rk.Array(rk.sort(y, rev=rev)).view(np.uint32), want.view(np.uint32))
             rk.sort_(y, rev=rev)
             assert np.array_equal(rk.Array(y).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int32])
+def test_sorts_by_quantiles_with_a_sample_that_misleads(rk, dtype):
+    """The keys that are sampled are spread and larger than nearly all the others, which go to the first bucket: the sample says that the buckets
+    fit, the count that they do not, and nothing has been moved yet.  The rule of the sample is that of the source, so that a change there shows here."""
+    import pathlib
+    text = (pathlib.Path(__file__).parent.parent / "amdgpu.jl_amd" / "csrc" / "rk_sort_quantiles.hpp").read_text()
+    for line in ("constexpr uint32_t SQ_GROUP = 16;", "uint32_t h = (g + 1u) * 0x9e3779b1u;", "h ^= h >> 15;", "h *= 0x85ebca77u;",
+                 "keys[a + __umulhi(h, b - a - (SQ_GROUP - 1u)) + s % SQ_GROUP]", "constexpr uint32_t SQ_SAMPLES = 256;", "constexpr uint32_t SQ_SAMPLES_EACH = 4;", "constexpr int64_t SQ_MEAN = 26624;"):
+        assert line in text, line
+    rng = np.random.default_rng(44)
+    n = QUANTILES[dtype] + 54321
+    groups = -(-n // (256 * 26624)) * 256 * 256 // 16
+    g, m = np.arange(groups, dtype=np.uint64), np.uint64(0xffffffff)
+    a, b = g * np.uint64(n) // np.uint64(groups), (g + np.uint64(1)) * np.uint64(n) // np.uint64(groups)
+    h = (g + np.uint64(1)) * np.uint64(0x9e3779b1) & m
+    h ^= h >> np.uint64(15)
+    h = h * np.uint64(0x85ebca77) & m
+    at = ((a + (h * (b - a - np.uint64(15)) >> np.uint64(32)))[:, None] + np.arange(16, dtype=np.uint64)).reshape(-1).astype(np.int64)
+    x = rng.integers(0, 1 << 20, n)
+    x[at] = (1 << 24) + rng.integers(0, 1 << 24, at.size)
+    x = (x * 1.5).astype(np.float32) if dtype == np.float32 else x.astype(np.int32)
+    assert not _moved_into_buckets(rk, x)
+    _device_sort_check(rk, x)
 
 
 @pytest.mark.parametrize("n", [1 << 24, 1 << 25, (1 << 26) - 24575, 1 << 26, (1 << 26) + 1])
