@@ -563,7 +563,7 @@ def main():
             run_row("permutedims(A, (3,2,1)) 2x8388608x2 Float32", n25, 8 * n25, run_permute3, reps)
             del sa, so
         # sort! (src/kernels/sorting.jl:1; perf/array.jl:143-149 sorts a Float32 vector): 8 B/key is the floor of
-        # any out-of-place permutation (one read, one write); the radix sort makes 4 digit passes plus 3 reads
+        # any out-of-place permutation (one read, one write); the keys are counted, moved into buckets once and sorted there
         if wanted("sort!"):
             m = 1 << 26
             ssrc = randn_f32(m)
@@ -573,7 +573,7 @@ def main():
             def run_sort():
                 RL.check(RL.lib.rk_sort(RL.RK_F32, skeys.ptr, m, 0, stmp.data_ptr(), stmp.numel(), stream_ptr()), "rk_sort")
             # sort! destroys its input: every launch is preceded by an untimed refill, so both figures are of
-            # individually timed calls (minimum and average); the call is six to fourteen kernels, not one
+            # individually timed calls (minimum and average); the call is twenty kernels, of which seven work, not one
             name = "sort!(Float32[2^26]); GB/s at 8 B/key"
             roctx.push(name)
             times = []
@@ -588,11 +588,12 @@ def main():
                 if i >= 3:
                     times.append(ev_a.elapsed_time(ev_b))
             roctx.pop()
-            # real traffic of the large sort: per digit pass a counting read (4 B/key) and the scatter pass (4 + 4 B/key)
+            # real traffic of this sort: the counting read (4 B/key), the scatter and the buckets (4 + 4 B/key each); by the counters 23, for the
+            # scatter's runs end inside lines (profiles/cases_kernels.txt)
             configs.append(entry(name, m, 8 * m, min(times), sum(times) / len(times), None,
                                  note="sort! destroys its input: refilled (untimed) before every call, so batch_avg_us is the average of individually timed calls too",
-                                 keys_per_s=m / (min(times) * 1e-3), real_traffic_bytes=48 * m,
-                                 GBps_real_traffic=round(48 * m / (min(times) * 1e-3) / 1e9, 1)))
+                                 keys_per_s=m / (min(times) * 1e-3), real_traffic_bytes=20 * m,
+                                 GBps_real_traffic=round(20 * m / (min(times) * 1e-3) / 1e9, 1)))
             del ssrc, skeys, stmp
         # cfg 4
         if wanted("cfg4"):
