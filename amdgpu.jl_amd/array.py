@@ -248,11 +248,10 @@ _UNSET_BYTES = np.full(SLOT_BYTES // 8, _UNSET, dtype=np.uint64).view(np.uint8)
 _WAIT_US = 200
 
 
-def scalar_words(dtype, more: int = 0) -> int:
+def scalar_words(dtype: np.dtype, more: int = 0) -> int:
     """``words`` of ``fill_slot`` for a result of ``dtype`` in word 0, and the words ``more``.  None for results that a kernel writes as 1
     or 2 bytes, every pattern of which is an ordinary value (of Bool two are): maximum of UInt8 that is 85 would wait 200 us in vain."""
-    dt = np.dtype(dtype)
-    return 1 | more if dt.itemsize >= 4 or dt == np.bool_ else 0
+    return 1 | more if dtype.itemsize >= 4 or dtype.kind == "b" else 0
 
 
 def fill_slot(slot, fn, name, args, words: int = 0) -> None:

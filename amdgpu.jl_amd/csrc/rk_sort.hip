@@ -594,11 +594,21 @@ __global__ __launch_bounds__(BLOCK, (sort_pass_waves<T, PERM, DIRECT>())) void s
     if (pass >= 0) step = sort_step(ctl, pass);
     if (pass < 0 || step.skip != 0u) {
         // all keys equal: no pass ran, and the last one writes the identity permutation, or the copy of the keys
-        if ((first_of_few || pass == (int)sizeof(T) - 1) && ctl->nexec == 0u && (PERM || (const void*)orig != (const void*)buf_a))
-            for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < (int64_t)n; i += (int64_t)gridDim.x * BLOCK) {
-                if (PERM) perm_out[i] = i + 1;
-                else ((T*)buf_a)[i] = orig[i];
+        if ((first_of_few || pass == (int)sizeof(T) - 1) && ctl->nexec == 0u && (PERM || (const void*)orig != (const void*)buf_a)) {
+            const int64_t step = (int64_t)gridDim.x * BLOCK;
+            for (int64_t i = (int64_t)blockIdx.x * BLOCK + tid; i < (int64_t)n; i += 4 * step) {
+                T k[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (!PERM && i + u * step < (int64_t)n) k[u] = orig[i + u * step];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (i + u * step >= (int64_t)n) continue;
+                    if (PERM) perm_out[i + u * step] = i + u * step + 1;
+                    else ((T*)buf_a)[i + u * step] = k[u];
+                }
             }
+        }
         return;
     }
     const bool first = (uint32_t)pass == step.first_pass, last = (uint32_t)pass == step.last_pass;

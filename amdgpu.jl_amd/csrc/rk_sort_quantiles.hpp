@@ -47,8 +47,9 @@ constexpr int64_t SQ_TILE = 6 * 4 * SQ_BLOCK;        // keys a tile: what LDS ho
 constexpr uint32_t SQ_CELLS = 4096;              // of the sampled range
 constexpr uint32_t SQ_MAX_K = 2560;              // buckets, a multiple of 64
 constexpr uint32_t SQ_GROUP = 16;                // neighbouring keys that are sampled together: a line of memory is fetched anyway
-// Samples a bucket: 512 take 3.5 + 2 us more of Float32[2^26] and make the buckets more alike, 186 for 190.
-constexpr uint32_t SQ_SAMPLES = 256;
+// Samples a bucket.  Half as many take 3.5 + 2 us less of Float32[2^26] and 1 + 0.5 of [2^24], and make the buckets less alike: of N(1000, 1), whose buckets are little more
+// than a cell, 485 -> 488 us a call of 2^26 keys and 177 -> 188 of 2^24.
+inline uint32_t sq_samples(int64_t n) { return n <= (int64_t)1 << 25 ? 512u : 256u; }
 constexpr uint32_t SQ_SAMPLES_EACH = 4;          // samples a thread fetches
 constexpr uint32_t SQ_TABLE_GRID = 64;
 constexpr uint32_t SQ_CHUNKS = 512;              // of tiles, at most
@@ -216,12 +217,13 @@ __device__ __forceinline__ void sq_add(uint32_t* cnt, uint32_t c) {
 // are: of 2^26 keys of N(1000, 1) 0.1 % zeros, or of N(1013, 10) 0.1 % NaN, are sorted by buckets then.
 template <bool REFINE>
 __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __restrict__ sample, uint32_t samples, const uint2* __restrict__ ends,
-                                                            uint32_t nends, uint32_t offset, uint32_t k, uint32_t too_many, int floats, uint32_t* hist, uint32_t* __restrict__ cells, SqCtl* sq) {
+                                                            uint32_t nends, uint32_t offset, uint32_t k, uint32_t each, uint32_t too_many, int floats, uint32_t* hist, uint32_t* __restrict__ cells, SqCtl* sq) {
     constexpr uint32_t PER = SQ_CELLS / SQ_BLOCK;
     __shared__ uint32_t h[SQ_CELLS], cnt[SQ_MAX_K];
     __shared__ uint32_t part[4][SQ_BLOCK / WAVE], lds_ticket;
-    constexpr uint32_t SQ_PICKS = 8;
-    __shared__ uint32_t found, end_cell[2], heavy_cell[SQ_FREQUENT], picked[SQ_FREQUENT], best[SQ_FREQUENT], pick[SQ_FREQUENT][SQ_PICKS];
+    constexpr uint32_t SQ_PICKS = 128;
+    __shared__ uint32_t found, end_cell[2], heavy_cell[SQ_FREQUENT], picked[SQ_FREQUENT], pick[SQ_FREQUENT][SQ_PICKS];
+    __shared__ uint32_t frequent, value[SQ_FREQUENT], value_cell[SQ_FREQUENT], value_same[SQ_FREQUENT];
     const uint32_t tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     if (sq->way == SQ_PLANNED || (REFINE && sq->heavies == 0u)) return;
     uint32_t lo = ~0u, hi = 0u, up = 0u;
@@ -332,29 +334,29 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __re
 #pragma unroll
             for (uint32_t j = 0; j < PER; ++j) {
                 const uint32_t behind = all - before - c[j];
-                if (before <= SQ_SAMPLES / 2u && before + c[j] > SQ_SAMPLES / 2u) end_cell[0] = tid * PER + j;
-                if (behind <= SQ_SAMPLES / 2u && behind + c[j] > SQ_SAMPLES / 2u) end_cell[1] = tid * PER + j;
+                if (before <= each / 2u && before + c[j] > each / 2u) end_cell[0] = tid * PER + j;
+                if (behind <= each / 2u && behind + c[j] > each / 2u) end_cell[1] = tid * PER + j;
                 before += c[j];
             }
         };
         // whether these leave an eighth of the range or less
         const auto few_cells = [&]() { return up < 20u && end_cell[0] <= end_cell[1] && end_cell[1] - end_cell[0] < SQ_CELLS / 8u; };
-        if (tid < SQ_FREQUENT) { picked[tid] = 0u; best[tid] = 0u; }
-        if (tid == 0u) { found = 0u; end_cell[0] = 0u; end_cell[1] = SQ_CELLS - 1u; }
+        if (tid < SQ_FREQUENT) picked[tid] = 0u;
+        if (tid == 0u) { found = 0u; frequent = 0u; end_cell[0] = 0u; end_cell[1] = SQ_CELLS - 1u; }
         __syncthreads();
         find_ends(before, all);
         // a cell far above its neighbours may hold such a value
 #pragma unroll
         for (uint32_t j = 0; j < PER; ++j) {
             const uint32_t at = tid * PER + j, beside = (at != 0u ? h[at - 1u] : 0u) + (at + 1u < SQ_CELLS ? h[at + 1u] : 0u);
-            if (c[j] >= beside + beside / 8u + SQ_SAMPLES / 2u) {
+            if (c[j] >= beside + beside / 8u + each / 2u) {
                 const uint32_t s = atomicAdd(&found, 1u);
                 if (s < SQ_FREQUENT) heavy_cell[s] = at;
             }
         }
         __syncthreads();
         const uint32_t heavy_cells = found <= SQ_FREQUENT ? found : 0u;
-        if (heavy_cells != 0u || few_cells()) {
+        if (range != 0u && (heavy_cells != 0u || few_cells())) {
             const auto add_heavy = [&](uint32_t v) {
                 if (is_heavy(v)) return;
 #pragma unroll
@@ -362,7 +364,7 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __re
                 ++map.heavies;
             };
             if (heavy_cells != 0u) {
-                // it is what a third of up to eight of the cell's samples are, and more than one
+                // up to 128 of the cell's samples: values that half a bucket's share of the samples, by these, are
                 constexpr uint32_t FROM = 4u * SQ_CHECKED, EACH = FROM / 4u / SQ_BLOCK;
 #pragma unroll 4
                 for (uint32_t u = 0; u < EACH; ++u) {
@@ -380,28 +382,37 @@ __global__ __launch_bounds__(SQ_BLOCK) void sq_table_kernel(const uint32_t* __re
                 if (tid < heavy_cells && picked[tid] > SQ_PICKS) picked[tid] = SQ_PICKS;
                 __syncthreads();
                 const uint32_t s = tid / SQ_PICKS, p = tid % SQ_PICKS;
+                static_assert(SQ_FREQUENT * SQ_PICKS <= SQ_BLOCK, "a thread a pick");
                 if (s < heavy_cells && p < picked[s]) {
-                    uint32_t same = 0u;
-                    for (uint32_t q = 0; q < SQ_PICKS; ++q) same += q < picked[s] && pick[s][q] == pick[s][p] ? 1u : 0u;
-                    atomicMax(&best[s], same << 8 | p);
+                    uint32_t same = 0u, in_front = 0u;
+                    for (uint32_t q = 0; q < picked[s]; ++q) {
+                        const bool is = pick[s][q] == pick[s][p];
+                        same += is ? 1u : 0u;
+                        in_front += is && q < p ? 1u : 0u;
+                    }
+                    if (in_front == 0u && same >= (picked[s] < 16u ? 2u : 3u) && (uint64_t)h[heavy_cell[s]] * same >= (uint64_t)(each / 2u) * picked[s]) {
+                        const uint32_t f = atomicAdd(&frequent, 1u);
+                        if (f < SQ_FREQUENT) { value[f] = pick[s][p]; value_cell[f] = s; value_same[f] = same; }
+                    }
                 }
-                __syncthreads();
-                if (tid < heavy_cells && (best[tid] >> 8 < 2u || (best[tid] >> 8) * 3u < picked[tid])) best[tid] = 0u;
                 if (tid == 0u) { end_cell[0] = 0u; end_cell[1] = SQ_CELLS - 1u; }
                 __syncthreads();
-                for (uint32_t t = 0; t < heavy_cells; ++t) {
-                    if (best[t] == 0u) continue;
-                    add_heavy(pick[t][best[t] & 0xffu]);
+                if (frequent <= SQ_FREQUENT) {
+                    for (uint32_t f = 0; f < frequent; ++f) {
+                        add_heavy(value[f]);
+                        const uint32_t t = value_cell[f];
 #pragma unroll
-                    for (uint32_t j = 0; j < PER; ++j)           // what remains
-                        if (heavy_cell[t] == tid * PER + j) c[j] = (uint32_t)((uint64_t)c[j] * (picked[t] - (best[t] >> 8)) / picked[t]);
+                        for (uint32_t j = 0; j < PER; ++j)       // what remains
+                            if (heavy_cell[t] == tid * PER + j) c[j] -= (uint32_t)((uint64_t)h[tid * PER + j] * value_same[f] / picked[t]);
+                    }
+                    uint32_t all_of = all;
+                    const uint32_t before_of = scan(c, all_of);
+                    find_ends(before_of, all_of);
+                    __syncthreads();
                 }
-                uint32_t all_of = all;
-                const uint32_t before_of = scan(c, all_of);
-                find_ends(before_of, all_of);
-                __syncthreads();
             }
-            if (few_cells()) {
+            // (of more such values at one place the buckets would not fit)
+            if (frequent <= SQ_FREQUENT && few_cells()) {
                 const uint32_t new_lo = lo + (end_cell[0] << (20u - up));
                 const uint64_t end = (uint64_t)lo + ((uint64_t)(end_cell[1] + 1u) << (20u - up)) - 1u;
                 const uint32_t new_hi = end < (uint64_t)hi ? (uint32_t)end : hi;
@@ -1336,7 +1347,7 @@ static SqLayout sq_layout(size_t off, int64_t n) {
     l.nchunks = (l.ntiles + l.chunk_tiles - 1u) / l.chunk_tiles;
     const float fit = (float)SQ_CAP * (float)SQ_CHECKED / (float)n;            // of the samples that are looked at, those of a bucket that just fits
     l.too_many = (uint32_t)(fit + 4.f * std::sqrt(fit));
-    l.sample_grid = l.k / (SQ_BLOCK * SQ_SAMPLES_EACH / SQ_SAMPLES);
+    l.sample_grid = l.k / (SQ_BLOCK * SQ_SAMPLES_EACH / sq_samples(n));
     const uint32_t k = l.k;
     const auto take = [&](size_t bytes) { const size_t at = off; off += (bytes + 255) & ~(size_t)255; return at; };
     l.sq_off = take(sizeof(SqCtl));
@@ -1374,9 +1385,9 @@ static int32_t sort_quantiles(const SqLayout& l, const void* keys, void* sorted_
     // from a key to the number whose multiples of 2^23 are binades
     const uint32_t offset = std::is_integral<T>::value ? 0u : flip != 0u ? 1u - 0x007fffffu : 0x007fffffu;
     const uint32_t samples = l.sample_grid * SQ_BLOCK * SQ_SAMPLES_EACH;
-    sq_table_kernel<false><<<SQ_TABLE_GRID, SQ_BLOCK, 0, stream>>>(moved, samples, ends, l.sample_grid, offset, k, l.too_many, floats, hist, cells, sq);
+    sq_table_kernel<false><<<SQ_TABLE_GRID, SQ_BLOCK, 0, stream>>>(moved, samples, ends, l.sample_grid, offset, k, sq_samples(n), l.too_many, floats, hist, cells, sq);
     RK_LAUNCH_CHECK();
-    sq_table_kernel<true><<<SQ_TABLE_GRID, SQ_BLOCK, 0, stream>>>(moved, samples, ends, l.sample_grid, offset, k, l.too_many, floats, hist, cells, sq);
+    sq_table_kernel<true><<<SQ_TABLE_GRID, SQ_BLOCK, 0, stream>>>(moved, samples, ends, l.sample_grid, offset, k, sq_samples(n), l.too_many, floats, hist, cells, sq);
     RK_LAUNCH_CHECK();
     sq_count_kernel<T><<<l.nchunks, SQ_BLOCK, 0, stream>>>((const T*)keys, (uint32_t)n, flip, k, cells, l.ntiles, l.chunk_tiles, (uint32_t*)rows, totals, seen, sq);
     RK_LAUNCH_CHECK();

@@ -547,11 +547,11 @@ def test_sorts_by_quantiles_with_a_sample_that_misleads(rk, dtype):
     import pathlib
     text = (pathlib.Path(__file__).parent.parent / "amdgpu.jl_amd" / "csrc" / "rk_sort_quantiles.hpp").read_text()
     for line in ("constexpr uint32_t SQ_GROUP = 16;", "uint32_t h = (g + 1u) * 0x9e3779b1u;", "h ^= h >> 15;", "h *= 0x85ebca77u;",
-                 "keys[a + __umulhi(h, b - a - (SQ_GROUP - 1u)) + s % SQ_GROUP]", "constexpr uint32_t SQ_SAMPLES = 256;", "constexpr uint32_t SQ_SAMPLES_EACH = 4;", "constexpr int64_t SQ_MEAN = 26624;"):
+                 "keys[a + __umulhi(h, b - a - (SQ_GROUP - 1u)) + s % SQ_GROUP]", "return n <= (int64_t)1 << 25 ? 512u : 256u;", "constexpr uint32_t SQ_SAMPLES_EACH = 4;", "constexpr int64_t SQ_MEAN = 26624;"):
         assert line in text, line
     rng = np.random.default_rng(44)
     n = QUANTILES[dtype] + 54321
-    groups = -(-n // (256 * 26624)) * 256 * 256 // 16
+    groups = -(-n // (256 * 26624)) * 256 * 512 // 16
     g, m = np.arange(groups, dtype=np.uint64), np.uint64(0xffffffff)
     a, b = g * np.uint64(n) // np.uint64(groups), (g + np.uint64(1)) * np.uint64(n) // np.uint64(groups)
     h = (g + np.uint64(1)) * np.uint64(0x9e3779b1) & m
