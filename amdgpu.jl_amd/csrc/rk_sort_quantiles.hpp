@@ -17,23 +17,23 @@
 // Radix passes -> so, us a call: sort Float32[2^23] 172 -> 128, [2^24] 248 -> 171, [2^26] 758 -> 449; Int32 of 32 bits [2^24] 265 -> 196,
 // [2^26] 811 -> 489, of 20 bits [2^24] 234 -> 188, [2^26] 740 -> 460.  The kernels of Float32[2^26]: 8 sample, 18 table, 50 count, 8 offsets, 155
 // scatter, 190 buckets; 512 MiB read and written are 81.  By counters (profiles/sort_quantiles_sq_counters.txt) the count is bound by its vector
-// instructions, 20 a key.  The scatter and the buckets are neither: vector units busy 43 and 59 %, LDS 35 and 40 % of the time (half of that bank
+// instructions, 20 a key.  The scatter and the buckets are neither: vector units busy 43 and 60 %, LDS 35 and 41 % of the time (half of that bank
 // conflicts), and over two fifths of a wave's time is waiting, in phases that one workgroup a compute unit does not overlap; the scatter also writes 367 MiB
-// for 256, runs of ten keys on the average (with tiles of 12288 keys and twice as many workgroups 181, 87 if nothing is written).  The fewer bytes a
+// for 256 (370 in Int32), runs of ten keys on the average (with tiles of 12288 keys and twice as many workgroups 181, 87 if nothing is written).  The fewer bytes a
 // key, the shorter the runs' lines: keys of 8 bytes, and sortperm, whose index would travel along, take two levels of splitters (rk_sort_split.hpp).
 // Below 2^22 keys the launches count: Float32[2^22] 91 in rk_sort_split.hpp, 95 so.  Int32[2^22] of 8 bits, one radix pass and eight launches
 // for nothing more, 69 -> 76, [2^23] 94 -> 96, [2^24] 132 -> 124; of 32 bits [2^22] 147 -> 108, which the others would pay for.
 //
 // Float32 around a number or with one in large numbers, radix passes / cells over the whole sampled range / so, us a call of 2^24 and of 2^26 keys: N(1000, 1) with
-// 0.1 % zeros 239 / 277 / 237 and 727 / 864 / 602; N(1013, 10) with 0.1 % NaN 241 / 282 / 225 and 734 / 878 / 542; N(20, 5) with 0.1 % -9999 239 / 209 / 225 and
-// 742 / 948 / 528; half zeros 248 / 289 / 212 and 743 / 885 / 505; nine in ten zeros 245 / 285 / 185 and 723 / 849 / 437.  Int32 ids with 0.01 % typemax
-// 265 / 741 / 217 and 777 / 1025 / 522.
+// 0.1 % zeros 239 / 277 / 243 and 727 / 864 / 604; N(1013, 10) with 0.1 % NaN 241 / 282 / 232 and 734 / 878 / 543; N(20, 5) with 0.1 % -9999 239 / 209 / 234 and
+// 742 / 948 / 527; half zeros 248 / 289 / 219 and 743 / 885 / 506; nine in ten zeros 245 / 285 / 194 and 723 / 849 / 437.  Int32 ids with 0.01 % typemax
+// 265 / 741 / 220 and 777 / 1025 / 522.  (Of 2^23 keys 0.95 to 1.2 times as fast as radix passes.)
 //
 // If a bucket exceeds what its workgroup holds (SQ_CAP) all the same, that is known before a key is moved, mostly from the sample, and the radix passes run
 // instead: their plan is there, or the plan says that none runs, and the kernels of the other way end at once.  So they do where the sample says that a bucket has
 // few values.  That costs them sample, table and launches, and above 2^24 keys passes whose workgroups take several tiles: Float32 of N(0, 1) rounded to 0.001
-// [2^24] 258 -> 294, [2^26] 776 -> 897; of 256 levels 242 -> 279, 719 -> 836; Int32 of a power law [2^24] 238 -> 284, of 16 bits [2^23] 120 -> 145,
-// [2^24] 164 -> 183, [2^26] 463 -> 497.
+// [2^24] 258 -> 294, [2^26] 776 -> 897; of 256 levels 242 -> 278, 719 -> 837; Int32 of a power law [2^23] 170 -> 211, [2^24] 238 -> 278, of 16 bits [2^23] 120 -> 138,
+// [2^24] 164 -> 181, [2^26] 463 -> 494.
 #pragma once
 
 #include <cmath>
